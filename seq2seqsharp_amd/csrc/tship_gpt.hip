@@ -168,6 +168,7 @@ struct TestHooks {
     int ffn_tiles = 0;        // TSHIP_FFN_TILES: 10, 15, 20, 30 or 40 = column tiles x 10 per block of the decode FFN up projection
     int patch_rows = 0;       // TSHIP_PATCH_ROWS: 1, 2, 4 or 8 row tiles per tile patch of the prefill GEMM
     long attn_splits = 0;     // TSHIP_ATTN_SPLITS: blocks per (sequence, KV head) pair in decode attention
+    int gemm_tile = -1;        // TSHIP_GEMM_TILE: tile of the prefill GEMMs (pick_gemm_tile); 0: the 256 x 256 tile from 256 rows on
     int attn_nq = 0;          // TSHIP_ATTN_NQ: 1 or 2 groups of 16 MFMA columns per wavefront in prefill attention
     bool no_kv_fuse = false;  // TSHIP_NO_KV_FUSE: the QKV projection of a prefill does not write the cache itself
     bool no_moe_batch = false;// TSHIP_NO_MOE_BATCH: one prefill GEMM launch per expert
@@ -186,6 +187,10 @@ static void refresh_test_hooks() {
     }
     if (const char* v = std::getenv("TSHIP_ATTN_SPLITS")) { h.attn_splits = std::atol(v); TSHIP_REQUIRE(h.attn_splits >= 1, "TSHIP_ATTN_SPLITS: a positive number"); }
     if (const char* v = std::getenv("TSHIP_ATTN_NQ")) { h.attn_nq = std::atoi(v); TSHIP_REQUIRE(h.attn_nq == 1 || h.attn_nq == 2, "TSHIP_ATTN_NQ: 1 or 2"); }
+    if (const char* v = std::getenv("TSHIP_GEMM_TILE")) {
+        h.gemm_tile = std::atoi(v);
+        TSHIP_REQUIRE(h.gemm_tile == 0 || h.gemm_tile == 11 || h.gemm_tile == 12 || h.gemm_tile == 14 || h.gemm_tile == 22 || h.gemm_tile == 24, "TSHIP_GEMM_TILE: 0, 11, 12, 14, 22 or 24");
+    }
     h.no_kv_fuse = std::getenv("TSHIP_NO_KV_FUSE") != nullptr;
     h.no_moe_batch = std::getenv("TSHIP_NO_MOE_BATCH") != nullptr;
     h.no_graph = std::getenv("TSHIP_NO_GRAPH") != nullptr;
@@ -513,16 +518,58 @@ static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const fl
     launch(m, name, gemm_f32_kernel, grid, dim3(256), g);
 }
 
-// Y = X * W for many rows (prefill), fp16: LDS-tiled MFMA kernels from 512 rows on, 128 x 128 tiles below.  X row-major
-// with at least round_up(R, 128) rows allocated (the small-tile kernel reads whole row tiles; rows from R on are never stored).
+// Tile of a prefill GEMM: 10 x (64-row groups) + 32-column tiles of mid_gemm_f16_kernel, or 0 for the 256 x 256 tile.
+// A launch takes rounds of tiles over the compute units x (a + b per k-tile) x a factor for the load of the shared parts
+// (L2, HBM, power).  a and b are fits to launches of 37 ... 16384 rows at seven (K, N) of 768 ... 22016: the choice costs
+// 0.3 % over the best tile on average of those 105 launches, and more than 8 % in one (21 us for 17).
+// own_cache_write: us that a launch saves with the 256 x 256 tile, which can write the key-value cache itself.
+static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) {
+    struct Cost { int tile, rows, cols; float a, b; };
+    static const Cost costs[] = {{11, 64, 1, 1.9f, 0.045f}, {12, 64, 2, 2.8f, 0.050f}, {14, 64, 4, 3.0f, 0.093f},
+                                 {22, 128, 2, 3.4f, 0.078f}, {24, 128, 4, 4.8f, 0.115f}, {0, 256, 8, 8.0f, 0.320f}};
+    const int forced = g_hooks.gemm_tile;
+    if (forced > 0 || (forced == 0 && R >= 256)) return forced;
+    const float ncu = (float)std::max(1, n_compute_units());
+    int best = 11; float best_us = 1e30f;
+    for (const Cost& c : costs) {
+        if (c.tile == 0 && R < 256) continue;
+        const float tiles = (float)(ceil_div(R, c.rows) * ceil_div(w.NT, c.cols)), rounds = std::ceil(tiles / ncu);
+        float us = rounds * (c.a + c.b * (float)w.KT) * (1.0f + 0.4f * tiles / (rounds * ncu));
+        if (c.tile == 0) us -= own_cache_write;
+        if (us < best_us) { best_us = us; best = c.tile; }
+    }
+    return best;
+}
+static void run_mid_gemm(TSHipGpt* m, const char* name, const BigArgs& e, int epi, int mid) {
+    auto go = [&](auto WRc, auto NJc) {
+        constexpr int WR = decltype(WRc)::value, NJ = decltype(NJc)::value;
+        const long tiles = ceil_div(e.NT, NJ) * ceil_div(e.R, 64 * WR);
+        const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8));
+        const unsigned shm = MidShape<WR, NJ>::SHM;
+        if (epi == BEPI_F32_BIAS) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_F32_BIAS, WR, NJ>, grid, dim3(512), shm, e);
+        else if (epi == BEPI_RESID) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_RESID, WR, NJ>, grid, dim3(512), shm, e);
+        else launch_shm(m, name, mid_gemm_f16_kernel<BEPI_ACT16, WR, NJ>, grid, dim3(512), shm, e);
+    };
+    typedef std::integral_constant<int, 1> c1; typedef std::integral_constant<int, 2> c2; typedef std::integral_constant<int, 4> c4;
+    switch (mid) {
+        case 11: go(c1{}, c1{}); break;
+        case 12: go(c1{}, c2{}); break;
+        case 14: go(c1{}, c4{}); break;
+        case 22: go(c2{}, c2{}); break;
+        case 24: go(c2{}, c4{}); break;
+        default: throw Error("internal: no such prefill GEMM tile");
+    }
+}
+
+// Y = X * W for many rows (prefill), fp16, X row-major.
 // n_problems > 1 (LDS-tiled asynchronous kernel only, see big_gemm_batched_ok): e.Wtab / rows_tab / strides describe that many
 // problems of the same shape and at most R rows each, run by one launch.
 static bool big_gemm_batched_ok(const GemmW& w, long R) { return R >= 512 && w.KT % 2 == 0; }
-static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, int n_problems = 1) {
-    const long Rp = round_up(R, 128);
+static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, int n_problems = 1, int tile = -1) {
     e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.R = (int)R;
+    const int mid = n_problems > 1 ? 0 : tile >= 0 ? tile : pick_gemm_tile(w, R);
     TSHIP_REQUIRE(n_problems == 1 || big_gemm_batched_ok(w, R), "internal: batched launch of a GEMM shape the LDS-tiled kernel does not take");
-    if (R >= 512) {       // LDS-tiled kernel, 256 x 256 block tile
+    if (!mid) {           // 256 x 256 block tile
         constexpr int CK = 4;
         const unsigned shm = 2u * 2u * 8u * CK * 1024u;
         // one-dimensional grid of 8-row x 4-column tile patches, 32 blocks each, rounded up to whole rounds of 8 patches
@@ -550,10 +597,7 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
         else launch_shm(m, name, big_gemm2_f16_kernel<BEPI_ACT16, CK>, grid, dim3(256), shm, e);
         return;
     }
-    dim3 grid((unsigned)ceil_div(w.NT, 4), (unsigned)(Rp / 128));
-    if (epi == BEPI_F32_BIAS) launch(m, name, big_gemm_f16_kernel<BEPI_F32_BIAS>, grid, dim3(256), e);
-    else if (epi == BEPI_RESID) launch(m, name, big_gemm_f16_kernel<BEPI_RESID>, grid, dim3(256), e);
-    else launch(m, name, big_gemm_f16_kernel<BEPI_ACT16>, grid, dim3(256), e);
+    run_mid_gemm(m, name, e, epi, mid);
 }
 
 typedef void (*AttnKernel)(AttnArgs);
@@ -1016,7 +1060,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     // Deferred RMSNorm (fp16 RMSNorm models, LDS-tiled GEMMs): no norm kernels.  The producer of the residual stream
     // stores half(gamma * x) and per-(32-column tile, row) sums of squares, a one-thread-per-row kernel turns those into
     // 1 / rms, and the consuming GEMMs scale their output rows by it.
-    const bool deferred = m->fused_norm && !m->ln && R >= 512;
+    const bool deferred = m->fused_norm && !m->ln;
     const int NTh = (int)(round_up(h, 32) / 32);
     DevBuf &pssq = m->pw_ssq, &prinv = m->pw_rinv;
     auto make_rinv = [&](const char* name) {
@@ -1045,7 +1089,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     auto producer = [&](BigArgs& e, const float* gamma) {        // residual GEMM that also emits the next GEMM's input
         e.xg16 = pxn.as<half_t>(); e.ld_xg = (int)m->ldh; e.gamma = gamma; e.ssq_out = pssq.as<float>(); e.ssq_ld = R;
     };
-    auto big = [&](const char* name, const GemmW& w, const void* X, long ldx, int epi, BigArgs e) { run_big_gemm(m, name, w, X, ldx, R, epi, e); };
+    auto big = [&](const char* name, const GemmW& w, const void* X, long ldx, int epi, BigArgs e, int tile = -1) { run_big_gemm(m, name, w, X, ldx, R, epi, e, 1, tile); };
     DevBuf& zero_bias = m->pw_zero_bias; zero_bias.reserve((size_t)std::max<long>(std::max<long>(qp, m->F13), round_up(h, 32)) * sizeof(float));
     for (int l = 0; l < c.n_layers; ++l) {
         LayerW& L = *m->L[l];
@@ -1056,7 +1100,9 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         // The LDS-tiled QKV projection writes keys and values into the fragment-major cache itself (rotation included)
         // when its wavefronts' 64 x 128 tiles are whole chunks of whole heads; otherwise a kernel of its own does.
         const int HD = c.n_heads * m->D, GD = c.n_kv_heads * m->D;
-        const bool fuse_kv = m->f16 && m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && R >= 512 && L.qkv.KT % 2 == 0 &&
+        // (the separate kernel: 9 us at 1.6 k rows, 80 us at 32 k)
+        const int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, 5.0f + 0.0023f * (float)R) : 0;
+        const bool fuse_kv = m->f16 && m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && !qkv_tile && L.qkv.KT % 2 == 0 &&
                              (m->D == 64 || m->D == 128) && !g_hooks.no_kv_fuse;
         if (m->f16) {
             BigArgs e; std::memset(&e, 0, sizeof(e));
@@ -1067,7 +1113,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
                 e.kcache = (half_t*)L.kc.p; e.vcache = (half_t*)L.vc.p; e.kv_max_len = m->ML; e.kv_col0 = HD; e.kv_gd = GD; e.kv_D = m->D;
                 e.kv_hkv = c.n_kv_heads; e.kv_Tq = Tp; e.kv_pos0 = pos0; e.rope_cos = aa.rope_cos; e.rope_sin = aa.rope_sin;
             }
-            big("p_gemm_qkv", L.qkv, pxn.p, m->ldh, BEPI_F32_BIAS, e);
+            big("p_gemm_qkv", L.qkv, pxn.p, m->ldh, BEPI_F32_BIAS, e, qkv_tile);
             aa.bias = zero_bias.as<float>();      // bias already added by the GEMM epilogue
         } else {
             run_gemm_f32(m, "p_gemm_qkv", L.qkv, pxn.as<float>(), m->ldh, (int)R, pqkv.as<float>(), qp, 0, 1);

@@ -131,14 +131,15 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
             e2.Wtab = (const half_t* const*)L.wtab2.p; e2.rows_tab = counts; e2.x_estride = mid_stride; e2.out_estride = y_stride;
             run_big_gemm(m, "moe_gemm2", *L.e2[0], mid, o.ld4h, n_max, BEPI_F32_BIAS, e2, E);
         } else {
+            const int tile = g_hooks.no_moe_batch ? 0 : -1;      // (the hook compares with the batched launches: same tile, same bits)
             for (int e = 0; e < E; ++e) {
                 if (n_e[e] == 0) continue;
                 BigArgs e1; std::memset(&e1, 0, sizeof(e1));
                 e1.bias = zero; e1.out16 = mid + e * mid_stride; e1.ld16 = (int)o.ld4h; e1.act = c.act; e1.gated = 0; e1.n_valid = 4 * h;
-                run_big_gemm(m, "moe_gemm1", *L.e1[e], xg + e * xg_stride, m->ldh, n_e[e], BEPI_ACT16, e1);
+                run_big_gemm(m, "moe_gemm1", *L.e1[e], xg + e * xg_stride, m->ldh, n_e[e], BEPI_ACT16, e1, 1, tile);
                 BigArgs e2; std::memset(&e2, 0, sizeof(e2));
                 e2.bias = zero; e2.out = y + e * y_stride; e2.ld_out = (int)o.ldy; e2.n_valid = h;
-                run_big_gemm(m, "moe_gemm2", *L.e2[e], mid + e * mid_stride, o.ld4h, n_e[e], BEPI_F32_BIAS, e2);
+                run_big_gemm(m, "moe_gemm2", *L.e2[e], mid + e * mid_stride, o.ld4h, n_e[e], BEPI_F32_BIAS, e2, 1, tile);
             }
         }
     } else if (m->f16) {

@@ -753,8 +753,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_f16_kernel(const half_t* 
 }
 
 // ------------------------------------------------------------------------------------------------
-// prefill GEMM, fp16 weights: many rows.  Block tile 128 rows x 128 columns; each wavefront owns one
-// 32-column weight tile (streamed from HBM/L2 as packed fragments) and 4 row tiles.  MFMA-bound.
+// prefill GEMMs, fp16 weights, row-major activations.  MFMA-bound from some hundred rows on.
 // ------------------------------------------------------------------------------------------------
 enum { BEPI_F32_BIAS = 0, BEPI_RESID = 1, BEPI_ACT16 = 2 };
 
@@ -794,54 +793,6 @@ struct BigArgs {
     // than eight patches and leave XCDs idle); 0 means 8
     int patch_rows;
 };
-
-template <int EPI>
-__global__ __launch_bounds__(256) void big_gemm_f16_kernel(BigArgs a) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int nt = blockIdx.x * 4 + w;
-    if (nt >= a.NT) return;
-    const int row0 = blockIdx.y * 128;
-    floatx16 acc[4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[rt][v] = 0.0f;
-    const half_t* wp = a.W + ((long)nt * a.KT * 64 + lane) * 8;
-    const half_t* xp = a.X + (long)(row0 + (lane & 31)) * a.ldx + (lane >> 5) * 8;
-#pragma unroll 2
-    for (int kt = 0; kt < a.KT; ++kt) {
-        half8 wf = *(const half8*)(wp + (long)kt * 512);
-        half8 xf[4];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) xf[rt] = *(const half8*)(xp + (long)rt * 32 * a.ldx + kt * 16);
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf, xf[rt], acc[rt], 0, 0, 0);
-    }
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int row = row0 + rt * 32 + (lane & 31);
-        if (row >= a.R) continue;
-        if (EPI == BEPI_ACT16 && a.gated) {
-#pragma unroll
-            for (int v = 0; v < 8; ++v) {
-                int nl = 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
-                int f = nt * 16 + nl;
-                if (f < a.n_valid)
-                    a.out16[(long)row * a.ld16 + f] = (half_t)(act_apply(a.act, acc[rt][v] + a.bias[f]) * (acc[rt][v + 8] + a.bias2[f]));
-            }
-        } else {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                int col = nt * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
-                if (col >= a.n_valid) continue;
-                float s = acc[rt][v] + a.bias[col];
-                if (EPI == BEPI_F32_BIAS) a.out[(long)row * a.ld_out + col] = s;
-                else if (EPI == BEPI_RESID) a.out[(long)row * a.ld_out + col] = s + a.out[(long)row * a.ld_out + col];
-                else a.out16[(long)row * a.ld16 + col] = (half_t)act_apply(a.act, s);
-            }
-        }
-    }
-}
 
 // Epilogue shared by the LDS-tiled prefill GEMMs.
 // Gated activation output of one wavefront (64 rows x 4 column tiles = 64 consecutive fp16 outputs per row) through LDS, so
@@ -1538,6 +1489,275 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     // wavefront owns 64 x 72 halfs of them for its epilogue, once every wavefront has passed this barrier)
     __builtin_amdgcn_s_barrier();
     big_gemm_store<EPI, 2>(a, acc, nt0, row0, wr, wn, lane, big_smem + w * (64 * 72));
+}
+
+// Prefill GEMM for launches that 256 x 256 tiles would leave most of the chip idle in (up to a few thousand rows).  Block tile
+// 64 WR rows x 32 NJ columns, eight wavefronts: a wavefront owns 64 rows x all the columns (NJ x 2 MFMA tiles of 32 x 32), and
+// the KG = 8 / WR wavefronts of a row group take the k-tiles in turn, so that a small tile still has two wavefronts per SIMD
+// and the fragment reads of a large one (NJ + 2 per 2 NJ MFMAs).  Staging, waits and the half-period offset between the two
+// wavefronts of a SIMD are those of big_gemm3_f16_kernel; a stage is KG k-tiles (a row's 128 or 256 contiguous bytes of
+// activations: whole lines).  The KG partial accumulators cross through the dead stages at the end, so outputs leave in line
+// layout.  Any number of k-tiles (those beyond the last are fetched again and not multiplied); rows and columns beyond the
+// matrix are clamped on load and dropped on store.
+// Bound by what a compute unit has in flight: about 64 KiB of requests, 70 KB per us into LDS, so a launch goes with the
+// bytes a tile requests and the rounds of tiles (the rule is pick_gemm_tile).  Measured, weights from HBM, us before (the
+// 256 x 256 tile from 512 rows on; below, 128 x 128 tiles whose fragments came straight from L2 without staging) -> now:
+//   37 rows    2048 x 3072  97 -> 8     2048 x 2048  97 -> 7    2048 x 11264   98 -> 15    5632 x 2048  253 -> 18
+//   1665 rows  2048 x 3072  45 -> 39    2048 x 2048  57 -> 27   2048 x 11264  109 (256 x 256)   5632 x 2048  124 -> 53
+// Two resident blocks per unit (three stages, half the reduction area) measured 8-25 % slower at one round of tiles and
+// gained only from three rounds on, where a larger tile is faster still.
+template <int NJ, int KG>
+__device__ __forceinline__ void mid_read_frags(unsigned wa, unsigned xa, half8 (&wf)[NJ], half8 (&xf)[2]) {
+    constexpr int XO = 32 * KG * 32;      // bytes of 32 rows of a stage
+    if constexpr (NJ == 4)
+        asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:%8\n\tds_read_b128 %2, %6 offset:%9\n\tds_read_b128 %3, %6 offset:%10\n\t"
+                     "ds_read_b128 %4, %7\n\tds_read_b128 %5, %7 offset:%11"
+                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(wf[2]), "=&v"(wf[3]), "=&v"(xf[0]), "=&v"(xf[1])
+                     : "v"(wa), "v"(xa), "n"(KG * 1024), "n"(2 * KG * 1024), "n"(3 * KG * 1024), "n"(XO) : "memory");
+    else if constexpr (NJ == 2)
+        asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:%6\n\tds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:%7"
+                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa), "n"(KG * 1024), "n"(XO) : "memory");
+    else
+        asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %4\n\tds_read_b128 %2, %4 offset:%5"
+                     : "=&v"(wf[0]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa), "n"(XO) : "memory");
+}
+template <int NJ>
+__device__ __forceinline__ void mid_wait_frags(half8 (&wf)[NJ], half8 (&xf)[2]) {
+    if constexpr (NJ == 4) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wf[0]), "+v"(wf[1]), "+v"(wf[2]), "+v"(wf[3]), "+v"(xf[0]), "+v"(xf[1])::"memory");
+    else if constexpr (NJ == 2) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wf[0]), "+v"(wf[1]), "+v"(xf[0]), "+v"(xf[1])::"memory");
+    else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wf[0]), "+v"(xf[0]), "+v"(xf[1])::"memory");
+}
+// stages and LDS bytes of a launch
+template <int WR, int NJ> struct MidShape {
+    static constexpr int KG = 8 / WR, STAGE = KG * (NJ + 2 * WR) * 1024, NST = STAGE > 40960 ? 3 : 4;
+    static constexpr int UP = NJ == 1 ? 2 : 4, RED = 8 * UP * 32 * 36 * 4;
+    static constexpr unsigned SHM = NST * STAGE > RED ? NST * STAGE : RED;
+};
+
+template <int EPI, int WR, int NJ>
+__global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
+    extern __shared__ __attribute__((aligned(16))) half_t big_smem[];
+    using S = MidShape<WR, NJ>;
+    constexpr int KG = S::KG, NST = S::NST, PF = NST - 1, STAGE = S::STAGE, LW = NJ * KG / 8, PPR = 2 * KG, LPC = LW + 2;      // LPC: loads per wavefront and chunk
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wr = WR == 2 ? w >> 2 : 0, kg = WR == 2 ? w & 3 : w;
+    // Block -> tile: every XCD takes one contiguous eighth of the tiles in an order with the row tiles fastest, so that the
+    // blocks it runs at a time share their weight tiles (read from HBM once) and one L2's copy of the activations.
+    const int CT = (a.NT + NJ - 1) / NJ, RT = (a.R + 64 * WR - 1) / (64 * WR), n_tiles = CT * RT;
+    const int per_xcd = (n_tiles + 7) >> 3, seq = blockIdx.x >> 3, tile = (int)(blockIdx.x & 7) * per_xcd + seq;
+    if (seq >= per_xcd || tile >= n_tiles) return;
+    const int nt0 = (tile / RT) * NJ;
+    const long row0 = (long)(tile % RT) * (64 * WR);
+    floatx16 acc[NJ][2];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[j][i][v] = 0.0f;
+
+    // 1 KiB pieces of a stage: NJ KG weight fragments [column tile][k-tile], then 16 pieces of activations (row-major, a row's
+    // 16-byte units at position unit ^ swz(row): the fragment reads of 32 rows x 2 units then spread evenly over the banks)
+    const half_t* wsrc[LW]; int wkt[LW];
+#pragma unroll
+    for (int i = 0; i < LW; ++i) {
+        const int p = i * 8 + w;
+        wsrc[i] = a.W + ((long)min(nt0 + p / KG, a.NT - 1) * a.KT * 64 + lane) * 8;
+        wkt[i] = p % KG;
+    }
+    auto swz = [](int row) { return KG == 4 ? (row >> 1) & 7 : row & 15; };
+    const half_t* xsrc[2]; int xkt[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int rl = (i * 8 + w) * (64 / PPR) + lane / PPR, s = (lane % PPR) ^ swz(rl);
+        xsrc[i] = a.X + min(row0 + rl, (long)a.R - 1) * (long)a.ldx + 8 * (s & 1);
+        xkt[i] = s >> 1;
+    }
+    typedef const void __attribute__((address_space(1)))* gptr_t;
+    typedef void __attribute__((address_space(3)))* lptr_t;
+    auto issue = [&](int c) {
+        char* st = (char*)big_smem + (c % NST) * STAGE;
+#pragma unroll
+        for (int i = 0; i < LW; ++i)
+            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (long)min(c * KG + wkt[i], a.KT - 1) * 512), (lptr_t)(st + (i * 8 + w) * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (long)min(c * KG + xkt[i], a.KT - 1) * 16), (lptr_t)(st + NJ * KG * 1024 + (i * 8 + w) * 1024), 16, 0, 0);
+    };
+    const int NC = (a.KT + KG - 1) / KG;
+    const unsigned lds0 = (unsigned)(size_t)(lptr_t)big_smem;
+    const int xr = 64 * wr + (lane & 31);
+    const unsigned woff = (unsigned)(kg * 1024 + lane * 16);
+    const unsigned xoff = (unsigned)(NJ * KG * 1024 + xr * (PPR * 16) + 16 * ((2 * kg + (lane >> 5)) ^ swz(xr)));
+    issue(0);
+    if (NC > 1) issue(1);
+    if (PF > 2 && NC > 2) issue(2);
+    half8 wf[NJ], xf[2];
+    auto wait_loads = [&](int c) {          // this wavefront's part of chunk c + 1 has landed
+        const int later = max(0, min(PF - 1, NC - 2 - c));
+        if (later == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPC) : "memory");
+        else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPC) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    auto R = [&](int c, bool wait_now) {
+        const unsigned sb = lds0 + (unsigned)((c % NST) * STAGE);
+        mid_read_frags<NJ, KG>(sb + woff, sb + xoff, wf, xf);
+        if (c + PF < NC) issue(c + PF);
+        if (wait_now) wait_loads(c);
+        mid_wait_frags<NJ>(wf, xf);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto M = [&](int c) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (c * KG + kg < a.KT) {           // (wavefront-uniform: the last chunk may hold fewer than KG k-tiles)
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[j], xf[i], acc[j][i], 0, 0, 0);
+            __builtin_amdgcn_s_setprio(0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    wait_loads(-1);
+    __builtin_amdgcn_s_barrier();                       // chunk 0 is in LDS
+    if ((w >> 2) == 0) {                                // the same number of barriers in both groups; see big_gemm3_f16_kernel
+        for (int c = 0; c < NC; ++c) {
+            if (c) { __builtin_amdgcn_s_barrier(); __builtin_amdgcn_sched_barrier(0); }
+            R(c, false);
+            M(c);
+            wait_loads(c);
+        }
+    } else {
+        R(0, true);
+        for (int c = 1; c < NC; ++c) {
+            __builtin_amdgcn_s_barrier();
+            M(c - 1);
+            R(c, true);
+        }
+        M(NC - 1);
+    }
+    __syncthreads();                                    // the stages are dead
+
+    // Sum of the KG partial accumulators, UP of the row group's 2 NJ MFMA tiles at a time: every wavefront writes its copies
+    // (row stride 36 floats), then KG / UP wavefronts per tile add them in order and finish the tile's rows in line layout:
+    // lane = (row, 4 consecutive columns), eight lanes per row.
+    constexpr int UP = S::UP, WPU = KG / UP, LDSROW = 36;
+    float* red = (float*)big_smem;
+    const int lh = lane >> 5, piece = lane & 7, rr = lane >> 3;
+    const int my_unit = kg / WPU, my_part = kg % WPU;
+    const bool ld_ok = (EPI == BEPI_ACT16 ? a.ld16 : a.ld_out) % 4 == 0 && (EPI != BEPI_RESID || !a.xg16 || a.ld_xg % 4 == 0);
+#pragma unroll
+    for (int ph = 0; ph < 2 * NJ / UP; ++ph) {
+        const int u = ph * UP + my_unit, nt = nt0 + (u >> 1);
+        const bool gated = EPI == BEPI_ACT16 && a.gated;
+        const int c0 = gated ? nt * 16 + 4 * (piece & 3) : nt * 32 + 4 * piece;      // first of this lane's four outputs (gated: of both factors)
+        const bool nt_ok = nt < a.NT, vec = ld_ok && c0 + 3 < a.n_valid;
+        // operands of this lane's outputs that do not depend on the products
+        floatx4 bb, gm = {0.0f, 0.0f, 0.0f, 0.0f}, old[4 / WPU];
+        float rv[4 / WPU];
+        const float* bsrc = gated && piece >= 4 ? a.bias2 : a.bias;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            bb[e] = bsrc[min(c0 + e, a.n_valid - 1)];
+            if (EPI == BEPI_RESID && a.xg16) gm[e] = a.gamma[min(c0 + e, a.n_valid - 1)];
+        }
+#pragma unroll
+        for (int q = 0; q < 4 / WPU; ++q) {
+            const long row = min(row0 + 64 * wr + 32 * (u & 1) + 8 * (my_part * (4 / WPU) + q) + rr, (long)a.R - 1);
+            rv[q] = a.rinv ? a.rinv[row] : 1.0f;
+            if (EPI == BEPI_RESID) {
+                const float* src = a.out + row * a.ld_out;
+                if (vec) old[q] = *(const floatx4*)(src + c0);
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) old[q][e] = src[min(c0 + e, a.n_valid - 1)];
+                }
+            }
+        }
+        if (ph) __syncthreads();
+#pragma unroll
+        for (int uu = 0; uu < UP; ++uu) {
+            const int j = (ph * UP + uu) >> 1, i = (ph * UP + uu) & 1;
+            float* dst = red + ((wr * UP + uu) * KG + kg) * (32 * LDSROW) + (lane & 31) * LDSROW + 4 * lh;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) *(floatx4*)(dst + 8 * g) = floatx4{acc[j][i][4 * g], acc[j][i][4 * g + 1], acc[j][i][4 * g + 2], acc[j][i][4 * g + 3]};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4 / WPU; ++q) {
+            const int rl = 8 * (my_part * (4 / WPU) + q) + rr;
+            const long row = row0 + 64 * wr + 32 * (u & 1) + rl;
+            const float* src = red + ((wr * UP + my_unit) * KG) * (32 * LDSROW) + rl * LDSROW + 4 * piece;
+            floatx4 s = *(const floatx4*)src;
+#pragma unroll
+            for (int k = 1; k < KG; ++k) {
+                const floatx4 p = *(const floatx4*)(src + k * (32 * LDSROW));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] += p[e];
+            }
+            const bool ok = nt_ok && row < a.R;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = s[e] * rv[q] + bb[e];
+            if (EPI == BEPI_ACT16) {
+                half4v o;
+                if (gated) {
+                    // columns 0-15 of a tile are the first factor, 16-31 the second: lanes four apart hold the two factors
+                    floatx4 z;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) z[e] = __shfl_xor(s[e], 4, 64);
+                    with_act(a.act, [&](auto A) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[e] = (half_t)(act_apply_c<decltype(A)::value>(s[e]) * z[e]);
+                    });
+                } else {
+                    with_act(a.act, [&](auto A) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[e] = (half_t)act_apply_c<decltype(A)::value>(s[e]);
+                    });
+                }
+                if (ok && (!gated || piece < 4)) {
+                    half_t* dst = a.out16 + row * a.ld16 + c0;
+                    if (vec) *(half4v*)dst = o;
+                    else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) if (c0 + e < a.n_valid) dst[e] = o[e];
+                    }
+                }
+                continue;
+            }
+            if (EPI == BEPI_RESID) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] = s[e] + old[q][e];
+            }
+            if (ok) {
+                float* dst = a.out + row * a.ld_out + c0;
+                if (vec) *(floatx4*)dst = s;
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) if (c0 + e < a.n_valid) dst[e] = s[e];
+                }
+            }
+            if (EPI == BEPI_RESID && a.xg16) {
+                half4v xg;
+                float sq = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { xg[e] = (half_t)(gm[e] * s[e]); sq += c0 + e < a.n_valid ? s[e] * s[e] : 0.0f; }
+                if (ok) {
+                    half_t* dst = a.xg16 + row * a.ld_xg + c0;
+                    if (vec) *(half4v*)dst = xg;
+                    else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) if (c0 + e < a.n_valid) dst[e] = xg[e];
+                    }
+                }
+                sq += __shfl_xor(sq, 1, 64);
+                sq += __shfl_xor(sq, 2, 64);
+                sq += __shfl_xor(sq, 4, 64);
+                if (ok && piece == 0) a.ssq_out[(long)nt * a.ssq_ld + row] = sq;
+            }
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------------------------

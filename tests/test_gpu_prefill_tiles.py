@@ -1,0 +1,77 @@
+"""Every tile of the prefill GEMMs (TSHIP_GEMM_TILE) at the edges of its range, against the oracle."""
+import numpy as np
+import pytest
+
+from seq2seqsharp_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+FP16_ABS = 3e-2      # the fp16 bar of the parity tests
+
+SHAPES = {
+    # hidden, heads, kv heads, ffn, attention, norm, activation; k-tiles of 16: 10 / 12.5 (a partial last one), 3 / 7, 32 / 44
+    "rms_gated": (160, 10, 5, 200, synth.GQA, synth.RMSNORM, synth.SWIGLU),
+    "layer_norm_relu": (48, 3, 3, 104, synth.MHA, synth.LAYERNORM, synth.RELU),
+    "rms_silu_wide": (512, 8, 2, 704, synth.GQA, synth.RMSNORM, synth.SILU),
+}
+
+
+@pytest.fixture(scope="module")
+def G():
+    from seq2seqsharp_amd import gpt
+    return gpt
+
+
+def _model(shape, batch, prompt):
+    hidden, heads, kv, ffn, attn, norm, act = SHAPES[shape]
+    cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=ffn, vocab=157, attn_type=attn, norm_type=norm, act=act,
+                     batch=batch, prompt=prompt, steps=2, dtype="f16")
+    return cfg, synth.make_weights(cfg, 41, random_bias=True), synth.make_prompts(cfg, 42)
+
+
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("batch,prompt", [(1, 1), (1, 33), (1, 64), (5, 13), (2, 65), (3, 90), (5, 128)])      # 1 ... 640 rows around 64, 128 and 256
+def test_prefill_gemm_tiles(G, oracle, monkeypatch, shape, batch, prompt):
+    """Logits, keys and values with each tile; one row, rows that end inside, at and behind a 64-row group, column counts that
+    are no multiple of a tile's columns, k-tile counts that are no multiple of a stage's.  Tile 0 applies from 256 rows on."""
+    cfg, w, seqs = _model(shape, batch, prompt)
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(seqs, use_cache=True)
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
+    for tile in (None, "11", "12", "14", "22", "24", "0"):
+        if tile is None:
+            monkeypatch.delenv("TSHIP_GEMM_TILE", raising=False)
+        else:
+            monkeypatch.setenv("TSHIP_GEMM_TILE", tile)
+        gpu.reset()
+        gpu.prefill(seqs)
+        got = gpu.logits()
+        assert np.abs(got - lg).max() <= FP16_ABS, tile
+        k, v = gpu.get_kv(1, 0), gpu.get_kv(1, 1)
+        if tile is None:
+            k0, v0 = k, v
+        # one fp16 rounding step of the stored value (2^-10 of it) and the same of the sums in front of it, in another order
+        assert np.abs(k - k0).max() <= 4e-3 * np.abs(k0).max() and np.abs(v - v0).max() <= 4e-3 * np.abs(v0).max(), tile
+    gpu.close()
+
+
+@pytest.mark.parametrize("hidden,heads,kv,batch,prompt", [(512, 8, 2, 5, 128), (1024, 8, 2, 3, 192), (512, 8, 4, 1, 544)])
+def test_large_tile_writes_the_cache_like_the_separate_kernel(G, monkeypatch, hidden, heads, kv, batch, prompt):
+    """The 256 x 256 tile forced: the QKV projection's own cache write (head sizes 64 and 128, a wavefront partly beyond the
+    rows) against the separate kernel, and the heights of the tile patches against each other, bit for bit."""
+    cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=2 * hidden, vocab=157, attn_type=synth.GQA,
+                     norm_type=synth.RMSNORM, act=synth.SWIGLU, batch=batch, prompt=prompt, steps=2, dtype="f16")
+    w = synth.make_weights(cfg, 77, random_bias=True)
+    seqs = synth.make_prompts(cfg, 78)
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
+    monkeypatch.setenv("TSHIP_GEMM_TILE", "0")
+    gpu.prefill(seqs)
+    want = [gpu.logits()] + [gpu.get_kv(l, i) for l in range(2) for i in range(2)]
+    for name, value in (("TSHIP_NO_KV_FUSE", "1"), ("TSHIP_PATCH_ROWS", "1"), ("TSHIP_PATCH_ROWS", "8")):
+        monkeypatch.setenv(name, value)
+        gpu.reset()
+        gpu.prefill(seqs)
+        monkeypatch.delenv(name)
+        got = [gpu.logits()] + [gpu.get_kv(l, i) for l in range(2) for i in range(2)]
+        assert all(np.array_equal(a, b) for a, b in zip(want, got)), (name, value)
+    gpu.close()
