@@ -169,6 +169,7 @@ struct TestHooks {
     int patch_rows = 0;       // TSHIP_PATCH_ROWS: 1, 2, 4 or 8 row tiles per tile patch of the prefill GEMM
     long attn_splits = 0;     // TSHIP_ATTN_SPLITS: blocks per (sequence, KV head) pair in decode attention
     int gemm_tile = -1;        // TSHIP_GEMM_TILE: tile of the prefill GEMMs (pick_gemm_tile); 0: the 256 x 256 tile from 256 rows on
+    int f32_tile = 0;         // TSHIP_F32_TILE: tile of the fp32 GEMMs from 33 rows on (pick_f32_tile)
     int attn_nq = 0;          // TSHIP_ATTN_NQ: 1 or 2 groups of 16 MFMA columns per wavefront in prefill attention
     bool no_kv_fuse = false;  // TSHIP_NO_KV_FUSE: the QKV projection of a prefill does not write the cache itself
     bool no_moe_batch = false;// TSHIP_NO_MOE_BATCH: one prefill GEMM launch per expert
@@ -190,6 +191,10 @@ static void refresh_test_hooks() {
     if (const char* v = std::getenv("TSHIP_GEMM_TILE")) {
         h.gemm_tile = std::atoi(v);
         TSHIP_REQUIRE(h.gemm_tile == 0 || h.gemm_tile == 11 || h.gemm_tile == 12 || h.gemm_tile == 14 || h.gemm_tile == 22 || h.gemm_tile == 24, "TSHIP_GEMM_TILE: 0, 11, 12, 14, 22 or 24");
+    }
+    if (const char* v = std::getenv("TSHIP_F32_TILE")) {
+        h.f32_tile = std::atoi(v);
+        TSHIP_REQUIRE(h.f32_tile == 11 || h.f32_tile == 21 || h.f32_tile == 22 || h.f32_tile == 42, "TSHIP_F32_TILE: 11, 21, 22 or 42");
     }
     h.no_kv_fuse = std::getenv("TSHIP_NO_KV_FUSE") != nullptr;
     h.no_moe_batch = std::getenv("TSHIP_NO_MOE_BATCH") != nullptr;
@@ -501,6 +506,23 @@ static void run_skinny(TSHipGpt* m, const char* name, const GemmW& w, const void
 #undef TSHIP_SK
 }
 
+// Tile of an fp32 GEMM from 33 rows on, 10 x (32-row) + (32-column) quadrants: the estimated time over the compute units'
+// rounds, fits to launches of 37 ... 4096 rows at six (K, N) of 512 ... 3072 (1.9 us + 2.0 + 0.0059 K per round of single
+// quadrants: 37 x 768 x 768 9.4 us, against 12.1, 18.7 and 29.8 with the larger tiles; 4 us + 0.8 + 0.033 K per round of the
+// largest: 4096 x 3072 x 768 162 us, 76 % of the matrix rate, against 306, 199 and 179 with the smaller ones).
+static int pick_f32_tile(int rows, int N, int K, int KS) {
+    if (g_hooks.f32_tile) return g_hooks.f32_tile;
+    struct Cost { int tile, rows, cols; float fixed, a, b; };
+    static const Cost costs[] = {{11, 32, 32, 1.9f, 2.0f, 0.0059f}, {21, 64, 32, 4.0f, 0.6f, 0.0101f}, {22, 64, 64, 4.0f, 1.0f, 0.0178f}, {42, 128, 64, 4.0f, 0.8f, 0.0331f}};
+    const long ncu = std::max(1, n_compute_units());
+    int best = 11; float best_us = 1e30f;
+    for (const Cost& c : costs) {
+        const long blocks = ceil_div((long)rows, c.rows) * ceil_div((long)N, c.cols) * KS;
+        const float us = c.fixed + (float)ceil_div(blocks, ncu) * (c.a + c.b * (float)ceil_div(K, KS));
+        if (us < best_us) { best_us = us; best = c.tile; }
+    }
+    return best;
+}
 static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const float* X, long ldx, int rows, float* out, long ld_out,
                          long split_stride, int KS, const float* bias = nullptr) {
     F32GemmArgs g;
@@ -514,8 +536,21 @@ static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const fl
         else launch(m, name, skinny_gemm_f32_kernel<32>, sgrid, dim3(256), g);
         return;
     }
-    dim3 grid((unsigned)ceil_div(w.N, 64), (unsigned)ceil_div(rows, 64), KS);
-    launch(m, name, gemm_f32_kernel, grid, dim3(256), g);
+    const bool vec = ((w.K | w.N) & 3) == 0 && ((ldx | w.ld) & 3) == 0 && (((uintptr_t)X | (uintptr_t)w.buf.p) & 15) == 0;
+    auto go = [&](auto QMc, auto QNc) {
+        constexpr int QM = decltype(QMc)::value, QN = decltype(QNc)::value;
+        const dim3 grid((unsigned)ceil_div(w.N, 32 * QN), (unsigned)ceil_div(rows, 32 * QM), KS);
+        const unsigned shm = MfmaF32Shape<QM, QN>::SHM;
+        if (vec) launch_shm(m, name, mfma_gemm_f32_kernel<QM, QN, true>, grid, dim3(512), shm, g);
+        else launch_shm(m, name, mfma_gemm_f32_kernel<QM, QN, false>, grid, dim3(512), shm, g);
+    };
+    typedef std::integral_constant<int, 1> c1; typedef std::integral_constant<int, 2> c2; typedef std::integral_constant<int, 4> c4;
+    switch (pick_f32_tile(rows, w.N, w.K, KS)) {
+        case 11: go(c1{}, c1{}); break;
+        case 21: go(c2{}, c1{}); break;
+        case 22: go(c2{}, c2{}); break;
+        default: go(c4{}, c2{}); break;
+    }
 }
 
 // Tile of a prefill GEMM: 10 x (64-row groups) + 32-column tiles of mid_gemm_f16_kernel, or 0 for the 256 x 256 tile.
@@ -601,17 +636,23 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
 }
 
 typedef void (*AttnKernel)(AttnArgs);
+template <typename CT, typename AT, int D, int G>
+static AttnKernel pick_attn_k(bool prefill) {
+    if constexpr (sizeof(CT) == 4) { if (prefill) return attn_prefill_f32_kernel<D, G>; }
+    else if (prefill) return attn_prefill_kernel<CT, AT, D, G>;
+    return attn_decode_kernel<CT, AT, D, G>;
+}
 template <typename CT, typename AT, int D>
 static AttnKernel pick_attn_g(int G, bool prefill) {
     switch (G) {
-        case 1: return prefill ? attn_prefill_kernel<CT, AT, D, 1> : attn_decode_kernel<CT, AT, D, 1>;
-        case 2: return prefill ? attn_prefill_kernel<CT, AT, D, 2> : attn_decode_kernel<CT, AT, D, 2>;
-        case 4: return prefill ? attn_prefill_kernel<CT, AT, D, 4> : attn_decode_kernel<CT, AT, D, 4>;
-        case 8: return prefill ? attn_prefill_kernel<CT, AT, D, 8> : attn_decode_kernel<CT, AT, D, 8>;
-        case 3: return prefill ? attn_prefill_kernel<CT, AT, D, 3> : attn_decode_kernel<CT, AT, D, 3>;
-        case 5: return prefill ? attn_prefill_kernel<CT, AT, D, 5> : attn_decode_kernel<CT, AT, D, 5>;
-        case 6: return prefill ? attn_prefill_kernel<CT, AT, D, 6> : attn_decode_kernel<CT, AT, D, 6>;
-        case 7: return prefill ? attn_prefill_kernel<CT, AT, D, 7> : attn_decode_kernel<CT, AT, D, 7>;
+        case 1: return pick_attn_k<CT, AT, D, 1>(prefill);
+        case 2: return pick_attn_k<CT, AT, D, 2>(prefill);
+        case 3: return pick_attn_k<CT, AT, D, 3>(prefill);
+        case 4: return pick_attn_k<CT, AT, D, 4>(prefill);
+        case 5: return pick_attn_k<CT, AT, D, 5>(prefill);
+        case 6: return pick_attn_k<CT, AT, D, 6>(prefill);
+        case 7: return pick_attn_k<CT, AT, D, 7>(prefill);
+        case 8: return pick_attn_k<CT, AT, D, 8>(prefill);
         default: throw Error("query heads per KV head must be 1 to 8");
     }
 }
@@ -1137,7 +1178,10 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             const int per_block = (16 / m->G) * 8 * nq;
             launch(m, "p_attn", pick_attn(m, true, false, host_lens != nullptr, nq), dim3((unsigned)ceil_div(Tp, per_block), m->Hv, B), dim3(512), aa);
         }
-        else launch(m, "p_attn", pick_attn(m, true), dim3(Tp, m->Hv, B), dim3(256), aa);
+        else if (!m->f16) {
+            const unsigned shm = m->D == 128 ? attn_prefill_f32_shm<128>() : m->D == 64 ? attn_prefill_f32_shm<64>() : m->D == 32 ? attn_prefill_f32_shm<32>() : attn_prefill_f32_shm<16>();
+            launch_shm(m, "p_attn", pick_attn(m, true), dim3((unsigned)ceil_div(Tp, 32 / m->G), m->Hv, B), dim3(256), shm, aa);
+        } else launch(m, "p_attn", pick_attn(m, true), dim3(Tp, m->Hv, B), dim3(256), aa);
         ResidNormArgs a2 = rn;
         a2.gamma = L.n2_g.as<float>(); a2.beta = L.n2_b.as<float>();
         if (m->f16) {

@@ -1761,8 +1761,7 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// fp32 GEMM (fp32 models: prefill and decode): C[ks][M][N] = A[M][K-range ks] * B[K-range][N], 64x64 tile,
-// k accumulated sequentially inside a split.
+// fp32 GEMM (fp32 models: prefill and decode): C[ks][M][N] = A[M][K-range ks] * B[K-range][N].
 // ------------------------------------------------------------------------------------------------
 struct F32GemmArgs {
     const float* A; long lda; const float* B; long ldb; float* C; long ldc; long split_stride;
@@ -1851,51 +1850,118 @@ __global__ __launch_bounds__(256) void skinny_gemm_f32_kernel(F32GemmArgs a) {
     }
 }
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(F32GemmArgs a) {
-    __shared__ float As[16][64 + 4];
-    __shared__ float Bs[16][64 + 4];
-    const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
-    const int col0 = blockIdx.x * 64, row0 = blockIdx.y * 64, ks = blockIdx.z;
+// The same product for more rows, on the fp32 matrix instructions (v_mfma_f32_32x32x2_f32: 256 multiply-adds per clock and
+// compute unit with fp32 operands and sums, against 128 of the vector pipes without packed fp32).  Block tile 32 QM x 32 QN,
+// eight wavefronts: QM x QN quadrants of 32 x 32 times KG wavefronts that share the k of a chunk and are added through LDS
+// at the end, so that small products (a 37 x 768 one is 48 quadrants) still give every SIMD two wavefronts.
+// Both operands go through registers, requested two chunks ahead, into two LDS stages; the row strides (4 resp. 8 floats
+// past a multiple of 32) keep the 16-byte reads of the rows and the 4-byte reads of the columns free of bank conflicts.
+// An instruction's two k are four apart (element j of a lane's 16 bytes), the same in both operands.
+// VEC: K, N and both leading dimensions are multiples of four and the operands 16-byte aligned.
+// Measured, us, 600 rows (a 64 x 64 tile of vector multiply-adds, one stage, before -> now): 768 x 768 91 -> 14,
+// 768 x 2304 107 -> 34, 768 x 3072 110 -> 35, 3072 x 768 357 -> 41 (120 tiles of 64 x 64 for 256 units).  The error against
+// 64 bits falls with the shorter chains of a wavefront's share (3072 x 768: 1.0e-6 of one chain, 2.2e-7 of eight).
+template <int QM, int QN>
+struct MfmaF32Shape {
+    static constexpr int KG = 8 / (QM * QN), KW = KG <= 2 ? 32 : 16, BK = KG * KW, TM = 32 * QM, TN = 32 * QN;
+    static constexpr int LDA = BK + 4, LDB = TN + 8, STAGE = TM * LDA + BK * LDB;
+    static constexpr unsigned SHM = 2u * STAGE * sizeof(float);
+    static_assert((KG - 1) * QM * QN * 1024 <= 2 * STAGE, "partial sums fit the stages");
+};
+template <int QM, int QN, bool VEC>
+__global__ __launch_bounds__(512) void mfma_gemm_f32_kernel(F32GemmArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float gf_smem[];
+    using S = MfmaF32Shape<QM, QN>;
+    constexpr int KG = S::KG, KW = S::KW, BK = S::BK, TM = S::TM, TN = S::TN, LDA = S::LDA, LDB = S::LDB, NQ = QM * QN;
+    constexpr int NA = TM * BK / 2048, NB = BK * TN / 2048;       // 16-byte pieces per thread and chunk
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, l32 = lane & 31, half = lane >> 5;
+    const int kg = w / NQ, q = w % NQ, qm = q / QN, qn = q % QN;
+    const int col0 = blockIdx.x * TN, row0 = blockIdx.y * TM, ks = blockIdx.z;
     const int kper = (int)round_up(ceil_div(a.K, a.KS), 16);
     const int kb = ks * kper, ke = min(a.K, kb + kper);
-    float acc[4][4];
+    auto load = [&](floatx4 (&r)[NA + NB], int k0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NA; ++i) {
+            const int p = t + 512 * i, row = min(row0 + p / (BK / 4), a.M - 1), k = k0 + 4 * (p % (BK / 4));
+            const float* src = a.A + (long)row * a.lda + k;
+            r[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (VEC) { if (k < ke) r[i] = *(const floatx4*)src; }
+            else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-    const int am = t >> 2, ak = (t & 3) * 4;
-    const int bk = t >> 4, bn = (t & 15) * 4;
-    for (int k0 = kb; k0 < ke; k0 += 16) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int r = row0 + am, k = k0 + ak + j;
-            As[ak + j][am] = (r < a.M && k < ke) ? a.A[(long)r * a.lda + k] : 0.0f;
-            int kk = k0 + bk, c = col0 + bn + j;
-            Bs[bk][bn + j] = (kk < ke && c < a.N) ? a.B[(long)kk * a.ldb + c] : 0.0f;
+                for (int c = 0; c < 4; ++c) if (k + c < ke) r[i][c] = src[c];
+            }
         }
-        __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            float av[4], bv[4];
+        for (int i = 0; i < NB; ++i) {
+            const int p = t + 512 * i, k = k0 + p / (TN / 4), c0 = col0 + 4 * (p % (TN / 4));
+            const float* src = a.B + (long)k * a.ldb + c0;
+            r[NA + i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (VEC) { if (k < ke && c0 < a.N) r[NA + i] = *(const floatx4*)src; }
+            else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) { av[i] = As[k][ty * 4 + i]; bv[i] = Bs[k][tx * 4 + i]; }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
+                for (int c = 0; c < 4; ++c) if (k < ke && c0 + c < a.N) r[NA + i][c] = src[c];
+            }
         }
+    };
+    auto store = [&](const floatx4 (&r)[NA + NB], float* sA) {
+        float* sB = sA + TM * LDA;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) { const int p = t + 512 * i; *(floatx4*)(sA + (p / (BK / 4)) * LDA + 4 * (p % (BK / 4))) = r[i]; }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) { const int p = t + 512 * i; *(floatx4*)(sB + (p / (TN / 4)) * LDB + 4 * (p % (TN / 4))) = r[NA + i]; }
+    };
+    floatx16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+    auto compute = [&](const float* sA) {
+        const float* pa = sA + (qm * 32 + l32) * LDA + kg * KW + 4 * half;
+        const float* pb = sA + TM * LDA + (kg * KW + 4 * half) * LDB + qn * 32 + l32;
+#pragma unroll
+        for (int s = 0; s < KW / 8; ++s) {
+            const floatx4 av = *(const floatx4*)(pa + 8 * s);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], pb[(8 * s + j) * LDB], acc, 0, 0, 0);
+        }
+    };
+    const int nc = max(1, (int)ceil_div(ke - kb, BK));
+    floatx4 r0[NA + NB], r1[NA + NB];
+    load(r0, kb);
+    load(r1, kb + BK);
+    store(r0, gf_smem);
+    // chunk c: stage c & 1 holds it, the other register set chunk c + 1; one barrier: what is written behind it was read
+    // before the barrier of the chunk in front
+    for (int c = 0; c < nc; c += 2) {
+        load(r0, kb + (c + 2) * BK);
         __syncthreads();
+        compute(gf_smem);
+        store(r1, gf_smem + S::STAGE);
+        if (c + 1 >= nc) break;
+        load(r1, kb + (c + 3) * BK);
+        __syncthreads();
+        compute(gf_smem + S::STAGE);
+        store(r0, gf_smem);
     }
-    float* C = a.C + ks * a.split_stride;
+    if constexpr (KG > 1) {       // the other wavefronts' sums, added in their order
+        __syncthreads();
+        if (kg > 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        int r = row0 + ty * 4 + i;
-        if (r >= a.M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int c = col0 + tx * 4 + j;
-            if (c < a.N) C[(long)r * a.ldc + c] = a.bias ? acc[i][j] + a.bias[c] : acc[i][j];
+            for (int i = 0; i < 16; ++i) gf_smem[(((kg - 1) * NQ + q) * 16 + i) * 64 + lane] = acc[i];
         }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; ++g)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] += gf_smem[((g * NQ + q) * 16 + i) * 64 + lane];
+    }
+    const int col = col0 + qn * 32 + l32;
+    if (col >= a.N) return;
+    const float bv = a.bias ? a.bias[col] : 0.0f;
+    float* C = a.C + ks * a.split_stride + col;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int row = row0 + qm * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+        if (row < a.M) C[(long)row * a.ldc] = a.bias ? acc[i] + bv : acc[i];
     }
 }
 
@@ -2597,6 +2663,136 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
     for (int idx = t; idx < G * D; idx += 256) out[idx] = (AT)sm.out[idx];
 }
 
+
+// The same for an fp32 cache (row-major), on the fp32 matrix instructions: grid (column tiles, Hkv, batch), a tile of 32
+// MFMA columns = 32 / G query positions x G heads, the longest tiles first.  The four wavefronts of a block take chunks of 32
+// cached positions in turn, each with an online softmax of its own, and are merged through LDS.
+//   S[32 t][32 col]  = K (A operand: lane row t, 16 bytes of it per load) x Q (B operand, in registers)
+//   O^T[D][32 col]  += V^T (A operand: lane row i is d = VD i + dt, VD = D / 32, so that a cached row is read whole) x P
+// The two k of an instruction are four apart: they are then d = 8 s + j and + 4 in S, and in O^T the t of the two rows that
+// the result layout of S leaves in a lane's register 4 g + j and its other half's: P goes back in without a shuffle.
+// No LDS for keys and values: a wavefront reads 4 D x 64 bytes per D x 64 clocks of matrix work, requested a product ahead.
+// A row-at-a-time kernel read the whole cache once per query: 38 us per layer for 2 x 300 positions of 12 heads of 64, now 15.5
+// (bound by the matrix instructions of the longest tile's wavefront and its start).  Masked positions have probability 0 and multiply their
+// values, as in the reference's full product; rows past the sequence are not read.
+template <int D, int G>
+__global__ __launch_bounds__(256) void attn_prefill_f32_kernel(AttnArgs a) {
+    constexpr int QB = 32 / G, VD = D >= 32 ? D / 32 : 1, LDQ = D + 4;
+    typedef float vrow_t __attribute__((ext_vector_type(VD)));
+    extern __shared__ __attribute__((aligned(16))) float af_smem[];       // queries [32][LDQ]; later O [4][D][33], then m, l [4][32]
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, l32 = lane & 31, half = lane >> 5;
+    const int kvh = blockIdx.y, b = blockIdx.z, kvc = a.kv_sub > 1 ? kvh / a.kv_sub : kvh;
+    const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * QB, nq = min(QB, a.Tq - q0);
+    for (int p = t; p < 32 * (D / 2); p += 256) {
+        const int c = p / (D / 2), i = p % (D / 2), tq = q0 + c / G;
+        float y0 = 0.0f, y1 = 0.0f;
+        if (c < nq * G) {
+            const long row = (long)b * a.Tq + tq;
+            const int col = (kvh * G + c % G) * D + 2 * i;
+            const float x0 = a.qkv[row * a.ldq + col] + a.bias[col], x1 = a.qkv[row * a.ldq + col + 1] + a.bias[col + 1];
+            y0 = x0; y1 = x1;
+            const long pos = a.pos0 + tq;
+            if (a.rope_cos) rope_pair(x0, x1, a.rope_cos[pos * (D / 2) + i], a.rope_sin[pos * (D / 2) + i], y0, y1);
+        }
+        af_smem[c * LDQ + 2 * i] = a.scale * y0; af_smem[c * LDQ + 2 * i + 1] = a.scale * y1;
+    }
+    __syncthreads();
+    floatx4 qf[D / 8];
+#pragma unroll
+    for (int s = 0; s < D / 8; ++s) qf[s] = *(const floatx4*)(af_smem + l32 * LDQ + 8 * s + 4 * half);
+    __syncthreads();
+    const int tq = q0 + min(l32 / G, nq - 1), n_pos = a.pos0 + a.Tq;       // (columns of no query repeat the last one's mask)
+    const bool all_masked = a.lens && tq >= a.lens[b];
+    const int T = all_masked ? n_pos : a.pos0 + tq + 1;      // this column's positions
+    int T_blk = a.pos0 + q0 + nq;                            // the block's
+    if (a.lens && q0 + nq - 1 >= a.lens[b]) T_blk = n_pos;
+    const float* Kb = (const float*)a.kcache + ((long)b * a.Hkv + kvc) * a.max_len * D;
+    const float* Vb = (const float*)a.vcache + ((long)b * a.Hkv + kvc) * a.max_len * D;
+    floatx16 o[VD];
+#pragma unroll
+    for (int dt = 0; dt < VD; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
+    float m = -INFINITY, l = 0.0f;
+    floatx4 kf[D / 8];
+    auto load_k = [&](int t0) {
+        const float* src = Kb + (long)min(t0 + l32, n_pos - 1) * D + 4 * half;
+#pragma unroll
+        for (int s = 0; s < D / 8; ++s) kf[s] = *(const floatx4*)(src + 8 * s);
+    };
+    int t0 = 32 * w;
+    if (t0 < T_blk) load_k(t0);
+    for (; t0 < T_blk; t0 += 128) {
+        vrow_t vf[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int tt = min(t0 + 8 * (i >> 2) + 4 * half + (i & 3), n_pos - 1);
+            if (D >= 32 || l32 < D) vf[i] = *(const vrow_t*)(Vb + (long)tt * D + VD * l32);
+            else
+#pragma unroll
+                for (int dt = 0; dt < VD; ++dt) vf[i][dt] = 0.0f;
+        }
+        floatx16 sc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < D / 8; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[s][j], qf[s][j], sc, 0, 0, 0);
+        if (t0 + 128 < T_blk) load_k(t0 + 128);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int tt = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
+            float v = sc[i];
+            if (all_masked) v = v + (-30000.0f);      // (a fully masked row: the float32 addition of the mask value rounds the score)
+            sc[i] = tt < T ? v : -INFINITY;
+            mx = fmaxf(mx, sc[i]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float mn = fmaxf(m, mx), base = mn == -INFINITY ? 0.0f : mn, corr = __expf(m - base);
+        m = mn;
+        float add = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) { sc[i] = __expf(sc[i] - base); add += sc[i]; }
+        l = l * corr + add;
+#pragma unroll
+        for (int dt = 0; dt < VD; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[dt][i] *= corr;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+            for (int dt = 0; dt < VD; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[i][dt], sc[i], o[dt], 0, 0, 0);
+    }
+    l += __shfl_xor(l, 32, 64);
+    float* sm_m = af_smem + 4 * D * 33;
+    float* sm_l = sm_m + 128;
+    if (half == 0) { sm_m[w * 32 + l32] = m; sm_l[w * 32 + l32] = l; }
+#pragma unroll
+    for (int dt = 0; dt < VD; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int row = 8 * (i >> 2) + 4 * half + (i & 3);
+            if (D >= 32 || row < D) af_smem[((long)w * D + VD * row + dt) * 33 + l32] = o[dt][i];
+        }
+    __syncthreads();
+    for (int idx = t; idx < nq * G * D; idx += 256) {
+        const int c = idx / D, d = idx % D;
+        float M = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) M = fmaxf(M, sm_m[i * 32 + c]);
+        float L = 0.0f, O = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float wgt = __expf(sm_m[i * 32 + c] - M);      // wavefronts that saw no position have m = -inf -> weight 0
+            L += sm_l[i * 32 + c] * wgt;
+            O += af_smem[(i * D + d) * 33 + c] * wgt;
+        }
+        ((float*)a.out)[((long)b * a.Tq + q0 + c / G) * a.ld_out + (kvh * G + c % G) * D + d] = O / L;
+    }
+}
+template <int D> constexpr unsigned attn_prefill_f32_shm() { return (unsigned)((4 * D * 33 + 256) * sizeof(float)); }
 
 // ------------------------------------------------------------------------------------------------
 // MFMA attention (fp16 cache, head_dim 64 or 128), decode: one block per (batch row, KV head); the G query heads of

@@ -1,0 +1,100 @@
+"""fp32 models from 33 rows on: the matrix-core GEMM (every tile, TSHIP_F32_TILE) and the tiled prefill attention, at the edges
+of their tiles, against the oracle."""
+import numpy as np
+import pytest
+
+from seq2seqsharp_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+FP32_REL = 1e-4      # the fp32 bar of the parity tests
+
+SHAPES = {
+    # hidden, heads, kv heads, ffn, attention, norm, activation; head sizes 16 / 32 / 64 / 128, one to eight query heads per KV head
+    "d16_g3": (144, 9, 3, 202, synth.GQA, synth.RMSNORM, synth.SWIGLU),          # odd FFN width: rows that are not 16-byte aligned
+    "d32_g5": (160, 5, 1, 72, synth.GQA, synth.LAYERNORM, synth.RELU),
+    "d64_g1": (192, 3, 3, 260, synth.MHA, synth.LAYERNORM, synth.RELU),
+    "d64_g7": (448, 7, 1, 96, synth.GQA, synth.RMSNORM, synth.SILU),
+    "d128_g2": (512, 4, 2, 136, synth.GQA, synth.RMSNORM, synth.SWIGLU),
+    "d16_g16": (256, 16, 1, 68, synth.GQA, synth.RMSNORM, synth.SILU),           # two groups of eight heads
+}
+
+
+@pytest.fixture(scope="module")
+def G():
+    from seq2seqsharp_amd import gpt
+    return gpt
+
+
+def _model(shape, batch, prompt):
+    hidden, heads, kv, ffn, attn, norm, act = SHAPES[shape]
+    cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=ffn, vocab=157, attn_type=attn, norm_type=norm, act=act,
+                     batch=batch, prompt=prompt, steps=2, dtype="f32")
+    w = synth.make_weights(cfg, 51, random_bias=True)
+    for k in list(w):                                        # attention far from uniform
+        if k.endswith((".Q", ".K", ".QKV")):
+            w[k] = w[k] * np.float32(6.0)
+    return cfg, w, synth.make_prompts(cfg, 52)
+
+
+def _check(gpu, orc, lg, what):
+    got = gpu.logits()
+    assert np.abs(got - lg).max() <= FP32_REL * np.abs(lg).max(), what
+
+
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("batch,prompt", [(1, 33), (3, 1), (5, 13), (1, 64), (2, 65), (3, 90), (1, 130)])
+def test_prefill(G, oracle, monkeypatch, shape, batch, prompt):
+    cfg, w, seqs = _model(shape, batch, prompt)
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(seqs, use_cache=True)
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
+    for tile in (None, "11", "21", "22", "42"):
+        if tile is None:
+            monkeypatch.delenv("TSHIP_F32_TILE", raising=False)
+        else:
+            monkeypatch.setenv("TSHIP_F32_TILE", tile)
+        gpu.reset()
+        gpu.prefill(seqs)
+        _check(gpu, orc, lg, tile)
+    gpu.close()
+
+
+@pytest.mark.parametrize("shape", ["d16_g3", "d64_g1", "d128_g2"])
+def test_prefill_behind_a_context_and_padded(G, oracle, shape):
+    """A second prompt behind cached positions, and prompts padded to one length (rows that see every position)."""
+    cfg, w, seqs = _model(shape, 3, 45 + 38)
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(seqs, use_cache=True)
+    gpu = G.HipGpt(cfg, w, max_batch=3, max_seq_len=96)
+    gpu.prefill(seqs[:, :45])
+    gpu.prefill(seqs[:, 45:])
+    _check(gpu, orc, lg, "turn")
+    lens = np.array([83, 20, 33], np.int32)
+    ids, _ = G.HipGpt.pad_sentences([list(s[:n]) for s, n in zip(seqs, lens)], pad_id=0)
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(ids, use_cache=True, lens=lens.astype(np.float32))
+    gpu.reset()
+    gpu.prefill(ids, lens=lens)
+    # (a padding row's scores are rounded to 2^-9: a score on the edge of a step moves its probability by 0.2 %)
+    err = np.abs(gpu.logits() - lg).max() / np.abs(lg).max()
+    assert err <= 10 * FP32_REL
+    gpu.close()
+
+
+def test_generate_with_more_than_32_rows(G, oracle):
+    """The same GEMM at decode (split K, replayed from a captured graph): 40 sequences, greedy."""
+    cfg, w, seqs = _model("d64_g1", 40, 3)
+    orc = oracle.OracleGpt(cfg, w)
+    p, _ = orc.step(seqs, use_cache=True)
+    gpu = G.HipGpt(cfg, w, max_batch=40, max_seq_len=16)
+    gpu.prefill(seqs)
+    ids, _ = gpu.generate(5)
+    cur = seqs
+    for i in range(5):
+        nxt = oracle.argmax(p).astype(np.int32)
+        assert np.array_equal(ids[i], nxt), i
+        cur = np.concatenate([cur, nxt[:, None]], 1)
+        p, lg = orc.step(cur, use_cache=True)
+    _check(gpu, orc, lg, "generate")
+    gpu.close()
