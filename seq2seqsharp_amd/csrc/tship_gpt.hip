@@ -122,6 +122,7 @@ struct TSHipGpt {
     DevBuf x, xn, o, a, part_qkv, part_h, part_f, logits, ids, d_pos, hidden;
     DevBuf moe_ws, topp_scratch, topp_uni, gen_buf, uni_buf, tile_count;
     DevBuf pw_lens, pw_ids, pw_x, pw_xn, pw_qkv, pw_o, pw_a, pw_f, pw_rowmap, pw_ssq, pw_rinv, pw_zero_bias, pw_moe;     // prefill workspace
+    DevBuf xn_rows, o_rows, a_rows, zero_qkv; // row-major activations of decode steps of more than 32 rows (xn, o and a hold packed ones)
     DevBuf ssq;                    // deferred-norm path: per-column-tile sums of squares [h/32][Bpad]
     bool fused_norm = false;       // fp16 + dense layers (RMSNorm; LayerNorm up to 32 rows): residual/norm folded into the GEMM tails
     bool ln = false;               // that path with LayerNorm: tile sums of x beside the sums of squares, folded constants per consumer
@@ -458,7 +459,8 @@ static void run_skinny(TSHipGpt* m, const char* name, const GemmW& w, const void
         TSHIP_REQUIRE(e.tile_count == m->tile_count.as<int>() && (size_t)w.NT * sizeof(int) <= m->tile_count.bytes,
                       "internal: too few tile counters");
     }
-    TSHIP_REQUIRE(epi != EPI_SPLIT_TAIL || (m->BT == 1 && e.tile_count), "internal: the split tail needs one batch tile and the tile counters");
+    TSHIP_REQUIRE((epi != EPI_SPLIT_TAIL && epi != EPI_RESID_TAIL) || m->BT == 1, "internal: a tail needs one batch tile");
+    TSHIP_REQUIRE(epi != EPI_SPLIT_TAIL || e.tile_count, "internal: the split tail needs the tile counters");
     dim3 grid(w.NT * e.KS);
     const int BT = m->BT;
     if (epi == EPI_ACT16 && BT == 1) {
@@ -499,10 +501,11 @@ static void run_skinny(TSHipGpt* m, const char* name, const GemmW& w, const void
 #define TSHIP_SK(BTV, NWV)                                                                                                  \
     if (epi == EPI_PARTIAL) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_PARTIAL, NWV>, grid, dim3(NWV * 64), e);        \
     else if (epi == EPI_F32_BIAS) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_F32_BIAS, NWV>, grid, dim3(NWV * 64), e); \
-    else if (epi == EPI_RESID_TAIL) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_RESID_TAIL, NWV, (BTV == 1 ? 16 : 8)>, grid, dim3(NWV * 64), e); \
-    else if (epi == EPI_SPLIT_TAIL) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_SPLIT_TAIL, NWV>, grid, dim3(NWV * 64), e); \
     else launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_ACT16, NWV>, grid, dim3(NWV * 64), e);
-    if (BT == 1) { TSHIP_SK(1, 8) } else if (BT == 2) { TSHIP_SK(2, 8) } else { TSHIP_SK(4, 4) }
+    // (tails with a norm behind them: models of up to 32 rows; larger ones take decode_step_rows)
+    if (epi == EPI_RESID_TAIL) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_RESID_TAIL, 8, 16>, grid, dim3(512), e);
+    else if (epi == EPI_SPLIT_TAIL) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_SPLIT_TAIL, 8>, grid, dim3(512), e);
+    else if (BT == 1) { TSHIP_SK(1, 8) } else if (BT == 2) { TSHIP_SK(2, 8) } else { TSHIP_SK(4, 4) }
 #undef TSHIP_SK
 }
 
@@ -840,6 +843,8 @@ static void record_history(TSHipGpt* m, const int* d_ids, int rows, int Tq, int 
 // normalise (RMSNormalization.Norm, Seq2SeqSharp/Layers/RMSNormalization.cs:33-37, folded into its neighbours).
 // ------------------------------------------------------------------------------------------------
 // first kernel of a decode step on the fused-norm path: embedding row x sqrt(h), the first layer's normalisation input, sums of squares
+// Models made for more than 32 rows (RMSNorm): the prefill's GEMM tiles on row-major activations (decode_step_rows)
+static bool decode_by_rows(const TSHipGpt* m) { return m->fused_norm && m->BT > 1; }
 static FnPrepArgs embed_prepare_args(TSHipGpt* m, const int* d_ids) {
     const int h = m->c.hidden;
     FnPrepArgs a; std::memset(&a, 0, sizeof(a));
@@ -847,7 +852,77 @@ static FnPrepArgs embed_prepare_args(TSHipGpt* m, const int* d_ids) {
     a.seg = m->seg.as<float>();      // (a cached decode step feeds one token per sequence: segment 0, Decoder.cs:661-673)
     a.gamma = m->L[0]->n1_g.as<float>(); a.xg16 = m->xn.as<half_t>(); a.xg_kt = (int)(m->ldh / 16); a.ssq_out = m->ssq.as<float>(); a.ssq_ld = m->Bpad;
     a.ln = m->ln ? 1 : 0;
+    if (decode_by_rows(m)) { a.xg16 = m->xn_rows.as<half_t>(); a.xg_kt = 0; a.xg_ld = m->ldh; }
     return a;
+}
+// The embedding rows of a decode step, unless the sampling kernel in front of it has prepared them.
+static void embed_prepare(TSHipGpt* m, const int* d_ids, int B) {
+    const int h = m->c.hidden;
+    if (m->embed_done) {
+        m->embed_done = false;        // (the greedy sampling kernel went on to embed the tokens it chose)
+    } else {
+        FnPrepArgs a = embed_prepare_args(m, d_ids);
+        if (h <= 2048) launch(m, "embed_prepare", fn_prepare_kernel<8>, dim3(B), dim3(256), a);
+        else if (h <= 4096) launch(m, "embed_prepare", fn_prepare_kernel<16>, dim3(B), dim3(256), a);
+        else launch(m, "embed_prepare", fn_prepare_kernel<32>, dim3(B), dim3(256), a);
+    }
+}
+// The same step of a model made for more than 32 rows (its packed activations are 64 or 128 rows at every batch): the
+// prefill's GEMMs (mid_gemm_f16_kernel) on row-major activations.  The kernels above read every activation fragment once per
+// column tile from L2, which outweighs the weights from two 32-row tiles on.  Still 5 launches per layer: the residual
+// projections need no split tail (the wavefronts of a block share K) and the consumers form 1 / rms themselves.
+// Measured, us per step at a context of 200, before -> now: 1B model, 33 / 64 / 96 / 128 rows 1125 / 1352 / 1914 / 2264 ->
+// 1060 / 1274 / 1362 / 1565; 8 layers of the 7B one, 40 / 128 rows 1258 / 2335 -> 1091 / 1716.  At 96 rows per layer of the 1B
+// model: QKV 9.7 -> 9.5, output 16.1 -> 8.9, up 28.7 -> 20.6, down (with a kernel that added its splits) 35.6 -> 25.
+static void decode_step_rows(TSHipGpt* m, const int* d_ids, int B) {
+    auto& c = m->c;
+    const int h = c.hidden, F = c.ffn_dim;
+    const long hp = round_up(h, 32), qp = round_up(m->Nqkv, 32), Vp = round_up(c.vocab, 32);
+    const int NTh = (int)(hp / 32);
+    float* ssq = m->ssq.as<float>();
+    // (the 256 x 256 tile neither forms 1 / rms nor fits these row counts: pick_gemm_tile offers it from 256 rows on)
+    auto gemm = [&](const char* name, const GemmW& w, const DevBuf& X, long ldx, int epi, BigArgs e) { run_big_gemm(m, name, w, X.p, ldx, B, epi, e, 1, pick_gemm_tile(w, B)); };
+    auto with_ssq = [&](BigArgs& e) { e.ssq = ssq; e.ssq_nt = NTh; e.ssq_in_ld = m->Bpad; e.inv_h = 1.0f / (float)h; e.eps = c.norm_eps; };
+    auto resid = [&](const char* name, const GemmW& w, const DevBuf& X, long ldx, const DevBuf& bias, const DevBuf& gamma) {
+        BigArgs e; std::memset(&e, 0, sizeof(e));
+        e.out = m->x.as<float>(); e.ld_out = h; e.bias = bias.as<float>(); e.n_valid = h;
+        e.xg16 = m->xn_rows.as<half_t>(); e.ld_xg = (int)m->ldh; e.gamma = gamma.as<float>(); e.ssq_out = ssq; e.ssq_ld = m->Bpad;
+        gemm(name, w, X, ldx, BEPI_RESID, e);
+    };
+    embed_prepare(m, d_ids, B);
+    for (int l = 0; l < c.n_layers; ++l) {
+        LayerW& L = *m->L[l];
+        {
+            BigArgs e; std::memset(&e, 0, sizeof(e));
+            e.out = m->part_qkv.as<float>(); e.ld_out = (int)qp; e.bias = L.bqkv.as<float>(); e.n_valid = m->Nqkv;
+            with_ssq(e);
+            gemm("gemm_qkv", L.qkv, m->xn_rows, m->ldh, BEPI_F32_BIAS, e);
+        }
+        {
+            AttnArgs a = attn_args(m, L);
+            a.qkv = m->part_qkv.as<float>(); a.KS = 1; a.split_stride = 0; a.ldq = qp;
+            a.bias = m->zero_qkv.as<float>();      // (added by the projection)
+            a.out = m->o_rows.p; a.ld_out = m->ldh;
+            launch_attn_decode(m, a, B);
+        }
+        resid("gemm_wo", L.wo, m->o_rows, m->ldh, L.bo, L.n2_g);
+        {
+            BigArgs e; std::memset(&e, 0, sizeof(e));
+            e.bias = L.b1.as<float>(); e.bias2 = L.b3.as<float>(); e.out16 = m->a_rows.as<half_t>(); e.ld16 = (int)m->ldF;
+            e.act = c.act; e.gated = m->gated; e.n_valid = F;
+            with_ssq(e);
+            gemm("gemm_ffn13", L.w13, m->xn_rows, m->ldh, BEPI_ACT16, e);
+        }
+        resid("gemm_ffn2", L.w2, m->a_rows, m->ldF, L.b2, l + 1 < c.n_layers ? m->L[l + 1]->n1_g : m->fn_g);
+    }
+    {
+        BigArgs e; std::memset(&e, 0, sizeof(e));
+        e.out = m->logits.as<float>(); e.ld_out = (int)Vp; e.bias = m->head_b.as<float>(); e.n_valid = c.vocab;
+        with_ssq(e);
+        e.advance_pos = m->d_pos.as<int>();
+        gemm("gemm_head", m->head, m->xn_rows, m->ldh, BEPI_F32_BIAS, e);
+    }
+    m->pos += 1;
 }
 static void decode_step_fn(TSHipGpt* m, const int* d_ids, int B) {
     auto& c = m->c;
@@ -862,14 +937,7 @@ static void decode_step_fn(TSHipGpt* m, const int* d_ids, int B) {
         e.xg16 = m->xn.as<half_t>(); e.xg_kt = xkt; e.ssq_out = ssq; e.ssq_out_ld = m->Bpad;
         e.ln = m->ln ? 1 : 0;      // (LayerNorm: the tails also store the tiles' plain sums)
     };
-    if (m->embed_done) {
-        m->embed_done = false;        // (the greedy sampling kernel went on to embed the tokens it chose)
-    } else {
-        FnPrepArgs a = embed_prepare_args(m, d_ids);
-        if (h <= 2048) launch(m, "embed_prepare", fn_prepare_kernel<8>, dim3(B), dim3(256), a);
-        else if (h <= 4096) launch(m, "embed_prepare", fn_prepare_kernel<16>, dim3(B), dim3(256), a);
-        else launch(m, "embed_prepare", fn_prepare_kernel<32>, dim3(B), dim3(256), a);
-    }
+    embed_prepare(m, d_ids, B);
     for (int l = 0; l < c.n_layers; ++l) {
         LayerW& L = *m->L[l];
         const long qstride = (long)m->Bpad * qp;
@@ -905,30 +973,13 @@ static void decode_step_fn(TSHipGpt* m, const int* d_ids, int B) {
             run_skinny(m, "gemm_ffn13", L.w13, m->xn.p, m->ldh, B, EPI_ACT16, e);
         }
         const float* next_gamma = l + 1 < c.n_layers ? m->L[l + 1]->n1_g.as<float>() : m->fn_g.as<float>();
-        if (L.w2.KS == 1) {
-            SkinnyArgs e; std::memset(&e, 0, sizeof(e));
-            tail(e, L.b2.as<float>(), next_gamma);
-            run_skinny(m, "gemm_ffn2", L.w2, m->a.p, m->ldF, B, EPI_RESID_TAIL, e);
-        } else if (m->BT == 1) {
+        {
             // long K: split across blocks so that every CU streams weights; the block of a column tile that finishes
             // last adds the partial sums and performs the tail
             SkinnyArgs e; std::memset(&e, 0, sizeof(e));
             tail(e, L.b2.as<float>(), next_gamma);
-            e.out = m->part_h.as<float>();       // exchange area [split][tile][1024]: 16 * Bpad * hp floats hold it for Bpad = 32
-            e.tile_count = m->tile_count.as<int>();
-            run_skinny(m, "gemm_ffn2", L.w2, m->a.p, m->ldF, B, EPI_SPLIT_TAIL, e);
-        } else {
-            // long K: split across blocks so that every CU streams weights, then a small tail kernel
-            SkinnyArgs e; std::memset(&e, 0, sizeof(e));
-            e.out = m->part_h.as<float>(); e.ld_out = (int)hp; e.split_stride = (long)m->Bpad * hp;
-            run_skinny(m, "gemm_ffn2", L.w2, m->a.p, m->ldF, B, EPI_PARTIAL, e);
-            ResidTailArgs r; std::memset(&r, 0, sizeof(r));
-            r.x = m->x.as<float>(); r.ldx = h; r.h = h; r.rows = B;
-            r.part = m->part_h.as<float>(); r.KS = L.w2.KS; r.split_stride = (long)m->Bpad * hp; r.ld_part = hp; r.bias = L.b2.as<float>();
-            r.gamma = next_gamma; r.xg16 = m->xn.as<half_t>(); r.xg_kt = xkt; r.ssq_out = ssq; r.ssq_ld = m->Bpad;
-            if (m->BT == 1) launch(m, "resid_tail", resid_tail_kernel<4>, dim3(NTh), dim3(256), r);
-            else if (m->BT == 2) launch(m, "resid_tail", resid_tail_kernel<8>, dim3(NTh), dim3(256), r);
-            else launch(m, "resid_tail", resid_tail_kernel<16>, dim3(NTh), dim3(256), r);
+            e.tile_count = m->tile_count.as<int>();      // (e.out: exchange area [split][tile][1024]; 16 * Bpad * hp floats hold it for Bpad = 32)
+            run_skinny(m, "gemm_ffn2", L.w2, m->a.p, m->ldF, B, L.w2.KS > 1 ? EPI_SPLIT_TAIL : EPI_RESID_TAIL, e);
         }
     }
     {
@@ -946,6 +997,7 @@ static void decode_step_fn(TSHipGpt* m, const int* d_ids, int B) {
 // decode step: tokens (device int32 [batch]) -> logits (device fp32 [batch][vocab])
 // ------------------------------------------------------------------------------------------------
 static void decode_step(TSHipGpt* m, const int* d_ids, int B) {
+    if (decode_by_rows(m)) { decode_step_rows(m, d_ids, B); return; }
     if (m->fused_norm) { decode_step_fn(m, d_ids, B); return; }
     auto& c = m->c;
     const int h = c.hidden, F = c.ffn_dim;
@@ -1364,6 +1416,12 @@ TSHIP_API int TSHip_GptCreate(const TSHipGptConfig* cfg, TSHipGpt** out) {
     // (LayerNorm: batches of up to 32 rows; the tails of larger batches do not store the tiles' plain sums)
     m->fused_norm = m->f16 && c.n_experts <= 1 && (c.norm_type == 0 || m->BT == 1);
     m->ln = m->fused_norm && c.norm_type == 1;
+    if (m->fused_norm && m->BT > 1) {
+        m->xn_rows.alloc((size_t)m->Bpad * m->ldh * m->esz());
+        m->o_rows.alloc((size_t)m->Bpad * m->ldh * m->esz());
+        m->a_rows.alloc((size_t)m->Bpad * m->ldF * m->esz());
+        m->zero_qkv.alloc((size_t)qp * sizeof(float));
+    }
     if (m->fused_norm) {
         m->ssq.alloc((size_t)(m->ln ? 2 : 1) * (hp / 32) * m->Bpad * sizeof(float));
         m->tile_count.alloc((size_t)(std::max<long>(hp, round_up(m->F13, 32)) / 32) * sizeof(int));     // zero-filled; every use returns it to zero

@@ -767,7 +767,10 @@ struct BigArgs {
     // deferred RMSNorm (LDS-tiled kernels only).  Consumers: X holds half(gamma * x) and every output row is scaled by
     // rinv[row] before the bias.  Producers (BEPI_RESID): besides the residual stream, store half(gamma * x) row-major
     // into xg16 and the sum of squares of every (32-column tile, row) into ssq_out[tile * ssq_ld + row].
+    // (mid_gemm_f16_kernel: with ssq instead of rinv it forms them itself from the ssq_nt tile sums [tile][ssq_in_ld rows])
     const float* rinv;
+    const float* ssq; int ssq_nt; long ssq_in_ld; float inv_h, eps;
+    int* advance_pos;      // mid_gemm_f16_kernel, optional: one thread of the launch increments this pair of device counters
     half_t* xg16; int ld_xg; const float* gamma; float* ssq_out; long ssq_ld;
     // QKV projection of a prefill (BEPI_F32_BIAS, LDS-tiled kernel) writing the cache itself: columns from kv_col0 on are
     // kv_gd key columns, then kv_gd value columns (head size kv_D, both counts multiples of 128); row r is position
@@ -1537,6 +1540,7 @@ template <int WR, int NJ> struct MidShape {
 template <int EPI, int WR, int NJ>
 __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     extern __shared__ __attribute__((aligned(16))) half_t big_smem[];
+    __shared__ float ssq_part[512];                     // [512 / (64 WR)][64 WR rows]: shares of the rows' sums of squares
     using S = MidShape<WR, NJ>;
     constexpr int KG = S::KG, NST = S::NST, PF = NST - 1, STAGE = S::STAGE, LW = NJ * KG / 8, PPR = 2 * KG, LPC = LW + 2;      // LPC: loads per wavefront and chunk
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1592,6 +1596,15 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     issue(0);
     if (NC > 1) issue(1);
     if (PF > 2 && NC > 2) issue(2);
+    if (a.ssq) {      // (behind the first requests: waiting for these sums then costs no round trip of its own)
+        const int rl = t & (64 * WR - 1), seg = t / (64 * WR);
+        const float* src = a.ssq + min(row0 + rl, (long)a.R - 1);
+        float s = 0.0f;
+#pragma unroll 8
+        for (int i = seg; i < a.ssq_nt; i += 8 / WR) s += src[i * a.ssq_in_ld];
+        ssq_part[t] = s;
+    }
+    if (a.advance_pos && blockIdx.x == 0 && t == 0) { a.advance_pos[0] += 1; a.advance_pos[1] += 1; }
     half8 wf[NJ], xf[2];
     auto wait_loads = [&](int c) {          // this wavefront's part of chunk c + 1 has landed
         const int later = max(0, min(PF - 1, NC - 2 - c));
@@ -1666,6 +1679,13 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
         for (int q = 0; q < 4 / WPU; ++q) {
             const long row = min(row0 + 64 * wr + 32 * (u & 1) + 8 * (my_part * (4 / WPU) + q) + rr, (long)a.R - 1);
             rv[q] = a.rinv ? a.rinv[row] : 1.0f;
+            if (a.ssq) {
+                const float* part = ssq_part + 64 * wr + 32 * (u & 1) + 8 * (my_part * (4 / WPU) + q) + rr;
+                float ss = part[0];
+#pragma unroll
+                for (int g = 1; g < 8 / WR; ++g) ss += part[g * 64 * WR];
+                rv[q] = 1.0f / sqrtf(ss * a.inv_h + a.eps);
+            }
             if (EPI == BEPI_RESID) {
                 const float* src = a.out + row * a.ld_out;
                 if (vec) old[q] = *(const floatx4*)(src + c0);
@@ -2176,50 +2196,6 @@ __global__ __launch_bounds__(256) void resid_norm_kernel(ResidNormArgs a) {
                 if (a.xn_kt > 0) ((AT*)a.xn)[xpack_index(r, c, a.xn_kt)] = (AT)y; else out[c] = (AT)y;
             }
         }
-    }
-}
-
-// Residual tail for a split-K projection on the deferred-norm path: one block per 32-column tile.
-// x[:, tile] += sum of the split-K partials (in split order) + bias; stores x, the next GEMM's packed input
-// half(gamma * x) and the tile's per-row sum of squares.  All loads of a thread are issued before the first use.
-struct ResidTailArgs {
-    float* x; long ldx; int h; int rows;
-    const float* part; int KS; long split_stride; long ld_part; const float* bias;
-    const float* gamma; half_t* xg16; int xg_kt; float* ssq_out; int ssq_ld;
-};
-template <int RPT>      // rows per thread: 256 threads cover 8 rows x 32 columns per pass
-__global__ __launch_bounds__(256) void resid_tail_kernel(ResidTailArgs a) {
-    const int nt = blockIdx.x, t = threadIdx.x, n = t & 31, b0 = t >> 5;
-    const int col = nt * 32 + n;
-    const bool okc = col < a.h;
-    float p[RPT][8], xv[RPT];
-    const float bias = okc ? a.bias[col] : 0.0f, gm = okc ? a.gamma[col] : 0.0f;
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-        const int b = b0 + 8 * i;
-        const bool ok = okc && b < a.rows;
-        xv[i] = ok ? a.x[(long)b * a.ldx + col] : 0.0f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) p[i][k] = (ok && k < a.KS) ? a.part[k * a.split_stride + (long)b * a.ld_part + col] : 0.0f;
-    }
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-        const int b = b0 + 8 * i;
-        if (b >= a.rows) continue;                       // uniform over the 32 lanes that share a row
-        float s = p[i][0];
-#pragma unroll
-        for (int k = 1; k < 8; ++k) if (k < a.KS) s += p[i][k];
-        for (int k = 8; k < a.KS; ++k) s += a.part[k * a.split_stride + (long)b * a.ld_part + col];
-        float v = 0.0f;
-        if (okc) {
-            v = (s + bias) + xv[i];
-            a.x[(long)b * a.ldx + col] = v;
-            a.xg16[xpack_index(b, col, a.xg_kt)] = (half_t)(gm * v);
-        }
-        float q = v * v;
-#pragma unroll
-        for (int o = 16; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
-        if (n == 0) a.ssq_out[(long)nt * a.ssq_ld + b] = q;
     }
 }
 
