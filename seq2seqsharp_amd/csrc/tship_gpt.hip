@@ -142,6 +142,11 @@ struct TSHipGpt {
     bool embed_done = false;       // the sampling kernel of this step has already done the next step's embedding (greedy_embed_kernel)
     DevBuf blocked;                // one byte per token, non-zero = DecodingOptions.BlockedTokens (allocated with the model: graphs keep its address)
     int cur_batch = 0;
+    // which prompt a cache row holds: rows of equal entries are equal in the first prompt_pos positions (rows that a beam
+    // search made from one prompt).  fresh_rows() after every other write of whole rows
+    std::vector<int> row_prompt; int prompt_pos = 0;
+    void fresh_rows() { row_prompt.resize(c.max_batch); for (int i = 0; i < c.max_batch; ++i) row_prompt[i] = i; prompt_pos = pos; }
+    DevBuf cache_table;            // addresses of every layer's key and value cache
     std::vector<std::string> last_symbols;      // launched symbols of the last profiled step, in launch order
     DevBuf beam_probs, beam_ids, beam_out, beam_uni, reorder_tmp, reorder_src;      // beam search: probabilities the picks consume, picks, gather temporaries
     Profiler* prof = nullptr;
@@ -1303,6 +1308,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         run_gemm_f32(m, "gemm_head", m->head, m->xn.as<float>(), m->ldh, B, m->logits.as<float>(), Vp, 0, 1, m->head_b.as<float>());
     }
     m->pos = pos0 + Tp;
+    m->fresh_rows();
     TSHIP_CHECK_HIP(hipMemcpyAsync(m->d_pos.p, &m->pos, sizeof(int), hipMemcpyHostToDevice, stream()));
     TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
     m->cur_batch = B;
@@ -1371,6 +1377,14 @@ TSHIP_API int TSHip_GptCreate(const TSHipGptConfig* cfg, TSHipGpt** out) {
         if (L.moe) for (int e = 0; e < c.n_experts; ++e) { L.e1.emplace_back(new GemmW()); L.e2.emplace_back(new GemmW()); }
         size_t cache_bytes = (size_t)c.max_batch * c.n_kv_heads * m->ML * m->D * m->esz();
         L.kc.alloc(cache_bytes); L.vc.alloc(cache_bytes);
+    }
+    {
+        std::vector<char*> at;
+        for (auto& L : m->L) { at.push_back((char*)L->kc.p); at.push_back((char*)L->vc.p); }
+        m->cache_table.alloc(at.size() * sizeof(char*));
+        TSHIP_CHECK_HIP(hipMemcpyAsync(m->cache_table.p, at.data(), at.size() * sizeof(char*), hipMemcpyHostToDevice, stream()));
+        TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
+        m->fresh_rows();
     }
     build_expected(m.get());
     // rotary table, computed exactly as the reference's expression (TensorApplyCPU.cs:1161-1164):
@@ -1510,7 +1524,7 @@ TSHIP_API int TSHip_GptFinalize(TSHipGpt* m) {
 TSHIP_API int TSHip_GptReset(TSHipGpt* m) {
     TSHIP_BEGIN
     TSHIP_REQUIRE(m, "TSHip_GptReset: null model");
-    m->pos = 0; m->cur_batch = 0;
+    m->pos = 0; m->cur_batch = 0; m->fresh_rows();
     TSHIP_CHECK_HIP(hipMemsetAsync(m->d_pos.p, 0, sizeof(int), stream()));
     if (m->tile_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->tile_count.p, 0, m->tile_count.bytes, stream()));
     if (m->last_pos.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->last_pos.p, 0xff, m->last_pos.bytes, stream()));      // -1: no token seen
@@ -1775,22 +1789,44 @@ TSHIP_API int TSHip_GptReorderRows(TSHipGpt* m, const int32_t* host_src_rows, in
         identity = identity && host_src_rows[i] == i;
     }
     if (!identity) {
-        m->reorder_src.reserve((size_t)m->c.max_batch * sizeof(int));
-        TSHIP_CHECK_HIP(hipMemcpyAsync(m->reorder_src.p, host_src_rows, (size_t)new_batch * sizeof(int), hipMemcpyHostToDevice, stream()));
-        TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));       // (the caller's array may go away)
         // cache rows: [batch][kv head][ML * D] elements; the first round_up(pos, 32) positions of every head are live
         // (fragment-major caches keep positions in chunks of 32)
-        const long head_bytes = (long)m->ML * m->D * (long)m->esz(), row_bytes = head_bytes * m->c.n_kv_heads;
-        const long used = std::min<long>(head_bytes, round_up(std::max(m->pos, 1), 32) * (long)m->D * (long)m->esz());
-        m->reorder_tmp.reserve((size_t)std::max<long>(row_bytes, m->last_pos.p ? m->last_ld * (long)sizeof(int) : 0) * m->c.max_batch);
-        const int* src = m->reorder_src.as<int>();
-        auto gather = [&](void* table, long stride, long chunk, long live, long pieces) {
-            launch(m, "rows_gather", rows_gather_kernel, dim3((unsigned)pieces, (unsigned)new_batch), dim3(256), (const char*)table, stride, chunk, live, src, m->reorder_tmp.as<char>(), 1);
-            launch(m, "rows_gather", rows_gather_kernel, dim3((unsigned)pieces, (unsigned)new_batch), dim3(256), (const char*)table, stride, chunk, live, src, m->reorder_tmp.as<char>(), 0);
-        };
-        for (auto& L : m->L) { gather(L->kc.p, row_bytes, head_bytes, used, m->c.n_kv_heads); gather(L->vc.p, row_bytes, head_bytes, used, m->c.n_kv_heads); }
-        if (m->last_pos.p) gather(m->last_pos.p, m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), 1);
-        TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
+        const long pos_bytes = (long)m->D * (long)m->esz(), head_bytes = m->ML * pos_bytes, row_bytes = head_bytes * m->c.n_kv_heads;
+        const long used = std::min<long>(head_bytes, round_up(std::max(m->pos, 1), 32) * pos_bytes);
+        const bool in_place = new_batch <= 16;       // (16 rows of 16 bytes fill 64 registers)
+        if (in_place) {
+            // rows of one prompt are equal up to its length: unless a row takes another prompt's place (or a new one), only
+            // what was decoded behind the prompts moves
+            bool same_prompt = true;
+            for (int i = 0; i < new_batch; ++i) same_prompt = same_prompt && i < m->cur_batch && m->row_prompt[i] == m->row_prompt[host_src_rows[i]];
+            RowsMoveArgs a; std::memset(&a, 0, sizeof(a));
+            a.caches = (char* const*)m->cache_table.p; a.row_stride = row_bytes; a.chunk = head_bytes; a.used = used; a.n = new_batch;
+            a.from = same_prompt ? std::min(m->pos, m->prompt_pos) / 32 * 32 * pos_bytes : 0;
+            for (int i = 0; i < new_batch; ++i) a.src[i] = host_src_rows[i];
+            const dim3 grid((unsigned)ceil_div(used - a.from, 4096), m->c.n_kv_heads, 2 * m->c.n_layers);
+            if (used > a.from) {
+                if (new_batch <= 4) launch(m, "rows_move", rows_move_kernel<4>, grid, dim3(256), a);
+                else if (new_batch <= 8) launch(m, "rows_move", rows_move_kernel<8>, grid, dim3(256), a);
+                else launch(m, "rows_move", rows_move_kernel<16>, grid, dim3(256), a);
+            }
+        }
+        if (!in_place || m->last_pos.p) {
+            m->reorder_src.reserve((size_t)m->c.max_batch * sizeof(int));
+            TSHIP_CHECK_HIP(hipMemcpyAsync(m->reorder_src.p, host_src_rows, (size_t)new_batch * sizeof(int), hipMemcpyHostToDevice, stream()));
+            TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));       // (the caller's array may go away)
+            m->reorder_tmp.reserve((size_t)std::max<long>(in_place ? 0 : row_bytes, m->last_pos.p ? m->last_ld * (long)sizeof(int) : 0) * m->c.max_batch);
+            const int* src = m->reorder_src.as<int>();
+            auto gather = [&](void* table, long stride, long chunk, long live, long pieces) {
+                launch(m, "rows_gather", rows_gather_kernel, dim3((unsigned)pieces, (unsigned)new_batch), dim3(256), (const char*)table, stride, chunk, live, src, m->reorder_tmp.as<char>(), 1);
+                launch(m, "rows_gather", rows_gather_kernel, dim3((unsigned)pieces, (unsigned)new_batch), dim3(256), (const char*)table, stride, chunk, live, src, m->reorder_tmp.as<char>(), 0);
+            };
+            if (!in_place) for (auto& L : m->L) { gather(L->kc.p, row_bytes, head_bytes, used, m->c.n_kv_heads); gather(L->vc.p, row_bytes, head_bytes, used, m->c.n_kv_heads); }
+            if (m->last_pos.p) gather(m->last_pos.p, m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), 1);
+            TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
+        }
+        std::vector<int> prompts(m->c.max_batch, -1);
+        for (int i = 0; i < new_batch; ++i) prompts[i] = m->row_prompt[host_src_rows[i]];
+        m->row_prompt = prompts;
     }
     m->cur_batch = new_batch;
     TSHIP_END
@@ -1894,7 +1930,7 @@ TSHIP_API int TSHip_GptSetSeqLen(TSHipGpt* m, int batch, int len) {
     TSHIP_BEGIN
     TSHIP_REQUIRE(m, "TSHip_GptSetSeqLen: null model");
     TSHIP_REQUIRE(batch >= 1 && batch <= m->c.max_batch && len >= 0 && len < m->c.max_seq_len, "TSHip_GptSetSeqLen: out of range");
-    m->pos = len; m->cur_batch = batch;
+    m->pos = len; m->cur_batch = batch; m->fresh_rows();
     TSHIP_CHECK_HIP(hipMemcpyAsync(m->d_pos.p, &m->pos, sizeof(int), hipMemcpyHostToDevice, stream()));
     TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
     TSHIP_END
@@ -1907,6 +1943,7 @@ TSHIP_API int TSHip_GptSetKV(TSHipGpt* m, int layer, int which, const float* hos
     TSHIP_REQUIRE(batch >= 1 && batch <= m->c.max_batch && len >= 0 && len <= m->c.max_seq_len, "TSHip_GptSetKV: out of range");
     const int G = m->c.n_kv_heads, D = m->D; const long ML = m->ML;
     char* base = (char*)(which ? m->L[layer]->vc.p : m->L[layer]->kc.p);
+    m->fresh_rows();
     const bool frag = m->vt;
     std::vector<char> tmp((size_t)ML * D * m->esz(), 0);
     for (int b = 0; b < batch; ++b) for (int g = 0; g < G; ++g) {
@@ -1984,7 +2021,7 @@ TSHIP_API int TSHip_GptRestoreRows(TSHipGpt* m, const TSHipGptSnapshot* sn) {
     }
     TSHIP_CHECK_HIP(hipMemcpyAsync(m->logits.p, sn->logits.p, sn->logits.bytes, hipMemcpyDeviceToDevice, stream()));
     if (m->last_pos.p) TSHIP_CHECK_HIP(hipMemcpyAsync(m->last_pos.p, sn->last_pos.p, (size_t)B * m->last_ld * sizeof(int), hipMemcpyDeviceToDevice, stream()));
-    m->pos = sn->len; m->cur_batch = B; m->embed_done = false;
+    m->pos = sn->len; m->cur_batch = B; m->embed_done = false; m->fresh_rows();
     TSHIP_CHECK_HIP(hipMemcpyAsync(m->d_pos.p, &m->pos, sizeof(int), hipMemcpyHostToDevice, stream()));
     TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
     TSHIP_END

@@ -1,4 +1,5 @@
-"""Decode steps of models made for more than 32 rows (row-major GEMM tiles), at the edges of their ranges."""
+"""Decode steps of models made for more than 32 rows (row-major GEMM tiles) and the in-place move of cache rows, at the edges
+of their ranges."""
 import numpy as np
 import pytest
 
@@ -50,3 +51,38 @@ def _steps(G, oracle, cfg, max_batch):
 def test_rows(G, oracle, shape, max_batch, batch):
     hidden, heads, kv, ffn, act = shape
     _steps(G, oracle, _cfg(hidden, heads, kv, ffn, synth.RMSNORM, act, batch, "f16"), max_batch)
+
+
+@pytest.mark.parametrize("dtype,hidden,heads", [("f32", 64, 4), ("f16", 64, 4), ("f16", 128, 2)])
+def test_reorder_rows(G, dtype, hidden, heads):
+    """Rows of shared prompts, of mixed ones and after a rewind, 1 ... 20 rows: the caches are the gathered ones."""
+    cfg = _cfg(hidden, heads, heads, 96, synth.RMSNORM, synth.RELU, 2, dtype, prompt=37)
+    w = synth.make_weights(cfg, 71, random_bias=True)
+    seqs = synth.make_prompts(cfg, 72)
+    gpu = G.HipGpt(cfg, w, max_batch=20, max_seq_len=64)
+    rng = np.random.default_rng(73)
+
+    def kv():
+        return [gpu.get_kv(l, i) for l in range(3) for i in range(2)]
+
+    def move(src):
+        before = kv()
+        gpu.reorder_rows(np.array(src, np.int32))
+        gpu.decode(rng.integers(4, 157, size=len(src)).astype(np.int32))
+        for a, b in zip(before, kv()):
+            assert np.array_equal(a[np.array(src)], b[:, :, :a.shape[2]]), src
+
+    gpu.prefill(seqs)
+    move([0, 1, 0, 1, 0, 1, 0, 1])                       # two prompts, four hypotheses each
+    move([2, 1, 0, 3, 2, 7, 0, 5])                       # inside the prompts: only what was decoded moves
+    move([3, 1, 0, 3, 2, 7, 0, 5])                       # a row takes the other prompt's place
+    move([7, 0])                                         # fewer rows
+    move([1, 0, 1, 1, 0, 0, 1, 0, 1, 1, 0, 0])
+    move(list(rng.integers(0, 12, size=16)))
+    move(list(rng.integers(0, 16, size=20)))             # more than the in-place kernel takes
+    gpu.set_seq_len(20, 20)                              # back into the prompt, then on with different tokens
+    gpu.decode(rng.integers(4, 157, size=20).astype(np.int32))
+    move(list(rng.integers(0, 20, size=7)))
+    gpu.prefill(rng.integers(4, 157, size=(7, 9)).astype(np.int32))
+    move([6, 5, 4, 3, 2, 1, 0])
+    gpu.close()
