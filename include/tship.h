@@ -276,7 +276,7 @@ TSHIP_API int TSHip_GptStepBytes(TSHipGpt* m, int batch, double* weight_bytes, d
  *   TSHIP_ATTN_SPLITS=n       decode attention: n blocks per (sequence, KV head) pair (default: chosen from the batch and context)
  *   TSHIP_FFN_TILES=10|15|20|30|40   decode FFN up projection: column tiles per block x 10 (15 = a tile and a half)
  *   TSHIP_GEMM_TILE=0|11|12|14|22|24   prefill GEMMs: tile of mid_gemm_f16_kernel (10 x 64-row groups + 32-column tiles), 0 = the
- *                             256 x 256 tile from 256 rows on (default: by estimated time)
+ *                             256 x 256 tile from 256 rows on; + 200 ... 400: so many blocks share a tile's K (default: by estimated time)
  *   TSHIP_F32_TILE=11|21|22|42    fp32 GEMMs from 33 rows on: tile in units of 32 rows (10 x) and 32 columns (default: by size)
  *   TSHIP_PATCH_ROWS=1|2|4|8  prefill GEMM: row tiles per tile patch of an XCD
  *   TSHIP_ATTN_NQ=1|2         prefill attention: groups of 16 MFMA columns per wavefront

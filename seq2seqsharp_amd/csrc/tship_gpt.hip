@@ -123,6 +123,9 @@ struct TSHipGpt {
     DevBuf moe_ws, topp_scratch, topp_uni, gen_buf, uni_buf, tile_count;
     DevBuf pw_lens, pw_ids, pw_x, pw_xn, pw_qkv, pw_o, pw_a, pw_f, pw_rowmap, pw_ssq, pw_rinv, pw_zero_bias, pw_moe;     // prefill workspace
     DevBuf xn_rows, o_rows, a_rows, zero_qkv; // row-major activations of decode steps of more than 32 rows (xn, o and a hold packed ones)
+    // prefill GEMMs whose tiles' K several blocks share: partial sums of up to 256 tiles x splits of 128 x 128, a counter per tile
+    static constexpr long MID_XCHG_TILES = 256;
+    DevBuf mid_xchg, mid_count;
     DevBuf ssq;                    // deferred-norm path: per-column-tile sums of squares [h/32][Bpad]
     bool fused_norm = false;       // fp16 + dense layers (RMSNorm; LayerNorm up to 32 rows): residual/norm folded into the GEMM tails
     bool ln = false;               // that path with LayerNorm: tile sums of x beside the sums of squares, folded constants per consumer
@@ -196,7 +199,9 @@ static void refresh_test_hooks() {
     if (const char* v = std::getenv("TSHIP_ATTN_NQ")) { h.attn_nq = std::atoi(v); TSHIP_REQUIRE(h.attn_nq == 1 || h.attn_nq == 2, "TSHIP_ATTN_NQ: 1 or 2"); }
     if (const char* v = std::getenv("TSHIP_GEMM_TILE")) {
         h.gemm_tile = std::atoi(v);
-        TSHIP_REQUIRE(h.gemm_tile == 0 || h.gemm_tile == 11 || h.gemm_tile == 12 || h.gemm_tile == 14 || h.gemm_tile == 22 || h.gemm_tile == 24, "TSHIP_GEMM_TILE: 0, 11, 12, 14, 22 or 24");
+        const int tile = h.gemm_tile % 100, splits = h.gemm_tile / 100;
+        TSHIP_REQUIRE((h.gemm_tile == 0 || tile == 11 || tile == 12 || tile == 14 || tile == 22 || tile == 24) && splits >= 0 && splits <= MID_SPLITS,
+                      "TSHIP_GEMM_TILE: 0, 11, 12, 14, 22 or 24, plus 100 x the blocks (2 to 4) that share a tile's K");
     }
     if (const char* v = std::getenv("TSHIP_F32_TILE")) {
         h.f32_tile = std::atoi(v);
@@ -566,28 +571,52 @@ static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const fl
 // (L2, HBM, power).  a and b are fits to launches of 37 ... 16384 rows at seven (K, N) of 768 ... 22016: the choice costs
 // 0.3 % over the best tile on average of those 105 launches, and more than 8 % in one (21 us for 17).
 // own_cache_write: us that a launch saves with the 256 x 256 tile, which can write the key-value cache itself.
+// A launch that leaves half of the units idle may have up to four blocks share the K of a tile (100 x their number in the
+// result); the exchange of their sums costs about 2 us and 0.3 us per block.
+// (5632 x 2048: 37 rows 18 -> 10 us with four blocks, 96 rows 25 -> 15; a decode step of 33 / 64 / 96 rows of the 1B model
+// 1060 / 1274 / 1362 -> 962 / 1110 / 1336 us.)
+// the most blocks up to `splits` that leave none of their ranges of whole chunks empty
+static int mid_splits(const GemmW& w, int tile, int splits) {
+    const int kg = tile >= 20 ? 4 : 8;
+    while (splits > 1 && (splits - 1) * (int)ceil_div(w.KT, kg * splits) * kg >= w.KT) --splits;
+    return splits;
+}
 static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) {
     struct Cost { int tile, rows, cols; float a, b; };
     static const Cost costs[] = {{11, 64, 1, 1.9f, 0.045f}, {12, 64, 2, 2.8f, 0.050f}, {14, 64, 4, 3.0f, 0.093f},
                                  {22, 128, 2, 3.4f, 0.078f}, {24, 128, 4, 4.8f, 0.115f}, {0, 256, 8, 8.0f, 0.320f}};
     const int forced = g_hooks.gemm_tile;
-    if (forced > 0 || (forced == 0 && R >= 256)) return forced;
+    if (forced == 0 && R >= 256) return 0;
+    if (forced > 0) {
+        const Cost& c = *std::find_if(std::begin(costs), std::end(costs), [&](const Cost& k) { return k.tile == forced % 100; });
+        const bool fits = ceil_div(R, c.rows) * ceil_div(w.NT, c.cols) * (forced / 100) <= TSHipGpt::MID_XCHG_TILES;
+        return forced % 100 + 100 * (forced >= 200 && fits ? mid_splits(w, forced % 100, forced / 100) : 1);
+    }
     const float ncu = (float)std::max(1, n_compute_units());
-    int best = 11; float best_us = 1e30f;
+    int best = 111; float best_us = 1e30f;
     for (const Cost& c : costs) {
         if (c.tile == 0 && R < 256) continue;
-        const float tiles = (float)(ceil_div(R, c.rows) * ceil_div(w.NT, c.cols)), rounds = std::ceil(tiles / ncu);
-        float us = rounds * (c.a + c.b * (float)w.KT) * (1.0f + 0.4f * tiles / (rounds * ncu));
-        if (c.tile == 0) us -= own_cache_write;
-        if (us < best_us) { best_us = us; best = c.tile; }
+        const long n_tiles = ceil_div(R, c.rows) * ceil_div(w.NT, c.cols);
+        for (int want = 1; want <= (c.tile ? MID_SPLITS : 1); ++want) {
+            const int splits = mid_splits(w, c.tile, want);
+            if (splits != want || (splits > 1 && (n_tiles * splits > TSHipGpt::MID_XCHG_TILES || n_tiles * splits > (long)ncu))) continue;
+            const float tiles = (float)(n_tiles * splits), rounds = std::ceil(tiles / ncu);
+            float us = rounds * (c.a + c.b * (float)ceil_div(w.KT, splits)) * (1.0f + 0.4f * tiles / (rounds * ncu));
+            if (splits > 1) us += 2.0f + 0.3f * (float)splits;
+            if (c.tile == 0) us -= own_cache_write;
+            if (us < best_us) { best_us = us; best = c.tile ? c.tile + 100 * splits : 0; }
+        }
     }
     return best;
 }
-static void run_mid_gemm(TSHipGpt* m, const char* name, const BigArgs& e, int epi, int mid) {
+static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int mid) {
+    e.splits = mid / 100; mid %= 100;
+    e.xchg = m->mid_xchg.as<float>(); e.tile_count = m->mid_count.as<int>();
     auto go = [&](auto WRc, auto NJc) {
         constexpr int WR = decltype(WRc)::value, NJ = decltype(NJc)::value;
         const long tiles = ceil_div(e.NT, NJ) * ceil_div(e.R, 64 * WR);
-        const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8));
+        TSHIP_REQUIRE(e.splits >= 1 && (e.splits == 1 || tiles * e.splits <= TSHipGpt::MID_XCHG_TILES), "internal: split-K exchange area too small");
+        const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8), (unsigned)e.splits);
         const unsigned shm = MidShape<WR, NJ>::SHM;
         if (epi == BEPI_F32_BIAS) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_F32_BIAS, WR, NJ>, grid, dim3(512), shm, e);
         else if (epi == BEPI_RESID) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_RESID, WR, NJ>, grid, dim3(512), shm, e);
@@ -1430,6 +1459,10 @@ TSHIP_API int TSHip_GptCreate(const TSHipGptConfig* cfg, TSHipGpt** out) {
     // (LayerNorm: batches of up to 32 rows; the tails of larger batches do not store the tiles' plain sums)
     m->fused_norm = m->f16 && c.n_experts <= 1 && (c.norm_type == 0 || m->BT == 1);
     m->ln = m->fused_norm && c.norm_type == 1;
+    if (m->f16) {
+        m->mid_xchg.alloc((size_t)TSHipGpt::MID_XCHG_TILES * 128 * 128 * sizeof(float));
+        m->mid_count.alloc((size_t)TSHipGpt::MID_XCHG_TILES * sizeof(int));      // zero-filled; every use returns it to zero
+    }
     if (m->fused_norm && m->BT > 1) {
         m->xn_rows.alloc((size_t)m->Bpad * m->ldh * m->esz());
         m->o_rows.alloc((size_t)m->Bpad * m->ldh * m->esz());
@@ -1527,6 +1560,7 @@ TSHIP_API int TSHip_GptReset(TSHipGpt* m) {
     m->pos = 0; m->cur_batch = 0; m->fresh_rows();
     TSHIP_CHECK_HIP(hipMemsetAsync(m->d_pos.p, 0, sizeof(int), stream()));
     if (m->tile_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->tile_count.p, 0, m->tile_count.bytes, stream()));
+    if (m->mid_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->mid_count.p, 0, m->mid_count.bytes, stream()));
     if (m->last_pos.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->last_pos.p, 0xff, m->last_pos.bytes, stream()));      // -1: no token seen
     if (m->attn_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->attn_count.p, 0, m->attn_count.bytes, stream()));
     if (m->moe_ws.p) TSHIP_CHECK_HIP(hipMemsetAsync((char*)m->moe_ws.p + moe_layout(m, m->Bpad).counts, 0, (size_t)m->c.n_experts * sizeof(int), stream()));

@@ -770,6 +770,7 @@ struct BigArgs {
     // (mid_gemm_f16_kernel: with ssq instead of rinv it forms them itself from the ssq_nt tile sums [tile][ssq_in_ld rows])
     const float* rinv;
     const float* ssq; int ssq_nt; long ssq_in_ld; float inv_h, eps;
+    int splits; float* xchg; int* tile_count;      // mid_gemm_f16_kernel: blocks that share a tile's K (0 or 1: one), their exchange area and counters
     int* advance_pos;      // mid_gemm_f16_kernel, optional: one thread of the launch increments this pair of device counters
     half_t* xg16; int ld_xg; const float* gamma; float* ssq_out; long ssq_ld;
     // QKV projection of a prefill (BEPI_F32_BIAS, LDS-tiled kernel) writing the cache itself: columns from kv_col0 on are
@@ -1530,6 +1531,7 @@ __device__ __forceinline__ void mid_wait_frags(half8 (&wf)[NJ], half8 (&xf)[2]) 
     else if constexpr (NJ == 2) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wf[0]), "+v"(wf[1]), "+v"(xf[0]), "+v"(xf[1])::"memory");
     else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wf[0]), "+v"(xf[0]), "+v"(xf[1])::"memory");
 }
+constexpr int MID_SPLITS = 4;        // at most so many blocks share the K of a tile
 // stages and LDS bytes of a launch
 template <int WR, int NJ> struct MidShape {
     static constexpr int KG = 8 / WR, STAGE = KG * (NJ + 2 * WR) * 1024, NST = STAGE > 40960 ? 3 : 4;
@@ -1550,6 +1552,9 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     const int CT = (a.NT + NJ - 1) / NJ, RT = (a.R + 64 * WR - 1) / (64 * WR), n_tiles = CT * RT;
     const int per_xcd = (n_tiles + 7) >> 3, seq = blockIdx.x >> 3, tile = (int)(blockIdx.x & 7) * per_xcd + seq;
     if (seq >= per_xcd || tile >= n_tiles) return;
+    // k-tiles of this block: all, or (a.splits > 1) one of as many ranges of whole chunks, blockIdx.y
+    const int kt_per = a.splits > 1 ? ((a.KT + KG * a.splits - 1) / (KG * a.splits)) * KG : a.KT;
+    const int kt_first = a.splits > 1 ? (int)blockIdx.y * kt_per : 0, kt_end = min(a.KT, kt_first + kt_per);      // (the host leaves no range empty)
     const int nt0 = (tile / RT) * NJ;
     const long row0 = (long)(tile % RT) * (64 * WR);
     floatx16 acc[NJ][2];
@@ -1583,12 +1588,12 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
         char* st = (char*)big_smem + (c % NST) * STAGE;
 #pragma unroll
         for (int i = 0; i < LW; ++i)
-            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (long)min(c * KG + wkt[i], a.KT - 1) * 512), (lptr_t)(st + (i * 8 + w) * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (long)min(kt_first + c * KG + wkt[i], kt_end - 1) * 512), (lptr_t)(st + (i * 8 + w) * 1024), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (long)min(c * KG + xkt[i], a.KT - 1) * 16), (lptr_t)(st + NJ * KG * 1024 + (i * 8 + w) * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (long)min(kt_first + c * KG + xkt[i], kt_end - 1) * 16), (lptr_t)(st + NJ * KG * 1024 + (i * 8 + w) * 1024), 16, 0, 0);
     };
-    const int NC = (a.KT + KG - 1) / KG;
+    const int NC = (kt_end - kt_first + KG - 1) / KG;
     const unsigned lds0 = (unsigned)(size_t)(lptr_t)big_smem;
     const int xr = 64 * wr + (lane & 31);
     const unsigned woff = (unsigned)(kg * 1024 + lane * 16);
@@ -1604,7 +1609,7 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
         for (int i = seg; i < a.ssq_nt; i += 8 / WR) s += src[i * a.ssq_in_ld];
         ssq_part[t] = s;
     }
-    if (a.advance_pos && blockIdx.x == 0 && t == 0) { a.advance_pos[0] += 1; a.advance_pos[1] += 1; }
+    if (a.advance_pos && blockIdx.x == 0 && blockIdx.y == 0 && t == 0) { a.advance_pos[0] += 1; a.advance_pos[1] += 1; }
     half8 wf[NJ], xf[2];
     auto wait_loads = [&](int c) {          // this wavefront's part of chunk c + 1 has landed
         const int later = max(0, min(PF - 1, NC - 2 - c));
@@ -1622,7 +1627,7 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     };
     auto M = [&](int c) {
         __builtin_amdgcn_sched_barrier(0);
-        if (c * KG + kg < a.KT) {           // (wavefront-uniform: the last chunk may hold fewer than KG k-tiles)
+        if (kt_first + c * KG + kg < kt_end) {           // (wavefront-uniform: the last chunk may hold fewer than KG k-tiles)
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
@@ -1660,8 +1665,15 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     const int lh = lane >> 5, piece = lane & 7, rr = lane >> 3;
     const int my_unit = kg / WPU, my_part = kg % WPU;
     const bool ld_ok = (EPI == BEPI_ACT16 ? a.ld16 : a.ld_out) % 4 == 0 && (EPI != BEPI_RESID || !a.xg16 || a.ld_xg % 4 == 0);
-#pragma unroll
-    for (int ph = 0; ph < 2 * NJ / UP; ++ph) {
+    // A split tile's blocks leave their sums in the exchange area [split][tile][4-float piece][thread]; the one that arrives
+    // last adds them in split order and finishes the tile (publication protocol of the split tail of the decode projections:
+    // write-through atomic stores, vmcnt(0), block barrier, atomic add, atomic loads; nobody waits for another block).
+    constexpr int NPH = 2 * NJ / UP, NPQ = 4 / WPU;
+    static_assert(NPH <= 2, "two phases at most");
+    auto phase = [&](auto ph_c, auto merge_c) __attribute__((always_inline)) {
+        constexpr int ph = decltype(ph_c)::value;
+        constexpr bool merge = decltype(merge_c)::value;
+        auto xat = [&](int k, int q) { return a.xchg + ((((long)k * n_tiles + tile) * NPH + ph) * NPQ + q) * 2048 + t; };
         const int u = ph * UP + my_unit, nt = nt0 + (u >> 1);
         const bool gated = EPI == BEPI_ACT16 && a.gated;
         const int c0 = gated ? nt * 16 + 4 * (piece & 3) : nt * 32 + 4 * piece;      // first of this lane's four outputs (gated: of both factors)
@@ -1695,26 +1707,50 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
                 }
             }
         }
-        if (ph) __syncthreads();
+        if constexpr (!merge) {
+            if (ph) __syncthreads();
 #pragma unroll
-        for (int uu = 0; uu < UP; ++uu) {
-            const int j = (ph * UP + uu) >> 1, i = (ph * UP + uu) & 1;
-            float* dst = red + ((wr * UP + uu) * KG + kg) * (32 * LDSROW) + (lane & 31) * LDSROW + 4 * lh;
+            for (int uu = 0; uu < UP; ++uu) {
+                const int j = (ph * UP + uu) >> 1, i = (ph * UP + uu) & 1;
+                float* dst = red + ((wr * UP + uu) * KG + kg) * (32 * LDSROW) + (lane & 31) * LDSROW + 4 * lh;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) *(floatx4*)(dst + 8 * g) = floatx4{acc[j][i][4 * g], acc[j][i][4 * g + 1], acc[j][i][4 * g + 2], acc[j][i][4 * g + 3]};
+                for (int g = 0; g < 4; ++g) *(floatx4*)(dst + 8 * g) = floatx4{acc[j][i][4 * g], acc[j][i][4 * g + 1], acc[j][i][4 * g + 2], acc[j][i][4 * g + 3]};
+            }
+            __syncthreads();
         }
-        __syncthreads();
 #pragma unroll
         for (int q = 0; q < 4 / WPU; ++q) {
             const int rl = 8 * (my_part * (4 / WPU) + q) + rr;
             const long row = row0 + 64 * wr + 32 * (u & 1) + rl;
             const float* src = red + ((wr * UP + my_unit) * KG) * (32 * LDSROW) + rl * LDSROW + 4 * piece;
-            floatx4 s = *(const floatx4*)src;
+            floatx4 s;
+            if constexpr (!merge) {
+                s = *(const floatx4*)src;
 #pragma unroll
-            for (int k = 1; k < KG; ++k) {
-                const floatx4 p = *(const floatx4*)(src + k * (32 * LDSROW));
+                for (int k = 1; k < KG; ++k) {
+                    const floatx4 p = *(const floatx4*)(src + k * (32 * LDSROW));
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s[e] += p[e];
+                    for (int e = 0; e < 4; ++e) s[e] += p[e];
+                }
+                if (a.splits > 1) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) __hip_atomic_store(xat(blockIdx.y, q) + 512 * e, s[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    continue;
+                }
+            } else {
+                float p[MID_SPLITS][4];      // requested together (the index clamped to the last split), added in order
+#pragma unroll
+                for (int k = 0; k < MID_SPLITS; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) p[k][e] = __hip_atomic_load(xat(min(k, a.splits - 1), q) + 512 * e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] = p[0][e];
+#pragma unroll
+                for (int k = 1; k < MID_SPLITS; ++k)
+                    if (k < a.splits) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) s[e] += p[k][e];
+                    }
             }
             const bool ok = nt_ok && row < a.R;
 #pragma unroll
@@ -1777,6 +1813,19 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
                 if (ok && piece == 0) a.ssq_out[(long)nt * a.ssq_ld + row] = sq;
             }
         }
+    };
+    phase(std::integral_constant<int, 0>(), std::false_type());
+    if constexpr (NPH > 1) phase(std::integral_constant<int, 1>(), std::false_type());
+    if (a.splits > 1) {
+        __shared__ int s_last;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // the stores have reached the point of coherence
+        __syncthreads();
+        if (t == 0) s_last = __hip_atomic_fetch_add(a.tile_count + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.splits - 1;
+        __syncthreads();
+        if (!s_last) return;
+        if (t == 0) __hip_atomic_store(a.tile_count + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);       // ready for the next launch
+        phase(std::integral_constant<int, 0>(), std::true_type());
+        if constexpr (NPH > 1) phase(std::integral_constant<int, 1>(), std::true_type());
     }
 }
 

@@ -86,3 +86,25 @@ def test_reorder_rows(G, dtype, hidden, heads):
     gpu.prefill(rng.integers(4, 157, size=(7, 9)).astype(np.int32))
     move([6, 5, 4, 3, 2, 1, 0])
     gpu.close()
+
+
+@pytest.mark.parametrize("hidden,heads,kv,ffn,norm,act", [(160, 10, 5, 1000, synth.RMSNORM, synth.SWIGLU), (512, 8, 2, 704, synth.LAYERNORM, synth.RELU)])
+@pytest.mark.parametrize("batch,prompt", [(1, 1), (1, 65), (3, 60), (2, 128)])
+def test_prefill_tiles_that_share_k(G, oracle, monkeypatch, hidden, heads, kv, ffn, norm, act, batch, prompt):
+    """Two to four blocks per tile (TSHIP_GEMM_TILE from 200 on), k-tile counts 10, 32, 44 and 62.5: ranges of unequal length,
+    and counts that leave fewer ranges than asked for; a second prefill finds the counters at zero."""
+    cfg = _cfg(hidden, heads, kv, ffn, norm, act, batch, "f16", prompt=prompt)
+    w = synth.make_weights(cfg, 81, random_bias=True)
+    seqs = synth.make_prompts(cfg, 82)
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(seqs, use_cache=True)
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
+    for tile in (211, 311, 411, 212, 414, 222, 322, 424):
+        monkeypatch.setenv("TSHIP_GEMM_TILE", str(tile))
+        got = []
+        for _ in range(2):
+            gpu.reset()
+            gpu.prefill(seqs)
+            got.append(gpu.logits())
+        assert np.abs(got[0] - lg).max() <= FP16_ABS and np.array_equal(got[0], got[1]), tile
+    gpu.close()
