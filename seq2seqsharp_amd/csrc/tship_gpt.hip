@@ -1224,13 +1224,15 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         aa.qkv = pqkv.as<float>(); aa.KS = 1; aa.split_stride = 0; aa.ldq = qp; aa.pos0 = pos0; aa.Tq = Tp;
         aa.out = po.p; aa.ld_out = m->ldh;
         aa.lens = host_lens ? m->pw_lens.as<int>() : nullptr;
-        // The LDS-tiled QKV projection writes keys and values into the fragment-major cache itself (rotation included)
-        // when its wavefronts' 64 x 128 tiles are whole chunks of whole heads; otherwise a kernel of its own does.
+        // The QKV projection with 256 x 256 tiles writes keys and values into the fragment-major cache itself (rotation included)
+        // when its wavefronts' 64 x 128 tiles are whole chunks of whole heads; otherwise a kernel of its own does, whose time
+        // (9 us at 1.6 k rows, 80 us at 32 k) counts for that tile only where it can do so.  (5 prompts of 333 tokens of the 1B
+        // model: 52 us a layer with the 256 x 256 tile, 44 with 128 x 128; the prefill 4.58 -> 4.44 ms.)
         const int HD = c.n_heads * m->D, GD = c.n_kv_heads * m->D;
-        // (the separate kernel: 9 us at 1.6 k rows, 80 us at 32 k)
-        const int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, 5.0f + 0.0023f * (float)R) : 0;
-        const bool fuse_kv = m->f16 && m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && !qkv_tile && L.qkv.KT % 2 == 0 &&
-                             (m->D == 64 || m->D == 128) && !g_hooks.no_kv_fuse;
+        const bool can_fuse_kv = m->f16 && m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && L.qkv.KT % 2 == 0 &&
+                                 (m->D == 64 || m->D == 128);
+        const int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, can_fuse_kv ? 5.0f + 0.0023f * (float)R : 0.0f) : 0;
+        const bool fuse_kv = can_fuse_kv && !qkv_tile && !g_hooks.no_kv_fuse;
         if (m->f16) {
             BigArgs e; std::memset(&e, 0, sizeof(e));
             e.out = pqkv.as<float>(); e.ld_out = (int)qp; e.bias = L.bqkv.as<float>(); e.n_valid = m->Nqkv;
