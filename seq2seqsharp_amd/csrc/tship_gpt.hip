@@ -1858,8 +1858,8 @@ TSHIP_API int TSHip_GptReorderRows(TSHipGpt* m, const int32_t* host_src_rows, in
             };
             if (!in_place) for (auto& L : m->L) { gather(L->kc.p, row_bytes, head_bytes, used, m->c.n_kv_heads); gather(L->vc.p, row_bytes, head_bytes, used, m->c.n_kv_heads); }
             if (m->last_pos.p) gather(m->last_pos.p, m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), 1);
-            TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
         }
+        TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));       // (the rows are in place when the call returns, and an error of the move is this call's)
         std::vector<int> prompts(m->c.max_batch, -1);
         for (int i = 0; i < new_batch; ++i) prompts[i] = m->row_prompt[host_src_rows[i]];
         m->row_prompt = prompts;
@@ -1980,6 +1980,7 @@ TSHIP_API int TSHip_GptSetKV(TSHipGpt* m, int layer, int which, const float* hos
     const int G = m->c.n_kv_heads, D = m->D; const long ML = m->ML;
     char* base = (char*)(which ? m->L[layer]->vc.p : m->L[layer]->kc.p);
     m->fresh_rows();
+    TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));       // (the copies below are not ordered behind the library's stream)
     const bool frag = m->vt;
     std::vector<char> tmp((size_t)ML * D * m->esz(), 0);
     for (int b = 0; b < batch; ++b) for (int g = 0; g < G; ++g) {

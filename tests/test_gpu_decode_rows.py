@@ -88,6 +88,24 @@ def test_reorder_rows(G, dtype, hidden, heads):
     gpu.close()
 
 
+@pytest.mark.parametrize("rows", [2, 8, 16])
+def test_set_kv_behind_a_move(G, rows):
+    """Keys and values handed in right behind a move of whole rows are what the cache holds: the move has ended by then."""
+    cfg = _cfg(512, 8, 8, 96, synth.RMSNORM, synth.RELU, rows, "f32")
+    w = synth.make_weights(cfg, 74)
+    gpu = G.HipGpt(cfg, w, max_batch=rows, max_seq_len=1024)
+    gpu.set_seq_len(rows, 1000)
+    rng = np.random.default_rng(75)
+    new = rng.standard_normal((rows, 8, 1000, 64), dtype=np.float32)
+    src = np.roll(np.arange(rows), 1)
+    for layer in (0, 2):
+        for which in (0, 1):
+            gpu.reorder_rows(src)
+            gpu.set_kv(layer, which, new)
+            assert np.array_equal(gpu.get_kv(layer, which), new), (layer, which)
+    gpu.close()
+
+
 @pytest.mark.parametrize("hidden,heads,kv,ffn,norm,act", [(160, 10, 5, 1000, synth.RMSNORM, synth.SWIGLU), (512, 8, 2, 704, synth.LAYERNORM, synth.RELU)])
 @pytest.mark.parametrize("batch,prompt", [(1, 1), (1, 65), (3, 60), (2, 128)])
 def test_prefill_tiles_that_share_k(G, oracle, monkeypatch, hidden, heads, kv, ffn, norm, act, batch, prompt):
