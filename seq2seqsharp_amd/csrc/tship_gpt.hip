@@ -1860,7 +1860,7 @@ TSHIP_API int TSHip_GptReorderRows(TSHipGpt* m, const int32_t* host_src_rows, in
             if (m->last_pos.p) gather(m->last_pos.p, m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), m->last_ld * (long)sizeof(int), 1);
         }
         TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));       // (the rows are in place when the call returns, and an error of the move is this call's)
-        std::vector<int> prompts(m->c.max_batch, -1);
+        std::vector<int> prompts = m->row_prompt;      // (rows from new_batch on keep what they hold)
         for (int i = 0; i < new_batch; ++i) prompts[i] = m->row_prompt[host_src_rows[i]];
         m->row_prompt = prompts;
     }

@@ -88,6 +88,23 @@ def test_reorder_rows(G, dtype, hidden, heads):
     gpu.close()
 
 
+def test_rows_left_behind_by_a_move_keep_their_own_prompts(G):
+    """A move to fewer rows, a step (profile_decode takes any batch) that takes the rows behind them in again, and a move
+    among those: they hold different prompts, so all of a row changes places."""
+    cfg = _cfg(64, 4, 4, 96, synth.RMSNORM, synth.RELU, 8, "f32", prompt=70)
+    w = synth.make_weights(cfg, 76, random_bias=True)
+    gpu = G.HipGpt(cfg, w, max_batch=8, max_seq_len=96)
+    gpu.prefill(synth.make_prompts(cfg, 77))
+    gpu.reorder_rows(np.array([1, 0, 2, 3], np.int32))
+    gpu.profile_decode(np.arange(4, 12, dtype=np.int32))
+    before = [gpu.get_kv(l, i) for l in range(3) for i in range(2)]
+    src = np.array([0, 1, 2, 3, 5, 4, 7, 6], np.int32)
+    gpu.reorder_rows(src)
+    for a, b in zip(before, [gpu.get_kv(l, i) for l in range(3) for i in range(2)]):
+        assert np.array_equal(a[src], b)
+    gpu.close()
+
+
 @pytest.mark.parametrize("rows", [2, 8, 16])
 def test_set_kv_behind_a_move(G, rows):
     """Keys and values handed in right behind a move of whole rows are what the cache holds: the move has ended by then."""
