@@ -1184,10 +1184,11 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     ResidNormArgs rn; std::memset(&rn, 0, sizeof(rn));
     rn.x = px.as<float>(); rn.ldx = h; rn.h = h; rn.eps = c.norm_eps; rn.norm_type = c.norm_type;
     rn.xn = pxn.p; rn.ldxn = m->ldh;
-    // Deferred RMSNorm (fp16 RMSNorm models, LDS-tiled GEMMs): no norm kernels.  The producer of the residual stream
+    // Deferred RMSNorm (fp16 RMSNorm models, from 512 rows on): no norm kernels.  The producer of the residual stream
     // stores half(gamma * x) and per-(32-column tile, row) sums of squares, a one-thread-per-row kernel turns those into
-    // 1 / rms, and the consuming GEMMs scale their output rows by it.
-    const bool deferred = m->fused_norm && !m->ln;
+    // 1 / rms, and the consuming GEMMs scale their output rows by it.  half(gamma * x) is infinite from 65504 on; prompts of
+    // fewer rows keep the norm kernels, which store normalised rows whatever the residual's size, in as many launches.
+    const bool deferred = m->fused_norm && !m->ln && R >= 512;
     const int NTh = (int)(round_up(h, 32) / 32);
     DevBuf &pssq = m->pw_ssq, &prinv = m->pw_rinv;
     auto make_rinv = [&](const char* name) {

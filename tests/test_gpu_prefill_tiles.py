@@ -75,3 +75,20 @@ def test_large_tile_writes_the_cache_like_the_separate_kernel(G, monkeypatch, hi
         got = [gpu.logits()] + [gpu.get_kv(l, i) for l in range(2) for i in range(2)]
         assert all(np.array_equal(a, b) for a, b in zip(want, got)), (name, value)
     gpu.close()
+
+
+@pytest.mark.parametrize("batch,prompt", [(1, 33), (3, 90), (7, 73)])       # up to 511 rows
+def test_short_prompts_keep_large_residuals(G, oracle, batch, prompt):
+    """A first token whose residual, times the norms' gain, is beyond the fp16 range: rows of a short prompt are normalised
+    before they are stored in 16 bits."""
+    cfg, w, seqs = _model("rms_gated", batch, prompt)
+    w["TgtEmbeddings"][5] = np.float16(2e4) * np.sign(w["TgtEmbeddings"][5])      # x sqrt(160): a residual of 2.5e5
+    seqs[seqs == 5] = 6
+    seqs[:, 0] = 5
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(seqs, use_cache=True)
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
+    gpu.prefill(seqs)
+    got = gpu.logits()
+    assert np.isfinite(got).all() and np.abs(got - lg).max() <= FP16_ABS
+    gpu.close()
