@@ -2698,8 +2698,10 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
 // the result layout of S leaves in a lane's register 4 g + j and its other half's: P goes back in without a shuffle.
 // No LDS for keys and values: a wavefront reads 4 D x 64 bytes per D x 64 clocks of matrix work, requested a product ahead.
 // A row-at-a-time kernel read the whole cache once per query: 38 us per layer for 2 x 300 positions of 12 heads of 64, now 15.5
-// (bound by the matrix instructions of the longest tile's wavefront and its start).  Masked positions have probability 0 and multiply their
-// values, as in the reference's full product; rows past the sequence are not read.
+// (bound by the matrix instructions of the longest tile's wavefront and its start).
+// A position that a column does not see has probability 0 there and multiplies its value by it.  So that an infinite or NaN value
+// does not reach the columns in front of it, the chunks that some column sees in part take such values out of the product and
+// add them to the columns that see them, one by one.  Rows past the sequence are not read.
 template <int D, int G>
 __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(AttnArgs a) {
     constexpr int QB = 32 / G, VD = D >= 32 ? D / 32 : 1, LDQ = D + 4;
@@ -2733,6 +2735,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(AttnArgs a) {
     if (a.lens && q0 + nq - 1 >= a.lens[b]) T_blk = n_pos;
     const float* Kb = (const float*)a.kcache + ((long)b * a.Hkv + kvc) * a.max_len * D;
     const float* Vb = (const float*)a.vcache + ((long)b * a.Hkv + kvc) * a.max_len * D;
+    const int T_min = a.pos0 + q0 + 1;                       // (the first column sees the fewest positions)
     floatx16 o[VD];
 #pragma unroll
     for (int dt = 0; dt < VD; ++dt)
@@ -2785,6 +2788,31 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(AttnArgs a) {
         for (int dt = 0; dt < VD; ++dt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[dt][i] *= corr;
+        if (t0 + 32 > T_min) {
+            float nan = 0.0f;                                // NaN if one of this lane's values is not finite
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll
+                for (int dt = 0; dt < VD; ++dt) nan = fmaf(vf[i][dt], 0.0f, nan);
+            if (__builtin_expect(__ballot(nan != 0.0f) != 0, 0)) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+#pragma unroll
+                    for (int dt = 0; dt < VD; ++dt) {
+                        const float v = vf[i][dt];
+                        const bool bad = v * 0.0f != 0.0f;
+                        for (unsigned long long left = __ballot(bad); left; left &= left - 1) {
+                            const int from = __builtin_ctzll(left), row = from & 31;      // that lane's position and row of O^T
+                            const float val = __shfl(v, from, 64), p = __shfl(sc[i], l32 + (from & 32), 64);
+                            const bool seen = t0 + 8 * (i >> 2) + 4 * (from >> 5) + (i & 3) < T && half == ((row >> 2) & 1);
+#pragma unroll
+                            for (int k = 0; k < 16; ++k)
+                                if (seen && k == 4 * (row >> 3) + (row & 3)) o[dt][k] = fmaf(p, val, o[dt][k]);
+                        }
+                        vf[i][dt] = bad ? 0.0f : v;
+                    }
+            }
+        }
 #pragma unroll
         for (int i = 0; i < 16; ++i)
 #pragma unroll

@@ -82,6 +82,30 @@ def test_prefill_behind_a_context_and_padded(G, oracle, shape):
     gpu.close()
 
 
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("at,bad", [(37, np.inf), (64, np.nan), (89, -np.inf)])      # inside a chunk of 32 positions, its first, the prompt's last
+def test_prefill_with_a_non_finite_row(G, shape, at, bad):
+    """A token whose key and value are not finite: the positions in front of it are those of a prompt without it, bit for bit."""
+    cfg, w, seqs = _model(shape, 2, 90)
+    w["TgtEmbeddings"][5] = bad
+    seqs[seqs == 5] = 6
+    gpu = G.HipGpt(cfg, w, max_batch=2, max_seq_len=104)
+
+    def run(ids):
+        gpu.reset()
+        gpu.prefill(ids)
+        return gpu.logits(), gpu.get_kv(1, 0), gpu.get_kv(1, 1)       # (the second layer's keys and values follow the first one's attention)
+
+    want = run(seqs)
+    seqs[1, at] = 5
+    got = run(seqs)
+    assert all(np.isfinite(x).all() for x in want) and np.array_equal(got[0][0], want[0][0])
+    for a, b in zip(want[1:], got[1:]):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1, :, :at], b[1, :, :at])
+        assert not np.isfinite(b[1, :, at:]).any()
+    gpu.close()
+
+
 def test_generate_with_more_than_32_rows(G, oracle):
     """The same GEMM at decode (split K, replayed from a captured graph): 40 sequences, greedy."""
     cfg, w, seqs = _model("d64_g1", 40, 3)
