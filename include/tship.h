@@ -278,6 +278,8 @@ TSHIP_API int TSHip_GptStepBytes(TSHipGpt* m, int batch, double* weight_bytes, d
  *   TSHIP_GEMM_TILE=0|11|12|14|22|24   prefill GEMMs: tile of mid_gemm_f16_kernel (10 x 64-row groups + 32-column tiles), 0 = the
  *                             256 x 256 tile from 256 rows on; + 200 ... 400: so many blocks share a tile's K (default: by estimated time)
  *   TSHIP_F32_TILE=11|21|22|42    fp32 GEMMs from 33 rows on: tile in units of 32 rows (10 x) and 32 columns (default: by size)
+ *   TSHIP_F32_ATTN=0|1        attention of fp32 prefills: a block per query, or tiles of 32 columns (default: by estimated time)
+ *   TSHIP_RECORD_SYMBOLS=1    TSHip_GptProfileSymbols gives the kernels launched since the last prefill began
  *   TSHIP_PATCH_ROWS=1|2|4|8  prefill GEMM: row tiles per tile patch of an XCD
  *   TSHIP_ATTN_NQ=1|2         prefill attention: groups of 16 MFMA columns per wavefront
  *   TSHIP_NO_KV_FUSE=1        prefill: the QKV projection leaves the cache write to a kernel of its own

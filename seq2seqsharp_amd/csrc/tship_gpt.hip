@@ -150,7 +150,7 @@ struct TSHipGpt {
     std::vector<int> row_prompt; int prompt_pos = 0;
     void fresh_rows() { row_prompt.resize(c.max_batch); for (int i = 0; i < c.max_batch; ++i) row_prompt[i] = i; prompt_pos = pos; }
     DevBuf cache_table;            // addresses of every layer's key and value cache
-    std::vector<std::string> last_symbols;      // launched symbols of the last profiled step, in launch order
+    std::vector<std::string> last_symbols;      // launched symbols of the last profiled step (TSHIP_RECORD_SYMBOLS: since the last prefill began), in launch order
     DevBuf beam_probs, beam_ids, beam_out, beam_uni, reorder_tmp, reorder_src;      // beam search: probabilities the picks consume, picks, gather temporaries
     Profiler* prof = nullptr;
 
@@ -179,9 +179,11 @@ struct TestHooks {
     long attn_splits = 0;     // TSHIP_ATTN_SPLITS: blocks per (sequence, KV head) pair in decode attention
     int gemm_tile = -1;        // TSHIP_GEMM_TILE: tile of the prefill GEMMs (pick_gemm_tile); 0: the 256 x 256 tile from 256 rows on
     int f32_tile = 0;         // TSHIP_F32_TILE: tile of the fp32 GEMMs from 33 rows on (pick_f32_tile)
+    int f32_attn = -1;        // TSHIP_F32_ATTN: attention of fp32 prefills: 0 a block per query, 1 tiles of 32 columns (f32_attn_by_query)
     int attn_nq = 0;          // TSHIP_ATTN_NQ: 1 or 2 groups of 16 MFMA columns per wavefront in prefill attention
     bool no_kv_fuse = false;  // TSHIP_NO_KV_FUSE: the QKV projection of a prefill does not write the cache itself
     bool no_moe_batch = false;// TSHIP_NO_MOE_BATCH: one prefill GEMM launch per expert
+    bool record_symbols = false;      // TSHIP_RECORD_SYMBOLS: TSHip_GptProfileSymbols gives the kernels launched since the last prefill began
     bool no_graph = false;    // TSHIP_NO_GRAPH: the generate loop launches its kernels one by one
 };
 static TestHooks g_hooks;
@@ -207,6 +209,8 @@ static void refresh_test_hooks() {
         h.f32_tile = std::atoi(v);
         TSHIP_REQUIRE(h.f32_tile == 11 || h.f32_tile == 21 || h.f32_tile == 22 || h.f32_tile == 42, "TSHIP_F32_TILE: 11, 21, 22 or 42");
     }
+    if (const char* v = std::getenv("TSHIP_F32_ATTN")) { h.f32_attn = std::atoi(v); TSHIP_REQUIRE(h.f32_attn == 0 || h.f32_attn == 1, "TSHIP_F32_ATTN: 0 or 1"); }
+    h.record_symbols = std::getenv("TSHIP_RECORD_SYMBOLS") != nullptr;
     h.no_kv_fuse = std::getenv("TSHIP_NO_KV_FUSE") != nullptr;
     h.no_moe_batch = std::getenv("TSHIP_NO_MOE_BATCH") != nullptr;
     h.no_graph = std::getenv("TSHIP_NO_GRAPH") != nullptr;
@@ -216,6 +220,7 @@ static void refresh_test_hooks() {
 template <typename... KArgs, typename... Args>
 static void launch(TSHipGpt* m, const char* name, void (*kernel)(KArgs...), dim3 grid, dim3 block, Args... args) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (m && g_hooks.record_symbols && !m->prof) m->last_symbols.push_back(kernel_symbol((const void*)kernel));
     if (m && m->prof) {
         TSHIP_CHECK_HIP(hipEventCreate(&e0));
         TSHIP_CHECK_HIP(hipEventCreate(&e1));
@@ -240,6 +245,7 @@ static void launch_shm(TSHipGpt* m, const char* name, void (*kernel)(KArgs...), 
         have = shm;
     }
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (m && g_hooks.record_symbols && !m->prof) m->last_symbols.push_back(kernel_symbol((const void*)kernel));
     if (m && m->prof) {
         TSHIP_CHECK_HIP(hipEventCreate(&e0));
         TSHIP_CHECK_HIP(hipEventCreate(&e1));
@@ -673,33 +679,33 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
 }
 
 typedef void (*AttnKernel)(AttnArgs);
+enum AttnKind { ATTN_DECODE, ATTN_PREFILL, ATTN_PREFILL_TILES };      // (tiles: fp32 caches)
 template <typename CT, typename AT, int D, int G>
-static AttnKernel pick_attn_k(bool prefill) {
-    if constexpr (sizeof(CT) == 4) { if (prefill) return attn_prefill_f32_kernel<D, G>; }
-    else if (prefill) return attn_prefill_kernel<CT, AT, D, G>;
-    return attn_decode_kernel<CT, AT, D, G>;
+static AttnKernel pick_attn_k(AttnKind kind) {
+    if constexpr (sizeof(CT) == 4) { if (kind == ATTN_PREFILL_TILES) return attn_prefill_f32_kernel<D, G>; }
+    return kind == ATTN_PREFILL ? attn_prefill_kernel<CT, AT, D, G> : attn_decode_kernel<CT, AT, D, G>;
 }
 template <typename CT, typename AT, int D>
-static AttnKernel pick_attn_g(int G, bool prefill) {
+static AttnKernel pick_attn_g(int G, AttnKind kind) {
     switch (G) {
-        case 1: return pick_attn_k<CT, AT, D, 1>(prefill);
-        case 2: return pick_attn_k<CT, AT, D, 2>(prefill);
-        case 3: return pick_attn_k<CT, AT, D, 3>(prefill);
-        case 4: return pick_attn_k<CT, AT, D, 4>(prefill);
-        case 5: return pick_attn_k<CT, AT, D, 5>(prefill);
-        case 6: return pick_attn_k<CT, AT, D, 6>(prefill);
-        case 7: return pick_attn_k<CT, AT, D, 7>(prefill);
-        case 8: return pick_attn_k<CT, AT, D, 8>(prefill);
+        case 1: return pick_attn_k<CT, AT, D, 1>(kind);
+        case 2: return pick_attn_k<CT, AT, D, 2>(kind);
+        case 3: return pick_attn_k<CT, AT, D, 3>(kind);
+        case 4: return pick_attn_k<CT, AT, D, 4>(kind);
+        case 5: return pick_attn_k<CT, AT, D, 5>(kind);
+        case 6: return pick_attn_k<CT, AT, D, 6>(kind);
+        case 7: return pick_attn_k<CT, AT, D, 7>(kind);
+        case 8: return pick_attn_k<CT, AT, D, 8>(kind);
         default: throw Error("query heads per KV head must be 1 to 8");
     }
 }
 template <typename CT, typename AT>
-static AttnKernel pick_attn_d(int D, int G, bool prefill) {
+static AttnKernel pick_attn_d(int D, int G, AttnKind kind) {
     switch (D) {
-        case 16: return pick_attn_g<CT, AT, 16>(G, prefill);
-        case 32: return pick_attn_g<CT, AT, 32>(G, prefill);
-        case 64: return pick_attn_g<CT, AT, 64>(G, prefill);
-        case 128: return pick_attn_g<CT, AT, 128>(G, prefill);
+        case 16: return pick_attn_g<CT, AT, 16>(G, kind);
+        case 32: return pick_attn_g<CT, AT, 32>(G, kind);
+        case 64: return pick_attn_g<CT, AT, 64>(G, kind);
+        case 128: return pick_attn_g<CT, AT, 128>(G, kind);
         default: throw Error("head_dim must be 16, 32, 64 or 128");
     }
 }
@@ -791,9 +797,26 @@ template <int D>
 static AttnDecodeKernel pick_attn_mfma_decode(int G, bool split, bool sub) {
     return sub ? pick_attn_mfma_decode_s<D, true>(G, split) : pick_attn_mfma_decode_s<D, false>(G, split);
 }
-static AttnKernel pick_attn(TSHipGpt* m, bool prefill, bool split = false, bool ragged = false, int nq = 1) {
+static AttnKernel pick_attn(TSHipGpt* m, AttnKind kind, bool split = false, bool ragged = false, int nq = 1) {
+    const bool prefill = kind != ATTN_DECODE;
     if (m->vt) return m->D == 64 ? pick_attn_mfma<64>(m->G, prefill, split, ragged, nq) : pick_attn_mfma<128>(m->G, prefill, split, ragged, nq);
-    return m->f16 ? pick_attn_d<half_t, half_t>(m->D, m->G, prefill) : pick_attn_d<float, float>(m->D, m->G, prefill);
+    return m->f16 ? pick_attn_d<half_t, half_t>(m->D, m->G, kind) : pick_attn_d<float, float>(m->D, m->G, kind);
+}
+// Kernel of an fp32 prefill's attention: a block per query that reads the cache with all lanes, or tiles of 32 columns on the
+// matrix cores.  A tile takes the positions in steps of 128 however few of its columns are queries, so few queries of small
+// heads are faster one by one.  One token behind 2000 positions, a block per query against tiles, us a layer: -19.5 with 2 x 2
+// heads of 16, -6.5 with 8 heads of 64, +56 with eight heads of 64 on one KV head; 64 tokens of 12 heads of 64: -3.7 behind
+// nothing, and in four sequences +109 behind 2000.  The estimates are fits to 1080 such pairs (four head sizes, one to eight
+// heads per KV head, 1 ... 256 tokens behind 0 ... 2000): the choice costs 0.3 us a layer over the faster kernel on average,
+// always tiles 2.2 and always a block per query 13.2 (profiles/prefill_f32_attention_kernels.txt).
+static bool f32_attn_by_query(const TSHipGpt* m, int B, int Tp, int pos0) {
+    if (g_hooks.f32_attn >= 0) return g_hooks.f32_attn == 0;
+    const long ncu = std::max(1, n_compute_units()), blocks = (long)Tp * m->Hv * B;
+    if (blocks > 4 * ncu) return false;
+    const float steps = (float)(pos0 + Tp) / 128.0f, shared = std::max(1.0f, (float)blocks / (float)(2 * ncu)) * (blocks > ncu && m->D >= 32 ? 1.5f : 1.0f);
+    const float by_query = steps * (float)(m->D / 8) * (0.083f + 0.063f * (float)m->G) * shared;
+    const float tiles = m->D == 128 ? 7.0f + 1.83f * steps : m->D == 64 ? 2.0f + 1.23f * steps : 1.15f * steps;
+    return by_query < tiles;
 }
 template <typename CT>
 static AttnKernel pick_kvw_t(int D) {
@@ -830,7 +853,7 @@ static int attn_splits(TSHipGpt* m, int B) {
     return (int)std::max<long>(1, std::min<long>(S, TSHipGpt::MAX_ATTN_SPLITS));
 }
 static void launch_attn_decode(TSHipGpt* m, AttnArgs a, int B) {
-    if (!m->vt) { launch(m, "attn_decode", pick_attn(m, false), dim3(m->Hv, B), dim3(1024), a); return; }
+    if (!m->vt) { launch(m, "attn_decode", pick_attn(m, ATTN_DECODE), dim3(m->Hv, B), dim3(1024), a); return; }
     const int S = attn_splits(m, B);
     const unsigned threads = m->D == 128 ? 256 : 512;
     dim3 grid(m->c.n_kv_heads, B, m->SG);       // (one block per pair: the groups of a KV head's query heads on z)
@@ -1140,6 +1163,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     const int h = c.hidden, F = c.ffn_dim;
     const long R = (long)B * Tp, Rp = round_up(R, 128);
     const long qp = round_up(m->Nqkv, 32);
+    if (g_hooks.record_symbols) m->last_symbols.clear();
     const int pos0 = m->pos;              // tokens are appended behind what the cache holds (nothing after Create / Reset)
     TSHIP_REQUIRE(pos0 == 0 || m->cur_batch == B, "TSHip_GptPrefill: batch differs from the cached sequences; call TSHip_GptReset first");
     TSHIP_REQUIRE(Tp >= 1 && pos0 + Tp < c.max_seq_len, "TSHip_GptPrefill: prompt length exceeds max_seq_len");
@@ -1265,12 +1289,12 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             int nq = (m->D == 128 && 16 % m->G == 0 && (long)ceil_div(Tp, (16 / m->G) * 16) * m->Hv * B >= 2048) ? 2 : 1;
             if (g_hooks.attn_nq && 16 % m->G == 0) nq = g_hooks.attn_nq;
             const int per_block = (16 / m->G) * 8 * nq;
-            launch(m, "p_attn", pick_attn(m, true, false, host_lens != nullptr, nq), dim3((unsigned)ceil_div(Tp, per_block), m->Hv, B), dim3(512), aa);
+            launch(m, "p_attn", pick_attn(m, ATTN_PREFILL, false, host_lens != nullptr, nq), dim3((unsigned)ceil_div(Tp, per_block), m->Hv, B), dim3(512), aa);
         }
-        else if (!m->f16) {
+        else if (!m->f16 && !f32_attn_by_query(m, B, Tp, pos0)) {
             const unsigned shm = m->D == 128 ? attn_prefill_f32_shm<128>() : m->D == 64 ? attn_prefill_f32_shm<64>() : m->D == 32 ? attn_prefill_f32_shm<32>() : attn_prefill_f32_shm<16>();
-            launch_shm(m, "p_attn", pick_attn(m, true), dim3((unsigned)ceil_div(Tp, 32 / m->G), m->Hv, B), dim3(256), shm, aa);
-        } else launch(m, "p_attn", pick_attn(m, true), dim3(Tp, m->Hv, B), dim3(256), aa);
+            launch_shm(m, "p_attn", pick_attn(m, ATTN_PREFILL_TILES), dim3((unsigned)ceil_div(Tp, 32 / m->G), m->Hv, B), dim3(256), shm, aa);
+        } else launch(m, "p_attn", pick_attn(m, ATTN_PREFILL), dim3(Tp, m->Hv, B), dim3(256), aa);
         ResidNormArgs a2 = rn;
         a2.gamma = L.n2_g.as<float>(); a2.beta = L.n2_b.as<float>();
         if (m->f16) {

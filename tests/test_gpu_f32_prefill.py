@@ -44,7 +44,7 @@ def _check(gpu, orc, lg, what):
 
 @pytest.mark.parametrize("shape", sorted(SHAPES))
 @pytest.mark.parametrize("batch,prompt", [(1, 33), (3, 1), (5, 13), (1, 64), (2, 65), (3, 90), (1, 130)])
-def test_prefill(G, oracle, monkeypatch, shape, batch, prompt):
+def test_prefill(G, oracle, attention, monkeypatch, shape, batch, prompt):
     cfg, w, seqs = _model(shape, batch, prompt)
     orc = oracle.OracleGpt(cfg, w)
     _, lg = orc.step(seqs, use_cache=True)
@@ -60,8 +60,14 @@ def test_prefill(G, oracle, monkeypatch, shape, batch, prompt):
     gpu.close()
 
 
+@pytest.fixture(params=["0", "1"], ids=["by_query", "tiles"])
+def attention(request, monkeypatch):
+    """Both attention kernels, whichever the rule takes."""
+    monkeypatch.setenv("TSHIP_F32_ATTN", request.param)
+
+
 @pytest.mark.parametrize("shape", ["d16_g3", "d64_g1", "d128_g2"])
-def test_prefill_behind_a_context_and_padded(G, oracle, shape):
+def test_prefill_behind_a_context_and_padded(G, oracle, attention, shape):
     """A second prompt behind cached positions, and prompts padded to one length (rows that see every position)."""
     cfg, w, seqs = _model(shape, 3, 45 + 38)
     orc = oracle.OracleGpt(cfg, w)
@@ -84,7 +90,7 @@ def test_prefill_behind_a_context_and_padded(G, oracle, shape):
 
 @pytest.mark.parametrize("shape", sorted(SHAPES))
 @pytest.mark.parametrize("at,bad", [(37, np.inf), (64, np.nan), (89, -np.inf)])      # inside a chunk of 32 positions, its first, the prompt's last
-def test_prefill_with_a_non_finite_row(G, shape, at, bad):
+def test_prefill_with_a_non_finite_row(G, attention, shape, at, bad):
     """A token whose key and value are not finite: the positions in front of it are those of a prompt without it, bit for bit."""
     cfg, w, seqs = _model(shape, 2, 90)
     w["TgtEmbeddings"][5] = bad
@@ -103,6 +109,23 @@ def test_prefill_with_a_non_finite_row(G, shape, at, bad):
     for a, b in zip(want[1:], got[1:]):
         assert np.array_equal(a[0], b[0]) and np.array_equal(a[1, :, :at], b[1, :, :at])
         assert not np.isfinite(b[1, :, at:]).any()
+    gpu.close()
+
+
+@pytest.mark.parametrize("hidden,heads,kv,batch,context,tokens,tiles", [
+    (64, 4, 2, 1, 400, 1, False), (64, 4, 2, 1, 400, 33, False), (512, 8, 8, 1, 400, 2, False), (256, 2, 2, 1, 0, 32, False),      # head sizes 16, 16, 64, 128
+    (512, 8, 1, 1, 400, 2, True), (512, 8, 8, 4, 0, 300, True), (64, 4, 2, 16, 400, 128, True)])
+def test_short_prompts_take_a_block_per_query(G, monkeypatch, hidden, heads, kv, batch, context, tokens, tiles):
+    """Few tokens behind a long context with small heads, against many tokens and against eight heads on a KV head."""
+    cfg = synth._cfg(n_layers=1, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=64, vocab=157, attn_type=synth.GQA, norm_type=synth.RMSNORM,
+                     act=synth.RELU, batch=batch, prompt=tokens, steps=1, dtype="f32")
+    gpu = G.HipGpt(cfg, synth.make_weights(cfg, 53), max_batch=batch, max_seq_len=context + tokens + 8)
+    if context:
+        gpu.set_seq_len(batch, context)
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
+    gpu.prefill(synth.make_prompts(cfg, 54))
+    kernels = gpu.profile_symbols()
+    assert any("attn_prefill_f32_kernel" in k for k in kernels) == tiles and any("attn_prefill_kernel" in k for k in kernels) != tiles, kernels
     gpu.close()
 
 
