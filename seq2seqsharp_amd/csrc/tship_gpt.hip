@@ -145,6 +145,12 @@ struct TSHipGpt {
     bool embed_done = false;       // the sampling kernel of this step has already done the next step's embedding (greedy_embed_kernel)
     DevBuf blocked;                // one byte per token, non-zero = DecodingOptions.BlockedTokens (allocated with the model: graphs keep its address)
     int cur_batch = 0;
+    // The arrival counters of the one-launch reductions are zero between launches; a step that ended in an error may have left
+    // them otherwise.
+    void clear_counters() {
+        for (DevBuf* b : {&tile_count, &attn_count, &mid_count})
+            if (b->p) TSHIP_CHECK_HIP(hipMemsetAsync(b->p, 0, b->bytes, stream()));
+    }
     // which prompt a cache row holds: rows of equal entries are equal in the first prompt_pos positions (rows that a beam
     // search made from one prompt).  fresh_rows() after every other write of whole rows
     std::vector<int> row_prompt; int prompt_pos = 0;
@@ -1586,10 +1592,8 @@ TSHIP_API int TSHip_GptReset(TSHipGpt* m) {
     TSHIP_REQUIRE(m, "TSHip_GptReset: null model");
     m->pos = 0; m->cur_batch = 0; m->fresh_rows();
     TSHIP_CHECK_HIP(hipMemsetAsync(m->d_pos.p, 0, sizeof(int), stream()));
-    if (m->tile_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->tile_count.p, 0, m->tile_count.bytes, stream()));
-    if (m->mid_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->mid_count.p, 0, m->mid_count.bytes, stream()));
+    m->clear_counters();
     if (m->last_pos.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->last_pos.p, 0xff, m->last_pos.bytes, stream()));      // -1: no token seen
-    if (m->attn_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->attn_count.p, 0, m->attn_count.bytes, stream()));
     if (m->moe_ws.p) TSHIP_CHECK_HIP(hipMemsetAsync((char*)m->moe_ws.p + moe_layout(m, m->Bpad).counts, 0, (size_t)m->c.n_experts * sizeof(int), stream()));
     TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
     TSHIP_END
@@ -1720,10 +1724,7 @@ static int generate_impl(TSHipGpt* m, int n_steps, int mode, float top_p, float 
         }
         if (!m->step_graph) {
             hipGraph_t graph = nullptr;
-            // the arrival counters of the one-launch reductions are zero between launches; a step that ended in an error
-            // may have left them otherwise, and every replay of the graph starts from what is there
-            if (m->tile_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->tile_count.p, 0, m->tile_count.bytes, stream()));
-            if (m->attn_count.p) TSHIP_CHECK_HIP(hipMemsetAsync(m->attn_count.p, 0, m->attn_count.bytes, stream()));
+            m->clear_counters();      // (every replay of the graph starts from what is there)
             TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
             TSHIP_CHECK_HIP(hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal));
             const int saved_pos = m->pos;
