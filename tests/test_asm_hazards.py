@@ -1,4 +1,4 @@
-"""The prefill attention kernel issues LDS reads and MFMAs as hand-written instructions whose results the compiler
+"""Some kernels issue LDS reads, and the prefill attention MFMAs too, as hand-written instructions whose results the compiler
 believes to be present as soon as the instruction has been issued.  Two classes of mistakes follow from that, both
 silent at compile time and sporadic at run time:
 
@@ -7,8 +7,10 @@ silent at compile time and sporadic at run time:
   * an instruction the compiler places reads an MFMA's result without the wait states the hardware needs between the
     two, because the compiler keeps that distance only for MFMAs it can see.
 
-This test compiles the kernels' translation unit to gfx950 assembly (no GPU needed) and scans every instance of the
-kernel for both.  The scanners are themselves checked against short listings that contain each mistake.
+These tests compile the kernels' translation unit to gfx950 assembly (no GPU needed).  The prefill attention is scanned in
+listing order for both, with the stricter rule that no branch is reached while a read is in flight; every kernel with
+hand-written reads (the prefill GEMMs fetch ahead under a branch between a read and its wait) is scanned for the first along
+all paths.  The scanners are themselves checked against short listings that contain each mistake.
 """
 import os
 import re
@@ -18,7 +20,8 @@ import pytest
 
 from seq2seqsharp_amd import build as B
 
-KERNEL = re.compile(r"^(_ZN5tship24attn_mfma_prefill_kernel\w+):")
+KERNEL = re.compile(r"^(_ZN5tship\w+):")
+ATTENTION = "attn_mfma_prefill_kernel"
 
 
 def _regs(tok):
@@ -84,6 +87,43 @@ def reads_in_flight(instrs):
     return bad
 
 
+def reads_in_flight_on_paths(instrs):
+    """The same for code that branches between a read and its wait: instructions that touch the destination of a hand-written
+    ds_read_b128 (or take their address from one) before a wait covers it, on any path through the branches."""
+    at = {s.split(":")[0]: i for i, (_, s, _) in enumerate(instrs) if s.startswith(".LBB")}
+    bad, seen, todo = set(), set(), [(0, ())]
+    while todo:
+        i, pend = todo.pop()
+        while i < len(instrs):
+            ln, s, inasm = instrs[i]
+            op = s.split()[0]
+            toks = [t.strip(",") for t in s.split()[1:]]
+            if s.startswith(".LBB"):
+                if (i, pend) in seen:
+                    break
+                seen.add((i, pend))
+            elif op == "s_waitcnt":
+                m = re.search(r"lgkmcnt\((\d+)\)", s)
+                if m:
+                    pend = pend[max(0, len(pend) - int(m.group(1))):]
+            elif op == "s_branch":
+                i = at[toks[0]]
+                continue
+            elif op.startswith("s_cbranch"):
+                todo.append((at[toks[0]], pend))
+            elif op == "s_endpgm":
+                break
+            else:
+                hand_read = op == "ds_read_b128" and inasm
+                hot = set().union(*pend) if pend else set()
+                if set().union(*[_regs(t) for t in toks[1 if hand_read else 0:]], set()) & hot:
+                    bad.add((ln, "'%s' touches registers of a read in flight" % s))
+                if hand_read:
+                    pend += (frozenset(_regs(toks[0])),)
+            i += 1
+    return sorted(bad)
+
+
 def mfma_results_read_early(instrs, distance=20):
     """Findings: instructions other than MFMAs that use the destination of a hand-written MFMA fewer than `distance`
     issue slots behind it (s_nop n counts n + 1; the hardware's largest requirement for this MFMA shape is below 20)."""
@@ -141,18 +181,45 @@ def test_scanners_find_each_mistake():
     assert mfma_results_read_early(_kernels(padded).popitem()[1]) == []
 
 
-@pytest.mark.timeout(900)
-def test_prefill_attention_assembly_has_neither_mistake(tmp_path):
+    # the same mistakes behind a branch that leaves the wait out, and a loop laid out behind another one
+    branch = lambda wait: _listing("\n".join([asm("ds_read_b128 v[2:5], v9 offset:0"), "\ts_cbranch_scc1 .LBB0_2", "\tv_add_f32_e32 v8, v7, v6",
+                                              asm("s_waitcnt lgkmcnt(0)") if wait else "\ts_nop 0", ".LBB0_3:", "\tv_mov_b32_e32 v10, v4", "\ts_endpgm",
+                                              ".LBB0_2:", asm("s_waitcnt lgkmcnt(0)"), "\ts_branch .LBB0_3"]))
+    assert reads_in_flight_on_paths(_kernels(branch(True)).popitem()[1]) == []
+    assert reads_in_flight_on_paths(_kernels(branch(False)).popitem()[1])
+    for listing in (late, count, edge):
+        assert reads_in_flight_on_paths(_kernels(listing).popitem()[1])
+    assert reads_in_flight_on_paths(_kernels(ok).popitem()[1]) == []
+    address = _listing("\n".join([asm("ds_read_b128 v[2:5], v9 offset:0"), asm("ds_read_b128 v[12:15], v3 offset:0"), asm("s_waitcnt lgkmcnt(0)")]))
+    assert reads_in_flight_on_paths(_kernels(address).popitem()[1])
+
+
+@pytest.fixture(scope="module")
+def assembly(tmp_path_factory):
     if not os.path.exists(B.HIPCC):
         pytest.skip("hipcc is not installed")
-    out = tmp_path / "tship_gpt.s"
+    out = tmp_path_factory.mktemp("asm") / "tship_gpt.s"
     cmd = [B.HIPCC] + B.FLAGS + ["--cuda-device-only", "-S", os.path.join(B.CSRC, "tship_gpt.hip"), "-o", str(out)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
-    kernels = _kernels(out.read_text())
+    return out.read_text()
+
+
+@pytest.mark.timeout(900)
+def test_prefill_attention_assembly_has_neither_mistake(assembly):
+    kernels = {n: i for n, i in _kernels(assembly).items() if ATTENTION in n}
     assert len(kernels) >= 32                      # head sizes 64 / 128, 1 / 2 / 4 / 8 query heads per KV head, plain / padded, one / two column groups
     for name, instrs in kernels.items():
         assert any(a and s.startswith("ds_read_b128") for _, s, a in instrs), name
         assert any(a and s.startswith("v_mfma") for _, s, a in instrs), name
         assert reads_in_flight(instrs) == [], name
         assert mfma_results_read_early(instrs) == [], name
+
+
+@pytest.mark.timeout(900)
+def test_no_kernel_touches_a_read_in_flight(assembly):
+    kernels = {n: i for n, i in _kernels(assembly).items() if any(a and s.startswith("ds_read_b128") for _, s, a in i)}
+    for kernel, instances in (("mid_gemm_f16_kernel", 15), ("big_gemm3_f16_kernel", 3), (ATTENTION, 32)):
+        assert sum(kernel in n for n in kernels) >= instances, kernel
+    for name, instrs in kernels.items():
+        assert reads_in_flight_on_paths(instrs) == [], name
