@@ -63,22 +63,27 @@ __global__ __launch_bounds__(256) void rows_gather_kernel(const char* __restrict
     for (long b = (long)threadIdx.x * 16; b < used; b += 256 * 16) *(uint4*)(to + b) = *(const uint4*)(from + b);
 }
 
-// The same in place for up to NR rows, all layers' keys and values in one launch: a thread holds its 16 bytes of every row in
-// registers before it writes the first, so no other thread meets them and nothing goes through a temporary.  Only bytes
-// from .. used of a head's region move (what lies in front of `from` is equal in all rows that change places).
+// The same in place for up to NR rows, all layers' keys and values in one launch: a thread requests its 16 bytes of every row
+// before it writes the first, so no other thread meets them and nothing goes through a temporary.  Only bytes from .. used of
+// a head's region move (what lies in front of `from` is equal in all rows that change places).  The requests are unconditional
+// (rows from n on: src is 0) and of a vector type, so that they are in registers and in flight together; a conditional fill of
+// a struct array went to scratch and waited for each row.
 // Bound by launches before (two per layer and cache, 7.7 us each at 8 rows of 320 positions x 768 floats: 24 layers' caches
-// 370 us a beam step); now one of 5 us behind a shared prompt.  grid (16-byte units / 256, kv heads, caches)
+// 370 us a beam step); now one behind a shared prompt.  grid (16-byte units / 256, kv heads, caches)
 struct RowsMoveArgs { char* const* caches; long row_stride, chunk, from, used; int n; int src[16]; };
 template <int NR>
 __global__ __launch_bounds__(256) void rows_move_kernel(RowsMoveArgs a) {
+    typedef unsigned unit_t __attribute__((ext_vector_type(4)));
     const long b = a.from + ((long)blockIdx.x * 256 + threadIdx.x) * 16;
     if (b >= a.used) return;
     char* p = a.caches[blockIdx.z] + blockIdx.y * a.chunk + b;
-    uint4 v[NR];
+    unit_t v[NR];
 #pragma unroll
-    for (int i = 0; i < NR; ++i) if (i < a.n) v[i] = *(const uint4*)(p + a.src[i] * a.row_stride);
+    for (int i = 0; i < NR; ++i) v[i] = *(const unit_t*)(p + a.src[i] * a.row_stride);
 #pragma unroll
-    for (int i = 0; i < NR; ++i) if (i < a.n && a.src[i] != i) *(uint4*)(p + i * a.row_stride) = v[i];
+    for (int i = 0; i < NR; ++i) asm volatile("" : "+v"(v[i]));       // (no request sinks to its store)
+#pragma unroll
+    for (int i = 0; i < NR; ++i) if (i < a.n && a.src[i] != i) *(unit_t*)(p + i * a.row_stride) = v[i];
 }
 
 // BeamSearch.GetTopNBSS (Utils/BeamSearch.cs:36-46): a FixedSizePriorityQueue (AdvUtils/FixedSizePriorityQueue.cs) with

@@ -124,6 +124,13 @@ def reads_in_flight_on_paths(instrs):
     return sorted(bad)
 
 
+def requests_before_the_first_wait(instrs):
+    """Vector loads in front of the first wait for one, and vector loads in all."""
+    ops = [s for _, s, _ in instrs]
+    first = next((i for i, s in enumerate(ops) if s.startswith("s_waitcnt") and "vmcnt" in s), len(ops))
+    return sum(s.startswith("global_load_dwordx4") for s in ops[:first]), sum(s.startswith("global_load_dwordx4") for s in ops)
+
+
 def mfma_results_read_early(instrs, distance=20):
     """Findings: instructions other than MFMAs that use the destination of a hand-written MFMA fewer than `distance`
     issue slots behind it (s_nop n counts n + 1; the hardware's largest requirement for this MFMA shape is below 20)."""
@@ -192,6 +199,8 @@ def test_scanners_find_each_mistake():
     assert reads_in_flight_on_paths(_kernels(ok).popitem()[1]) == []
     address = _listing("\n".join([asm("ds_read_b128 v[2:5], v9 offset:0"), asm("ds_read_b128 v[12:15], v3 offset:0"), asm("s_waitcnt lgkmcnt(0)")]))
     assert reads_in_flight_on_paths(_kernels(address).popitem()[1])
+    serial = _listing("\tglobal_load_dwordx4 v[2:5], v[0:1], off\n\ts_waitcnt vmcnt(0)\n\tglobal_load_dwordx4 v[6:9], v[0:1], off")
+    assert requests_before_the_first_wait(_kernels(serial).popitem()[1]) == (1, 2)
 
 
 @pytest.fixture(scope="module")
@@ -223,3 +232,15 @@ def test_no_kernel_touches_a_read_in_flight(assembly):
         assert sum(kernel in n for n in kernels) >= instances, kernel
     for name, instrs in kernels.items():
         assert reads_in_flight_on_paths(instrs) == [], name
+
+
+@pytest.mark.timeout(900)
+def test_moved_cache_rows_are_in_flight_together(assembly):
+    """rows_move_kernel: a thread's 16 bytes of all rows are requested before it waits for the first, and stay in registers."""
+    kernels = {n: i for n, i in _kernels(assembly).items() if "rows_move_kernel" in n}
+    rows = sorted(int(re.search(r"rows_move_kernelILi(\d+)", n).group(1)) for n in kernels)
+    assert rows == [4, 8, 16]
+    for name, instrs in kernels.items():
+        n = int(re.search(r"rows_move_kernelILi(\d+)", name).group(1))
+        assert requests_before_the_first_wait(instrs) == (n, n), name
+        assert not any("scratch_" in s or s.startswith("ds_") for _, s, _ in instrs), name
