@@ -580,13 +580,13 @@ static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const fl
 
 // Tile of a prefill GEMM: 10 x (64-row groups) + 32-column tiles of mid_gemm_f16_kernel, or 0 for the 256 x 256 tile.
 // A launch takes rounds of tiles over the compute units x (a + b per k-tile) x a factor for the load of the shared parts
-// (L2, HBM, power).  a and b are fits to launches of 37 ... 16384 rows at seven (K, N) of 768 ... 22016: the choice costs
-// 0.3 % over the best tile on average of those 105 launches, and more than 8 % in one (21 us for 17).
+// (L2, HBM, power).  A launch that leaves half of the units idle may have up to four blocks share the K of a tile (100 x their
+// number in the result); the exchange costs 1.2 us, a little per block and 0.7 us per 64 x 32 values of the tile that each
+// block stores and the last one adds.
 // own_cache_write: us that a launch saves with the 256 x 256 tile, which can write the key-value cache itself.
-// A launch that leaves half of the units idle may have up to four blocks share the K of a tile (100 x their number in the
-// result); the exchange of their sums costs about 2 us and 0.3 us per block.
-// (5632 x 2048: 37 rows 18 -> 10 us with four blocks, 96 rows 25 -> 15; a decode step of 33 / 64 / 96 rows of the 1B model
-// 1060 / 1274 / 1362 -> 962 / 1110 / 1336 us.)
+// a, b and the exchange are fits to 7227 times (33 ... 16384 rows, 27 pairs of K and N from 128 to 22016, every tile and
+// split; profiles/prefill_gemm_tiles.txt): over the best tile of each of the 696 sizes the choice costs 0.6 % on average,
+// more than 15 % in 6.  Without the exchange's growth with the tile it was 2.5 % and 53: 4096 x 1024 at 1024 rows 27.5 us for 17.5.
 // the most blocks up to `splits` that leave none of their ranges of whole chunks empty
 static int mid_splits(const GemmW& w, int tile, int splits) {
     const int kg = tile >= 20 ? 4 : 8;
@@ -595,8 +595,8 @@ static int mid_splits(const GemmW& w, int tile, int splits) {
 }
 static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) {
     struct Cost { int tile, rows, cols; float a, b; };
-    static const Cost costs[] = {{11, 64, 1, 1.9f, 0.045f}, {12, 64, 2, 2.8f, 0.050f}, {14, 64, 4, 3.0f, 0.093f},
-                                 {22, 128, 2, 3.4f, 0.078f}, {24, 128, 4, 4.8f, 0.115f}, {0, 256, 8, 8.0f, 0.320f}};
+    static const Cost costs[] = {{11, 64, 1, 3.5f, 0.031f}, {12, 64, 2, 4.4f, 0.046f}, {14, 64, 4, 6.5f, 0.077f},
+                                 {22, 128, 2, 5.2f, 0.072f}, {24, 128, 4, 8.1f, 0.111f}, {0, 256, 8, 7.0f, 0.285f}};
     const int forced = g_hooks.gemm_tile;
     if (forced == 0 && R >= 256) return 0;
     if (forced > 0) {
@@ -613,8 +613,8 @@ static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) 
             const int splits = mid_splits(w, c.tile, want);
             if (splits != want || (splits > 1 && (n_tiles * splits > TSHipGpt::MID_XCHG_TILES || n_tiles * splits > (long)ncu))) continue;
             const float tiles = (float)(n_tiles * splits), rounds = std::ceil(tiles / ncu);
-            float us = rounds * (c.a + c.b * (float)ceil_div(w.KT, splits)) * (1.0f + 0.4f * tiles / (rounds * ncu));
-            if (splits > 1) us += 2.0f + 0.3f * (float)splits;
+            float us = rounds * (c.a + c.b * (float)ceil_div(w.KT, splits)) * (1.0f + (c.tile ? 0.2f : 0.65f) * tiles / (rounds * ncu));
+            if (splits > 1) us += 1.16f + 0.08f * (float)splits + 0.7f * (float)(c.rows * c.cols) / 64.0f;
             if (c.tile == 0) us -= own_cache_write;
             if (us < best_us) { best_us = us; best = c.tile ? c.tile + 100 * splits : 0; }
         }
@@ -1255,15 +1255,16 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         aa.qkv = pqkv.as<float>(); aa.KS = 1; aa.split_stride = 0; aa.ldq = qp; aa.pos0 = pos0; aa.Tq = Tp;
         aa.out = po.p; aa.ld_out = m->ldh;
         aa.lens = host_lens ? m->pw_lens.as<int>() : nullptr;
-        // The QKV projection with 256 x 256 tiles writes keys and values into the fragment-major cache itself (rotation included)
-        // when its wavefronts' 64 x 128 tiles are whole chunks of whole heads; otherwise a kernel of its own does, whose time
-        // (9 us at 1.6 k rows, 80 us at 32 k) counts for that tile only where it can do so.  (5 prompts of 333 tokens of the 1B
-        // model: 52 us a layer with the 256 x 256 tile, 44 with 128 x 128; the prefill 4.58 -> 4.44 ms.)
+        // The QKV projection with 256 x 256 tiles can write keys and values into the fragment-major cache itself (rotation
+        // included) when its wavefronts' 64 x 128 tiles are whole chunks of whole heads.  That takes it about 7.5 us longer and
+        // saves a kernel whose time goes with rows x columns of keys and values (profiles/prefill_gemm_tiles.txt: 1024 columns,
+        // 1024 rows 49.0 + 7.4 against 62.5 us, 16384 rows 202 + 37 against 211); a kernel of its own does it where that is less.
         const int HD = c.n_heads * m->D, GD = c.n_kv_heads * m->D;
         const bool can_fuse_kv = m->f16 && m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && L.qkv.KT % 2 == 0 &&
                                  (m->D == 64 || m->D == 128);
-        const int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, can_fuse_kv ? 5.0f + 0.0023f * (float)R : 0.0f) : 0;
-        const bool fuse_kv = can_fuse_kv && !qkv_tile && !g_hooks.no_kv_fuse;
+        const float fuse_saves = 1.9e-6f * (float)(R * 2 * GD) - 7.5f;
+        const int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, can_fuse_kv ? std::max(0.0f, fuse_saves) : 0.0f) : 0;
+        const bool fuse_kv = can_fuse_kv && !qkv_tile && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
         if (m->f16) {
             BigArgs e; std::memset(&e, 0, sizeof(e));
             e.out = pqkv.as<float>(); e.ld_out = (int)qp; e.bias = L.bqkv.as<float>(); e.n_valid = m->Nqkv;
