@@ -95,7 +95,7 @@ def test_cfg1_fp32_full_depth_greedy_tokens(G, oracle):
 
 
 def test_cfg1_fp16_full_width(G, oracle):
-    """Configuration 1's fp16 variant at full width, 4 layers, batch 8, prompt 96 (768 prompt rows: the LDS-tiled GEMMs)."""
+    """Configuration 1's fp16 variant at full width, 4 layers, batch 8, prompt 96 (768 prompt rows)."""
     cfg = dict(synth.CONFIGS["cfg1_gpt2small_f16"], n_layers=4, prompt=96)
     _, gpu, out, _ = teacher_forced(G, oracle, cfg, 3, 4)
     check_fp16(out)
@@ -342,19 +342,37 @@ def test_cfg3_full_depth_graph_replay_equals_stepwise(G):
     step.close()
 
 
+@pytest.fixture
+def large_tile(monkeypatch):
+    """The 256 x 256 tile of the prefill GEMMs, which prompts of these tests' sizes do not take by themselves, and a check
+    of the kernels that the last prefill launched."""
+    monkeypatch.setenv("TSHIP_GEMM_TILE", "0")
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
+
+    def launched(gpu, cache_write=None):
+        kernels = gpu.profile_symbols()
+        assert any("big_gemm" in k for k in kernels) and not any("mid_gemm" in k for k in kernels), kernels
+        if cache_write is not None:
+            assert any("kv_write_frag_kernel" in k for k in kernels) == cache_write, kernels
+    return launched
+
+
+@pytest.mark.parametrize("tile", ["by_size", "large"])
 @pytest.mark.parametrize("batch,prompt,hidden,heads,kv,ffn,act", [
     (3, 200, 192, 3, 3, 256, synth.SWIGLU),        # 600 rows: partial 256-row tiles; 6 and 8 column tiles (partial groups of four)
     (2, 300, 256, 4, 2, 264, synth.SWIGLU_SILU),   # odd number of k-tiles in the down projection (the register-staged kernel)
     (5, 128, 512, 8, 2, 1024, synth.SWIGLU),       # 640 rows, whole 64-row blocks, whole groups of four column tiles (line stores)
     (9, 64, 128, 2, 1, 512, synth.RELU),           # 576 rows, ungated activation
 ])
-def test_prefill_tile_edges_against_oracle(G, oracle, batch, prompt, hidden, heads, kv, ffn, act):
-    """Prompts of 512 rows and more take the LDS-tiled prefill GEMMs, whose epilogues write whole 64 x 128-byte blocks
-    through LDS where a wavefront's block is complete and element-wise elsewhere: row counts that are no multiple of
-    the tile sizes and widths that leave partial column groups, against the oracle."""
+def test_prefill_tile_edges_against_oracle(G, oracle, request, tile, batch, prompt, hidden, heads, kv, ffn, act):
+    """The prefill GEMMs' epilogues write whole lines (256 x 256 tile: 64 x 128-byte blocks through LDS) where a
+    wavefront's block is complete and element-wise elsewhere: row counts that are no multiple of the tile sizes and
+    widths that leave partial column groups, against the oracle."""
+    launched = request.getfixturevalue("large_tile") if tile == "large" else lambda gpu: None
     cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=ffn, vocab=211, attn_type=synth.GQA,
                      norm_type=synth.RMSNORM, act=act, batch=batch, prompt=prompt, steps=2, dtype="f16")
     _, gpu, out, _ = teacher_forced(G, oracle, cfg, 31, 2)
+    launched(gpu)
     check_fp16(out)
     gpu.close()
 
@@ -362,7 +380,7 @@ def test_prefill_tile_edges_against_oracle(G, oracle, batch, prompt, hidden, hea
 @pytest.mark.parametrize("dtype,hidden,heads,kv,batch,prompt", [
     ("f16", 512, 8, 1, 5, 70),        # head size 64, eight query heads on one KV head: the MFMA attention kernels
     ("f16", 1024, 8, 1, 33, 40),      # head size 128
-    ("f16", 1024, 16, 2, 3, 530),     # two KV heads; 530 rows of prompt take the LDS-tiled prefill GEMMs
+    ("f16", 1024, 16, 2, 3, 530),     # two KV heads; 1590 rows of prompt
     ("f32", 256, 8, 1, 4, 37),        # the fp32 (VALU) attention kernels
     ("f16", 256, 8, 1, 2, 33),        # head size 32: VALU kernels on an fp16 cache
 ])
@@ -384,9 +402,9 @@ def test_eight_query_heads_per_kv_head(G, oracle, dtype, hidden, heads, kv, batc
     (1024, 8, 2, 3, 192),      # head size 128: a wavefront's 128 columns are one head, written in two passes
     (512, 8, 4, 1, 544),       # one sequence of 17 chunks: the last wavefront's second chunk lies beyond the rows
 ])
-def test_projection_writes_the_cache_like_the_separate_kernel(G, oracle, monkeypatch, hidden, heads, kv, batch, prompt):
-    """From 512 rows on, with whole 32-position chunks, the QKV projection's epilogue rotates the keys and writes keys and
-    values into the fragment-major cache itself.  Same cache contents and logits as with the separate cache-write kernel
+def test_projection_writes_the_cache_like_the_separate_kernel(G, oracle, monkeypatch, large_tile, hidden, heads, kv, batch, prompt):
+    """With the 256 x 256 tile and whole 32-position chunks, the QKV projection's epilogue rotates the keys and writes keys
+    and values into the fragment-major cache itself.  Same cache contents and logits as with the separate cache-write kernel
     (TSHIP_NO_KV_FUSE=1), and the cache against the oracle's keys and values."""
     cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=2 * hidden, vocab=157, attn_type=synth.GQA,
                      norm_type=synth.RMSNORM, act=synth.SWIGLU, batch=batch, prompt=prompt, steps=2, dtype="f16")
@@ -394,11 +412,13 @@ def test_projection_writes_the_cache_like_the_separate_kernel(G, oracle, monkeyp
     seqs = synth.make_prompts(cfg, 78)
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 136)
     gpu.prefill(seqs)
+    large_tile(gpu, cache_write=False)
     fused = [(gpu.get_kv(l, 0), gpu.get_kv(l, 1)) for l in range(2)]
     lg_fused = gpu.logits()
     monkeypatch.setenv("TSHIP_NO_KV_FUSE", "1")
     gpu.reset()
     gpu.prefill(seqs)
+    large_tile(gpu, cache_write=True)
     monkeypatch.delenv("TSHIP_NO_KV_FUSE")
     for l in range(2):
         k, v = gpu.get_kv(l, 0), gpu.get_kv(l, 1)
@@ -406,11 +426,13 @@ def test_projection_writes_the_cache_like_the_separate_kernel(G, oracle, monkeyp
         assert np.array_equal(fused[l][1], v), "values of layer %d" % l
     assert np.array_equal(lg_fused, gpu.logits())
     # appended tokens behind the fused prefill continue the same cache: 128 more per sequence (with three or five sequences
-    # again 512 rows or more, written by the projection at a cache offset; with one sequence by the separate kernel)
+    # written by the projection at a cache offset; the 128 rows of one sequence take smaller tiles and the separate kernel)
     more = synth.make_prompts(dict(cfg, prompt=128), 79)
     gpu.reset()
     gpu.prefill(seqs)
     gpu.prefill(more)
+    if batch > 1:
+        large_tile(gpu, cache_write=False)
     lg_app = gpu.logits()
     k_app = gpu.get_kv(1, 0)
     orc = oracle.OracleGpt(cfg, w)
@@ -426,8 +448,8 @@ def test_projection_writes_the_cache_like_the_separate_kernel(G, oracle, monkeyp
 
 
 @pytest.mark.parametrize("patch_rows", ["1", "2", "4", "8"])
-def test_prefill_tile_patch_heights_give_the_same_bits(G, monkeypatch, patch_rows):
-    """The LDS-tiled prefill GEMM maps its blocks to tiles in patches of (8, 4, 2 or 1) x 4 tiles per XCD, chosen from the
+def test_prefill_tile_patch_heights_give_the_same_bits(G, monkeypatch, large_tile, patch_rows):
+    """The 256 x 256 prefill GEMM maps its blocks to tiles in patches of (8, 4, 2 or 1) x 4 tiles per XCD, chosen from the
     launch size; the mapping must not change any result.  1536 rows x 512 columns: 6 x 2 tiles, fewer than eight patches at
     every height, against the height the launch code picks."""
     cfg = synth._cfg(n_layers=2, hidden=512, n_heads=8, n_kv_heads=2, ffn_dim=1024, vocab=157, attn_type=synth.GQA,
@@ -440,6 +462,7 @@ def test_prefill_tile_patch_heights_give_the_same_bits(G, monkeypatch, patch_row
     monkeypatch.setenv("TSHIP_PATCH_ROWS", patch_rows)
     gpu.reset()
     gpu.prefill(seqs)
+    large_tile(gpu)
     monkeypatch.delenv("TSHIP_PATCH_ROWS")
     assert np.array_equal(want, gpu.logits())
     gpu.close()

@@ -3,11 +3,14 @@ of their ranges."""
 import numpy as np
 import pytest
 
+from parity_util import FP16_SENSITIVE_REL, sensitive
 from seq2seqsharp_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-FP16_ABS = 3e-2      # the fp16 bar of the parity tests
+# hidden, heads, kv heads, ffn, activation
+SHAPES = [(160, 10, 5, 200, synth.SWIGLU), (48, 3, 1, 104, synth.RELU), (512, 8, 2, 704, synth.SILU), (256, 2, 2, 96, synth.SWIGLU_SILU)]
+SPLIT_SHAPES = [(160, 10, 5, 1000, synth.RMSNORM, synth.SWIGLU), (512, 8, 2, 704, synth.LAYERNORM, synth.RELU)]
 
 
 @pytest.fixture(scope="module")
@@ -21,36 +24,58 @@ def _cfg(hidden, heads, kv, ffn, norm, act, batch, dtype, attn=synth.GQA, prompt
                       batch=batch, prompt=prompt, steps=4, dtype=dtype)
 
 
-def _steps(G, oracle, cfg, max_batch):
-    w = synth.make_weights(cfg, 61, random_bias=True)
+def _within(gl, lg, what):
+    assert np.abs(gl - lg).max() <= FP16_SENSITIVE_REL * np.abs(lg).max(), what
+
+
+# the tile by size, every tile by itself, and tiles whose K several blocks share (their counters go through graph replays)
+TILES = ("", "11", "12", "14", "22", "24", "411", "412", "322", "424")
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("max_batch,batch", [(33, 33), (64, 1), (64, 64), (100, 65), (128, 128)])
+def test_rows(G, oracle, monkeypatch, shape, max_batch, batch):
+    """Steps one by one against the oracle, and the generate loop with and without its captured graph: the same tokens and the
+    same bits as those steps.  (A new model per tile: a captured step keeps the tiles it was captured with.)"""
+    hidden, heads, kv, ffn, act = shape
+    cfg = _cfg(hidden, heads, kv, ffn, synth.RMSNORM, act, batch, "f16")
+    w = sensitive(synth.make_weights(cfg, 61, random_bias=True), hidden)
     seqs = synth.make_prompts(cfg, 62)
     orc = oracle.OracleGpt(cfg, w)
-    gpu = G.HipGpt(cfg, w, max_batch=max_batch, max_seq_len=24)
     p, lg = orc.step(seqs, use_cache=True)
-    gpu.prefill(seqs)
-    cur = seqs
-    for i in range(4):
-        nxt = oracle.argmax(p).astype(np.int32)
-        cur = np.concatenate([cur, nxt[:, None]], 1)
+    want, fed, cur = [lg], [], seqs
+    for _ in range(4):
+        fed.append(oracle.argmax(p).astype(np.int32))
+        cur = np.concatenate([cur, fed[-1][:, None]], 1)
         p, lg = orc.step(cur, use_cache=True)
-        gpu.decode(nxt)
-        assert np.abs(gpu.logits() - lg).max() <= FP16_ABS, i
-    assert gpu.seq_len() == seqs.shape[1] + 4
-    # the same steps from the generate loop's captured graph: same kernels, same bits
-    want = gpu.logits()
-    gpu.reset()
-    gpu.prefill(seqs)
-    ids, _ = gpu.generate(4)
-    if np.array_equal(ids.T, cur[:, -4:]):       # (an fp16 model may choose another token where two are close)
-        assert np.array_equal(gpu.logits(), want)
-    gpu.close()
-
-
-@pytest.mark.parametrize("shape", [(160, 10, 5, 200, synth.SWIGLU), (48, 3, 1, 104, synth.RELU), (512, 8, 2, 704, synth.SILU), (256, 2, 2, 96, synth.SWIGLU_SILU)])
-@pytest.mark.parametrize("max_batch,batch", [(33, 33), (64, 1), (64, 64), (100, 65), (128, 128)])
-def test_rows(G, oracle, shape, max_batch, batch):
-    hidden, heads, kv, ffn, act = shape
-    _steps(G, oracle, _cfg(hidden, heads, kv, ffn, synth.RMSNORM, act, batch, "f16"), max_batch)
+        want.append(lg)
+    for tile in TILES:
+        if tile:
+            monkeypatch.setenv("TSHIP_GEMM_TILE", tile)
+        gpu = G.HipGpt(cfg, w, max_batch=max_batch, max_seq_len=24)
+        gpu.prefill(seqs)
+        _within(gpu.logits(), want[0], tile)
+        for nxt, lg in zip(fed, want[1:]):
+            gpu.decode(nxt)
+            _within(gpu.logits(), lg, tile)
+        assert gpu.seq_len() == seqs.shape[1] + 4
+        runs = []
+        for graph in (True, False):
+            if not graph:
+                monkeypatch.setenv("TSHIP_NO_GRAPH", "1")
+            gpu.reset()
+            gpu.prefill(seqs)
+            ids, _ = gpu.generate(4)
+            runs.append((ids, gpu.logits()))
+        monkeypatch.delenv("TSHIP_NO_GRAPH")
+        gpu.reset()
+        gpu.prefill(seqs)
+        for nxt in runs[0][0]:
+            assert np.array_equal(gpu.sample(), nxt), tile
+            gpu.decode(nxt)
+        for ids, logits in runs:
+            assert np.array_equal(ids, runs[0][0]) and np.array_equal(logits, gpu.logits()), tile
+        gpu.close()
 
 
 @pytest.mark.parametrize("dtype,hidden,heads", [("f32", 64, 4), ("f16", 64, 4), ("f16", 128, 2)])
@@ -123,13 +148,13 @@ def test_set_kv_behind_a_move(G, rows):
     gpu.close()
 
 
-@pytest.mark.parametrize("hidden,heads,kv,ffn,norm,act", [(160, 10, 5, 1000, synth.RMSNORM, synth.SWIGLU), (512, 8, 2, 704, synth.LAYERNORM, synth.RELU)])
+@pytest.mark.parametrize("hidden,heads,kv,ffn,norm,act", SPLIT_SHAPES)
 @pytest.mark.parametrize("batch,prompt", [(1, 1), (1, 65), (3, 60), (2, 128)])
 def test_prefill_tiles_that_share_k(G, oracle, monkeypatch, hidden, heads, kv, ffn, norm, act, batch, prompt):
     """Two to four blocks per tile (TSHIP_GEMM_TILE from 200 on), k-tile counts 10, 32, 44 and 62.5: ranges of unequal length,
     and counts that leave fewer ranges than asked for; a second prefill finds the counters at zero."""
     cfg = _cfg(hidden, heads, kv, ffn, norm, act, batch, "f16", prompt=prompt)
-    w = synth.make_weights(cfg, 81, random_bias=True)
+    w = sensitive(synth.make_weights(cfg, 81, random_bias=True), hidden)
     seqs = synth.make_prompts(cfg, 82)
     orc = oracle.OracleGpt(cfg, w)
     _, lg = orc.step(seqs, use_cache=True)
@@ -141,5 +166,6 @@ def test_prefill_tiles_that_share_k(G, oracle, monkeypatch, hidden, heads, kv, f
             gpu.reset()
             gpu.prefill(seqs)
             got.append(gpu.logits())
-        assert np.abs(got[0] - lg).max() <= FP16_ABS and np.array_equal(got[0], got[1]), tile
+        _within(got[0], lg, tile)
+        assert np.array_equal(got[0], got[1]), tile
     gpu.close()

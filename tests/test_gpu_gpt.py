@@ -175,7 +175,7 @@ def test_generate_matches_stepwise_and_is_deterministic(G):
 
 @pytest.mark.parametrize("batch", [4, 8])
 def test_decode_equals_prefill_recompute(G, batch):
-    """(batch 8: 768 and 800 prompt rows, which takes the LDS-tiled prefill GEMM; batch 4 takes the direct one.)
+    """(batch 8: 768 and 800 prompt rows, half of them with batch 4: prefill GEMM tiles of different heights.)
     Size-independent property at the real head shape (GQA 32/8 heads of 64): prefill(P) + decode(tokens) must give
     the logits of prefill(P + n).  It exercises cache positions, the RoPE offset and the decode GEMM against the
     prefill GEMM on a model wide enough to use full MFMA tiles."""
@@ -237,10 +237,13 @@ def test_full_size_cfg2_properties(G):
     b.close()
 
 
+@pytest.mark.parametrize("tile", ["by_size", "0"])
 @pytest.mark.parametrize("name", ["odd_sizes", "gqa_leaky_d32_g4", "mha_ln_relu"])
-def test_fp16_long_prompt_prefill_against_oracle(G, oracle, name):
-    """More than 512 prompt rows: the prefill projections run on the LDS-tiled GEMM (ragged row, column and k tiles
-    with these sizes).  Logits of the last position and the whole KV cache of the last layer against the oracle."""
+def test_fp16_long_prompt_prefill_against_oracle(G, oracle, monkeypatch, name, tile):
+    """655 prompt rows: the prefill projections with the tile picked by size, and with 256 x 256 tiles (ragged row, column
+    and k tiles with these sizes).  Logits of the last position and the whole KV cache of the last layer against the oracle."""
+    if tile != "by_size":
+        monkeypatch.setenv("TSHIP_GEMM_TILE", tile)
     cfg = synth.tiny_config(dtype="f16", **dict(TINY[name], batch=5, prompt=131))
     w = synth.make_weights(cfg, 21, random_bias=True)
     orc = oracle.OracleGpt(cfg, w)
@@ -360,8 +363,8 @@ def test_moe_model(G, oracle, dtype, act):
 @pytest.mark.parametrize("dtype,batch,prompt", [("f16", 4, 330), ("f16", 3, 70), ("f32", 2, 40)])
 def test_moe_prefill_runs_the_experts_on_gathered_rows(G, oracle, dtype, batch, prompt):
     """Prefill of a model with MoE layers: all prompt rows are routed at once, every expert runs the prefill GEMMs on the
-    rows gathered for it (about 660 rows per expert in the first case: the LDS-tiled kernel; fewer than 512 in the
-    others), and the scaled outputs are added back in expert order.  Logits of the last position and the routing of the
+    rows gathered for it (about 660 rows per expert in the first case: one launch for all experts; fewer than 512 in the
+    others: one per expert), and the scaled outputs are added back in expert order.  Logits of the last position and the routing of the
     last position against the oracle, then decode steps on top of the cache the prefill wrote."""
     cfg = synth.tiny_config(n_layers=3, n_experts=4, experts_per_token=2, norm_type=synth.LAYERNORM, act=synth.RELU, dtype=dtype,
                             batch=batch, prompt=prompt, vocab=300)
@@ -426,7 +429,7 @@ def test_full_width_layer_against_oracle(G, oracle):
 @pytest.mark.parametrize("kv_heads,batch,prompt", [(1, 3, 40), (2, 8, 70)])
 def test_head_dim_128_against_oracle(G, oracle, kv_heads, batch, prompt):
     """The 7B configuration's head shape (head_dim 128, 4 or 2 query heads per KV head) on a narrow model: prefill
-    (the second case has 560 prompt rows: LDS-tiled GEMM and MFMA prefill attention over several chunks) and decode
+    (the second case has 560 prompt rows: MFMA prefill attention over several chunks) and decode
     steps across a 32-position chunk boundary, fp16, against the oracle."""
     cfg = synth.tiny_config(dtype="f16", hidden=512, n_heads=4, n_kv_heads=kv_heads, ffn_dim=1024, vocab=512, batch=batch, prompt=prompt)
     orc, gpu, out, _ = _teacher_forced(G, oracle, cfg, 71, 4)
@@ -489,8 +492,8 @@ def test_decode_ffn_up_projection_several_tiles_per_block(G, oracle, monkeypatch
 def test_prefill_appends_to_cached_sequences(G, oracle, dtype, hidden, heads, kv_heads, first, second):
     """A second prefill continues the cached sequences (the next turn of a dialogue whose cache was kept): the logits
     and the cache are those of one prefill of the concatenation, and decoding goes on from there.  Covers a first part
-    that ends on a 32-position boundary (whole fragments written) and ones that do not, head_dim 64 and 128, and the
-    LDS-tiled GEMMs (530 x 2 rows)."""
+    that ends on a 32-position boundary (whole fragments written) and ones that do not, head_dim 64 and 128, and
+    a second part of 530 x 2 rows."""
     cfg = synth.tiny_config(dtype=dtype, hidden=hidden, n_heads=heads, n_kv_heads=kv_heads, ffn_dim=2 * hidden, vocab=300, batch=2, prompt=first + second)
     w = synth.make_weights(cfg, 91, random_bias=True)
     orc = oracle.OracleGpt(cfg, w)
@@ -615,7 +618,7 @@ def test_argument_errors(G):
 ])
 def test_moe_prefill_one_launch_for_all_experts_equals_one_per_expert(G, oracle, monkeypatch, experts, k, batch, prompt, router_bias):
     """From 512 prompt rows on, the prefill of an fp16 model never reads the experts' row counts back: each projection of
-    all experts is one launch of the LDS-tiled kernel over the experts' row tiles packed one behind the other (weights by
+    all experts is one launch of the 256 x 256 kernel over the experts' row tiles packed one behind the other (weights by
     pointer table, the problem of a tile found on the device from the counts), and the up projection reads its rows
     through the token lists.  Same logits, bit for bit, as the path with the counts on the host, gathered rows and one
     launch per expert (TSHIP_NO_MOE_BATCH=1): with an expert that holds far fewer rows than the largest one, one with no

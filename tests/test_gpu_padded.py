@@ -63,16 +63,23 @@ def test_padded_batch_fp32(G, oracle, kw):
     gpu.close()
 
 
+@pytest.mark.parametrize("tile", ["by_size", "large"])
 @pytest.mark.parametrize("hidden,heads,kv_heads,lens", [(256, 4, 2, [70, 33, 1, 64, 2]), (512, 4, 1, [40, 9, 31]), (256, 4, 4, [130, 129, 5, 64]),
-                                                        # 9 x 64 = 576 padded rows in whole 32-position chunks: the LDS-tiled GEMMs, and the QKV
+                                                        # 9 x 64 = 576 padded rows in whole 32-position chunks: with the 256 x 256 tile the QKV
                                                         # projection writes the cache (padding positions included) from its epilogue
                                                         (512, 8, 4, [64, 17, 1, 33, 64, 50, 2, 31, 48]), (512, 4, 2, [64, 3, 40, 64, 20, 9, 33, 1, 60])])
-def test_padded_batch_fp16_mfma_attention(G, oracle, hidden, heads, kv_heads, lens):
+def test_padded_batch_fp16_mfma_attention(G, oracle, monkeypatch, hidden, heads, kv_heads, lens, tile):
     """head_dim 64 and 128 (the MFMA prefill attention): lengths on both sides of 32-position chunk boundaries, a row of
-    length 1, rows of full length."""
+    length 1, rows of full length; the prefill GEMMs' tile by size, and the 256 x 256 one (from 256 rows on)."""
+    if tile == "large":
+        monkeypatch.setenv("TSHIP_GEMM_TILE", "0")
+        monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
     lens = np.array(lens, np.int32)
     cfg = synth.tiny_config(dtype="f16", hidden=hidden, n_heads=heads, n_kv_heads=kv_heads, ffn_dim=2 * hidden, vocab=300, batch=len(lens))
     orc, gpu, out, ids = _run(G, oracle, cfg, lens, 9)
+    if tile == "large" and lens.size == 9:      # (symbols since the prefill: the steps launch no cache write of this kind)
+        kernels = gpu.profile_symbols()
+        assert any("big_gemm" in k for k in kernels) and not any("kv_write_frag_kernel" in k for k in kernels), kernels
     fr = []
     for lg, gl in out:
         assert np.abs(gl - lg).max() <= 3e-2

@@ -177,8 +177,8 @@ def test_moe_expert_counts_beyond_eight(oracle, experts, k, batch, dtype):
 
 
 def _big_prefill_cfg(seed):
-    """512 to 1700 prompt rows in whole 32-position chunks, key and value widths multiples of 128: the shapes where the
-    LDS-tiled prefill kernels, their adaptive tile patches and the cache write from the QKV projection are in use."""
+    """512 to 1700 prompt rows in whole 32-position chunks, key and value widths multiples of 128: shapes that the 256 x 256
+    prefill tile with its adaptive tile patches and the cache write from the QKV projection takes."""
     rng = np.random.default_rng(3000 + seed)
     while True:
         d = int(rng.choice([64, 128]))
@@ -197,18 +197,29 @@ def _big_prefill_cfg(seed):
 @pytest.mark.parametrize("seed", range(16))
 def test_large_prefill_paths_agree_bit_for_bit(monkeypatch, seed):
     """The cache written by the QKV projection's epilogue and the tile patches chosen from the launch size, against the
-    separate cache-write kernel and fixed 8 x 4 patches: same logits, keys and values."""
+    separate cache-write kernel and fixed 8 x 4 patches: same logits, keys and values.  (The 256 x 256 tile is forced: most
+    of these sizes take smaller ones by themselves.)"""
     from seq2seqsharp_amd import gpt as G
     cfg = _big_prefill_cfg(seed)
     w = synth.make_weights(cfg, 100 + seed, random_bias=True)
     seqs = synth.make_prompts(cfg, 200 + seed)
     gpu = G.HipGpt(cfg, w, max_batch=cfg["batch"], max_seq_len=cfg["prompt"] + 8)
+    monkeypatch.setenv("TSHIP_GEMM_TILE", "0")
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
+
+    def launched(cache_write):
+        kernels = gpu.profile_symbols()
+        assert any("big_gemm3" in x for x in kernels) and not any("mid_gemm" in x for x in kernels), kernels
+        assert any("kv_write_frag_kernel" in x for x in kernels) == cache_write, kernels
+
     gpu.prefill(seqs)
+    launched(False)
     lg, k, v = gpu.logits(), gpu.get_kv(1, 0), gpu.get_kv(1, 1)
     assert np.isfinite(lg).all()
     monkeypatch.setenv("TSHIP_NO_KV_FUSE", "1")
     monkeypatch.setenv("TSHIP_PATCH_ROWS", "8")
     gpu.reset()
     gpu.prefill(seqs)
+    launched(True)
     assert np.array_equal(lg, gpu.logits()) and np.array_equal(k, gpu.get_kv(1, 0)) and np.array_equal(v, gpu.get_kv(1, 1))
     gpu.close()
