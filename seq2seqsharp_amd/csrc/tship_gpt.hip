@@ -122,7 +122,7 @@ struct TSHipGpt {
     DevBuf x, xn, o, a, part_qkv, part_h, part_f, logits, ids, d_pos, hidden;
     DevBuf moe_ws, topp_scratch, topp_uni, gen_buf, uni_buf, tile_count;
     DevBuf pw_lens, pw_ids, pw_x, pw_xn, pw_qkv, pw_o, pw_a, pw_f, pw_rowmap, pw_ssq, pw_rinv, pw_zero_bias, pw_moe;     // prefill workspace
-    DevBuf xn_rows, o_rows, a_rows, zero_qkv; // row-major activations of decode steps of more than 32 rows (xn, o and a hold packed ones)
+    DevBuf xn_rows, o_rows, a_rows, zero_qkv; // row-major activations of models that step by rows (xn, and o and a of the other models, hold packed ones)
     // prefill GEMMs whose tiles' K several blocks share: partial sums of up to 256 tiles x splits of 128 x 128, a counter per tile
     static constexpr long MID_XCHG_TILES = 256;
     DevBuf mid_xchg, mid_count;
@@ -932,11 +932,11 @@ static void embed_prepare(TSHipGpt* m, const int* d_ids, int B) {
 }
 // The same step of a model made for more than 32 rows (its packed activations are 64 or 128 rows at every batch): the
 // prefill's GEMMs (mid_gemm_f16_kernel) on row-major activations.  The kernels above read every activation fragment once per
-// column tile from L2, which outweighs the weights from two 32-row tiles on.  Still 5 launches per layer: the residual
-// projections need no split tail (the wavefronts of a block share K) and the consumers form 1 / rms themselves.
-// Measured, us per step at a context of 200, before -> now: 1B model, 33 / 64 / 96 / 128 rows 1125 / 1352 / 1914 / 2264 ->
-// 1060 / 1274 / 1362 / 1565; 8 layers of the 7B one, 40 / 128 rows 1258 / 2335 -> 1091 / 1716.  At 96 rows per layer of the 1B
-// model: QKV 9.7 -> 9.5, output 16.1 -> 8.9, up 28.7 -> 20.6, down (with a kernel that added its splits) 35.6 -> 25.
+// column tile from L2, which outweighs the weights from two 32-row tiles on.  Still 5 launches per layer: where blocks share the
+// K of a residual projection's tile, the last one adds it up and finishes it, and the consumers form 1 / rms themselves.
+// Measured, us per step at a context of 200, before -> now: 1B model, 33 / 64 / 96 / 128 rows 1072 / 1258 / 1780 / 2091 ->
+// 915 / 1021 / 1175 / 1309; 8 layers of the 7B one, 40 / 128 rows 1187 / 2153 -> 945 / 1358.  At 96 rows per layer of the 1B
+// model: QKV 9.0 -> 9.1, output 15.5 -> 8.7, up 27.7 -> 20.1, down (with a kernel that added its splits) 34.4 -> 13.2.
 static void decode_step_rows(TSHipGpt* m, const int* d_ids, int B) {
     auto& c = m->c;
     const int h = c.hidden, F = c.ffn_dim;
@@ -1470,8 +1470,6 @@ TSHIP_API int TSHip_GptCreate(const TSHipGptConfig* cfg, TSHipGpt** out) {
     const long hp = round_up(h, 32), qp = round_up(m->Nqkv, 32), Vp = round_up(c.vocab, 32);
     m->x.alloc((size_t)m->Bpad * h * sizeof(float));
     m->xn.alloc((size_t)m->Bpad * m->ldh * m->esz());
-    m->o.alloc((size_t)m->Bpad * m->ldh * m->esz());
-    m->a.alloc((size_t)m->Bpad * m->ldF * m->esz());
     m->part_qkv.alloc((size_t)16 * m->Bpad * qp * sizeof(float));
     m->part_h.alloc((size_t)16 * m->Bpad * hp * sizeof(float));
     if (!m->f16) m->part_f.alloc((size_t)16 * m->Bpad * m->F13 * sizeof(float));
@@ -1497,11 +1495,14 @@ TSHIP_API int TSHip_GptCreate(const TSHipGptConfig* cfg, TSHipGpt** out) {
         m->mid_xchg.alloc((size_t)TSHipGpt::MID_XCHG_TILES * 128 * 128 * sizeof(float));
         m->mid_count.alloc((size_t)TSHipGpt::MID_XCHG_TILES * sizeof(int));      // zero-filled; every use returns it to zero
     }
-    if (m->fused_norm && m->BT > 1) {
+    if (decode_by_rows(m.get())) {
         m->xn_rows.alloc((size_t)m->Bpad * m->ldh * m->esz());
         m->o_rows.alloc((size_t)m->Bpad * m->ldh * m->esz());
         m->a_rows.alloc((size_t)m->Bpad * m->ldF * m->esz());
         m->zero_qkv.alloc((size_t)qp * sizeof(float));
+    } else {
+        m->o.alloc((size_t)m->Bpad * m->ldh * m->esz());
+        m->a.alloc((size_t)m->Bpad * m->ldF * m->esz());
     }
     if (m->fused_norm) {
         m->ssq.alloc((size_t)(m->ln ? 2 : 1) * (hp / 32) * m->Bpad * sizeof(float));
@@ -1536,21 +1537,15 @@ TSHIP_API int TSHip_GptFinalize(TSHipGpt* m) {
     for (auto& n : m->expected)
         if (!m->seen.count(n)) throw Error("TSHip_GptFinalize: weight '" + n + "' was never set");
     // RMSNorm has no beta (Layers/RMSNormalization.cs:33-37): keep null pointers there
-    if (m->fused_norm) {
-        // deferred-norm path: the output projection runs unsplit with the residual tail in its epilogue; the FFN down
-        // projection keeps its K split only when K is long enough to need more than two passes per wavefront
-        for (auto& L : m->L) {
-            // residual-tail projections (N = hidden): split K so that the launch has about one block per compute unit
-            // (more blocks than that run in a second wave, which measured 2 us slower); BT > 1 keeps them unsplit
-            auto tail_ks = [&](const GemmW& w) {
-                if (m->BT != 1) return 1;
-                int ks = std::max(1, n_compute_units() / std::max(1, w.NT));
-                ks = std::min(ks, std::max(1, w.KT / 8));           // at least one k-tile per wavefront
-                return std::min(ks, 16);
-            };
-            L->wo.KS = tail_ks(L->wo);
-            L->w2.KS = m->BT == 1 ? tail_ks(L->w2) : (L->w2.KS <= 2 ? 1 : L->w2.KS);
-        }
+    if (m->fused_norm && !decode_by_rows(m)) {
+        // residual-tail projections (N = hidden): split K so that the launch has about one block per compute unit
+        // (more blocks than that run in a second wave, which measured 2 us slower)
+        auto tail_ks = [&](const GemmW& w) {
+            int ks = std::max(1, n_compute_units() / std::max(1, w.NT));
+            ks = std::min(ks, std::max(1, w.KT / 8));           // at least one k-tile per wavefront
+            return std::min(ks, 16);
+        };
+        for (auto& L : m->L) { L->wo.KS = tail_ks(L->wo); L->w2.KS = tail_ks(L->w2); }
     }
     if (m->ln) {
         // deferred LayerNorm: every consumer of a normalised row gets the norm's gamma and beta folded through its weights
