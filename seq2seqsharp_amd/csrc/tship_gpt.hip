@@ -10,6 +10,7 @@
 // with a preallocated compact KV cache instead of concat-and-reallocate, and with only token ids
 // crossing PCIe per step.
 #include "tship_gpt_kernels.h"
+#include "tship_f32_step.h"
 #include "tship_moe_kernels.h"
 #include "tship_sample_kernels.h"
 
@@ -129,6 +130,8 @@ struct TSHipGpt {
     DevBuf ssq;                    // deferred-norm path: per-column-tile sums of squares [h/32][Bpad]
     bool fused_norm = false;       // fp16 + dense layers (RMSNorm; LayerNorm up to 32 rows): residual/norm folded into the GEMM tails
     bool ln = false;               // that path with LayerNorm: tile sums of x beside the sums of squares, folded constants per consumer
+    bool f32_step = false;         // dense fp32 models of up to 32 rows: the decode step of tship_f32_step.h
+    DevBuf row_stats;              // statistics of the residual stream in that step, [32-column tile][32 rows]
     DevBuf ln_head;                // [2][round_up(vocab, 32)]: d then c of the vocabulary projection behind the final norm
     bool vt = false;               // fp16 cache with head_dim 64/128: keys and values stored fragment-major for the MFMA attention kernels
     long ML = 0;                   // cache rows per (sequence, KV head): max_seq_len rounded up to 32
@@ -685,39 +688,47 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
 }
 
 typedef void (*AttnKernel)(AttnArgs);
-enum AttnKind { ATTN_DECODE, ATTN_PREFILL, ATTN_PREFILL_TILES };      // (tiles: fp32 caches)
-template <typename CT, typename AT, int D, int G>
-static AttnKernel pick_attn_k(AttnKind kind) {
-    if constexpr (sizeof(CT) == 4) { if (kind == ATTN_PREFILL_TILES) return attn_prefill_f32_kernel<D, G>; }
-    return kind == ATTN_PREFILL ? attn_prefill_kernel<CT, AT, D, G> : attn_decode_kernel<CT, AT, D, G>;
-}
-template <typename CT, typename AT, int D>
-static AttnKernel pick_attn_g(int G, AttnKind kind) {
-    switch (G) {
-        case 1: return pick_attn_k<CT, AT, D, 1>(kind);
-        case 2: return pick_attn_k<CT, AT, D, 2>(kind);
-        case 3: return pick_attn_k<CT, AT, D, 3>(kind);
-        case 4: return pick_attn_k<CT, AT, D, 4>(kind);
-        case 5: return pick_attn_k<CT, AT, D, 5>(kind);
-        case 6: return pick_attn_k<CT, AT, D, 6>(kind);
-        case 7: return pick_attn_k<CT, AT, D, 7>(kind);
-        case 8: return pick_attn_k<CT, AT, D, 8>(kind);
-        default: throw Error("query heads per KV head must be 1 to 8");
+enum AttnKind { ATTN_PREFILL, ATTN_PREFILL_TILES };      // (tiles: fp32 caches)
+// calls f(head size, query heads per block) with both as compile-time constants
+template <typename F>
+static auto with_heads(int D, int G, F&& f) {
+    auto heads = [&](auto Dc) {
+        switch (G) {
+            case 1: return f(Dc, std::integral_constant<int, 1>{});
+            case 2: return f(Dc, std::integral_constant<int, 2>{});
+            case 3: return f(Dc, std::integral_constant<int, 3>{});
+            case 4: return f(Dc, std::integral_constant<int, 4>{});
+            case 5: return f(Dc, std::integral_constant<int, 5>{});
+            case 6: return f(Dc, std::integral_constant<int, 6>{});
+            case 7: return f(Dc, std::integral_constant<int, 7>{});
+            case 8: return f(Dc, std::integral_constant<int, 8>{});
+            default: throw Error("query heads per KV head must be 1 to 8");
+        }
+    };
+    switch (D) {
+        case 16: return heads(std::integral_constant<int, 16>{});
+        case 32: return heads(std::integral_constant<int, 32>{});
+        case 64: return heads(std::integral_constant<int, 64>{});
+        case 128: return heads(std::integral_constant<int, 128>{});
+        default: throw Error("head_dim must be 16, 32, 64 or 128");
     }
 }
 template <typename CT, typename AT>
 static AttnKernel pick_attn_d(int D, int G, AttnKind kind) {
-    switch (D) {
-        case 16: return pick_attn_g<CT, AT, 16>(G, kind);
-        case 32: return pick_attn_g<CT, AT, 32>(G, kind);
-        case 64: return pick_attn_g<CT, AT, 64>(G, kind);
-        case 128: return pick_attn_g<CT, AT, 128>(G, kind);
-        default: throw Error("head_dim must be 16, 32, 64 or 128");
-    }
+    return with_heads(D, G, [&](auto Dc, auto Gc) -> AttnKernel {
+        if constexpr (sizeof(CT) == 4) { if (kind == ATTN_PREFILL_TILES) return attn_prefill_f32_kernel<decltype(Dc)::value, decltype(Gc)::value>; }
+        return attn_prefill_kernel<CT, AT, decltype(Dc)::value, decltype(Gc)::value>;
+    });
+}
+// decode attention of caches without the fragment layout
+typedef void (*AttnStepKernel)(const int*, const float*, void*, void*, const float*, const float*, int, unsigned, int, int, AttnArgs);
+template <typename T>
+static AttnStepKernel pick_attn_step(int D, int G) {
+    return with_heads(D, G, [&](auto Dc, auto Gc) -> AttnStepKernel { return attn_decode_kernel<T, T, decltype(Dc)::value, decltype(Gc)::value>; });
 }
 template <int D>
-static AttnKernel pick_attn_mfma(int G, bool prefill, bool split, bool ragged, int nq = 1) {
-    if (prefill && nq == 2) {
+static AttnKernel pick_attn_mfma_prefill(int G, bool ragged, int nq) {
+    if (nq == 2) {
         if (ragged) {
             switch (G) {
                 case 1: return attn_mfma_prefill_kernel<D, 1, true, 2>;
@@ -735,7 +746,7 @@ static AttnKernel pick_attn_mfma(int G, bool prefill, bool split, bool ragged, i
             default: throw Error("internal: two column groups per wavefront are for 1, 2, 4 or 8 query heads per KV head");
         }
     }
-    if (prefill && ragged) {
+    if (ragged) {
         switch (G) {
             case 1: return attn_mfma_prefill_kernel<D, 1, true>;
             case 2: return attn_mfma_prefill_kernel<D, 2, true>;
@@ -748,8 +759,6 @@ static AttnKernel pick_attn_mfma(int G, bool prefill, bool split, bool ragged, i
             default: throw Error("query heads per KV head must be 1 to 8");
         }
     }
-    TSHIP_REQUIRE(prefill, "internal: the MFMA decode kernels are picked by pick_attn_mfma_decode");
-    (void)split;
     switch (G) {
         case 1: return attn_mfma_prefill_kernel<D, 1>;
         case 2: return attn_mfma_prefill_kernel<D, 2>;
@@ -803,9 +812,8 @@ template <int D>
 static AttnDecodeKernel pick_attn_mfma_decode(int G, bool split, bool sub) {
     return sub ? pick_attn_mfma_decode_s<D, true>(G, split) : pick_attn_mfma_decode_s<D, false>(G, split);
 }
-static AttnKernel pick_attn(TSHipGpt* m, AttnKind kind, bool split = false, bool ragged = false, int nq = 1) {
-    const bool prefill = kind != ATTN_DECODE;
-    if (m->vt) return m->D == 64 ? pick_attn_mfma<64>(m->G, prefill, split, ragged, nq) : pick_attn_mfma<128>(m->G, prefill, split, ragged, nq);
+static AttnKernel pick_attn_prefill(TSHipGpt* m, AttnKind kind, bool ragged = false, int nq = 1) {
+    if (m->vt) return m->D == 64 ? pick_attn_mfma_prefill<64>(m->G, ragged, nq) : pick_attn_mfma_prefill<128>(m->G, ragged, nq);
     return m->f16 ? pick_attn_d<half_t, half_t>(m->D, m->G, kind) : pick_attn_d<float, float>(m->D, m->G, kind);
 }
 // Kernel of an fp32 prefill's attention: a block per query that reads the cache with all lanes, or tiles of 32 columns on the
@@ -859,7 +867,14 @@ static int attn_splits(TSHipGpt* m, int B) {
     return (int)std::max<long>(1, std::min<long>(S, TSHipGpt::MAX_ATTN_SPLITS));
 }
 static void launch_attn_decode(TSHipGpt* m, AttnArgs a, int B) {
-    if (!m->vt) { launch(m, "attn_decode", pick_attn(m, ATTN_DECODE), dim3(m->Hv, B), dim3(1024), a); return; }
+    if (!m->vt) {
+        TSHIP_REQUIRE(a.max_len < (1L << 31) && a.ldq < (1L << 31) && a.split_stride < (1L << 31) && a.H < 256 && a.Hkv < 256 && a.KS < 256 && a.kv_sub >= 0 && a.kv_sub < 32,
+                      "internal: attention counts beyond their packed fields");
+        const unsigned counts = (unsigned)a.H | ((unsigned)a.Hkv << 8) | ((unsigned)a.KS << 16) | ((unsigned)a.kv_sub << 24);
+        launch(m, "attn_decode", m->f16 ? pick_attn_step<half_t>(m->D, m->G) : pick_attn_step<float>(m->D, m->G), dim3(m->Hv, B), dim3(1024),
+               a.d_pos, a.qkv, a.kcache, a.vcache, a.rope_cos, a.rope_sin, (int)a.max_len, counts, (int)a.ldq, (int)a.split_stride, a);
+        return;
+    }
     const int S = attn_splits(m, B);
     const unsigned threads = m->D == 128 ? 256 : 512;
     dim3 grid(m->c.n_kv_heads, B, m->SG);       // (one block per pair: the groups of a KV head's query heads on z)
@@ -1057,9 +1072,89 @@ static void decode_step_fn(TSHipGpt* m, const int* d_ids, int B) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// decode step of dense fp32 models (tship_f32_step.h)
+// ------------------------------------------------------------------------------------------------
+static int f32_step_range(int K, int KS) { return (int)round_up(ceil_div(K, KS), 4); }      // k per split, whole groups of four
+template <int SRC, int EPI>
+static void run_step_f32(TSHipGpt* m, const char* name, const GemmW& w, const float* X, long ldx, int rows, F32StepArgs a) {
+    a.X = X; a.W = w.buf.as<float>(); a.ldx = ldx; a.ldb = w.ld; a.K = w.K; a.N = w.N; a.NT = (int)ceil_div(w.N, 32); a.rows = rows;
+    a.KS = EPI == F32_BIAS ? 1 : w.KS; a.kper = f32_step_range(w.K, a.KS);
+    a.st = (const floatx2*)m->row_stats.p; a.st_nt = m->c.hidden / 32; a.inv_h = 1.0f / (float)m->c.hidden; a.eps = m->c.norm_eps; a.ln = m->c.norm_type;
+    const bool vec = ((w.N | w.ld) & 3) == 0;
+    constexpr bool ACT = SRC == F32_ACT || SRC == F32_GATE;
+    TSHIP_REQUIRE(rows <= F32_STEP_ROWS && w.K % 4 == 0 && ldx % 4 == 0 && a.KS <= 16 && (vec || EPI == F32_BIAS), "internal: shape of an fp32 decode projection");
+    if (EPI == F32_TAIL)
+        TSHIP_REQUIRE((size_t)a.KS * a.NT * 32 * round_up(rows, 16) * sizeof(float) <= m->part_h.bytes && (size_t)2 * a.NT * sizeof(int) <= m->tile_count.bytes,
+                      "internal: split-K exchange area too small");
+    auto go = [&](auto MRc, auto Uc) {
+        constexpr int MR = decltype(MRc)::value, U = decltype(Uc)::value;
+        const dim3 grid((unsigned)round_up(a.NT, 8), (unsigned)a.KS, (unsigned)ceil_div(rows, MR));
+        auto kernel = step_gemm_f32_kernel<MR, U, SRC, EPI>;
+        if constexpr (EPI == F32_BIAS) { if (!vec) kernel = step_gemm_f32_kernel<MR, U, SRC, EPI, false>; }
+        launch(m, name, kernel, grid, dim3(256), a.W, a.X, ACT ? (const floatx2*)a.X2 : a.st, (int)a.ldb, (int)a.ldx, a.g, a.b, a.K, a.kper, a.NT, a.rows, a);
+    };
+    typedef std::integral_constant<int, 1> c1; typedef std::integral_constant<int, 2> c2; typedef std::integral_constant<int, 4> c4;
+    typedef std::integral_constant<int, 8> c8; typedef std::integral_constant<int, 16> c16;
+    // groups of four k in flight per thread (128 k of the block each): the block's range in one batch; four only without a norm
+    // (its operands take the registers: 6.4 against 5.7 us at 8 x 768 x 3072) and up to eight rows
+    auto batches = [&](auto MRc) {
+        if constexpr (EPI == F32_BIAS) go(MRc, c2{});
+        else if (a.kper <= 128) go(MRc, c1{});
+        else if (a.kper <= 256 || SRC == F32_NORM || decltype(MRc)::value > 8) go(MRc, c2{});
+        else if constexpr (SRC != F32_NORM && decltype(MRc)::value <= 8) go(MRc, c4{});
+    };
+    if (rows == 1) batches(c1{}); else if (rows == 2) batches(c2{}); else if (rows <= 4) batches(c4{}); else if (rows <= 8) batches(c8{}); else batches(c16{});
+}
+static F32EmbedArgs f32_embed_args(TSHipGpt* m, const int* d_ids) {
+    F32EmbedArgs a;
+    a.x = m->x.as<float>(); a.ldx = m->c.hidden; a.h = m->c.hidden; a.ids = d_ids; a.emb = m->emb.as<float>(); a.emb_scale = (float)std::sqrt((double)m->c.hidden);
+    a.seg = m->seg.as<float>();      // (a cached decode step feeds one token per sequence: segment 0, Decoder.cs:661-673)
+    a.st = (floatx2*)m->row_stats.p;
+    return a;
+}
+static void decode_step_f32(TSHipGpt* m, const int* d_ids, int B) {
+    auto& c = m->c;
+    const int h = c.hidden;
+    const long qp = round_up(m->Nqkv, 32), qstride = (long)m->Bpad * qp, fstride = (long)m->Bpad * m->F13, Vp = round_up(c.vocab, 32);
+    auto norm = [&](const DevBuf& gamma, const DevBuf& beta) { F32StepArgs e; std::memset(&e, 0, sizeof(e)); e.g = gamma.as<float>(); e.b = beta.as<float>(); return e; };
+    auto tail = [&](F32StepArgs& e, const DevBuf& bias) {
+        e.bias = bias.as<float>(); e.x = m->x.as<float>(); e.ld_x = h; e.st_out = (floatx2*)m->row_stats.p; e.xchg = m->part_h.as<float>(); e.count = m->tile_count.as<int>();
+    };
+    if (m->embed_done) m->embed_done = false;
+    else launch(m, "embed_prepare", f32_embed_kernel, dim3(B), dim3(256), f32_embed_args(m, d_ids));
+    for (int l = 0; l < c.n_layers; ++l) {
+        LayerW& L = *m->L[l];
+        F32StepArgs e = norm(L.n1_g, L.n1_b);
+        e.out = m->part_qkv.as<float>(); e.ld_out = qp; e.split_stride = qstride;
+        run_step_f32<F32_NORM, F32_PARTIAL>(m, "gemm_qkv", L.qkv, m->x.as<float>(), h, B, e);
+        AttnArgs a = attn_args(m, L);
+        a.qkv = m->part_qkv.as<float>(); a.KS = L.qkv.KS; a.split_stride = qstride; a.ldq = qp;
+        a.out = m->o.p; a.ld_out = m->ldh;
+        launch_attn_decode(m, a, B);
+        std::memset(&e, 0, sizeof(e));
+        tail(e, L.bo);
+        run_step_f32<F32_PLAIN, F32_TAIL>(m, "gemm_wo", L.wo, m->o.as<float>(), m->ldh, B, e);
+        e = norm(L.n2_g, L.n2_b);
+        e.out = m->part_f.as<float>(); e.ld_out = m->F13; e.split_stride = fstride;
+        run_step_f32<F32_NORM, F32_PARTIAL>(m, "gemm_ffn13", L.w13, m->x.as<float>(), h, B, e);
+        std::memset(&e, 0, sizeof(e));
+        const float* up = m->part_f.as<float>();
+        e.X2 = up + (L.w13.KS - 1) * fstride; e.g = L.b1.as<float>(); e.b = L.b3.as<float>(); e.act = c.act;
+        tail(e, L.b2);
+        if (m->gated) run_step_f32<F32_GATE, F32_TAIL>(m, "gemm_ffn2", L.w2, up, m->F13, B, e);
+        else run_step_f32<F32_ACT, F32_TAIL>(m, "gemm_ffn2", L.w2, up, m->F13, B, e);
+    }
+    F32StepArgs e = norm(m->fn_g, m->fn_b);
+    e.xn_out = m->xn.as<float>(); e.ld_xn = m->ldh; e.out = m->logits.as<float>(); e.ld_out = Vp; e.bias = m->head_b.as<float>(); e.advance_pos = m->d_pos.as<int>();
+    run_step_f32<F32_NORM, F32_BIAS>(m, "gemm_head", m->head, m->x.as<float>(), h, B, e);
+    m->pos += 1;
+}
+
+// ------------------------------------------------------------------------------------------------
 // decode step: tokens (device int32 [batch]) -> logits (device fp32 [batch][vocab])
 // ------------------------------------------------------------------------------------------------
 static void decode_step(TSHipGpt* m, const int* d_ids, int B) {
+    if (m->f32_step) { decode_step_f32(m, d_ids, B); return; }
     if (decode_by_rows(m)) { decode_step_rows(m, d_ids, B); return; }
     if (m->fused_norm) { decode_step_fn(m, d_ids, B); return; }
     auto& c = m->c;
@@ -1296,12 +1391,12 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             int nq = (m->D == 128 && 16 % m->G == 0 && (long)ceil_div(Tp, (16 / m->G) * 16) * m->Hv * B >= 2048) ? 2 : 1;
             if (g_hooks.attn_nq && 16 % m->G == 0) nq = g_hooks.attn_nq;
             const int per_block = (16 / m->G) * 8 * nq;
-            launch(m, "p_attn", pick_attn(m, ATTN_PREFILL, false, host_lens != nullptr, nq), dim3((unsigned)ceil_div(Tp, per_block), m->Hv, B), dim3(512), aa);
+            launch(m, "p_attn", pick_attn_prefill(m, ATTN_PREFILL, host_lens != nullptr, nq), dim3((unsigned)ceil_div(Tp, per_block), m->Hv, B), dim3(512), aa);
         }
         else if (!m->f16 && !f32_attn_by_query(m, B, Tp, pos0)) {
             const unsigned shm = m->D == 128 ? attn_prefill_f32_shm<128>() : m->D == 64 ? attn_prefill_f32_shm<64>() : m->D == 32 ? attn_prefill_f32_shm<32>() : attn_prefill_f32_shm<16>();
-            launch_shm(m, "p_attn", pick_attn(m, ATTN_PREFILL_TILES), dim3((unsigned)ceil_div(Tp, 32 / m->G), m->Hv, B), dim3(256), shm, aa);
-        } else launch(m, "p_attn", pick_attn(m, ATTN_PREFILL), dim3(Tp, m->Hv, B), dim3(256), aa);
+            launch_shm(m, "p_attn", pick_attn_prefill(m, ATTN_PREFILL_TILES), dim3((unsigned)ceil_div(Tp, 32 / m->G), m->Hv, B), dim3(256), shm, aa);
+        } else launch(m, "p_attn", pick_attn_prefill(m, ATTN_PREFILL), dim3(Tp, m->Hv, B), dim3(256), aa);
         ResidNormArgs a2 = rn;
         a2.gamma = L.n2_g.as<float>(); a2.beta = L.n2_b.as<float>();
         if (m->f16) {
@@ -1491,6 +1586,11 @@ TSHIP_API int TSHip_GptCreate(const TSHipGptConfig* cfg, TSHipGpt** out) {
     // (LayerNorm: batches of up to 32 rows; the tails of larger batches do not store the tiles' plain sums)
     m->fused_norm = m->f16 && c.n_experts <= 1 && (c.norm_type == 0 || m->BT == 1);
     m->ln = m->fused_norm && c.norm_type == 1;
+    m->f32_step = !m->f16 && c.n_experts <= 1 && m->BT == 1 && h % 32 == 0 && h <= 32 * F32_STEP_TILES && c.ffn_dim % 32 == 0 && m->Nqkv % 32 == 0;
+    if (m->f32_step) {
+        m->row_stats.alloc((size_t)F32_STEP_TILES * F32_STEP_ROWS * sizeof(floatx2));
+        m->tile_count.alloc((size_t)(2 * F32_STEP_TILES) * sizeof(int));     // (a counter per tile and group of 16 rows) zero-filled; every use returns it to zero
+    }
     if (m->f16) {
         m->mid_xchg.alloc((size_t)TSHipGpt::MID_XCHG_TILES * 128 * 128 * sizeof(float));
         m->mid_count.alloc((size_t)TSHipGpt::MID_XCHG_TILES * sizeof(int));      // zero-filled; every use returns it to zero
@@ -1546,6 +1646,20 @@ TSHIP_API int TSHip_GptFinalize(TSHipGpt* m) {
             return std::min(ks, 16);
         };
         for (auto& L : m->L) { L->wo.KS = tail_ks(L->wo); L->w2.KS = tail_ks(L->w2); }
+    }
+    if (m->f32_step) {
+        // Blocks per column tile.  Projections that store partial sums: up to one block per compute unit (the next kernel adds
+        // them on its way; the activation two at most).  Projections with a tail: fewer, every split costs the last block
+        // an exchange.  us per launch at 768 x 768 for 4 / 6 / 8 / 10 splits 5.5 / 5.5 / 5.8 / 6.2 (8 rows), 3072 x 768 for
+        // 6 / 8 / 10 / 16 6.9 / 6.9 / 7.3 / 7.9, 512 x 512 for 4 / 8 / 16 4.2 / 5.0 / 6.4 (one row).
+        auto splits = [&](GemmW& w, int most) { w.KS = (int)ceil_div(w.K, f32_step_range(w.K, std::max(1, std::min(most, w.K / 128)))); };
+        for (auto& L : m->L) {
+            const int ncu = std::max(1, n_compute_units()), tiles_h = (int)(m->c.hidden / 32);
+            splits(L->qkv, std::min(16, ncu / (int)ceil_div(L->qkv.N, 32)));
+            splits(L->w13, std::min(2, ncu / (int)ceil_div(L->w13.N, 32)));
+            splits(L->wo, std::min(8, 3 * ncu / 4 / tiles_h));
+            splits(L->w2, std::min(8, 3 * ncu / 4 / tiles_h));
+        }
     }
     if (m->ln) {
         // deferred LayerNorm: every consumer of a normalised row gets the norm's gamma and beta folded through its weights

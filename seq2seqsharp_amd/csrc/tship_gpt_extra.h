@@ -246,6 +246,11 @@ static void sample_tokens(TSHipGpt* m, int mode, float top_p, float temperature,
             m->embed_done = true;
             return;
         }
+        if (embed_next && m->f32_step) {
+            launch(m, "greedy_embed", greedy_embed_f32_kernel, dim3(B), dim3(1024), lg, Vp, m->c.vocab, ids, gen_out, d_step, lastp, m->last_ld, dpos, bl, f32_embed_args(m, ids));
+            m->embed_done = true;
+            return;
+        }
         launch(m, "greedy", greedy_kernel, dim3(B), dim3(1024), lg, Vp, m->c.vocab, ids, gen_out, d_step, lastp, m->last_ld, dpos, bl);
         return;
     }

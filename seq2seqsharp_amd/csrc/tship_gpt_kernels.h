@@ -2351,108 +2351,11 @@ struct AttnArgs {
     int kv_sub;
 };
 
-// Single-query attention of G query heads that share one KV head over T cached positions.
-// Lanes are grouped LPR to a cache row (16-byte loads, head_dim contiguous); a wavefront covers RPW rows per
-// load and keeps UR loads of keys and of values in flight, refilling each register as soon as it is consumed.
-// Every lane group keeps its own online-softmax state over the rows it visits; the groups of a wavefront are
-// merged with lane shuffles and the NW wavefronts through LDS.
-// sQ: LDS [G][D] queries, already rotated and scaled.  Result (fp32) is written to sOut [G][D] in LDS.
-// ONCE: the launch reads every cached row once (a decode step), see load_once; a prefill's blocks share them through L2.
-template <typename CT, int D, int G, int NW, bool ONCE = false>
-__device__ __forceinline__ void attn_core(const float* sQ, const CT* Kb, const CT* Vb, int T, float* sM, float* sL, float* sAcc,
-                                          float* sOut, bool quant = false) {
-    constexpr int EPL = 16 / (int)sizeof(CT);
-    constexpr int LPR = D / EPL;
-    constexpr int RPW = 64 / LPR;
-    constexpr int UR = 4;
-    constexpr int SWEEP = NW * RPW * UR;
-    typedef CT vec_t __attribute__((ext_vector_type(EPL)));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int sub = lane % LPR, rg = lane / LPR;
-    auto kv_load = [](const vec_t* p) { if constexpr (ONCE) return load_once(p); else return *p; };
-
-    // fp16 cache: queries are kept as packed halves and the dot product uses v_dot2_f32_f16 (fp32 accumulate);
-    // fp32 cache: plain fp32 multiply-add
-    constexpr bool H16 = sizeof(CT) == 2;
-    float q[H16 ? 1 : G][H16 ? 1 : EPL];
-    half2v q2[H16 ? G : 1][H16 ? EPL / 2 : 1];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        if constexpr (H16) {
-#pragma unroll
-            for (int e = 0; e < EPL / 2; ++e) {
-                q2[g][e][0] = (half_t)sQ[g * D + sub * EPL + 2 * e];
-                q2[g][e][1] = (half_t)sQ[g * D + sub * EPL + 2 * e + 1];
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) q[g][e] = sQ[g * D + sub * EPL + e];
-        }
-    }
-    float m[G], l[G], acc[G][EPL];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        m[g] = -INFINITY; l[g] = 0.0f;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
-    }
-    vec_t kv[UR], vv[UR];
-    int tt[UR];
-#pragma unroll
-    for (int u = 0; u < UR; ++u) {
-        tt[u] = (u * NW + wave) * RPW + rg;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) { kv[u][e] = (CT)0.0f; vv[u][e] = (CT)0.0f; }
-        if (tt[u] < T) {
-            kv[u] = kv_load((const vec_t*)(Kb + (long)tt[u] * D + sub * EPL));
-            vv[u] = kv_load((const vec_t*)(Vb + (long)tt[u] * D + sub * EPL));
-        }
-    }
-    for (int base = 0; base < T; base += SWEEP) {
-#pragma unroll
-        for (int u = 0; u < UR; ++u) {
-            const bool ok = tt[u] < T;
-            const vec_t kc = kv[u];
-            float vf[EPL];
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) vf[e] = (float)vv[u][e];
-            tt[u] += SWEEP;
-            if (tt[u] < T) {
-                kv[u] = kv_load((const vec_t*)(Kb + (long)tt[u] * D + sub * EPL));
-                vv[u] = kv_load((const vec_t*)(Vb + (long)tt[u] * D + sub * EPL));
-            }
-            float s[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float d = 0.0f;
-                if constexpr (H16) {
-#pragma unroll
-                    for (int e = 0; e < EPL / 2; ++e) {
-                        half2v kp; kp[0] = (half_t)kc[2 * e]; kp[1] = (half_t)kc[2 * e + 1];
-                        d = __builtin_amdgcn_fdot2(q2[g][e], kp, d, false);
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < EPL; ++e) d = fmaf(q[g][e], (float)kc[e], d);
-                }
-#pragma unroll
-                for (int o = LPR / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
-                s[g] = quant ? d + (-30000.0f) : d;      // (a fully masked row: the float32 addition of the mask value rounds the score)
-            }
-            if (ok) {
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    float mn = fmaxf(m[g], s[g]);
-                    float corr = __expf(m[g] - mn);
-                    float p = __expf(s[g] - mn);
-                    l[g] = l[g] * corr + p;
-#pragma unroll
-                    for (int e = 0; e < EPL; ++e) acc[g][e] = acc[g][e] * corr + p * vf[e];
-                    m[g] = mn;
-                }
-            }
-        }
-    }
+// The online-softmax states (m, l, acc) of the row groups of a block's NW wavefronts (attn_core), merged: [G][D] results to sOut.
+template <typename CT, int D, int G, int NW>
+__device__ __forceinline__ void attn_merge(float (&m)[G], float (&l)[G], float (&acc)[G][16 / (int)sizeof(CT)], float* sM, float* sL, float* sAcc, float* sOut) {
+    constexpr int EPL = 16 / (int)sizeof(CT), LPR = D / EPL;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane % LPR, rg = lane / LPR;
     // merge the row groups of this wavefront
 #pragma unroll
     for (int o = LPR; o < 64; o <<= 1) {
@@ -2492,6 +2395,109 @@ __device__ __forceinline__ void attn_core(const float* sQ, const CT* Kb, const C
     __syncthreads();
 }
 
+
+// Single-query attention of G query heads that share one KV head over T cached positions.
+// Lanes are grouped LPR to a cache row (16-byte loads, head_dim contiguous); a wavefront covers RPW rows per
+// load and keeps UR loads of keys and of values in flight, refilling each register as soon as it is consumed.
+// Every lane group keeps its own online-softmax state over the rows it visits; the groups of a wavefront are
+// merged with lane shuffles and the NW wavefronts through LDS.
+// sQ: LDS [G][D] queries, already rotated and scaled.  Result (fp32) is written to sOut [G][D] in LDS.
+template <typename CT, int D, int G, int NW>
+__device__ __forceinline__ void attn_core(const float* sQ, const CT* Kb, const CT* Vb, int T, float* sM, float* sL, float* sAcc,
+                                          float* sOut, bool quant = false) {
+    constexpr int EPL = 16 / (int)sizeof(CT);
+    constexpr int LPR = D / EPL;
+    constexpr int RPW = 64 / LPR;
+    constexpr int UR = 4;
+    constexpr int SWEEP = NW * RPW * UR;
+    typedef CT vec_t __attribute__((ext_vector_type(EPL)));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int sub = lane % LPR, rg = lane / LPR;
+    // fp16 cache: queries are kept as packed halves and the dot product uses v_dot2_f32_f16 (fp32 accumulate);
+    // fp32 cache: plain fp32 multiply-add
+    constexpr bool H16 = sizeof(CT) == 2;
+    float q[H16 ? 1 : G][H16 ? 1 : EPL];
+    half2v q2[H16 ? G : 1][H16 ? EPL / 2 : 1];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        if constexpr (H16) {
+#pragma unroll
+            for (int e = 0; e < EPL / 2; ++e) {
+                q2[g][e][0] = (half_t)sQ[g * D + sub * EPL + 2 * e];
+                q2[g][e][1] = (half_t)sQ[g * D + sub * EPL + 2 * e + 1];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) q[g][e] = sQ[g * D + sub * EPL + e];
+        }
+    }
+    float m[G], l[G], acc[G][EPL];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        m[g] = -INFINITY; l[g] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
+    }
+    vec_t kv[UR], vv[UR];
+    int tt[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+        tt[u] = (u * NW + wave) * RPW + rg;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) { kv[u][e] = (CT)0.0f; vv[u][e] = (CT)0.0f; }
+        if (tt[u] < T) {
+            kv[u] = *(const vec_t*)(Kb + (long)tt[u] * D + sub * EPL);
+            vv[u] = *(const vec_t*)(Vb + (long)tt[u] * D + sub * EPL);
+        }
+    }
+    for (int base = 0; base < T; base += SWEEP) {
+#pragma unroll
+        for (int u = 0; u < UR; ++u) {
+            const bool ok = tt[u] < T;
+            const vec_t kc = kv[u];
+            float vf[EPL];
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) vf[e] = (float)vv[u][e];
+            tt[u] += SWEEP;
+            if (tt[u] < T) {
+                kv[u] = *(const vec_t*)(Kb + (long)tt[u] * D + sub * EPL);
+                vv[u] = *(const vec_t*)(Vb + (long)tt[u] * D + sub * EPL);
+            }
+            float s[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                float d = 0.0f;
+                if constexpr (H16) {
+#pragma unroll
+                    for (int e = 0; e < EPL / 2; ++e) {
+                        half2v kp; kp[0] = (half_t)kc[2 * e]; kp[1] = (half_t)kc[2 * e + 1];
+                        d = __builtin_amdgcn_fdot2(q2[g][e], kp, d, false);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) d = fmaf(q[g][e], (float)kc[e], d);
+                }
+#pragma unroll
+                for (int o = LPR / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+                s[g] = quant ? d + (-30000.0f) : d;      // (a fully masked row: the float32 addition of the mask value rounds the score)
+            }
+            if (ok) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    float mn = fmaxf(m[g], s[g]);
+                    float corr = __expf(m[g] - mn);
+                    float p = __expf(s[g] - mn);
+                    l[g] = l[g] * corr + p;
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) acc[g][e] = acc[g][e] * corr + p * vf[e];
+                    m[g] = mn;
+                }
+            }
+        }
+    }
+    attn_merge<CT, D, G, NW>(m, l, acc, sM, sL, sAcc, sOut);
+}
+
 template <typename CT, int D, int G, int NW>
 struct AttnSmem {
     float in[(G + 2) * D];
@@ -2506,58 +2512,169 @@ struct AttnSmem {
 // key/value to the cache in place, then attends over pos+1 positions.
 // Replaces: AsContiguous head split, RoPE, GQA Expand, Concate(cache), MulBatch, Softmax, MulBatch, transpose
 // (Seq2SeqSharp/Layers/GroupQueryAttention.cs:121-224, Layers/MultiHeadAttention.cs:133-230).
+// A small launch (8 heads, 100 positions) is a chain of round trips, so they are taken side by side: the leading arguments
+// are preloaded, the position heads the longest chain, and the first sweep of cached rows (16 wavefronts x 4 requests each)
+// and the rotation are requested before the partial sums are waited for; the new row is attended from LDS, not read back.
 template <typename CT, typename AT, int D, int G>
-__global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs a) {
+__global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict__ d_pos_, const float* __restrict__ qkv_, void* kcache_, void* vcache_,
+                                                           const float* __restrict__ rope_cos_, const float* __restrict__ rope_sin_, int max_len_, unsigned counts_, int ldq_, int split_stride_, AttnArgs a) {
     constexpr int NW = 16, NTH = NW * 64;
+    constexpr int EPL = 16 / (int)sizeof(CT), LPR = D / EPL, RPW = 64 / LPR, UR = 4, SWEEP = NW * RPW * UR;
+    typedef CT vec_t __attribute__((ext_vector_type(EPL)));
     __shared__ AttnSmem<CT, D, G, NW> sm;
-    const int kvh = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
-    const int kvc = a.kv_sub > 1 ? kvh / a.kv_sub : kvh;       // the KV head whose cache this group of query heads reads
-    const int pos = *a.d_pos;
-    const int HD = a.H * D, GD = a.Hkv * D;
-    float rinv = 1.0f, mean = 0.0f;
-    if (a.ssq) {
-        float s = 0.0f;
-        for (int tt = (t & 63); tt < a.ssq_nt; tt += 64) s += a.ssq[(long)tt * a.ssq_ld + b];
-        s = wave_sum(s);                                   // same butterfly in every wavefront: identical result
-        if (a.ln) {
-            float sv = 0.0f;
-            for (int tt = (t & 63); tt < a.ssq_nt; tt += 64) sv += a.ssq[(long)(a.ssq_nt + tt) * a.ssq_ld + b];
-            mean = wave_sum(sv) * a.inv_h;
-            rinv = 1.0f / sqrtf(fmaxf(s * a.inv_h - mean * mean, 0.0f) + a.eps);
-        } else {
-            rinv = 1.0f / sqrtf(s * a.inv_h + a.eps);
+    __shared__ __align__(16) CT s_k[D], s_v[D];
+    const int H = counts_ & 255, Hkv = (counts_ >> 8) & 255, KS = (counts_ >> 16) & 255, kv_sub = counts_ >> 24;      // (as in AttnArgs)
+    const int kvh = blockIdx.x, b = blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6, sub = lane % LPR, rg = lane / LPR;
+    const int kvc = kv_sub > 1 ? kvh / kv_sub : kvh;       // the KV head whose cache this group of query heads reads
+    const int pos = *d_pos_;
+    CT* Kb = (CT*)kcache_ + ((long)b * Hkv + kvc) * max_len_ * D;
+    CT* Vb = (CT*)vcache_ + ((long)b * Hkv + kvc) * max_len_ * D;
+    const int HD = H * D, GD = Hkv * D;
+    // the projection's sums: thread t takes columns t and t + 1024 of the group's (G + 2) D
+    constexpr int NC = ((G + 2) * D + NTH - 1) / NTH, NP = ((G + 1) * D / 2 + NTH - 1) / NTH;
+    int col[NC]; float p0[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int idx = min(t + i * NTH, (G + 2) * D - 1);
+        col[i] = idx < G * D ? kvh * G * D + idx : idx < (G + 1) * D ? HD + kvc * D + (idx - G * D) : HD + GD + kvc * D + (idx - (G + 1) * D);
+        p0[i] = qkv_[(long)b * ldq_ + col[i]];
+    }
+    float rc[NP], rs[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int p = (t + i * NTH) % (D / 2);
+        rc[i] = rope_cos_ ? rope_cos_[(long)pos * (D / 2) + p] : 1.0f; rs[i] = rope_cos_ ? rope_sin_[(long)pos * (D / 2) + p] : 0.0f;
+    }
+    vec_t kv[UR], vv[UR];
+    int tt[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+        tt[u] = (u * NW + wave) * RPW + rg;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) { kv[u][e] = (CT)0.0f; vv[u][e] = (CT)0.0f; }
+        if (tt[u] < pos) {
+            kv[u] = load_once((const vec_t*)(Kb + (long)tt[u] * D + sub * EPL));
+            vv[u] = load_once((const vec_t*)(Vb + (long)tt[u] * D + sub * EPL));
         }
     }
-    for (int idx = t; idx < (G + 2) * D; idx += NTH) {
-        int col;
-        if (idx < G * D) col = kvh * G * D + idx;
-        else if (idx < (G + 1) * D) col = HD + kvc * D + (idx - G * D);
-        else col = HD + GD + kvc * D + (idx - (G + 1) * D);
+    float rinv = 1.0f, mean = 0.0f;
+    if constexpr (sizeof(CT) == 2) {
+        if (a.ssq) {
+            float s = 0.0f;
+            for (int tt = lane; tt < a.ssq_nt; tt += 64) s += a.ssq[(long)tt * a.ssq_ld + b];
+            s = wave_sum(s);                                   // same butterfly in every wavefront: identical result
+            if (a.ln) {
+                float sv = 0.0f;
+                for (int tt = lane; tt < a.ssq_nt; tt += 64) sv += a.ssq[(long)(a.ssq_nt + tt) * a.ssq_ld + b];
+                mean = wave_sum(sv) * a.inv_h;
+                rinv = 1.0f / sqrtf(fmaxf(s * a.inv_h - mean * mean, 0.0f) + a.eps);
+            } else {
+                rinv = 1.0f / sqrtf(s * a.inv_h + a.eps);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
         // split-K partials in index order, eight requested at a time (unconditionally, the index clamped to the last split)
-        float s = a.qkv[(long)b * a.ldq + col];
-        for (int k = 1; k < a.KS; k += 8) {
+        float s = p0[i];
+        for (int k = 1; k < KS; k += 8) {
             float pk[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pk[j] = a.qkv[min(k + j, a.KS - 1) * a.split_stride + (long)b * a.ldq + col];
+            for (int j = 0; j < 8; ++j) pk[j] = qkv_[min(k + j, KS - 1) * (long)split_stride_ + (long)b * ldq_ + col[i]];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) if (k + j < a.KS) s += pk[j];
+            for (int j = 0; j < 8; ++j) if (k + j < KS) s += pk[j];
         }
-        sm.in[idx] = a.ln ? (s - mean * a.bias[a.ldq + col]) * rinv + a.bias[col] : s * rinv + a.bias[col];
+        if (t + i * NTH < (G + 2) * D) sm.in[t + i * NTH] = a.ln ? (s - mean * a.bias[ldq_ + col[i]]) * rinv + a.bias[col[i]] : s * rinv + a.bias[col[i]];
     }
     __syncthreads();
-    CT* Kb = (CT*)a.kcache + ((long)b * a.Hkv + kvc) * a.max_len * D;
-    CT* Vb = (CT*)a.vcache + ((long)b * a.Hkv + kvc) * a.max_len * D;
-    for (int p = t; p < (G + 1) * D / 2; p += NTH) {
-        int vec = p / (D / 2), i = p % (D / 2);
-        float x0 = sm.in[vec * D + 2 * i], x1 = sm.in[vec * D + 2 * i + 1], y0 = x0, y1 = x1;
-        if (a.rope_cos) rope_pair(x0, x1, a.rope_cos[(long)pos * (D / 2) + i], a.rope_sin[(long)pos * (D / 2) + i], y0, y1);
-        if (vec < G) { sm.q[vec * D + 2 * i] = a.scale * y0; sm.q[vec * D + 2 * i + 1] = a.scale * y1; }
-        else { Kb[(long)pos * D + 2 * i] = (CT)y0; Kb[(long)pos * D + 2 * i + 1] = (CT)y1; }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int p = t + i * NTH;
+        if (p < (G + 1) * D / 2) {
+            const int vec = p / (D / 2), j = p % (D / 2);
+            const float x0 = sm.in[vec * D + 2 * j], x1 = sm.in[vec * D + 2 * j + 1];
+            float y0 = x0, y1 = x1;
+            if (rope_cos_) rope_pair(x0, x1, rc[i], rs[i], y0, y1);
+            if (vec < G) { sm.q[vec * D + 2 * j] = a.scale * y0; sm.q[vec * D + 2 * j + 1] = a.scale * y1; }
+            else {
+                CT* dst = Kb + (long)pos * D + 2 * j;
+                s_k[2 * j] = dst[0] = (CT)y0; s_k[2 * j + 1] = dst[1] = (CT)y1;
+            }
+        }
     }
-    for (int d = t; d < D; d += NTH) Vb[(long)pos * D + d] = (CT)sm.in[(G + 1) * D + d];
-    __threadfence_block();
+    for (int d = t; d < D; d += NTH) Vb[(long)pos * D + d] = s_v[d] = (CT)sm.in[(G + 1) * D + d];
     __syncthreads();
-    attn_core<CT, D, G, NW, true>(sm.q, Kb, Vb, pos + 1, sm.m, sm.l, sm.acc, sm.out);
+
+    // fp16 cache: queries as packed halves and v_dot2_f32_f16 (fp32 accumulate); fp32 cache: fp32 multiply-add
+    constexpr bool H16 = sizeof(CT) == 2;
+    float q[H16 ? 1 : G][H16 ? 1 : EPL];
+    half2v q2[H16 ? G : 1][H16 ? EPL / 2 : 1];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        if constexpr (H16) {
+#pragma unroll
+            for (int e = 0; e < EPL / 2; ++e) {
+                q2[g][e][0] = (half_t)sm.q[g * D + sub * EPL + 2 * e];
+                q2[g][e][1] = (half_t)sm.q[g * D + sub * EPL + 2 * e + 1];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) q[g][e] = sm.q[g * D + sub * EPL + e];
+        }
+    }
+    float m[G], l[G], acc[G][EPL];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        m[g] = -INFINITY; l[g] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
+    }
+    auto take = [&](const vec_t& kc, const vec_t& vc, bool ok) {
+        float s[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            float d = 0.0f;
+            if constexpr (H16) {
+#pragma unroll
+                for (int e = 0; e < EPL / 2; ++e) {
+                    half2v kp; kp[0] = (half_t)kc[2 * e]; kp[1] = (half_t)kc[2 * e + 1];
+                    d = __builtin_amdgcn_fdot2(q2[g][e], kp, d, false);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) d = fmaf(q[g][e], (float)kc[e], d);
+            }
+#pragma unroll
+            for (int o = LPR / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+            s[g] = d;
+        }
+        if (ok) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const float mn = fmaxf(m[g], s[g]);
+                const float corr = __expf(m[g] - mn), p = __expf(s[g] - mn);
+                l[g] = l[g] * corr + p;
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) acc[g][e] = acc[g][e] * corr + p * (float)vc[e];
+                m[g] = mn;
+            }
+        }
+    };
+    for (int base = 0; base < pos; base += SWEEP) {
+#pragma unroll
+        for (int u = 0; u < UR; ++u) {
+            const bool ok = tt[u] < pos;
+            const vec_t kc = kv[u], vc = vv[u];
+            tt[u] += SWEEP;
+            if (tt[u] < pos) {
+                kv[u] = load_once((const vec_t*)(Kb + (long)tt[u] * D + sub * EPL));
+                vv[u] = load_once((const vec_t*)(Vb + (long)tt[u] * D + sub * EPL));
+            }
+            if ((base / RPW + u * NW + wave) * RPW < pos) take(kc, vc, ok);      // (a wavefront whose rows are all behind the last one skips them)
+        }
+    }
+    if (wave == 0) take(*(const vec_t*)&s_k[sub * EPL], *(const vec_t*)&s_v[sub * EPL], rg == 0);      // the new position
+    attn_merge<CT, D, G, NW>(m, l, acc, sm.m, sm.l, sm.acc, sm.out);
     if (a.out_kt > 0) {
         for (int idx = t; idx < G * D; idx += NTH) ((AT*)a.out)[xpack_index(b, kvh * G * D + idx, a.out_kt)] = (AT)sm.out[idx];
     } else {
