@@ -184,7 +184,7 @@ namespace tship {
 // the model (refresh_test_hooks), never inside the per-layer code.
 struct TestHooks {
     int ffn_tiles = 0;        // TSHIP_FFN_TILES: 10, 15, 20, 30 or 40 = column tiles x 10 per block of the decode FFN up projection
-    int patch_rows = 0;       // TSHIP_PATCH_ROWS: 1, 2, 4 or 8 row tiles per tile patch of the prefill GEMM
+    int patch_rows = 0;       // TSHIP_PATCH_ROWS: 1, 2, 4 or 8: most row tiles of a band of tiles of the prefill GEMM (xcd_tile)
     long attn_splits = 0;     // TSHIP_ATTN_SPLITS: blocks per (sequence, KV head) pair in decode attention
     int gemm_tile = -1;        // TSHIP_GEMM_TILE: tile of the prefill GEMMs (pick_gemm_tile); 0: the 256 x 256 tile from 256 rows on
     int f32_tile = 0;         // TSHIP_F32_TILE: tile of the fp32 GEMMs from 33 rows on (pick_f32_tile)
@@ -631,7 +631,7 @@ static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int 
         constexpr int WR = decltype(WRc)::value, NJ = decltype(NJc)::value;
         const long tiles = ceil_div(e.NT, NJ) * ceil_div(e.R, 64 * WR);
         TSHIP_REQUIRE(e.splits >= 1 && (e.splits == 1 || tiles * e.splits <= TSHipGpt::MID_XCHG_TILES), "internal: split-K exchange area too small");
-        const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8), (unsigned)e.splits);
+        const dim3 grid((unsigned)xcd_tile_blocks(tiles), (unsigned)e.splits);
         const unsigned shm = MidShape<WR, NJ>::SHM;
         if (epi == BEPI_F32_BIAS) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_F32_BIAS, WR, NJ>, grid, dim3(512), shm, e);
         else if (epi == BEPI_RESID) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_RESID, WR, NJ>, grid, dim3(512), shm, e);
@@ -659,19 +659,8 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
     if (!mid) {           // 256 x 256 block tile
         constexpr int CK = 4;
         const unsigned shm = 2u * 2u * 8u * CK * 1024u;
-        // one-dimensional grid of 8-row x 4-column tile patches, 32 blocks each, rounded up to whole rounds of 8 patches
-        const long CT = ceil_div(w.NT, 8), RT = ceil_div(R, 256);
-        long patches = ceil_div(CT, 4) * ceil_div(RT, 8);
-        dim3 grid((unsigned)(round_up(patches, 8) * 32));
-        if (w.KT % 2 == 0 && n_problems == 1) {
-            // fewer than eight patches would leave XCDs without work: flatter patches (4, 2 or 1 row tiles)
-            int ph = 8;
-            while (ph > 1 && ceil_div(CT, 4) * ceil_div(RT, ph) < 8) ph /= 2;
-            if (g_hooks.patch_rows) ph = g_hooks.patch_rows;
-            patches = ceil_div(CT, 4) * ceil_div(RT, ph);
-            e.patch_rows = ph;
-            grid.x = (unsigned)(round_up(patches, 8) * 4 * ph);
-        }
+        dim3 grid((unsigned)xcd_tile_blocks(ceil_div(w.NT, 8) * ceil_div(R, 256)));
+        e.patch_rows = g_hooks.patch_rows;
         if (n_problems > 1 && !e.packed_problems) { e.blocks_per_problem = (int)grid.x; grid.x *= (unsigned)n_problems; }
         if (w.KT % 2 == 0) {      // asynchronous staging: four stages of two k-tiles, eight wavefronts
             if (epi == BEPI_F32_BIAS) launch_shm(m, name, big_gemm3_f16_kernel<BEPI_F32_BIAS>, grid, dim3(512), shm, e);

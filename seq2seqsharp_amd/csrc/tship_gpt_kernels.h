@@ -755,6 +755,36 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_f16_kernel(const half_t* 
 // ------------------------------------------------------------------------------------------------
 // prefill GEMMs, fp16 weights, row-major activations.  MFMA-bound from some hundred rows on.
 // ------------------------------------------------------------------------------------------------
+// Block -> tile of an RT x CT grid of tiles.  Workgroups go to the 8 XCDs round robin (id % 8) and each XCD has its own L2.
+// The tiles are numbered band by band (bands of up to `band` row tiles, as even as
+// they come), inside a band with the rows fastest; 32 consecutive ones, what an XCD runs at a time, share their operands in
+// its L2.  Whole rounds of 256 tiles go to the XCDs in runs of 32 and what is left in equal parts, so that no XCD has a tile
+// more than another.  (Whole 8 x 4 patches dealt to the XCDs gave one or three of them two patches in the only round: the
+// gated 2048 x 11264 at 2500 rows, 440 tiles for 256 units, took 165 us.)
+// False: no tile.  The grid has at least xcd_tile_blocks(RT x CT) blocks.
+__host__ __device__ inline long xcd_tile_blocks(long tiles) { return round_up(tiles, 8); }
+__device__ __forceinline__ bool xcd_tile(unsigned bid, int RT, int CT, int band, int& rtile, int& ctile) {
+    const int n = RT * CT, whole = n >> 8, xcd = (int)(bid & 7), seq = (int)(bid >> 3), part = (n - (whole << 8) + 7) >> 3;
+    int i;
+    if (seq < whole * 32) i = ((seq >> 5) << 8) + xcd * 32 + (seq & 31);
+    else {
+        const int s = seq - whole * 32;
+        i = (whole << 8) + xcd * part + s;
+        if (s >= part || i >= n) return false;
+    }
+    if (RT <= band) {      // (one band)
+        ctile = RT == 1 ? i : i / RT; rtile = i - ctile * RT;
+        return true;
+    }
+    const int bands = (RT + band - 1) / band, ph = (RT + bands - 1) / bands, last = (bands - 1) * ph;
+    int b = i / (ph * CT);
+    const int h = b >= bands - 1 ? RT - last : ph;
+    if (b >= bands - 1) b = bands - 1;
+    const int j = i - b * ph * CT;
+    ctile = j / h; rtile = b * ph + j % h;
+    return true;
+}
+
 enum { BEPI_F32_BIAS = 0, BEPI_RESID = 1, BEPI_ACT16 = 2 };
 
 struct BigArgs {
@@ -793,9 +823,7 @@ struct BigArgs {
     // Optional (LDS-tiled asynchronous kernel): row r of problem e is row row_idx[e * idx_estride + r] of X (the rows an
     // expert was given, read where they lie instead of being copied together first)
     const int* row_idx; long idx_estride;
-    // LDS-tiled asynchronous kernel: row tiles per XCD patch (8, or fewer for launches that would otherwise fill fewer
-    // than eight patches and leave XCDs idle); 0 means 8
-    int patch_rows;
+    int patch_rows;        // LDS-tiled asynchronous kernel: most row tiles of a band (xcd_tile); 0 means 8
 };
 
 // Epilogue shared by the LDS-tiled prefill GEMMs.
@@ -1229,14 +1257,8 @@ __global__ __launch_bounds__(256) void big_gemm2_f16_kernel(BigArgs a) {
     half_t* sX = big_smem + 2 * FR * 512;            // [2][FR * 512]
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = w >> 1, wn = w & 1;
-    // Block -> tile: workgroups go to the 8 XCDs round robin (id % 8) and each XCD has its own L2, so the 32 blocks an
-    // XCD runs at a time are laid out as one patch of 8 row tiles x 4 column tiles (12 distinct operand tiles for 32
-    // blocks); consecutive patches go to different XCDs.
-    const int CT = (a.NT + 7) / 8, RT = (int)((a.R + 255) / 256), PC = (CT + 3) / 4;
-    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int patch = (seq >> 5) * 8 + xcd, q = seq & 31;
-    const int ctile = (patch % PC) * 4 + (q & 3), rtile = (patch / PC) * 8 + (q >> 2);
-    if (ctile >= CT || rtile >= RT) return;
+    int rtile, ctile;
+    if (!xcd_tile(blockIdx.x, (int)((a.R + 255) / 256), (a.NT + 7) / 8, 8, rtile, ctile)) return;
     const int nt0 = ctile * 8;
     const long row0 = (long)rtile * 256;
     floatx16 acc[4][4];
@@ -1366,16 +1388,16 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
         const int e = (int)(bid / (unsigned)a.blocks_per_problem);
         bid -= (unsigned)e * (unsigned)a.blocks_per_problem;
         take_problem(e);
-        rot = e;      // a problem with fewer than eight patches would leave XCDs idle: problem e starts on XCD e % 8
+        rot = e;      // a problem with fewer than eight tiles would leave XCDs idle: problem e starts on XCD e % 8
     }
-    const int CT = (a.NT + 7) / 8, PC = (CT + 3) / 4;
-    const int RT = a.packed_problems ? a.packed_rt : (int)((a.R + 255) / 256);
-    const int xcd = (int)((bid - (unsigned)rot) & 7), seq = (int)(bid >> 3);
-    const int PH = a.patch_rows ? a.patch_rows : 8;          // a patch: PH row tiles x 4 column tiles
-    const int patch = (seq / (4 * PH)) * 8 + xcd, q = seq % (4 * PH);
-    const int ctile = (patch % PC) * 4 + (q & 3);
-    int rtile = (patch / PC) * PH + (q >> 2);
-    if (ctile >= CT || rtile >= RT) return;
+    const int CT = (a.NT + 7) / 8;
+    int RT = (int)((a.R + 255) / 256);
+    if (a.packed_problems) {
+        RT = 0;
+        for (int i = 0; i < a.packed_problems; ++i) RT += (a.rows_tab[i] + 255) / 256;
+    }
+    int rtile, ctile;
+    if (!xcd_tile(bid - (unsigned)rot, RT, CT, a.patch_rows ? a.patch_rows : 8, rtile, ctile)) return;
     if (a.packed_problems) {
         // the problem whose tiles hold packed row tile `rtile` (block-uniform: the counts sit in scalar registers)
         int e = -1, first = 0;
@@ -1384,7 +1406,6 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
             if (e < 0 && rtile < first + tiles) { e = i; rtile -= first; }
             first += tiles;
         }
-        if (e < 0) return;
         take_problem(e);
     }
     const int nt0 = ctile * 8;
@@ -1546,17 +1567,16 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     using S = MidShape<WR, NJ>;
     constexpr int KG = S::KG, NST = S::NST, PF = NST - 1, STAGE = S::STAGE, LW = NJ * KG / 8, PPR = 2 * KG, LPC = LW + 2;      // LPC: loads per wavefront and chunk
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wr = WR == 2 ? w >> 2 : 0, kg = WR == 2 ? w & 3 : w;
-    // Block -> tile: every XCD takes one contiguous eighth of the tiles in an order with the row tiles fastest, so that the
-    // blocks it runs at a time share their weight tiles (read from HBM once) and one L2's copy of the activations.
+    const int wr = w / KG, kg = w % KG;
     const int CT = (a.NT + NJ - 1) / NJ, RT = (a.R + 64 * WR - 1) / (64 * WR), n_tiles = CT * RT;
-    const int per_xcd = (n_tiles + 7) >> 3, seq = blockIdx.x >> 3, tile = (int)(blockIdx.x & 7) * per_xcd + seq;
-    if (seq >= per_xcd || tile >= n_tiles) return;
+    int rtile, ctile;
+    if (!xcd_tile(blockIdx.x, RT, CT, 8, rtile, ctile)) return;
+    const int tile = ctile * RT + rtile;
     // k-tiles of this block: all, or (a.splits > 1) one of as many ranges of whole chunks, blockIdx.y
     const int kt_per = a.splits > 1 ? ((a.KT + KG * a.splits - 1) / (KG * a.splits)) * KG : a.KT;
     const int kt_first = a.splits > 1 ? (int)blockIdx.y * kt_per : 0, kt_end = min(a.KT, kt_first + kt_per);      // (the host leaves no range empty)
-    const int nt0 = (tile / RT) * NJ;
-    const long row0 = (long)(tile % RT) * (64 * WR);
+    const int nt0 = ctile * NJ;
+    const long row0 = (long)rtile * (64 * WR);
     floatx16 acc[NJ][2];
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
