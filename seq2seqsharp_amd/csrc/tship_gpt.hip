@@ -587,42 +587,72 @@ static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const fl
 // number in the result); the exchange costs 1.2 us, a little per block and 0.7 us per 64 x 32 values of the tile that each
 // block stores and the last one adds.
 // own_cache_write: us that a launch saves with the 256 x 256 tile, which can write the key-value cache itself.
-// a, b and the exchange are fits to 7227 times (33 ... 16384 rows, 27 pairs of K and N from 128 to 22016, every tile and
-// split; profiles/prefill_gemm_tiles.txt): over the best tile of each of the 696 sizes the choice costs 0.6 % on average,
-// more than 15 % in 6.  Without the exchange's growth with the tile it was 2.5 % and 53: 4096 x 1024 at 1024 rows 27.5 us for 17.5.
+// a, b and the exchange are fits to 8707 times (33 ... 16384 rows, 27 pairs of K and N from 128 to 22016, every tile and
+// split; profiles/prefill_gemm_tiles.txt): over the best tile of each of the 916 sizes the choice costs 0.6 % on average,
+// more than 15 % in 9.  Without the exchange's growth with the tile it was 2.5 % and 53: 4096 x 1024 at 1024 rows 27.5 us for 17.5.
+struct GemmTile { int tile; float us; };      // (tile as above, plus 100 x the blocks that share its K)
 // the most blocks up to `splits` that leave none of their ranges of whole chunks empty
-static int mid_splits(const GemmW& w, int tile, int splits) {
+static int mid_splits(int KT, int tile, int splits) {
     const int kg = tile >= 20 ? 4 : 8;
-    while (splits > 1 && (splits - 1) * (int)ceil_div(w.KT, kg * splits) * kg >= w.KT) --splits;
+    while (splits > 1 && (splits - 1) * (int)ceil_div(KT, kg * splits) * kg >= KT) --splits;
     return splits;
 }
-static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) {
-    struct Cost { int tile, rows, cols; float a, b; };
+struct GemmCost { int tile, rows, cols; float a, b; };
+static const std::vector<GemmCost>& gemm_costs() {
+    typedef GemmCost Cost;
     static const Cost costs[] = {{11, 64, 1, 3.5f, 0.031f}, {12, 64, 2, 4.4f, 0.046f}, {14, 64, 4, 6.5f, 0.077f},
-                                 {22, 128, 2, 5.2f, 0.072f}, {24, 128, 4, 8.1f, 0.111f}, {0, 256, 8, 7.0f, 0.285f}};
-    const int forced = g_hooks.gemm_tile;
-    if (forced == 0 && R >= 256) return 0;
-    if (forced > 0) {
-        const Cost& c = *std::find_if(std::begin(costs), std::end(costs), [&](const Cost& k) { return k.tile == forced % 100; });
-        const bool fits = ceil_div(R, c.rows) * ceil_div(w.NT, c.cols) * (forced / 100) <= TSHipGpt::MID_XCHG_TILES;
-        return forced % 100 + 100 * (forced >= 200 && fits ? mid_splits(w, forced % 100, forced / 100) : 1);
-    }
-    const float ncu = (float)std::max(1, n_compute_units());
-    int best = 111; float best_us = 1e30f;
-    for (const Cost& c : costs) {
+                                 {22, 128, 2, 5.2f, 0.072f}, {24, 128, 4, 8.1f, 0.111f}, {0, 256, 8, 11.0f, 0.315f}};
+    static const std::vector<GemmCost> v(std::begin(costs), std::end(costs));
+    return v;
+}
+static float gemm_tile_us(const GemmCost& c, int KT, long n_tiles, int splits) {
+    const float ncu = (float)std::max(1, n_compute_units()), tiles = (float)(n_tiles * splits), rounds = std::ceil(tiles / ncu);
+    float us = rounds * (c.a + c.b * (float)ceil_div(KT, splits)) * (1.0f + (c.tile ? 0.2f : 0.35f) * tiles / (rounds * ncu));
+    if (splits > 1) us += 1.16f + 0.08f * (float)splits + 0.7f * (float)(c.rows * c.cols) / 64.0f;
+    return us;
+}
+static GemmTile best_gemm_tile(int KT, int NT, long R, float own_cache_write = 0.0f) {
+    GemmTile best = {111, 1e30f};
+    for (const GemmCost& c : gemm_costs()) {
         if (c.tile == 0 && R < 256) continue;
-        const long n_tiles = ceil_div(R, c.rows) * ceil_div(w.NT, c.cols);
-        for (int want = 1; want <= (c.tile ? MID_SPLITS : 1); ++want) {
-            const int splits = mid_splits(w, c.tile, want);
-            if (splits != want || (splits > 1 && (n_tiles * splits > TSHipGpt::MID_XCHG_TILES || n_tiles * splits > (long)ncu))) continue;
-            const float tiles = (float)(n_tiles * splits), rounds = std::ceil(tiles / ncu);
-            float us = rounds * (c.a + c.b * (float)ceil_div(w.KT, splits)) * (1.0f + (c.tile ? 0.2f : 0.65f) * tiles / (rounds * ncu));
-            if (splits > 1) us += 1.16f + 0.08f * (float)splits + 0.7f * (float)(c.rows * c.cols) / 64.0f;
-            if (c.tile == 0) us -= own_cache_write;
-            if (us < best_us) { best_us = us; best = c.tile ? c.tile + 100 * splits : 0; }
+        const long n_tiles = ceil_div(R, c.rows) * ceil_div(NT, c.cols);
+        for (int splits = 1; splits <= (c.tile ? MID_SPLITS : 1); ++splits) {
+            if (mid_splits(KT, c.tile, splits) != splits || (splits > 1 && (n_tiles * splits > TSHipGpt::MID_XCHG_TILES || n_tiles * splits > n_compute_units()))) continue;
+            const float us = gemm_tile_us(c, KT, n_tiles, splits) - (c.tile == 0 ? own_cache_write : 0.0f);
+            if (us < best.us) best = {c.tile ? c.tile + 100 * splits : 0, us};
         }
     }
     return best;
+}
+static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) {
+    const int forced = g_hooks.gemm_tile;
+    if (forced == 0 && R >= 256) return 0;
+    if (forced > 0) {
+        const GemmCost& c = *std::find_if(gemm_costs().begin(), gemm_costs().end(), [&](const GemmCost& k) { return k.tile == forced % 100; });
+        const bool fits = ceil_div(R, c.rows) * ceil_div(w.NT, c.cols) * (forced / 100) <= TSHipGpt::MID_XCHG_TILES;
+        return forced % 100 + 100 * (forced >= 200 && fits ? mid_splits(w.KT, forced % 100, forced / 100) : 1);
+    }
+    return best_gemm_tile(w.KT, w.NT, R, own_cache_write).tile;
+}
+// A launch whose last round holds few tiles leaves most of the chip idle for as long as a whole round takes: instead, the first
+// `cols` 32-column tiles in whole rounds of one tile, and the other columns in a launch of their own with the tile that is best for
+// them.  cols 0: one launch.  The second launch costs 2 us.  ms per prompt, one launch per projection -> two: 1B model, 1500 / 1665 /
+// 2200 / 5000 / 8750 rows 4.4 / 4.5 / 6.6 / 10.4 / 17.9 -> 3.9 / 4.2 / 5.3 / 9.5 / 15.8 (with the tiles' even shares of xcd_tile);
+// 8 layers of the 7B one, 700 / 4400 rows 3.6 / 17.0 -> 3.1 / 13.9; the 768-wide one, 6000 rows 3.8 -> 3.3.
+struct GemmMix { int tile, cols, rest; float us; };
+static GemmMix pick_gemm_mix(const GemmW& w, long R) {
+    const long ncu = std::max(1, n_compute_units());
+    const GemmTile one = best_gemm_tile(w.KT, w.NT, R);
+    GemmMix mix = {one.tile, 0, 0, one.us};
+    for (const GemmCost& c : gemm_costs()) {
+        if (c.tile == 0 && R < 256) continue;
+        const long RT = ceil_div(R, c.rows), CT = ceil_div(w.NT, c.cols), cols = RT * CT / ncu * ncu / RT;      // column tiles of whole rounds
+        if (cols < 1 || cols >= CT) continue;
+        const GemmTile rest = best_gemm_tile(w.KT, w.NT - (int)(cols * c.cols), R);
+        const float us = gemm_tile_us(c, w.KT, RT * cols, 1) + rest.us + 2.0f;
+        if (us < mix.us && us < 0.97f * one.us) mix = {c.tile ? c.tile + 100 : 0, (int)(cols * c.cols), rest.tile, us};
+    }
+    return mix;
 }
 static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int mid) {
     e.splits = mid / 100; mid %= 100;
@@ -648,21 +678,16 @@ static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int 
     }
 }
 
-// Y = X * W for many rows (prefill), fp16, X row-major.
-// n_problems > 1 (LDS-tiled asynchronous kernel only, see big_gemm_batched_ok): e.Wtab / rows_tab / strides describe that many
-// problems of the same shape and at most R rows each, run by one launch.
-static bool big_gemm_batched_ok(const GemmW& w, long R) { return R >= 512 && w.KT % 2 == 0; }
-static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, int n_problems = 1, int tile = -1) {
-    e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.R = (int)R;
-    const int mid = n_problems > 1 ? 0 : tile >= 0 ? tile : pick_gemm_tile(w, R);
-    TSHIP_REQUIRE(n_problems == 1 || big_gemm_batched_ok(w, R), "internal: batched launch of a GEMM shape the LDS-tiled kernel does not take");
-    if (!mid) {           // 256 x 256 block tile
+static bool big_gemm_batched_ok(int KT, long R) { return R >= 512 && KT % 2 == 0; }
+static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int tile, int n_problems = 1) {
+    TSHIP_REQUIRE(n_problems == 1 || (!tile && big_gemm_batched_ok(e.KT, e.R)), "internal: batched launch of a GEMM shape the LDS-tiled kernel does not take");
+    if (!tile) {          // 256 x 256 block tile
         constexpr int CK = 4;
         const unsigned shm = 2u * 2u * 8u * CK * 1024u;
-        dim3 grid((unsigned)xcd_tile_blocks(ceil_div(w.NT, 8) * ceil_div(R, 256)));
+        dim3 grid((unsigned)xcd_tile_blocks(ceil_div(e.NT, 8) * ceil_div((long)e.R, 256)));
         e.patch_rows = g_hooks.patch_rows;
         if (n_problems > 1 && !e.packed_problems) { e.blocks_per_problem = (int)grid.x; grid.x *= (unsigned)n_problems; }
-        if (w.KT % 2 == 0) {      // asynchronous staging: four stages of two k-tiles, eight wavefronts
+        if (e.KT % 2 == 0) {      // asynchronous staging: four stages of two k-tiles, eight wavefronts
             if (epi == BEPI_F32_BIAS) launch_shm(m, name, big_gemm3_f16_kernel<BEPI_F32_BIAS>, grid, dim3(512), shm, e);
             else if (epi == BEPI_RESID) launch_shm(m, name, big_gemm3_f16_kernel<BEPI_RESID>, grid, dim3(512), shm, e);
             else launch_shm(m, name, big_gemm3_f16_kernel<BEPI_ACT16>, grid, dim3(512), shm, e);
@@ -673,7 +698,33 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
         else launch_shm(m, name, big_gemm2_f16_kernel<BEPI_ACT16, CK>, grid, dim3(256), shm, e);
         return;
     }
-    run_mid_gemm(m, name, e, epi, mid);
+    run_mid_gemm(m, name, e, epi, tile);
+}
+
+// Y = X * W for many rows (prefill), fp16, X row-major.
+// n_problems > 1 (LDS-tiled asynchronous kernel only, see big_gemm_batched_ok): e.Wtab / rows_tab / strides describe that many
+// problems of the same shape and at most R rows each, run by one launch.
+static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, int n_problems = 1, int tile = -1) {
+    e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.R = (int)R;
+    if (n_problems == 1 && tile < 0 && g_hooks.gemm_tile < 0) {
+        const GemmMix mix = pick_gemm_mix(w, R);
+        tile = mix.tile;
+        if (mix.cols) {
+            const int off = epi == BEPI_ACT16 && e.gated ? 16 * mix.cols : 32 * mix.cols;       // outputs of the first part
+            TSHIP_REQUIRE(!e.kcache && !e.advance_pos && !e.ssq && off < e.n_valid, "internal: columns of this projection stay together");
+            BigArgs r = e;
+            e.NT = mix.cols; e.n_valid = off;
+            r.W += (long)mix.cols * w.KT * 512; r.NT -= mix.cols; r.n_valid -= off; r.bias += off;
+            if (r.bias2) r.bias2 += off;
+            if (epi == BEPI_ACT16) r.out16 += off; else r.out += off;
+            if (epi == BEPI_RESID && r.xg16) { r.xg16 += off; r.gamma += off; r.ssq_out += mix.cols * r.ssq_ld; }
+            launch_big_gemm(m, name, e, epi, mix.tile);
+            launch_big_gemm(m, name, r, epi, mix.rest);
+            return;
+        }
+    }
+    if (n_problems == 1 && tile < 0) tile = pick_gemm_tile(w, R);
+    launch_big_gemm(m, name, e, epi, n_problems > 1 ? 0 : tile, n_problems);
 }
 
 typedef void (*AttnKernel)(AttnArgs);
@@ -1347,7 +1398,12 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         const bool can_fuse_kv = m->f16 && m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && L.qkv.KT % 2 == 0 &&
                                  (m->D == 64 || m->D == 128);
         const float fuse_saves = 1.9e-6f * (float)(R * 2 * GD) - 7.5f;
-        const int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, can_fuse_kv ? std::max(0.0f, fuse_saves) : 0.0f) : 0;
+        const float own_write = can_fuse_kv ? std::max(0.0f, fuse_saves) : 0.0f;
+        int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, own_write) : 0;
+        if (m->f16 && g_hooks.gemm_tile < 0) {      // (two launches of different tiles, -1, where that is less than the saved kernel)
+            const GemmMix mix = pick_gemm_mix(L.qkv, R);
+            if (mix.cols && mix.us < best_gemm_tile(L.qkv.KT, L.qkv.NT, R, own_write).us) qkv_tile = -1;
+        }
         const bool fuse_kv = can_fuse_kv && !qkv_tile && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
         if (m->f16) {
             BigArgs e; std::memset(&e, 0, sizeof(e));

@@ -80,7 +80,7 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
     // fp16 decode steps: the router kernel also takes the row's place in its experts' batches and writes the row there
     const bool fused_route = m->f16 && h % 4 == 0 && !batched && k <= 64;
     if (fused_route) { r.xg16 = (half_t*)(base + o.xg); r.xg_estride = xg_stride; r.packed_kt = (int)(m->ldh / 16); r.counts = counts; r.slot = slot; r.max_rows = (int)Bp; }
-    const bool packed = batched && m->f16 && h % 4 == 0 && rows >= 512 && big_gemm_batched_ok(*L.e1[0], rows) && big_gemm_batched_ok(*L.e2[0], rows) &&
+    const bool packed = batched && m->f16 && h % 4 == 0 && rows >= 512 && big_gemm_batched_ok(L.e1[0]->KT, rows) && big_gemm_batched_ok(L.e2[0]->KT, rows) &&
                         L.wtab1.p && L.wtab2.p && !g_hooks.no_moe_batch;
     if (packed) { r.xn16 = (half_t*)(base + o.xg); r.ld_xn16 = m->ldh; }       // (the gathered rows' area holds them: E * cap rows are reserved)
     const unsigned router_shm = (unsigned)((2L * h + (r.router_lds ? (long)E * h : 0)) * sizeof(float));
@@ -119,7 +119,7 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
         launch(m, "moe_gather", moe_gather_kernel<half_t>, dim3(rows, E), dim3(256), (const float*)xn32, h, (const int*)counts, (const int*)lists, (int)Bp, xg,
                m->ldh, xg_stride, 0);
         const int n_max = *std::max_element(n_e.begin(), n_e.end());
-        if (big_gemm_batched_ok(*L.e1[0], n_max) && big_gemm_batched_ok(*L.e2[0], n_max) && L.wtab1.p && L.wtab2.p && !g_hooks.no_moe_batch) {
+        if (big_gemm_batched_ok(L.e1[0]->KT, n_max) && big_gemm_batched_ok(L.e2[0]->KT, n_max) && L.wtab1.p && L.wtab2.p && !g_hooks.no_moe_batch) {
             // all experts in one launch per projection (row counts read on the device): the down projection of one expert
             // is 64 tiles at 8 x 4096 rows, a quarter of the compute units
             BigArgs e1; std::memset(&e1, 0, sizeof(e1));

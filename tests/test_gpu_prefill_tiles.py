@@ -93,3 +93,30 @@ def test_short_prompts_keep_large_residuals(G, oracle, batch, prompt):
     got = gpu.logits()
     assert np.isfinite(got).all() and np.abs(got - lg).max() <= FP16_ABS
     gpu.close()
+
+
+@pytest.mark.parametrize("norm,act", [(synth.RMSNORM, synth.SWIGLU), (synth.LAYERNORM, synth.RELU)])
+@pytest.mark.parametrize("batch,prompt", [(5, 300), (4, 549)])       # QKV and up, and output and down, in two launches
+def test_columns_in_two_launches(G, monkeypatch, norm, act, batch, prompt):
+    """Projections whose columns are taken by two launches of different tiles, against one tile for all of them: keys and values
+    of the second layer stand on every row and column of the first one's projections."""
+    ffn = 5632 if act == synth.SWIGLU else 11264
+    cfg = synth._cfg(n_layers=2, hidden=2048, n_heads=32, n_kv_heads=8, ffn_dim=ffn, vocab=157, attn_type=synth.GQA, norm_type=norm, act=act,
+                     batch=batch, prompt=prompt, steps=2, dtype="f16")
+    w = synth.make_weights(cfg, 91, random_bias=True)
+    seqs = synth.make_prompts(cfg, 92)
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
+    got = []
+    for tile in (None, "24"):
+        if tile:
+            monkeypatch.setenv("TSHIP_GEMM_TILE", tile)
+        gpu.reset()
+        gpu.prefill(seqs)
+        n = sum("gemm" in s for s in gpu.profile_symbols())
+        got.append((n, gpu.logits(), gpu.get_kv(1, 0), gpu.get_kv(1, 1)))
+    gpu.close()
+    assert got[1][0] == 4 * 2 + 1 and got[0][0] >= 6 * 2 + 1
+    assert np.abs(got[0][1] - got[1][1]).max() <= FP16_SENSITIVE_REL * np.abs(got[1][1]).max()
+    for a, b in zip(got[0][2:], got[1][2:]):      # (fp16 steps of the values and of the sums in front of them, in another order)
+        assert np.abs(a - b).max() <= 4e-3 * np.abs(b).max()
