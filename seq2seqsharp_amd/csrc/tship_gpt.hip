@@ -142,7 +142,6 @@ struct TSHipGpt {
     int pos = 0;                   // host mirror of *d_pos
     // repeat penalty of top-p sampling (DecodingOptions.RepeatPenalty): last sequence index of every token, per sequence
     DevBuf last_pos; long last_ld = 0; float repeat_penalty = 0.0f; float graph_penalty = 0.0f;
-    static constexpr int MAX_ATTN_SPLITS = 16;
     DevBuf attn_xchg, attn_count;  // decode attention with several blocks per (row, KV head): partial sums and one counter per pair
     bool any_blocked = false;
     bool embed_done = false;       // the sampling kernel of this step has already done the next step's embedding (greedy_embed_kernel)
@@ -900,11 +899,10 @@ static int attn_splits(TSHipGpt* m, int B) {
     const int NW = m->D == 128 ? 4 : 8;
     const long pairs = (long)B * m->Hv;
     long S = n_compute_units() / std::max<long>(pairs, 1);                  // fill the CUs
-    // Splitting pays when a wavefront still walks many chunks: at a context of 1 k the launch is bound by its fixed
-    // costs and the exchange adds 0.7 us (measured: 16.8 vs 15.9 us at 4 rows); at 8 k it gains 2.5 %.
-    S = std::min<long>(S, (m->ML / 32) / (NW * 8L));
+    S = std::min<long>(std::min<long>(S, (m->ML / 32) / NW), MAX_ATTN_SPLITS);      // at least one chunk per wavefront (the kernel decides by the position)
+    if (m->ML / 32 <= attn_split_chunks(m->D, (int)S)) S = 1;
     if (g_hooks.attn_splits) S = g_hooks.attn_splits;      // (testing: force the number of blocks per pair)
-    return (int)std::max<long>(1, std::min<long>(S, TSHipGpt::MAX_ATTN_SPLITS));
+    return (int)std::max<long>(1, std::min<long>(S, MAX_ATTN_SPLITS));
 }
 static void launch_attn_decode(TSHipGpt* m, AttnArgs a, int B) {
     if (!m->vt) {
@@ -923,7 +921,7 @@ static void launch_attn_decode(TSHipGpt* m, AttnArgs a, int B) {
         const long pairs = (long)B * m->Hv, per = (long)m->G * m->D + 2 * m->G;
         TSHIP_REQUIRE((size_t)(pairs * S * per) * sizeof(float) <= m->attn_xchg.bytes && (size_t)pairs * sizeof(int) <= m->attn_count.bytes,
                       "internal: attention exchange area too small");
-        a.S = S; a.xchg = m->attn_xchg.as<float>(); a.xcount = m->attn_count.as<int>();
+        a.S = S; a.s_fixed = g_hooks.attn_splits != 0; a.xchg = m->attn_xchg.as<float>(); a.xcount = m->attn_count.as<int>();
         grid.z = (unsigned)S;
     }
     AttnDecodeKernel k = m->D == 64 ? pick_attn_mfma_decode<64>(m->G, S > 1, m->SG > 1) : pick_attn_mfma_decode<128>(m->G, S > 1, m->SG > 1);
@@ -1619,7 +1617,7 @@ TSHIP_API int TSHip_GptCreate(const TSHipGptConfig* cfg, TSHipGpt** out) {
     if (m->vt) {
         const long pairs = (long)c.max_batch * m->Hv, per = (long)m->G * m->D + 2 * m->G;
         // at most as many blocks as CUs (or one per pair) ever share the area
-        const long blocks = std::max<long>(pairs, std::min<long>(pairs * TSHipGpt::MAX_ATTN_SPLITS, 2L * n_compute_units()));
+        const long blocks = std::max<long>(pairs, std::min<long>(pairs * MAX_ATTN_SPLITS, 2L * n_compute_units()));
         m->attn_xchg.alloc((size_t)(blocks * per) * sizeof(float));
         m->attn_count.alloc((size_t)pairs * sizeof(int));
         TSHIP_CHECK_HIP(hipMemset(m->attn_count.p, 0, m->attn_count.bytes));

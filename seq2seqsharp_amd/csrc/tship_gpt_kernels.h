@@ -2358,7 +2358,7 @@ struct AttnArgs {
     int ln;      // deferred LayerNorm (see SkinnyArgs): plain sums behind the sums of squares, `bias` holds d[ldq] followed by c[ldq]
     int vt;      // 1: keys and values are stored fragment-major (kfrag_index / vfrag_index) for the MFMA attention kernels
     // decode with several blocks per (row, KV head): their number, the exchange area [pairs][S][G D + 2 G] floats and one counter per pair
-    int S; float* xchg; int* xcount;
+    int S; float* xchg; int* xcount; int s_fixed;      // (s_fixed: all S take part whatever the position, for tests)
     // prefill of sequences padded to one length (Decoder.cs:656, 687-690): original lengths [batch], null = none were padded.
     // Query row r of sequence b sees columns c <= r while r < lens[b] (BuildSelfTriMask, TensorApplyCPU.cs:1040-1065); a row
     // from lens[b] on has every column masked, which after the softmax means: it attends to ALL columns of the padded
@@ -2996,7 +2996,8 @@ template <int D> constexpr unsigned attn_prefill_f32_shm() { return (unsigned)((
 // SPLIT: a.S blocks (blockIdx.z) share one (batch row, KV head); chunks go round robin over all their wavefronts, every
 // block leaves its unnormalised sums in an exchange area and the block that arrives last merges them in block order
 // (same publication protocol as the split-K projections: agent-scope atomic stores, wait, counter; no spinning).
-// For launches with fewer (row, head) pairs than CUs.
+// For launches with fewer (row, head) pairs than CUs.  How many of the a.S blocks take part is decided on the device from the
+// position, so that a cache made for long conversations costs short ones nothing.
 // The leading scalar arguments are everything the prologue's requests depend on: they are preloaded into scalar registers
 // at wavefront start (see skinny_gemm_f16_kernel; at most 14 of them), so that no request waits for the argument struct.
 // To fit, the pointers travel as one base (the key cache) and offsets from it in units of 256 bytes (every one of them is
@@ -3007,6 +3008,13 @@ struct AttnPacked {
     int max_len; unsigned counts;     // H | Hkv << 8 | KS << 16 | (ssq ? 1 : 0) << 24 | (rope ? 1 : 0) << 25 | (ln ? 1 : 0) << 26
     int ldq, split_stride; unsigned ssq_dims;   // ssq_nt | ssq_ld << 16
 };
+constexpr int MAX_ATTN_SPLITS = 16;
+// Most chunks of 32 positions that one block of a pair takes by itself: a round of chunks of all its wavefronts takes 1.1 us, the
+// exchange 2 (head size 128: 3).  Two or three blocks per pair mean that most of the chip's bandwidth is in use already.  One
+// block -> several, ms per 17 steps: 1B model, one row at 300 / 600 / 1000 / 2000 positions 10.39 / 10.72 / 11.21 / 12.44 -> (one) /
+// 10.75 (so one) / 10.91 / 11.06, 8 rows at 1500 12.30 -> 11.84, 16 rows at 1500 (two blocks) 12.87 -> 13.07 (so one); 8 layers of the
+// 7B one, one row at 1000 12.86 -> 12.22, 8 rows at 500 12.43 -> 12.57 (so one), 3 rows at 3000 14.01 -> 12.90.
+__host__ __device__ constexpr int attn_split_chunks(int D, int S) { return S < 4 ? (D == 128 ? 63 : 127) : (D == 128 ? 20 : 24); }
 template <int D, int G, bool SPLIT, bool SUB = false>      // SUB: groups of query heads share a KV head (AttnArgs::kv_sub > 1)
 __global__ __launch_bounds__(D == 128 ? 256 : 512) void attn_mfma_kernel(void* kcache_, int d_vcache, int d_qkv, int d_pos, int d_bias, int d_ssq, int d_rope_cos,
                                                                        int d_rope_sin, int max_len_, unsigned counts, int ldq_, int split_stride_,
@@ -3030,7 +3038,7 @@ __global__ __launch_bounds__(D == 128 ? 256 : 512) void attn_mfma_kernel(void* k
     __shared__ float sO[NW][D][16];
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     // wavefront slot among all wavefronts of the pair, and their number
-    const int gw = SPLIT ? (int)blockIdx.z * NW + w : w, GS = SPLIT ? a.S * NW : NW;
+    const int gw = SPLIT ? (int)blockIdx.z * NW + w : w;
     const int r16 = lane & 15, q = lane >> 4;
     const int HD = a.H * D, GD = a.Hkv * D;
     // Groups of query heads that share a KV head (AttnArgs::kv_sub).  One block per pair: grid (Hkv, batch, kv_sub), so
@@ -3071,7 +3079,7 @@ __global__ __launch_bounds__(D == 128 ? 256 : 512) void attn_mfma_kernel(void* k
     // is unconditional so that the waits below are counted exactly; a first chunk that holds the row being appended
     // is requested again after the prologue.
     for (int i = t; i < 16 * D; i += NTH) (&sQ[0][0])[i] = 0.0f;
-    int T, nchunks, n_own; bool validA;
+    int T, nchunks, n_own, S = 1, GS = NW; bool validA;
     {
         constexpr int CPT = ((G + 2) * D + NTH - 1) / NTH;        // projection columns per thread
         constexpr int PPT = ((G + 1) * D / 2 + NTH - 1) / NTH;    // rotary pairs per thread
@@ -3115,6 +3123,13 @@ __global__ __launch_bounds__(D == 128 ? 256 : 512) void attn_mfma_kernel(void* k
         __builtin_amdgcn_sched_barrier(0);
         const int pos = pos_base;
         T = pos_base + 1; nchunks = (T + 31) / 32;
+        if constexpr (SPLIT) {
+            // Blocks that take part: as many as leave each wavefront one chunk, or one.  The others leave; their requests
+            // above land in registers that nobody reads.
+            S = a.s_fixed ? a.S : nchunks > attn_split_chunks(D, a.S) ? min(a.S, nchunks / NW) : 1;
+            if ((int)blockIdx.z >= S) return;
+            GS = S * NW;
+        }
         n_own = nchunks > gw ? (nchunks - gw + GS - 1) / GS : 0;
         validA = gw < nchunks - 1;
         float rc[PPT], rs[PPT];
@@ -3274,7 +3289,7 @@ __global__ __launch_bounds__(D == 128 ? 256 : 512) void attn_mfma_kernel(void* k
 #pragma unroll
         for (int i = 0; i < 4; ++i) sO[w][dt * 16 + 4 * q + i][r16] = acc_o[dt][i];
     __syncthreads();
-    if constexpr (SPLIT) {
+    if (SPLIT && S > 1) {
         // block sums relative to the block maximum -> exchange area [pair][block][NCOL D + 2 NCOL] floats
         __shared__ int s_last;
         const int pair = b * (int)gridDim.x + kvh;
@@ -3302,22 +3317,33 @@ __global__ __launch_bounds__(D == 128 ? 256 : 512) void attn_mfma_kernel(void* k
         // rests on: write-through atomic stores, vmcnt(0), block barrier, atomic add, atomic loads in the last arriver)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // the stores have reached the point of coherence
         __syncthreads();
-        if (t == 0) s_last = __hip_atomic_fetch_add(a.xcount + pair, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.S - 1;
+        if (t == 0) s_last = __hip_atomic_fetch_add(a.xcount + pair, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
         __syncthreads();
         if (!s_last) return;
         // every block of the pair has published (its count came after its stores): merge in block order
         const float* base = a.xchg + (long)pair * a.S * per;
         for (int idx = t; idx < NCOL * D; idx += NTH) {
             const int col = idx % NCOL, d = idx / NCOL;
-            float M = -INFINITY;
-            for (int s = 0; s < a.S; ++s) M = fmaxf(M, __hip_atomic_load(base + s * per + NCOL * D + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            float L = 0.0f, O = 0.0f;
-            for (int s = 0; s < a.S; ++s) {
-                const float ms = __hip_atomic_load(base + s * per + NCOL * D + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const float wgt = (ms == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
-                L += __hip_atomic_load(base + s * per + NCOL * D + NCOL + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * wgt;
-                O += __hip_atomic_load(base + s * per + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * wgt;
+            // all blocks' sums requested together (clamped to the last block): one round trip, not two per block
+            float ms[MAX_ATTN_SPLITS], ls[MAX_ATTN_SPLITS], os[MAX_ATTN_SPLITS];
+#pragma unroll
+            for (int s = 0; s < MAX_ATTN_SPLITS; ++s) {
+                const float* p = base + min(s, S - 1) * per;
+                ms[s] = __hip_atomic_load(p + NCOL * D + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                ls[s] = __hip_atomic_load(p + NCOL * D + NCOL + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                os[s] = __hip_atomic_load(p + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+            float M = ms[0];
+#pragma unroll
+            for (int s = 1; s < MAX_ATTN_SPLITS; ++s) M = fmaxf(M, ms[s]);
+            float L = 0.0f, O = 0.0f;
+#pragma unroll
+            for (int s = 0; s < MAX_ATTN_SPLITS; ++s)
+                if (s < S) {
+                    const float wgt = (ms[s] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ms[s] - M);
+                    L += ls[s] * wgt;
+                    O += os[s] * wgt;
+                }
             const float o = O / L;
             const int kcol = (kvh * G + col) * D + d;
             if (a.out_kt > 0) ((half_t*)a.out)[xpack_index(b, kcol, a.out_kt)] = (half_t)o;

@@ -445,7 +445,7 @@ def test_head_dim_128_against_oracle(G, oracle, kv_heads, batch, prompt):
                                                                       (256, 4, 2, 3, 90, 16), (1024, 16, 1, 1, 200, 2)])
 def test_decode_attention_split_over_blocks(G, oracle, monkeypatch, hidden, heads, kv_heads, batch, prompt, splits):
     """Few (row, KV head) pairs and a long context: several blocks share a pair and the last one to arrive merges their
-    sums.  The library only splits at contexts of several thousand positions; the environment variable forces it here
+    sums.  The library only splits longer contexts; the environment variable forces it here
     (head_dim 64 and 128, two and three blocks, sixteen blocks most of which have no chunk at all, and sixteen query heads
     on one KV head, served as two groups of eight that each split in two).  fp16, against
     the oracle, with decode steps across a 32-position chunk boundary; then decode against the prefill path, which does
@@ -461,6 +461,40 @@ def test_decode_attention_split_over_blocks(G, oracle, monkeypatch, hidden, head
     gpu.prefill(cur)
     assert np.abs(gpu.logits() - last).max() <= 2e-2
     gpu.close()
+
+
+@pytest.mark.parametrize("hidden,heads,kv_heads,batch,at", [(256, 4, 2, 1, 768), (256, 2, 1, 2, 640), (512, 8, 8, 5, 768)])
+def test_decode_attention_takes_more_blocks_as_the_context_grows(G, monkeypatch, hidden, heads, kv_heads, batch, at):
+    """Head sizes 64 and 128: the captured step goes on from the last position that one block of a pair takes by itself to the
+    first that several share.  Against one block throughout, and against the prefill path."""
+    cfg = synth.tiny_config(dtype="f16", hidden=hidden, n_heads=heads, n_kv_heads=kv_heads, ffn_dim=2 * hidden, vocab=300, batch=batch, prompt=at - 3)
+    w = synth.make_weights(cfg, 83, random_bias=True)
+    seqs = synth.make_prompts(cfg, 84)
+    got = []
+    for splits in (None, "1"):
+        if splits:
+            monkeypatch.setenv("TSHIP_ATTN_SPLITS", splits)
+        gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=1100)
+        gpu.prefill(seqs)
+        ids, _ = gpu.generate(6)
+        ids = ids.reshape(6, batch)
+        gpu.set_seq_len(batch, at - 3)
+        steps = []
+        for i in range(6):
+            gpu.decode(ids[i])
+            steps.append(gpu.logits())
+        got.append(steps)
+        if not splits:
+            first = ids
+            gpu.reset()
+            gpu.prefill(np.concatenate([seqs, ids.T], 1))
+            assert np.abs(gpu.logits() - steps[-1]).max() <= 2e-2
+        else:
+            assert np.array_equal(ids, first)
+        gpu.close()
+    for a, b in zip(*got):      # (fp16 outputs of fp32 sums in another order)
+        assert np.abs(a - b).max() <= 4e-3 * np.abs(b).max()
+    assert np.array_equal(got[0][0], got[1][0]) and not np.array_equal(got[0][-1], got[1][-1])
 
 
 @pytest.mark.parametrize("name,tiles", [("gqa_rms_gate", 20), ("gqa_rms_gate", 30), ("gqa_rms_gate_silu", 40), ("mha_ln_relu", 20),
