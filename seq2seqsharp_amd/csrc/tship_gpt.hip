@@ -471,6 +471,20 @@ static void run_resid_norm(TSHipGpt* m, const char* name, int rows, ResidNormArg
 #undef TSHIP_RN
 }
 
+// Fragments a wavefront of a decode GEMM requests at a time.  Batches are requested whole (fragments beyond the wavefront's pw
+// are clamped duplicates), every further batch waits for the one before, and with several rounds of blocks smaller batches leave
+// room for more of them.  us per launch, 8 rows, batches of 2 / 4 / 8: vocabulary projection of 32 000 columns, pw = 6 (768 wide) 10.5 /
+// 11.9 / 12.9, 8 (1024) 13.7 / 13.0 / 14.5, 16 (2048) 23.5 / 22.5 / 22.7, 32 (4096) 44.2 / 43.3 / 41.5; 2048 x 3072 in two splits, pw = 8
+// - / 4.97 / 4.78; 5632 x 2048 in four, pw = 11 - / 8.15 / 8.58.
+static int skinny_batch(int pw, long blocks) {
+    int best = 8; float least = 1e30f;
+    for (int u : {8, 4, 2}) {
+        const int n = (int)ceil_div(pw, u);
+        const float cost = (float)(n * u) * (u == 8 && pw <= 16 && blocks > 2L * n_compute_units() ? 1.1f : 1.0f) + 0.5f * (float)(n - 1);
+        if (cost < least) { least = cost; best = u; }
+    }
+    return best;
+}
 // Y = X * W for <= 128 rows.  fp16: MFMA kernel; epilogue per `epi`.  fp32: tiled GEMM into partials.
 static void run_skinny(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, int rows, int epi, SkinnyArgs e) {
     TSHIP_REQUIRE(m->f16, "internal: run_skinny is the fp16 path");
@@ -507,30 +521,24 @@ static void run_skinny(TSHipGpt* m, const char* name, const GemmW& w, const void
         TSHIP_REQUIRE(best == 10, "internal: column tiles per block");
     }
     TSHIP_REQUIRE(!e.Wtab, "internal: batched problems go through the kernel's BATCHED instantiations");
-    if (BT == 1 && (epi == EPI_PARTIAL || epi == EPI_SPLIT_TAIL)) {
-        // the first batch of a wavefront is requested whole (fragments beyond its k range are clamped duplicates): a batch as
-        // long as the range keeps the requested bytes at the needed ones
-        const long pw = ceil_div(ceil_div(w.KT, e.KS), 8);
-        if (pw <= 2) {
-            if (epi == EPI_PARTIAL) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_PARTIAL, 8, 2>, grid, dim3(512), e);
-            else launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_SPLIT_TAIL, 8, 2>, grid, dim3(512), e);
-            return;
-        }
-        if (pw <= 4) {
-            if (epi == EPI_PARTIAL) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_PARTIAL, 8, 4>, grid, dim3(512), e);
-            else launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_SPLIT_TAIL, 8, 4>, grid, dim3(512), e);
-            return;
-        }
-    }
-#define TSHIP_SK(BTV, NWV)                                                                                                  \
-    if (epi == EPI_PARTIAL) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_PARTIAL, NWV>, grid, dim3(NWV * 64), e);        \
-    else if (epi == EPI_F32_BIAS) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_F32_BIAS, NWV>, grid, dim3(NWV * 64), e); \
-    else launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_ACT16, NWV>, grid, dim3(NWV * 64), e);
+    auto go = [&](auto BTc, auto Uc) {
+        constexpr int BTV = decltype(BTc)::value, U = decltype(Uc)::value, NW = BTV == 4 ? 4 : 8;
+        if (epi == EPI_PARTIAL) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_PARTIAL, NW, U>, grid, dim3(NW * 64), e);
+        else if (epi == EPI_F32_BIAS) launch_skinny(m, name, skinny_gemm_f16_kernel<BTV, EPI_F32_BIAS, NW, U>, grid, dim3(NW * 64), e);
+        else if constexpr (BTV == 1) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_SPLIT_TAIL, 8, U>, grid, dim3(512), e);
+    };
+    typedef std::integral_constant<int, 1> c1; typedef std::integral_constant<int, 2> c2; typedef std::integral_constant<int, 4> c4; typedef std::integral_constant<int, 8> c8;
     // (tails with a norm behind them: models of up to 32 rows; larger ones take decode_step_rows)
     if (epi == EPI_RESID_TAIL) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_RESID_TAIL, 8, 16>, grid, dim3(512), e);
-    else if (epi == EPI_SPLIT_TAIL) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_SPLIT_TAIL, 8>, grid, dim3(512), e);
-    else if (BT == 1) { TSHIP_SK(1, 8) } else if (BT == 2) { TSHIP_SK(2, 8) } else { TSHIP_SK(4, 4) }
-#undef TSHIP_SK
+    else if (epi == EPI_ACT16) {
+        if (BT == 1) launch_skinny(m, name, skinny_gemm_f16_kernel<1, EPI_ACT16, 8>, grid, dim3(512), e);
+        else if (BT == 2) launch_skinny(m, name, skinny_gemm_f16_kernel<2, EPI_ACT16, 8>, grid, dim3(512), e);
+        else launch_skinny(m, name, skinny_gemm_f16_kernel<4, EPI_ACT16, 4>, grid, dim3(256), e);
+    } else {
+        const int U = skinny_batch((int)ceil_div(ceil_div(w.KT, e.KS), BT == 4 ? 4 : 8), (long)w.NT * e.KS);
+        auto batch = [&](auto BTc) { if (U == 2) go(BTc, c2{}); else if (U == 4) go(BTc, c4{}); else go(BTc, c8{}); };
+        if (BT == 1) batch(c1{}); else if (BT == 2) batch(c2{}); else batch(c4{});
+    }
 }
 
 // Tile of an fp32 GEMM from 33 rows on, 10 x (32-row) + (32-column) quadrants: the estimated time over the compute units'
@@ -1683,10 +1691,12 @@ TSHIP_API int TSHip_GptFinalize(TSHipGpt* m) {
     if (m->fused_norm && !decode_by_rows(m)) {
         // residual-tail projections (N = hidden): split K so that the launch has about one block per compute unit
         // (more blocks than that run in a second wave, which measured 2 us slower)
+        // (and every split costs the last block an exchange: us at 8 rows for 2 / 4 / 6 / 8 / 10 splits, 768 x 768 5.2 / 5.0 / 5.3 / 5.7 /
+        // 6.6, 3072 x 768 6.5 / 5.9 / 5.8 / 6.1 / 7.0)
         auto tail_ks = [&](const GemmW& w) {
             int ks = std::max(1, n_compute_units() / std::max(1, w.NT));
-            ks = std::min(ks, std::max(1, w.KT / 8));           // at least one k-tile per wavefront
-            return std::min(ks, 16);
+            ks = std::min(ks, std::max(1, w.KT / 12));
+            return std::min(ks, 6);
         };
         for (auto& L : m->L) { L->wo.KS = tail_ks(L->wo); L->w2.KS = tail_ks(L->w2); }
     }
