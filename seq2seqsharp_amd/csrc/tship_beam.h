@@ -12,6 +12,7 @@
 
 namespace tship {
 
+// (picks of the general form below: sampled ones, or more than BEAM_PICKS)
 // probabilities of every row of logits: (float)exp(x - max) / sum (TensorApplyCPU.cs:1230-1268), after the division by the
 // temperature when sampling (Decoder.cs:720-723).  grid (rows), 1024 threads.
 __global__ __launch_bounds__(1024) void beam_probs_kernel(const float* __restrict__ logits, long ld, int V, float temperature, int divide,
@@ -49,6 +50,89 @@ __global__ void beam_take_kernel(float* __restrict__ probs, long ldp, const int*
     ids_out[r] = id;
     logp_out[r] = logf(probs[(long)r * ldp + id]);
     probs[(long)r * ldp + id] = 0.0f;
+}
+
+// Up to BEAM_PICKS greedy picks of every row at once: what that many rounds of (argmax, take) give.  After the row statistics of
+// topp_rowmax_kernel / topp_rowsum_kernel every segment of 1024 tokens lists its first n picks, and one block per row merges
+// the lists; no probability is stored.  8 rows of 32 000 tokens, 4 picks: one block per row for the softmax and a launch pair per
+// pick took 72 us, these four launches 27.
+// A token's key orders as the picks do: higher probability, then lower index; a blocked token behind every other, a NaN never
+// (0).  A picked token goes on with probability 0, as ScatterFill leaves it.
+constexpr int BEAM_PICKS = 8;
+typedef unsigned long long beam_key_t;
+__device__ __forceinline__ beam_key_t beam_key(float p, int id, bool blocked) {
+    if (!blocked && !(p >= 0.0f)) return 0;
+    return ((beam_key_t)(blocked ? 0u : __float_as_uint(p) + 1u) << 32) | (unsigned)~id;
+}
+// the block's largest key (256 threads)
+__device__ __forceinline__ beam_key_t beam_block_max(beam_key_t k, beam_key_t* s) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { const beam_key_t other = __shfl_xor(k, o, 64); if (other > k) k = other; }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = k;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 4; ++w) if (s[w] > k) k = s[w];
+    return k;
+}
+__device__ __forceinline__ float beam_row_sum(const TopPArgs& a, int r) {
+    const float* ss = a.accp + (long)r * a.Vs + a.nseg;
+    float sum = ss[0];
+    for (int s2 = 1; s2 < a.nseg; ++s2) sum += ss[s2];
+    return sum;
+}
+// grid (nseg, rows), 256 threads, four tokens per thread
+__global__ __launch_bounds__(256) void beam_segment_kernel(TopPArgs a, int n, beam_key_t* __restrict__ lists) {
+    __shared__ beam_key_t s[4];
+    const int seg = blockIdx.x, r = blockIdx.y, t = threadIdx.x;
+    const float* row = a.in + (long)r * a.ld;
+    const float mx = topp_row_max(a, r), sum = beam_row_sum(a, r);
+    beam_key_t k[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int id = seg * TOPP_SEG + i * 256 + t;
+        k[i] = id < a.V ? beam_key(expf(row[id] / a.temperature - mx) / sum, id, a.blocked && a.blocked[id]) : 0;
+    }
+    for (int j = 0; j < n; ++j) {
+        beam_key_t best = k[0];
+#pragma unroll
+        for (int i = 1; i < 4; ++i) if (k[i] > best) best = k[i];
+        best = beam_block_max(best, s);
+        if (t == 0) lists[((long)r * a.nseg + seg) * n + j] = best;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) if (k[i] == best) k[i] = 0;
+    }
+}
+// grid (rows), 256 threads; ids_out, logp_out [n][rows]
+__global__ __launch_bounds__(256) void beam_merge_kernel(TopPArgs a, int n, const beam_key_t* __restrict__ lists, int* __restrict__ ids_out, float* __restrict__ logp_out) {
+    __shared__ beam_key_t s[4];
+    const int r = blockIdx.x, t = threadIdx.x, rows = gridDim.x, total = a.nseg * n;
+    const float* row = a.in + (long)r * a.ld;
+    const float mx = topp_row_max(a, r), sum = beam_row_sum(a, r);
+    constexpr int PER = 256 * BEAM_PICKS / 256;       // (rows of up to 262144 tokens: 256 segments)
+    beam_key_t k[PER], extra = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) k[i] = t + i * 256 < total ? lists[(long)r * total + t + i * 256] : 0;
+    int picked[BEAM_PICKS];
+#pragma unroll
+    for (int j = 0; j < BEAM_PICKS; ++j) {
+        picked[j] = -1;
+        if (j >= n) continue;
+        beam_key_t best = extra;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) if (k[i] > best) best = k[i];
+        best = beam_block_max(best, s);
+        const int id = best ? (int)~(unsigned)best : 0;      // (a row of NaNs: the reference's scan never moves off index 0)
+        float p = expf(row[id] / a.temperature - mx) / sum;
+#pragma unroll
+        for (int i = 0; i < BEAM_PICKS; ++i) if (i < j && picked[i] == id) p = 0.0f;
+        picked[j] = id;
+        const beam_key_t again = beam_key(0.0f, id, a.blocked && a.blocked[id]);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) if (best && k[i] == best) k[i] = again;
+        if (!best && t == 0) extra = again;
+        if (t == 0) { ids_out[(long)j * rows + r] = id; logp_out[(long)j * rows + r] = logf(p); }
+    }
 }
 
 // rows of a [rows][row_stride] table gathered into a dense temporary and back: dst row i = old row src[i].  Only the first

@@ -1963,15 +1963,35 @@ TSHIP_API int TSHip_GptBeamPick(TSHipGpt* m, int n_picks, int mode, float top_p,
     TSHIP_REQUIRE(temperature > 0.0f, "temperature must be positive");
     const int B = m->cur_batch, V = m->c.vocab;
     const long Vp = round_up(V, 32);
-    m->beam_probs.reserve((size_t)m->Bpad * Vp * sizeof(float));
-    m->beam_ids.reserve((size_t)m->Bpad * sizeof(int));
     m->beam_out.reserve((size_t)n_picks * B * (sizeof(int) + sizeof(float)));
     int* d_ids_out = m->beam_out.as<int>(); float* d_logp = (float*)(d_ids_out + (size_t)n_picks * B);
+    const unsigned char* blocked = m->any_blocked ? (const unsigned char*)m->blocked.p : nullptr;
+    auto deliver = [&]() {
+        TSHIP_CHECK_HIP(hipMemcpyAsync(host_ids_out, d_ids_out, (size_t)n_picks * B * sizeof(int), hipMemcpyDeviceToHost, stream()));
+        TSHIP_CHECK_HIP(hipMemcpyAsync(host_logp_out, d_logp, (size_t)n_picks * B * sizeof(float), hipMemcpyDeviceToHost, stream()));
+        TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
+    };
+    if (mode == TSHIP_GREEDY && n_picks <= BEAM_PICKS && V <= 262144) {
+        const size_t need = topp_scratch_bytes(m->Bpad, V);
+        if (m->topp_scratch.bytes < need) m->topp_scratch.alloc(need);
+        TopPArgs a; std::memset(&a, 0, sizeof(a));
+        a.in = m->logits.as<float>(); a.ld = Vp; a.V = V; a.in_is_logits = 1; a.temperature = 1.0f; a.blocked = blocked;
+        topp_carve(a, m->topp_scratch.p, m->Bpad, V);
+        beam_key_t* lists = (beam_key_t*)a.hist;      // (256 words per segment; a list takes 16)
+        const dim3 segs((unsigned)a.nseg, (unsigned)B);
+        launch(m, "beam_rowmax", topp_rowmax_kernel, segs, dim3(256), a);
+        launch(m, "beam_rowsum", topp_rowsum_kernel, segs, dim3(256), a);
+        launch(m, "beam_segment", beam_segment_kernel, segs, dim3(256), a, n_picks, lists);
+        launch(m, "beam_merge", beam_merge_kernel, dim3(B), dim3(256), a, n_picks, (const beam_key_t*)lists, d_ids_out, d_logp);
+        deliver();
+        return 1;
+    }
+    m->beam_probs.reserve((size_t)m->Bpad * Vp * sizeof(float));
+    m->beam_ids.reserve((size_t)m->Bpad * sizeof(int));
     float* probs = m->beam_probs.as<float>();
     // Decoder.cs:720-723: the logits are divided by the temperature only when sampling
     launch(m, "beam_probs", beam_probs_kernel, dim3(B), dim3(1024), (const float*)m->logits.as<float>(), Vp, V, temperature,
            (int)(mode == TSHIP_TOPP && temperature != 1.0f), probs, Vp);
-    const unsigned char* blocked = m->any_blocked ? (const unsigned char*)m->blocked.p : nullptr;
     if (mode == TSHIP_TOPP) {
         m->beam_uni.reserve((size_t)n_picks * B * sizeof(float));
         TSHIP_CHECK_HIP(hipMemcpyAsync(m->beam_uni.p, host_uniforms, (size_t)n_picks * B * sizeof(float), hipMemcpyHostToDevice, stream()));
@@ -1997,9 +2017,7 @@ TSHIP_API int TSHip_GptBeamPick(TSHipGpt* m, int n_picks, int mode, float top_p,
         launch(m, "beam_take", beam_take_kernel, dim3((unsigned)ceil_div(B, 64)), dim3(64), probs, Vp, (const int*)m->beam_ids.as<int>(), B,
                d_ids_out + (size_t)i * B, d_logp + (size_t)i * B);
     }
-    TSHIP_CHECK_HIP(hipMemcpyAsync(host_ids_out, d_ids_out, (size_t)n_picks * B * sizeof(int), hipMemcpyDeviceToHost, stream()));
-    TSHIP_CHECK_HIP(hipMemcpyAsync(host_logp_out, d_logp, (size_t)n_picks * B * sizeof(float), hipMemcpyDeviceToHost, stream()));
-    TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
+    deliver();
     TSHIP_END
 }
 

@@ -223,8 +223,14 @@ static void run_moe_ffn_prefill(TSHipGpt* m, LayerW& L, int rows, const ResidNor
 // top-p pick whose block goes on with the next decode step's first kernel for its row (as greedy_embed_kernel does)
 template <int NPT>
 __global__ __launch_bounds__(PICK_THREADS) void topp_pick_embed_kernel(TopPArgs a, FnPrepArgs pa) {
+    if (topp_done(a, blockIdx.x)) return;
     const int tok = topp_pick_scan_row(a);
     fn_prepare_row<NPT, PICK_THREADS>(pa, blockIdx.x, tok, threadIdx.x);
+}
+template <int NPT>
+__global__ __launch_bounds__(PICK_THREADS) void topp_top_embed_kernel(TopPArgs a, FnPrepArgs pa) {
+    const int tok = topp_top_row(a);
+    if (tok >= 0) fn_prepare_row<NPT, PICK_THREADS>(pa, blockIdx.x, tok, threadIdx.x);
 }
 
 // embed_next: a decode step on these tokens follows at once (the generate loop): on the fused-norm path the greedy kernel
@@ -278,12 +284,14 @@ static void sample_tokens(TSHipGpt* m, int mode, float top_p, float temperature,
     a.repeat_penalty = m->repeat_penalty; a.last_pos = last; a.last_ld = m->last_ld; a.d_len = m->d_pos.as<int>(); a.record = record ? 1 : 0;
     auto run = [&](const char* name, void (*kernel)(TopPArgs), dim3 grid, dim3 block, const TopPArgs& args) { launch(m, name, kernel, grid, block, args); };
     if (embed_next && m->fused_norm && m->c.hidden <= 8192) {
-        const TopPArgs pick = topp_run(a, B, run, false);
         const FnPrepArgs pa = embed_prepare_args(m, m->ids.as<int>());
+        auto go = [&](auto NPTc) {
+            constexpr int NPT = decltype(NPTc)::value;
+            topp_run(a, B, run, [&](const TopPArgs& k) { launch(m, "topp_top_embed", topp_top_embed_kernel<NPT>, dim3(B), dim3(PICK_THREADS), k, pa); },
+                     [&](const TopPArgs& k) { launch(m, "topp_pick_embed", topp_pick_embed_kernel<NPT>, dim3(B), dim3(PICK_THREADS), k, pa); });
+        };
         const int h = m->c.hidden;
-        if (h <= 2048) launch(m, "topp_pick_embed", topp_pick_embed_kernel<4>, dim3(B), dim3(PICK_THREADS), pick, pa);
-        else if (h <= 4096) launch(m, "topp_pick_embed", topp_pick_embed_kernel<8>, dim3(B), dim3(PICK_THREADS), pick, pa);
-        else launch(m, "topp_pick_embed", topp_pick_embed_kernel<16>, dim3(B), dim3(PICK_THREADS), pick, pa);
+        if (h <= 2048) go(std::integral_constant<int, 4>{}); else if (h <= 4096) go(std::integral_constant<int, 8>{}); else go(std::integral_constant<int, 16>{});
         m->embed_done = true;
         return;
     }

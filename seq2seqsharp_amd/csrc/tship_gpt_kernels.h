@@ -3789,22 +3789,29 @@ __device__ __forceinline__ int greedy_row(const float* __restrict__ logits, long
     const int b = blockIdx.x, t = threadIdx.x;
     const float* row = logits + (long)b * ld;
     float best = -INFINITY; int bi = 0x7fffffff;
-    for (int i0 = t; i0 < V; i0 += 1024 * 8) {
-        float v[8];
-        // (unconditional requests with clamped indices: all eight are in flight before the first comparison)
+    // eight 16-byte requests per thread at a time, all in flight before the first comparison (32 768 logits: one round trip;
+    // 4-byte requests took four); rows start at multiples of 32 floats, the indices are clamped to the row's last 16 bytes
+    for (int i0 = 4 * t; i0 < V; i0 += 1024 * 4 * 8) {
+        floatx4 v[8];
+        const int last = (V - 1) & ~3;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = row[min(i0 + u * 1024, V - 1)];
+        for (int u = 0; u < 8; ++u) v[u] = *(const floatx4*)(row + min(i0 + u * 4096, last));
         if (blocked) {
-            unsigned char bl[8];
+            unsigned bl[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) bl[u] = blocked[min(i0 + u * 1024, V - 1)];
+            for (int u = 0; u < 8; ++u) bl[u] = *(const unsigned*)(blocked + min(i0 + u * 4096, last));
 #pragma unroll
-            for (int u = 0; u < 8; ++u) if (bl[u]) v[u] = -INFINITY;
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) if ((bl[u] >> (8 * e)) & 255u) v[u][e] = -INFINITY;
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) if (i0 + u * 1024 >= V) v[u] = -INFINITY;
+        for (int u = 0; u < 8; ++u)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) { int i = i0 + u * 1024; if (i < V && (v[u] > best || (v[u] == best && i < bi))) { best = v[u]; bi = i; } }
+            for (int e = 0; e < 4; ++e) {
+                const int i = i0 + u * 4096 + e;
+                if (i < V && (v[u][e] > best || (v[u][e] == best && i < bi))) { best = v[u][e]; bi = i; }
+            }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {

@@ -39,7 +39,16 @@ struct TopPArgs {
     // one byte per token, non-zero = blocked: the reference adds -1 to such a probability (Decoder.cs:745-753), so it is
     // <= 0 and never a candidate.  May be null.
     const unsigned char* blocked;
+    // logits only: rows whose candidates of at least 2^-9 reach top_p are finished by topp_top_kernel; the sort kernels behind
+    // it leave such rows alone (topp_done)
+    int guarded;
 };
+// At most 512 of a softmax's values are 2^-9 or more.  Their keys are collected in the row's slice of keysB / idxB (free until
+// the first sort pass), their number and the row's state in the words of `accp` behind the segment sums.
+constexpr int TOPP_TOP = 512;
+constexpr unsigned TOPP_TOP_KEY = ~0x3b000000u;       // key of 2^-9: larger probabilities have smaller keys
+__device__ __forceinline__ int* topp_state(const TopPArgs& a, int r) { return (int*)(a.accp + (long)r * a.Vs) + 2 * a.nseg; }      // [0] candidates, [1] 1 = the row needs the sort
+__device__ __forceinline__ bool topp_done(const TopPArgs& a, int r) { return a.guarded && topp_state(a, r)[1] == 0; }
 
 __device__ __forceinline__ int topp_seq_len(const TopPArgs& a, int r) { return a.row_lens ? a.row_lens[r] : (a.d_len ? *a.d_len : a.len); }
 
@@ -92,6 +101,7 @@ static __global__ __launch_bounds__(256) void topp_rowmax_kernel(TopPArgs a) {
     }
     const float m = block_max_256(lm, sred);
     if (t == 0) a.accp[(long)r * a.Vs + seg] = m;
+    if (a.guarded && seg == 0 && t == 0) topp_state(a, r)[0] = 0;
 }
 
 __device__ __forceinline__ float topp_row_max(const TopPArgs& a, int r) {
@@ -183,6 +193,10 @@ static __global__ __launch_bounds__(256) void topp_keys_kernel(TopPArgs a) {
         const unsigned k = s_key[e];
         kA[i] = k; iA[i] = i;
         atomicAdd(&s_hist[k & 255u], 1);
+        if (a.guarded && k <= TOPP_TOP_KEY) {
+            const int slot = atomicAdd(topp_state(a, r), 1);
+            if (slot < TOPP_TOP) { a.keysB[(long)r * a.Vs + slot] = k; a.idxB[(long)r * a.Vs + slot] = i; }
+        }
     }
     __syncthreads();
     a.hist[((long)r * a.nseg + seg) * 256 + t] = s_hist[t];
@@ -192,6 +206,7 @@ static __global__ __launch_bounds__(256) void topp_keys_kernel(TopPArgs a) {
 static __global__ __launch_bounds__(256) void topp_hist_kernel(TopPArgs a) {
     __shared__ int h[256];
     const int seg = blockIdx.x, r = blockIdx.y, t = threadIdx.x;
+    if (topp_done(a, r)) return;
     const unsigned* k = a.keysA + (long)r * a.Vs;
     h[t] = 0;
     __syncthreads();
@@ -208,6 +223,7 @@ static __global__ __launch_bounds__(256) void topp_hist_kernel(TopPArgs a) {
 static __global__ __launch_bounds__(256) void topp_scan_kernel(TopPArgs a) {
     __shared__ int tot[256];
     const int r = blockIdx.x, d = threadIdx.x;
+    if (topp_done(a, r)) return;
     int* h = a.hist + (long)r * a.nseg * 256;
     // (loads in batches of eight: a load-modify-store loop would wait for memory once per segment)
     int run = 0;
@@ -246,6 +262,7 @@ static __global__ __launch_bounds__(256) void topp_scan_kernel(TopPArgs a) {
 static __global__ __launch_bounds__(256) void topp_scatter_kernel(TopPArgs a) {
     __shared__ int wh[16][256];
     const int seg = blockIdx.x, r = blockIdx.y, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    if (topp_done(a, r)) return;
     const unsigned* kin = a.keysA + (long)r * a.Vs; const int* iin = a.idxA + (long)r * a.Vs;
     unsigned* kout = a.keysB + (long)r * a.Vs; int* iout = a.idxB + (long)r * a.Vs;
     for (int i = t; i < 16 * 256; i += 256) (&wh[0][0])[i] = 0;
@@ -574,20 +591,81 @@ __device__ __forceinline__ int topp_pick_scan_row(const TopPArgs& a) {
     __syncthreads();
     return s_id;
 }
-static __global__ __launch_bounds__(PICK_THREADS) void topp_pick_scan_kernel(TopPArgs a) { topp_pick_scan_row(a); }
+static __global__ __launch_bounds__(PICK_THREADS) void topp_pick_scan_kernel(TopPArgs a) { if (!topp_done(a, blockIdx.x)) topp_pick_scan_row(a); }
 
-// the whole pipeline; `launch_fn(name, kernel, grid, block, args)` puts one kernel on the library stream
-// with_pick = false: everything but the last kernel; returns the arguments that kernel takes (the caller launches a pick
-// kernel of its own, see topp_pick_embed_kernel)
-template <typename LaunchFn>
-inline TopPArgs topp_run(TopPArgs a, int rows, LaunchFn&& launch_fn, bool with_pick = true) {
+// The pick from a row's candidates of at least 2^-9, when they reach top_p by themselves (a trained model's distribution does):
+// sorted by counting the smaller ones, added one by one in the order and with the arithmetic of topp_pick_scan_row, whose
+// result this is bit for bit.  Otherwise the row is left to the sort.  Returns the token, or -1.  16 rows of 32 000 tokens, us a
+// step: the eight launches of the sort and its pick 70 -> 7 here and about 2 for each of them to find its rows done.
+// grid (rows), PICK_THREADS = TOPP_TOP threads
+__device__ __forceinline__ int topp_top_row(const TopPArgs& a) {
+    __shared__ uint2 s_in[TOPP_TOP];
+    __shared__ float s_val[TOPP_TOP], s_acc[TOPP_TOP];
+    __shared__ int s_idx[TOPP_TOP], s_used, s_first[PICK_WAVES];
+    static_assert(TOPP_TOP == PICK_THREADS, "a candidate per thread");
+    const int r = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int n = topp_state(a, r)[0];
+    const long slot = (a.d_step ? (long)*a.d_step * gridDim.x : 0) + r;
+    const float u = a.uniforms[slot];
+    unsigned key = 0xffffffffu; int id = 0;
+    if (t < n && n <= TOPP_TOP) { key = a.keysB[(long)r * a.Vs + t]; id = a.idxB[(long)r * a.Vs + t]; s_in[t] = uint2{key, (unsigned)id}; }
+    if (t == 0) s_used = -1;
+    __syncthreads();
+    if (n <= TOPP_TOP) {
+        if (t < n) {
+            int rank = 0;
+            for (int j = 0; j < n; ++j) { const uint2 o = s_in[j]; rank += o.x < key || (o.x == key && (int)o.y < id); }
+            s_val[rank] = __uint_as_float(~key); s_idx[rank] = id;
+        }
+        __syncthreads();
+        if (w == 0) {
+            float acc = 0.0f; int used = -1;
+            for (int k0 = 0; k0 < n && used < 0; k0 += 64) {
+                const float v = s_val[min(k0 + lane, n - 1)];
+                const int m = min(64, n - k0);
+                for (int i = 0; i < m; ++i) {
+                    acc += __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), i));
+                    if (lane == 0) s_acc[k0 + i] = acc;
+                    if (acc >= a.top_p) { used = k0 + i + 1; break; }
+                }
+            }
+            if (lane == 0) s_used = used;
+        }
+        __syncthreads();
+    }
+    const int used = s_used;
+    if (t == 0) topp_state(a, r)[1] = used < 0 ? 1 : 0;
+    if (used < 0) return -1;
+    const unsigned long long hit = __ballot(t < used && s_acc[min(t, used - 1)] / s_acc[used - 1] >= u);
+    if (lane == 0) s_first[w] = hit ? 64 * w + __ffsll(hit) - 1 : 0x7fffffff;
+    __syncthreads();
+    int first = s_first[0];
+#pragma unroll
+    for (int i = 1; i < PICK_WAVES; ++i) first = min(first, s_first[i]);
+    const int tok = first == 0x7fffffff ? 0 : s_idx[first];
+    if (t == 0) {
+        if (a.next_ids) a.next_ids[r] = tok;
+        if (a.gen_out) a.gen_out[slot] = tok;
+        if (a.out_f32) a.out_f32[r] = (float)tok;
+        if (a.record && a.last_pos) a.last_pos[(long)r * a.last_ld + tok] = topp_seq_len(a, r);     // the new token's index
+    }
+    return tok;
+}
+static __global__ __launch_bounds__(PICK_THREADS) void topp_top_kernel(TopPArgs a) { topp_top_row(a); }
+
+// the whole pipeline; `launch_fn(name, kernel, grid, block, args)` puts one kernel on the library stream.  top_fn(args) and
+// pick_fn(args) launch the two kernels that choose tokens (the first for logits only), in the plain form or one that goes on
+template <typename LaunchFn, typename TopFn, typename PickFn>
+inline void topp_run(TopPArgs a, int rows, LaunchFn&& launch_fn, TopFn&& top_fn, PickFn&& pick_fn) {
     const dim3 segs((unsigned)a.nseg, (unsigned)rows);
+    a.guarded = a.in_is_logits;
     if (a.in_is_logits) {
         launch_fn("topp_rowmax", topp_rowmax_kernel, segs, dim3(256), a);
         launch_fn("topp_rowsum", topp_rowsum_kernel, segs, dim3(256), a);
     }
     a.scan_in_scatter = a.nseg <= 64 ? 1 : 0;      // (beyond that every block of a row would re-read too many counts)
     launch_fn("topp_keys", topp_keys_kernel, segs, dim3(256), a);          // also the digit counts of pass 0
+    if (a.in_is_logits) top_fn(a);
     for (int pass = 0; pass < 4; ++pass) {
         a.shift = pass * 8;
         if (pass > 0) launch_fn("topp_hist", topp_hist_kernel, dim3((unsigned)a.nseg, (unsigned)rows), dim3(256), a);
@@ -596,8 +674,12 @@ inline TopPArgs topp_run(TopPArgs a, int rows, LaunchFn&& launch_fn, bool with_p
         unsigned* tk = a.keysA; a.keysA = a.keysB; a.keysB = tk;
         int* ti = a.idxA; a.idxA = a.idxB; a.idxB = ti;
     }
-    if (with_pick) launch_fn("topp_pick", topp_pick_scan_kernel, dim3((unsigned)rows), dim3(PICK_THREADS), a);
-    return a;
+    pick_fn(a);
+}
+template <typename LaunchFn>
+inline void topp_run(TopPArgs a, int rows, LaunchFn&& launch_fn) {
+    auto choose = [&](const char* name, void (*kernel)(TopPArgs)) { return [&launch_fn, rows, name, kernel](const TopPArgs& k) { launch_fn(name, kernel, dim3((unsigned)rows), dim3(PICK_THREADS), k); }; };
+    topp_run(a, rows, launch_fn, choose("topp_top", topp_top_kernel), choose("topp_pick", topp_pick_scan_kernel));
 }
 
 }  // namespace tship
