@@ -191,6 +191,8 @@ struct TestHooks {
     int attn_nq = 0;          // TSHIP_ATTN_NQ: 1 or 2 groups of 16 MFMA columns per wavefront in prefill attention
     bool no_kv_fuse = false;  // TSHIP_NO_KV_FUSE: the QKV projection of a prefill does not write the cache itself
     bool no_moe_batch = false;// TSHIP_NO_MOE_BATCH: one prefill GEMM launch per expert
+    int moe_router_rows = 1024;       // TSHIP_MOE_ROUTER_ROWS: prefills of more rows route a row per wavefront
+    int moe_rest = 0;         // TSHIP_MOE_REST: tile of a launch of its own for the experts' last rows (see run_packed_gemm)
     bool record_symbols = false;      // TSHIP_RECORD_SYMBOLS: TSHip_GptProfileSymbols gives the kernels launched since the last prefill began
     bool no_graph = false;    // TSHIP_NO_GRAPH: the generate loop launches its kernels one by one
 };
@@ -221,6 +223,11 @@ static void refresh_test_hooks() {
     h.record_symbols = std::getenv("TSHIP_RECORD_SYMBOLS") != nullptr;
     h.no_kv_fuse = std::getenv("TSHIP_NO_KV_FUSE") != nullptr;
     h.no_moe_batch = std::getenv("TSHIP_NO_MOE_BATCH") != nullptr;
+    if (const char* v = std::getenv("TSHIP_MOE_ROUTER_ROWS")) { h.moe_router_rows = std::atoi(v); TSHIP_REQUIRE(h.moe_router_rows >= 0, "TSHIP_MOE_ROUTER_ROWS: a number of rows"); }
+    if (const char* v = std::getenv("TSHIP_MOE_REST")) {
+        h.moe_rest = std::atoi(v);
+        TSHIP_REQUIRE(h.moe_rest == 11 || h.moe_rest == 12 || h.moe_rest == 14 || h.moe_rest == 22 || h.moe_rest == 24, "TSHIP_MOE_REST: 11, 12, 14, 22 or 24");
+    }
     h.no_graph = std::getenv("TSHIP_NO_GRAPH") != nullptr;
     g_hooks = h;
 }
@@ -668,9 +675,10 @@ static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int 
         constexpr int WR = decltype(WRc)::value, NJ = decltype(NJc)::value;
         const long tiles = ceil_div(e.NT, NJ) * ceil_div(e.R, 64 * WR);
         TSHIP_REQUIRE(e.splits >= 1 && (e.splits == 1 || tiles * e.splits <= TSHipGpt::MID_XCHG_TILES), "internal: split-K exchange area too small");
-        const dim3 grid((unsigned)xcd_tile_blocks(tiles), (unsigned)e.splits);
+        const dim3 grid((unsigned)xcd_tile_blocks(tiles), (unsigned)e.splits, (unsigned)std::max(1, e.packed_problems));
         const unsigned shm = MidShape<WR, NJ>::SHM;
-        if (epi == BEPI_F32_BIAS) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_F32_BIAS, WR, NJ>, grid, dim3(512), shm, e);
+        if (e.packed_problems) launch_shm(m, name, epi == BEPI_F32_BIAS ? mid_gemm_f16_kernel<BEPI_F32_BIAS, WR, NJ, true> : mid_gemm_f16_kernel<BEPI_ACT16, WR, NJ, true>, grid, dim3(512), shm, e);
+        else if (epi == BEPI_F32_BIAS) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_F32_BIAS, WR, NJ>, grid, dim3(512), shm, e);
         else if (epi == BEPI_RESID) launch_shm(m, name, mid_gemm_f16_kernel<BEPI_RESID, WR, NJ>, grid, dim3(512), shm, e);
         else launch_shm(m, name, mid_gemm_f16_kernel<BEPI_ACT16, WR, NJ>, grid, dim3(512), shm, e);
     };
@@ -687,7 +695,7 @@ static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int 
 
 static bool big_gemm_batched_ok(int KT, long R) { return R >= 512 && KT % 2 == 0; }
 static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int tile, int n_problems = 1) {
-    TSHIP_REQUIRE(n_problems == 1 || (!tile && big_gemm_batched_ok(e.KT, e.R)), "internal: batched launch of a GEMM shape the LDS-tiled kernel does not take");
+    TSHIP_REQUIRE(n_problems == 1 || (!tile && (e.packed_problems ? e.KT % 2 == 0 : big_gemm_batched_ok(e.KT, e.R))), "internal: batched launch of a GEMM shape the LDS-tiled kernel does not take");
     if (!tile) {          // 256 x 256 block tile
         constexpr int CK = 4;
         const unsigned shm = 2u * 2u * 8u * CK * 1024u;
@@ -732,6 +740,33 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
     }
     if (n_problems == 1 && tile < 0) tile = pick_gemm_tile(w, R);
     launch_big_gemm(m, name, e, epi, n_problems > 1 ? 0 : tile, n_problems);
+}
+
+// The experts of a MoE layer, e.packed_problems of them with `total` rows together (the device knows which has how many): one
+// launch of the 256 x 256 tile over all their row tiles, or their whole row tiles in one launch and the last rows of each, less
+// than 256, in another with a smaller tile.  Two where every expert's nearly empty last tile makes a round of tiles more: 32 768
+// rows over 8 experts, 4096 x 1024: 528 tiles are three rounds, 330 us; 496 and the rest 250 + 32.  The line is drawn by gemm_tile_us for
+// 128 rows per expert in the last tile.
+static void run_packed_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long total, int epi, BigArgs e) {
+    const int E = e.packed_problems;
+    e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.splits = 1;
+    const GemmCost& whole = gemm_costs().back();
+    const long CT = ceil_div(w.NT, whole.cols), half_tiles = E * CT / 2, tiles = total / whole.rows * CT;
+    int rest = 0; float rest_us = 1e30f;
+    for (const GemmCost& c : gemm_costs()) {
+        if (!c.tile) continue;
+        const float us = gemm_tile_us(c, w.KT, E * (c.rows + 256) / (2 * c.rows) * ceil_div(w.NT, c.cols), 1);
+        if (us < rest_us) { rest_us = us; rest = c.tile; }
+    }
+    bool two = tiles > half_tiles && gemm_tile_us(whole, w.KT, tiles - half_tiles, 1) + rest_us + 2.0f < 0.97f * gemm_tile_us(whole, w.KT, tiles + half_tiles, 1);
+    if (g_hooks.moe_rest) { two = true; rest = g_hooks.moe_rest; }
+    e.packed_whole = two ? 1 : 0;
+    e.R = (int)(256 * (total / 256 + (two ? 0 : E)));      // >= 256 x the sum over the experts of their (whole) row tiles
+    if (e.R) launch_big_gemm(m, name, e, epi, 0, E);
+    if (two) {
+        e.R = 255;
+        run_mid_gemm(m, name, e, epi, rest + 100);
+    }
 }
 
 typedef void (*AttnKernel)(AttnArgs);

@@ -85,7 +85,17 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
     if (packed) { r.xn16 = (half_t*)(base + o.xg); r.ld_xn16 = m->ldh; }       // (the gathered rows' area holds them: E * cap rows are reserved)
     const unsigned router_shm = (unsigned)((2L * h + (r.router_lds ? (long)E * h : 0)) * sizeof(float));
     if (m->f16 && h % 4 == 0) {      // tree-order sums: an fp16 model's routing input is not the reference's to the last bit anyway
-        if (h <= 1024) launch(m, "moe_router", moe_router_fast_kernel<1>, dim3(rows), dim3(256), r);
+        // a row per wavefront for a prefill's rows, the matrix in 64 KiB of LDS; a block per row for the others, whose launch does not
+        // wait for the matrix: 1024 columns, 8 experts, 512 / 1024 / 1536 / 2048 / 4096 / 8192 rows 7.3 / 9.7 / 12.0 / 14.7 / 24.6 / 50.4 us
+        // with it, 9.2 / 9.3 / 9.7 / 10.3 / 14.3 / 22.2 per wavefront
+        const long shm = (h * round_up(E, 8) + 2L * h) * 4;
+        if (batched && rows > g_hooks.moe_router_rows && !r.part && k <= 4 && h * round_up(E, 8) <= 16384) {
+            r.rows = rows;
+            const dim3 blocks((unsigned)std::min<long>(ceil_div(rows, 8), 2L * n_compute_units()));
+            if (h <= 1024) launch_shm(m, "moe_router", moe_router_rows_kernel<4>, blocks, dim3(512), (unsigned)shm, r);
+            else if (h <= 2048) launch_shm(m, "moe_router", moe_router_rows_kernel<8>, blocks, dim3(512), (unsigned)shm, r);
+            else launch_shm(m, "moe_router", moe_router_rows_kernel<16>, blocks, dim3(512), (unsigned)shm, r);
+        } else if (h <= 1024) launch(m, "moe_router", moe_router_fast_kernel<1>, dim3(rows), dim3(256), r);
         else if (h <= 2048) launch(m, "moe_router", moe_router_fast_kernel<2>, dim3(rows), dim3(256), r);
         else launch(m, "moe_router", moe_router_fast_kernel<4>, dim3(rows), dim3(256), r);
     } else launch_shm(m, "moe_router", moe_router_kernel, dim3(rows), dim3(256), router_shm, r);
@@ -96,17 +106,16 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
     std::vector<int> n_e(E, rows);
     if (packed) {
         half_t* xn16 = (half_t*)(base + o.xg); half_t* mid = (half_t*)(base + o.mid);
-        const int rt_bound = (int)((long)rows * k / 256 + E);      // >= the sum over the experts of ceil(count / 256)
         BigArgs e1; std::memset(&e1, 0, sizeof(e1));
         e1.bias = zero; e1.out16 = mid; e1.ld16 = (int)o.ld4h; e1.act = c.act; e1.gated = 0; e1.n_valid = 4 * h;
         e1.Wtab = (const half_t* const*)L.wtab1.p; e1.rows_tab = counts; e1.x_estride = 0; e1.out16_estride = mid_stride;
-        e1.row_idx = lists; e1.idx_estride = Bp; e1.packed_problems = E; e1.packed_rt = rt_bound;
-        run_big_gemm(m, "moe_gemm1", *L.e1[0], xn16, m->ldh, (long)rt_bound * 256, BEPI_ACT16, e1, E);
+        e1.row_idx = lists; e1.idx_estride = Bp; e1.packed_problems = E;
+        run_packed_gemm(m, "moe_gemm1", *L.e1[0], xn16, m->ldh, (long)rows * k, BEPI_ACT16, e1);
         BigArgs e2; std::memset(&e2, 0, sizeof(e2));
         e2.bias = zero; e2.out = y; e2.ld_out = (int)o.ldy; e2.n_valid = h;
         e2.Wtab = (const half_t* const*)L.wtab2.p; e2.rows_tab = counts; e2.x_estride = mid_stride; e2.out_estride = y_stride;
-        e2.packed_problems = E; e2.packed_rt = rt_bound;
-        run_big_gemm(m, "moe_gemm2", *L.e2[0], mid, o.ld4h, (long)rt_bound * 256, BEPI_F32_BIAS, e2, E);
+        e2.packed_problems = E;
+        run_packed_gemm(m, "moe_gemm2", *L.e2[0], mid, o.ld4h, (long)rows * k, BEPI_F32_BIAS, e2);
     } else if (batched) {
         TSHIP_CHECK_HIP(hipMemcpyAsync(n_e.data(), counts, E * sizeof(int), hipMemcpyDeviceToHost, stream()));
         TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));

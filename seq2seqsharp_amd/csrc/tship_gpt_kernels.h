@@ -815,11 +815,13 @@ struct BigArgs {
     // device; blocks beyond it leave at once) and its activations / outputs at fixed strides.  0: one problem.
     int blocks_per_problem; const half_t* const* Wtab; const int* rows_tab; long x_estride, out_estride, out16_estride;
     // The same with the problems' row tiles packed one behind the other (packed_problems > 0; blocks_per_problem unused): the
-    // launch covers packed_rt row tiles, an upper bound of the sum over the problems of ceil(rows_tab[e] / 256) that the host
+    // launch covers R / 256 row tiles, an upper bound of the sum over the problems of ceil(rows_tab[e] / 256) that the host
     // knows without reading the counts (the sum of the rows / 256 + the number of problems); every block finds its problem
     // from the counts, blocks beyond the last problem's tiles leave at once.  Consecutive row tiles mostly belong to one
     // problem, so a patch still shares its weight tiles.
-    int packed_problems; int packed_rt;
+    // packed_whole: whole row tiles only; the problems' last rows, from the last multiple of 256 on, run in a launch of
+    // mid_gemm_f16_kernel.
+    int packed_problems; int packed_whole;
     // Optional (LDS-tiled asynchronous kernel): row r of problem e is row row_idx[e * idx_estride + r] of X (the rows an
     // expert was given, read where they lie instead of being copied together first)
     const int* row_idx; long idx_estride;
@@ -1392,9 +1394,10 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     }
     const int CT = (a.NT + 7) / 8;
     int RT = (int)((a.R + 255) / 256);
+    const int packed_up = a.packed_whole ? 0 : 255;
     if (a.packed_problems) {
         RT = 0;
-        for (int i = 0; i < a.packed_problems; ++i) RT += (a.rows_tab[i] + 255) / 256;
+        for (int i = 0; i < a.packed_problems; ++i) RT += (a.rows_tab[i] + packed_up) / 256;
     }
     int rtile, ctile;
     if (!xcd_tile(bid - (unsigned)rot, RT, CT, a.patch_rows ? a.patch_rows : 8, rtile, ctile)) return;
@@ -1402,7 +1405,7 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
         // the problem whose tiles hold packed row tile `rtile` (block-uniform: the counts sit in scalar registers)
         int e = -1, first = 0;
         for (int i = 0; i < a.packed_problems; ++i) {
-            const int tiles = (a.rows_tab[i] + 255) / 256;
+            const int tiles = (a.rows_tab[i] + packed_up) / 256;
             if (e < 0 && rtile < first + tiles) { e = i; rtile -= first; }
             first += tiles;
         }
@@ -1560,7 +1563,8 @@ template <int WR, int NJ> struct MidShape {
     static constexpr unsigned SHM = NST * STAGE > RED ? NST * STAGE : RED;
 };
 
-template <int EPI, int WR, int NJ>
+// PACKED: the last rows of several problems (BigArgs::packed_whole), problem = blockIdx.z
+template <int EPI, int WR, int NJ, bool PACKED = false>
 __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     extern __shared__ __attribute__((aligned(16))) half_t big_smem[];
     __shared__ float ssq_part[512];                     // [512 / (64 WR)][64 WR rows]: shares of the rows' sums of squares
@@ -1568,7 +1572,17 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     constexpr int KG = S::KG, NST = S::NST, PF = NST - 1, STAGE = S::STAGE, LW = NJ * KG / 8, PPR = 2 * KG, LPC = LW + 2;      // LPC: loads per wavefront and chunk
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = w / KG, kg = w % KG;
-    const int CT = (a.NT + NJ - 1) / NJ, RT = (a.R + 64 * WR - 1) / (64 * WR), n_tiles = CT * RT;
+    int first = 0;      // first row
+    if constexpr (PACKED) {
+        const int e = blockIdx.z;
+        a.R = a.rows_tab[e]; a.W = a.Wtab[e]; a.X += e * a.x_estride;
+        if (a.out) a.out += e * a.out_estride;
+        if (a.out16) a.out16 += e * a.out16_estride;
+        if (a.row_idx) a.row_idx += e * a.idx_estride;
+        first = a.R & ~255;
+        if (first == a.R) return;
+    }
+    const int CT = (a.NT + NJ - 1) / NJ, RT = (a.R - first + 64 * WR - 1) / (64 * WR), n_tiles = CT * RT;
     int rtile, ctile;
     if (!xcd_tile(blockIdx.x, RT, CT, 8, rtile, ctile)) return;
     const int tile = ctile * RT + rtile;
@@ -1576,7 +1590,7 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     const int kt_per = a.splits > 1 ? ((a.KT + KG * a.splits - 1) / (KG * a.splits)) * KG : a.KT;
     const int kt_first = a.splits > 1 ? (int)blockIdx.y * kt_per : 0, kt_end = min(a.KT, kt_first + kt_per);      // (the host leaves no range empty)
     const int nt0 = ctile * NJ;
-    const long row0 = (long)rtile * (64 * WR);
+    const long row0 = first + (long)rtile * (64 * WR);
     floatx16 acc[NJ][2];
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
@@ -1599,7 +1613,9 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int rl = (i * 8 + w) * (64 / PPR) + lane / PPR, s = (lane % PPR) ^ swz(rl);
-        xsrc[i] = a.X + min(row0 + rl, (long)a.R - 1) * (long)a.ldx + 8 * (s & 1);
+        long row = min(row0 + rl, (long)a.R - 1);
+        if (PACKED && a.row_idx) row = a.row_idx[row];
+        xsrc[i] = a.X + row * (long)a.ldx + 8 * (s & 1);
         xkt[i] = s >> 1;
     }
     typedef const void __attribute__((address_space(1)))* gptr_t;

@@ -26,6 +26,7 @@ struct MoeRouterArgs {
     // fast kernel only, when xn16 is set (prefill): the normalised row leaves as fp16, row-major with ld_xn16 elements per
     // row, where the experts' up projection reads it through the token lists; xn32 is not written
     half_t* xn16; long ld_xn16;
+    int rows;            // moe_router_rows_kernel
 };
 
 __device__ __forceinline__ float tree8(float v) {
@@ -441,6 +442,137 @@ __global__ __launch_bounds__(256) void moe_router_fast_kernel(MoeRouterArgs a) {
                     *(half4*)(dst + xpack_index(sl, c, a.packed_kt)) = hv;       // (four neighbouring columns are neighbours in a fragment)
                 }
             }
+        }
+    }
+}
+
+// The same routing for the many rows of a prefill (no pending output, k <= 4): a wavefront per row, so that nothing waits at a block
+// barrier, and the norm's parameters and the router matrix, eight times a row's bytes, in LDS for as long as the block lives.  A
+// lane's columns are 4 (lane + 64 i) ... + 3; the matrix lies as [column % 4][four experts][column / 4], so that lanes read
+// neighbouring 16 bytes.  Sums are trees over a lane's columns as well.  The next row is requested before the current one's sums.
+// Bound by the instructions of a row; us at 16 384 rows of 1024 columns and 8 experts: 97 with a block per row (three barriers, a
+// serial TopK that three of its wavefronts wait for, 32 KiB of weights from L2), 109 when such blocks go on over several rows, 42 now.
+// grid: up to a block per eight rows, 512 threads; dynamic LDS (h round_up(E, 8) + 2 h) floats
+template <int NG>      // NG * 256 >= hidden
+__global__ __launch_bounds__(512) void moe_router_rows_kernel(MoeRouterArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float router_smem[];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, h = a.h, E = a.E, EP = (E + 7) & ~7, h4 = h >> 2;
+    float* sW = router_smem;
+    float* sg = sW + (long)h * EP;
+    float* sb = sg + h;
+    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+    for (int c = t; c < h; c += 512) {
+        floatx4 wgt[2];
+        for (int e0 = 0; e0 < EP; e0 += 8) {
+            const float* src = a.router + (long)c * E + e0;
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                if ((E & 3) == 0) wgt[f] = e0 + 4 * f < E ? *(const floatx4*)(src + 4 * f) : zero4;
+                else {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) wgt[f][u] = e0 + 4 * f + u < E ? src[4 * f + u] : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int f = 0; f < 2; ++f) *(floatx4*)(sW + ((long)((c & 3) * (EP >> 2) + (e0 >> 2) + f) * h4 + (c >> 2)) * 4) = wgt[f];
+        }
+        sg[c] = a.gamma[c]; sb[c] = a.beta[c];
+    }
+    __syncthreads();
+    const int step = gridDim.x * 8;
+    floatx4 next[NG];
+    auto request = [&](int r) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) { const int c = 4 * (lane + 64 * i); next[i] = c < h ? *(const floatx4*)(a.x + (long)r * a.ldx + c) : zero4; }
+    };
+    auto tree = [](float (&v)[NG]) {
+#pragma unroll
+        for (int o = NG / 2; o > 0; o >>= 1)
+#pragma unroll
+            for (int i = 0; i < o; ++i) v[i] += v[i + o];
+        return v[0];
+    };
+    int r = blockIdx.x * 8 + w;
+    if (r < a.rows) request(r);
+    for (; r < a.rows; r += step) {
+        floatx4 v[NG];
+#pragma unroll
+        for (int i = 0; i < NG; ++i) v[i] = next[i];
+        if (r + step < a.rows) request(r + step);
+        float part[NG];
+#pragma unroll
+        for (int i = 0; i < NG; ++i) part[i] = (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);          // (columns beyond h hold zeros)
+        const float mean = wave_sum(tree(part)) / (float)h;
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            float d[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) { d[q] = v[i][q] - mean; d[q] *= d[q]; }
+            part[i] = 4 * (lane + 64 * i) < h ? (d[0] + d[1]) + (d[2] + d[3]) : 0.0f;
+        }
+        const float sigma = sqrtf(a.eps + wave_sum(tree(part)) / (float)h);
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            const int c = 4 * (lane + 64 * i);
+            if (c >= h) continue;
+            const floatx4 g = *(const floatx4*)(sg + c), b = *(const floatx4*)(sb + c);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[i][q] = g[q] * ((v[i][q] - mean) / sigma) + b[q];
+            if (a.xn16) {
+                half4 hv = {(half_t)v[i][0], (half_t)v[i][1], (half_t)v[i][2], (half_t)v[i][3]};
+                *(half4*)(a.xn16 + (long)r * a.ld_xn16 + c) = hv;
+            } else *(floatx4*)(a.xn32 + (long)r * h + c) = v[i];
+        }
+        float lg = -INFINITY;
+        for (int e0 = 0; e0 < E; e0 += 8) {
+            float level[5][8];       // sums of 1, 2, 4, ... column groups that wait for their other half
+#pragma unroll
+            for (int i = 0; i < NG; ++i) {
+                const int c = 4 * (lane + 64 * i);
+                float acc[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) acc[u] = 0.0f;
+                if (c < h) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int f = 0; f < 2; ++f) {
+                            const floatx4 wgt = *(const floatx4*)(sW + ((long)(q * (EP >> 2) + (e0 >> 2) + f) * h4 + (c >> 2)) * 4);
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) acc[4 * f + u] += v[i][q] * wgt[u];
+                        }
+                }
+                int l = 0;
+#pragma unroll
+                for (int n = i; n & 1; n >>= 1, ++l)
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) acc[u] += level[l][u];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) level[l][u] = acc[u];
+            }
+            constexpr int TOP = NG == 4 ? 2 : NG == 8 ? 3 : 4;
+            const float tot = wave_sum8(level[TOP], lane);
+            const float mine = __shfl(tot, ((lane >> 2) & 1) * 32 + ((lane >> 1) & 1) * 16 + (lane & 1) * 8, 64);      // expert lane % 8
+            if ((lane >> 3) == (e0 >> 3) && lane < E) lg = (mine + a.router_b[lane]) + (-65000.0f);
+        }
+        // softmax and TopK as in moe_router_fast_kernel: lane e holds expert e
+        const float mx = wave_max(lg);
+        const float ex = lane < E ? (float)exp((double)(lg - mx)) : 0.0f;
+        float ssum = 0.0f;
+        for (int e = 0; e < E; ++e) ssum += lane_value(ex, e);
+        const float p = ex / ssum;
+        if (lane < E) a.probs[(long)r * E + lane] = p;
+        float ov[4], oi[4];
+        switch (a.k) {
+            case 1: topk_by_insertion<1>(p, E, ov, oi); break;
+            case 2: topk_by_insertion<2>(p, E, ov, oi); break;
+            case 3: topk_by_insertion<3>(p, E, ov, oi); break;
+            default: topk_by_insertion<4>(p, E, ov, oi); break;
+        }
+        if (lane == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) if (i < a.k) { a.top_val[(long)r * a.k + i] = ov[i]; a.top_idx[(long)r * a.k + i] = oi[i]; }
         }
     }
 }
