@@ -773,7 +773,7 @@ __device__ __forceinline__ bool xcd_tile(unsigned bid, int RT, int CT, int band,
         if (s >= part || i >= n) return false;
     }
     if (RT <= band) {      // (one band)
-        ctile = RT == 1 ? i : i / RT; rtile = i - ctile * RT;
+        ctile = RT <= 2 ? i >> (RT - 1) : i / RT; rtile = i - ctile * RT;      // (no division in a decode step)
         return true;
     }
     const int bands = (RT + band - 1) / band, ph = (RT + bands - 1) / bands, last = (bands - 1) * ph;

@@ -451,7 +451,7 @@ __global__ __launch_bounds__(256) void moe_router_fast_kernel(MoeRouterArgs a) {
 // lane's columns are 4 (lane + 64 i) ... + 3; the matrix lies as [column % 4][four experts][column / 4], so that lanes read
 // neighbouring 16 bytes.  Sums are trees over a lane's columns as well.  The next row is requested before the current one's sums.
 // Bound by the instructions of a row; us at 16 384 rows of 1024 columns and 8 experts: 97 with a block per row (three barriers, a
-// serial TopK that three of its wavefronts wait for, 32 KiB of weights from L2), 109 when such blocks go on over several rows, 42 now.
+// serial TopK that three of its wavefronts wait for, 32 KiB of weights from L2), 109 when such blocks go on over several rows, 37 now.
 // grid: up to a block per eight rows, 512 threads; dynamic LDS (h round_up(E, 8) + 2 h) floats
 template <int NG>      // NG * 256 >= hidden
 __global__ __launch_bounds__(512) void moe_router_rows_kernel(MoeRouterArgs a) {
