@@ -949,9 +949,9 @@ static int attn_splits(TSHipGpt* m, int B) {
 }
 static void launch_attn_decode(TSHipGpt* m, AttnArgs a, int B) {
     if (!m->vt) {
-        TSHIP_REQUIRE(a.max_len < (1L << 31) && a.ldq < (1L << 31) && a.split_stride < (1L << 31) && a.H < 256 && a.Hkv < 256 && a.KS < 256 && a.kv_sub >= 0 && a.kv_sub < 32,
-                      "internal: attention counts beyond their packed fields");
-        const unsigned counts = (unsigned)a.H | ((unsigned)a.Hkv << 8) | ((unsigned)a.KS << 16) | ((unsigned)a.kv_sub << 24);
+        TSHIP_REQUIRE(a.max_len < (1L << 31) && a.ldq < (1L << 31) && a.split_stride < (1L << 31) && a.H < 1024 && a.Hkv < 1024 && a.KS < 32 && a.kv_sub >= 0 && a.kv_sub < 32,
+                      "internal: attention counts beyond their packed fields");      // (at most 512 heads of 16, 16 splits, 31 groups)
+        const unsigned counts = (unsigned)a.H | ((unsigned)a.Hkv << 10) | ((unsigned)a.KS << 20) | ((unsigned)a.kv_sub << 25);
         launch(m, "attn_decode", m->f16 ? pick_attn_step<half_t>(m->D, m->G) : pick_attn_step<float>(m->D, m->G), dim3(m->Hv, B), dim3(1024),
                a.d_pos, a.qkv, a.kcache, a.vcache, a.rope_cos, a.rope_sin, (int)a.max_len, counts, (int)a.ldq, (int)a.split_stride, a);
         return;

@@ -2563,7 +2563,7 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
     typedef CT vec_t __attribute__((ext_vector_type(EPL)));
     __shared__ AttnSmem<CT, D, G, NW> sm;
     __shared__ __align__(16) CT s_k[D], s_v[D];
-    const int H = counts_ & 255, Hkv = (counts_ >> 8) & 255, KS = (counts_ >> 16) & 255, kv_sub = counts_ >> 24;      // (as in AttnArgs)
+    const int H = counts_ & 1023, Hkv = (counts_ >> 10) & 1023, KS = (counts_ >> 20) & 31, kv_sub = counts_ >> 25;      // (as in AttnArgs)
     const int kvh = blockIdx.x, b = blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6, sub = lane % LPR, rg = lane / LPR;
     const int kvc = kv_sub > 1 ? kvh / kv_sub : kvh;       // the KV head whose cache this group of query heads reads
     const int pos = *d_pos_;
