@@ -693,15 +693,14 @@ static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int 
     }
 }
 
-static bool big_gemm_batched_ok(int KT, long R) { return R >= 512 && KT % 2 == 0; }
-static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int tile, int n_problems = 1) {
-    TSHIP_REQUIRE(n_problems == 1 || (!tile && (e.packed_problems ? e.KT % 2 == 0 : big_gemm_batched_ok(e.KT, e.R))), "internal: batched launch of a GEMM shape the LDS-tiled kernel does not take");
+static bool big_gemm_packed_ok(int KT, long R) { return R >= 512 && KT % 2 == 0; }
+static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int tile) {
+    TSHIP_REQUIRE(!e.packed_problems || (!tile && e.KT % 2 == 0), "internal: packed launch of a GEMM shape the LDS-tiled kernel does not take");
     if (!tile) {          // 256 x 256 block tile
         constexpr int CK = 4;
         const unsigned shm = 2u * 2u * 8u * CK * 1024u;
-        dim3 grid((unsigned)xcd_tile_blocks(ceil_div(e.NT, 8) * ceil_div((long)e.R, 256)));
+        const dim3 grid((unsigned)xcd_tile_blocks(ceil_div(e.NT, 8) * ceil_div((long)e.R, 256)));
         e.patch_rows = g_hooks.patch_rows;
-        if (n_problems > 1 && !e.packed_problems) { e.blocks_per_problem = (int)grid.x; grid.x *= (unsigned)n_problems; }
         if (e.KT % 2 == 0) {      // asynchronous staging: four stages of two k-tiles, eight wavefronts
             if (epi == BEPI_F32_BIAS) launch_shm(m, name, big_gemm3_f16_kernel<BEPI_F32_BIAS>, grid, dim3(512), shm, e);
             else if (epi == BEPI_RESID) launch_shm(m, name, big_gemm3_f16_kernel<BEPI_RESID>, grid, dim3(512), shm, e);
@@ -717,11 +716,9 @@ static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, i
 }
 
 // Y = X * W for many rows (prefill), fp16, X row-major.
-// n_problems > 1 (LDS-tiled asynchronous kernel only, see big_gemm_batched_ok): e.Wtab / rows_tab / strides describe that many
-// problems of the same shape and at most R rows each, run by one launch.
-static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, int n_problems = 1, int tile = -1) {
+static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, int tile = -1) {
     e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.R = (int)R;
-    if (n_problems == 1 && tile < 0 && g_hooks.gemm_tile < 0) {
+    if (tile < 0 && g_hooks.gemm_tile < 0) {
         const GemmMix mix = pick_gemm_mix(w, R);
         tile = mix.tile;
         if (mix.cols) {
@@ -738,8 +735,8 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
             return;
         }
     }
-    if (n_problems == 1 && tile < 0) tile = pick_gemm_tile(w, R);
-    launch_big_gemm(m, name, e, epi, n_problems > 1 ? 0 : tile, n_problems);
+    if (tile < 0) tile = pick_gemm_tile(w, R);
+    launch_big_gemm(m, name, e, epi, tile);
 }
 
 // The experts of a MoE layer, e.packed_problems of them with `total` rows together (the device knows which has how many): one
@@ -762,7 +759,7 @@ static void run_packed_gemm(TSHipGpt* m, const char* name, const GemmW& w, const
     if (g_hooks.moe_rest) { two = true; rest = g_hooks.moe_rest; }
     e.packed_whole = two ? 1 : 0;
     e.R = (int)(256 * (total / 256 + (two ? 0 : E)));      // >= 256 x the sum over the experts of their (whole) row tiles
-    if (e.R) launch_big_gemm(m, name, e, epi, 0, E);
+    if (e.R) launch_big_gemm(m, name, e, epi, 0);
     if (two) {
         e.R = 255;
         run_mid_gemm(m, name, e, epi, rest + 100);
@@ -1040,7 +1037,7 @@ static void decode_step_rows(TSHipGpt* m, const int* d_ids, int B) {
     const int NTh = (int)(hp / 32);
     float* ssq = m->ssq.as<float>();
     // (the 256 x 256 tile neither forms 1 / rms nor fits these row counts: pick_gemm_tile offers it from 256 rows on)
-    auto gemm = [&](const char* name, const GemmW& w, const DevBuf& X, long ldx, int epi, BigArgs e) { run_big_gemm(m, name, w, X.p, ldx, B, epi, e, 1, pick_gemm_tile(w, B)); };
+    auto gemm = [&](const char* name, const GemmW& w, const DevBuf& X, long ldx, int epi, BigArgs e) { run_big_gemm(m, name, w, X.p, ldx, B, epi, e, pick_gemm_tile(w, B)); };
     auto with_ssq = [&](BigArgs& e) { e.ssq = ssq; e.ssq_nt = NTh; e.ssq_in_ld = m->Bpad; e.inv_h = 1.0f / (float)h; e.eps = c.norm_eps; };
     auto resid = [&](const char* name, const GemmW& w, const DevBuf& X, long ldx, const DevBuf& bias, const DevBuf& gamma) {
         BigArgs e; std::memset(&e, 0, sizeof(e));
@@ -1423,7 +1420,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     auto producer = [&](BigArgs& e, const float* gamma) {        // residual GEMM that also emits the next GEMM's input
         e.xg16 = pxn.as<half_t>(); e.ld_xg = (int)m->ldh; e.gamma = gamma; e.ssq_out = pssq.as<float>(); e.ssq_ld = R;
     };
-    auto big = [&](const char* name, const GemmW& w, const void* X, long ldx, int epi, BigArgs e, int tile = -1) { run_big_gemm(m, name, w, X, ldx, R, epi, e, 1, tile); };
+    auto big = [&](const char* name, const GemmW& w, const void* X, long ldx, int epi, BigArgs e, int tile = -1) { run_big_gemm(m, name, w, X, ldx, R, epi, e, tile); };
     DevBuf& zero_bias = m->pw_zero_bias; zero_bias.reserve((size_t)std::max<long>(std::max<long>(qp, m->F13), round_up(h, 32)) * sizeof(float));
     for (int l = 0; l < c.n_layers; ++l) {
         LayerW& L = *m->L[l];

@@ -80,7 +80,7 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
     // fp16 decode steps: the router kernel also takes the row's place in its experts' batches and writes the row there
     const bool fused_route = m->f16 && h % 4 == 0 && !batched && k <= 64;
     if (fused_route) { r.xg16 = (half_t*)(base + o.xg); r.xg_estride = xg_stride; r.packed_kt = (int)(m->ldh / 16); r.counts = counts; r.slot = slot; r.max_rows = (int)Bp; }
-    const bool packed = batched && m->f16 && h % 4 == 0 && rows >= 512 && big_gemm_batched_ok(L.e1[0]->KT, rows) && big_gemm_batched_ok(L.e2[0]->KT, rows) &&
+    const bool packed = batched && m->f16 && h % 4 == 0 && rows >= 512 && big_gemm_packed_ok(L.e1[0]->KT, rows) && big_gemm_packed_ok(L.e2[0]->KT, rows) &&
                         L.wtab1.p && L.wtab2.p && !g_hooks.no_moe_batch;
     if (packed) { r.xn16 = (half_t*)(base + o.xg); r.ld_xn16 = m->ldh; }       // (the gathered rows' area holds them: E * cap rows are reserved)
     const unsigned router_shm = (unsigned)((2L * h + (r.router_lds ? (long)E * h : 0)) * sizeof(float));
@@ -127,29 +127,15 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
         half_t* xg = (half_t*)(base + o.xg); half_t* mid = (half_t*)(base + o.mid);
         launch(m, "moe_gather", moe_gather_kernel<half_t>, dim3(rows, E), dim3(256), (const float*)xn32, h, (const int*)counts, (const int*)lists, (int)Bp, xg,
                m->ldh, xg_stride, 0);
-        const int n_max = *std::max_element(n_e.begin(), n_e.end());
-        if (big_gemm_batched_ok(L.e1[0]->KT, n_max) && big_gemm_batched_ok(L.e2[0]->KT, n_max) && L.wtab1.p && L.wtab2.p && !g_hooks.no_moe_batch) {
-            // all experts in one launch per projection (row counts read on the device): the down projection of one expert
-            // is 64 tiles at 8 x 4096 rows, a quarter of the compute units
+        const int tile = g_hooks.no_moe_batch ? 0 : -1;      // (the hook compares with the batched launches: same tile, same bits)
+        for (int e = 0; e < E; ++e) {
+            if (n_e[e] == 0) continue;
             BigArgs e1; std::memset(&e1, 0, sizeof(e1));
-            e1.bias = zero; e1.out16 = mid; e1.ld16 = (int)o.ld4h; e1.act = c.act; e1.gated = 0; e1.n_valid = 4 * h;
-            e1.Wtab = (const half_t* const*)L.wtab1.p; e1.rows_tab = counts; e1.x_estride = xg_stride; e1.out16_estride = mid_stride;
-            run_big_gemm(m, "moe_gemm1", *L.e1[0], xg, m->ldh, n_max, BEPI_ACT16, e1, E);
+            e1.bias = zero; e1.out16 = mid + e * mid_stride; e1.ld16 = (int)o.ld4h; e1.act = c.act; e1.gated = 0; e1.n_valid = 4 * h;
+            run_big_gemm(m, "moe_gemm1", *L.e1[e], xg + e * xg_stride, m->ldh, n_e[e], BEPI_ACT16, e1, tile);
             BigArgs e2; std::memset(&e2, 0, sizeof(e2));
-            e2.bias = zero; e2.out = y; e2.ld_out = (int)o.ldy; e2.n_valid = h;
-            e2.Wtab = (const half_t* const*)L.wtab2.p; e2.rows_tab = counts; e2.x_estride = mid_stride; e2.out_estride = y_stride;
-            run_big_gemm(m, "moe_gemm2", *L.e2[0], mid, o.ld4h, n_max, BEPI_F32_BIAS, e2, E);
-        } else {
-            const int tile = g_hooks.no_moe_batch ? 0 : -1;      // (the hook compares with the batched launches: same tile, same bits)
-            for (int e = 0; e < E; ++e) {
-                if (n_e[e] == 0) continue;
-                BigArgs e1; std::memset(&e1, 0, sizeof(e1));
-                e1.bias = zero; e1.out16 = mid + e * mid_stride; e1.ld16 = (int)o.ld4h; e1.act = c.act; e1.gated = 0; e1.n_valid = 4 * h;
-                run_big_gemm(m, "moe_gemm1", *L.e1[e], xg + e * xg_stride, m->ldh, n_e[e], BEPI_ACT16, e1, 1, tile);
-                BigArgs e2; std::memset(&e2, 0, sizeof(e2));
-                e2.bias = zero; e2.out = y + e * y_stride; e2.ld_out = (int)o.ldy; e2.n_valid = h;
-                run_big_gemm(m, "moe_gemm2", *L.e2[e], mid + e * mid_stride, o.ld4h, n_e[e], BEPI_F32_BIAS, e2, 1, tile);
-            }
+            e2.bias = zero; e2.out = y + e * y_stride; e2.ld_out = (int)o.ldy; e2.n_valid = h;
+            run_big_gemm(m, "moe_gemm2", *L.e2[e], mid + e * mid_stride, o.ld4h, n_e[e], BEPI_F32_BIAS, e2, tile);
         }
     } else if (m->f16) {
         half_t* xg = (half_t*)(base + o.xg); half_t* mid = (half_t*)(base + o.mid);

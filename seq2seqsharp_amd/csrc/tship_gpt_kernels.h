@@ -810,18 +810,16 @@ struct BigArgs {
     // [sequence][kv_hkv heads][kv_max_len x kv_D]; only the query columns are stored to `out`.  kcache null: off.
     half_t* kcache; half_t* vcache; long kv_max_len; int kv_col0, kv_gd, kv_D, kv_hkv, kv_Tq, kv_pos0;
     const float* rope_cos; const float* rope_sin;
-    // Several independent problems in one launch of the LDS-tiled kernel (the experts of a MoE layer at prefill): problem
-    // e = blockIdx.x / blocks_per_problem takes its weights from Wtab[e], its row count from rows_tab[e] (read on the
-    // device; blocks beyond it leave at once) and its activations / outputs at fixed strides.  0: one problem.
-    int blocks_per_problem; const half_t* const* Wtab; const int* rows_tab; long x_estride, out_estride, out16_estride;
-    // The same with the problems' row tiles packed one behind the other (packed_problems > 0; blocks_per_problem unused): the
-    // launch covers R / 256 row tiles, an upper bound of the sum over the problems of ceil(rows_tab[e] / 256) that the host
-    // knows without reading the counts (the sum of the rows / 256 + the number of problems); every block finds its problem
-    // from the counts, blocks beyond the last problem's tiles leave at once.  Consecutive row tiles mostly belong to one
-    // problem, so a patch still shares its weight tiles.
+    // Several problems of one shape in one launch (the experts of a MoE layer at prefill; packed_problems > 0): problem e takes its
+    // weights from Wtab[e], its row count from rows_tab[e] (read on the device) and its activations / outputs at fixed strides.
+    // The LDS-tiled asynchronous kernel packs the problems' row tiles one behind the other: the launch covers R / 256 row tiles,
+    // an upper bound of the sum over the problems of ceil(rows_tab[e] / 256) that the host knows without reading the counts (the sum
+    // of the rows / 256 + the number of problems); every block finds its problem from the counts, blocks beyond the last
+    // problem's tiles leave at once.  Consecutive row tiles mostly belong to one problem, so a run of tiles still shares its
+    // weight tiles.
     // packed_whole: whole row tiles only; the problems' last rows, from the last multiple of 256 on, run in a launch of
     // mid_gemm_f16_kernel.
-    int packed_problems; int packed_whole;
+    int packed_problems; int packed_whole; const half_t* const* Wtab; const int* rows_tab; long x_estride, out_estride, out16_estride;
     // Optional (LDS-tiled asynchronous kernel): row r of problem e is row row_idx[e * idx_estride + r] of X (the rows an
     // expert was given, read where they lie instead of being copied together first)
     const int* row_idx; long idx_estride;
@@ -1378,20 +1376,6 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     constexpr int STAGE = 2 * FR * 512;                  // halfs per stage: weight fragments, then activation fragments
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = w >> 1, wn = w & 1;                   // 4 x 2 wavefronts
-    unsigned bid = blockIdx.x;
-    int rot = 0;
-    auto take_problem = [&](int e) {
-        a.R = a.rows_tab[e]; a.W = a.Wtab[e]; a.X += e * a.x_estride;
-        if (a.out) a.out += e * a.out_estride;
-        if (a.out16) a.out16 += e * a.out16_estride;
-        if (a.row_idx) a.row_idx += e * a.idx_estride;
-    };
-    if (a.blocks_per_problem && !a.packed_problems) {
-        const int e = (int)(bid / (unsigned)a.blocks_per_problem);
-        bid -= (unsigned)e * (unsigned)a.blocks_per_problem;
-        take_problem(e);
-        rot = e;      // a problem with fewer than eight tiles would leave XCDs idle: problem e starts on XCD e % 8
-    }
     const int CT = (a.NT + 7) / 8;
     int RT = (int)((a.R + 255) / 256);
     const int packed_up = a.packed_whole ? 0 : 255;
@@ -1400,7 +1384,7 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
         for (int i = 0; i < a.packed_problems; ++i) RT += (a.rows_tab[i] + packed_up) / 256;
     }
     int rtile, ctile;
-    if (!xcd_tile(bid - (unsigned)rot, RT, CT, a.patch_rows ? a.patch_rows : 8, rtile, ctile)) return;
+    if (!xcd_tile(blockIdx.x, RT, CT, a.patch_rows ? a.patch_rows : 8, rtile, ctile)) return;
     if (a.packed_problems) {
         // the problem whose tiles hold packed row tile `rtile` (block-uniform: the counts sit in scalar registers)
         int e = -1, first = 0;
@@ -1409,7 +1393,10 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
             if (e < 0 && rtile < first + tiles) { e = i; rtile -= first; }
             first += tiles;
         }
-        take_problem(e);
+        a.R = a.rows_tab[e]; a.W = a.Wtab[e]; a.X += e * a.x_estride;
+        if (a.out) a.out += e * a.out_estride;
+        if (a.out16) a.out16 += e * a.out16_estride;
+        if (a.row_idx) a.row_idx += e * a.idx_estride;
     }
     const int nt0 = ctile * 8;
     const long row0 = (long)rtile * 256;

@@ -43,3 +43,10 @@ def test_every_tile_once_and_equal_shares(tmp_path):
     subprocess.run(["g++", "-O2", "-o", str(exe), str(src)], check=True)
     r = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
     assert r.returncode == 0, r.stdout
+
+
+def test_kernels_hand_over_the_block_id_itself():
+    """xcd_tile covers every tile for block ids 0 ... xcd_tile_blocks - 1 only: shifted ids leave tiles out."""
+    text = open(os.path.join(ROOT, "seq2seqsharp_amd", "csrc", "tship_gpt_kernels.h")).read()
+    first = re.findall(r"!xcd_tile\(([^,]*),", text)
+    assert len(first) >= 3 and set(first) == {"blockIdx.x"}
