@@ -93,8 +93,7 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
             r.rows = rows;
             const dim3 blocks((unsigned)std::min<long>(ceil_div(rows, 8), 2L * n_compute_units()));
             if (h <= 1024) launch_shm(m, "moe_router", moe_router_rows_kernel<4>, blocks, dim3(512), (unsigned)shm, r);
-            else if (h <= 2048) launch_shm(m, "moe_router", moe_router_rows_kernel<8>, blocks, dim3(512), (unsigned)shm, r);
-            else launch_shm(m, "moe_router", moe_router_rows_kernel<16>, blocks, dim3(512), (unsigned)shm, r);
+            else launch_shm(m, "moe_router", moe_router_rows_kernel<8>, blocks, dim3(512), (unsigned)shm, r);      // (h <= 2048 by the matrix's size)
         } else if (h <= 1024) launch(m, "moe_router", moe_router_fast_kernel<1>, dim3(rows), dim3(256), r);
         else if (h <= 2048) launch(m, "moe_router", moe_router_fast_kernel<2>, dim3(rows), dim3(256), r);
         else launch(m, "moe_router", moe_router_fast_kernel<4>, dim3(rows), dim3(256), r);

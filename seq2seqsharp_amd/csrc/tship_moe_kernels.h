@@ -455,6 +455,7 @@ __global__ __launch_bounds__(256) void moe_router_fast_kernel(MoeRouterArgs a) {
 // grid: up to a block per eight rows, 512 threads; dynamic LDS (h round_up(E, 8) + 2 h) floats
 template <int NG>      // NG * 256 >= hidden
 __global__ __launch_bounds__(512) void moe_router_rows_kernel(MoeRouterArgs a) {
+    static_assert(NG == 4 || NG == 8, "column groups of a lane");
     extern __shared__ __attribute__((aligned(16))) float router_smem[];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, h = a.h, E = a.E, EP = (E + 7) & ~7, h4 = h >> 2;
     float* sW = router_smem;
@@ -526,7 +527,7 @@ __global__ __launch_bounds__(512) void moe_router_rows_kernel(MoeRouterArgs a) {
         }
         float lg = -INFINITY;
         for (int e0 = 0; e0 < E; e0 += 8) {
-            float level[5][8];       // sums of 1, 2, 4, ... column groups that wait for their other half
+            float level[4][8];       // sums of 1, 2, 4, ... column groups that wait for their other half
 #pragma unroll
             for (int i = 0; i < NG; ++i) {
                 const int c = 4 * (lane + 64 * i);
@@ -551,7 +552,7 @@ __global__ __launch_bounds__(512) void moe_router_rows_kernel(MoeRouterArgs a) {
 #pragma unroll
                 for (int u = 0; u < 8; ++u) level[l][u] = acc[u];
             }
-            constexpr int TOP = NG == 4 ? 2 : NG == 8 ? 3 : 4;
+            constexpr int TOP = NG == 4 ? 2 : 3;
             const float tot = wave_sum8(level[TOP], lane);
             const float mine = __shfl(tot, ((lane >> 2) & 1) * 32 + ((lane >> 1) & 1) * 16 + (lane & 1) * 8, 64);      // expert lane % 8
             if ((lane >> 3) == (e0 >> 3) && lane < E) lg = (mine + a.router_b[lane]) + (-65000.0f);

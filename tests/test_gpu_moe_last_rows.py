@@ -37,17 +37,23 @@ def test_last_rows_by_themselves(G, oracle, monkeypatch, experts, k, batch, prom
     gpu.close()
 
 
-# hidden sizes that fill no row of lanes, one to sixteen column groups per lane, expert counts around eight; more rows than wavefronts
-@pytest.mark.parametrize("hidden,heads,kv,experts,k,batch,prompt", [(48, 3, 1, 2, 1, 1, 3), (64, 4, 2, 9, 4, 3, 90), (528, 33, 11, 8, 2, 2, 40), (1056, 33, 11, 12, 3, 1, 17),
-                                                                    (2080, 65, 13, 7, 2, 1, 9), (64, 4, 4, 64, 4, 1, 60), (64, 4, 2, 8, 2, 9, 500), (272, 17, 17, 16, 2, 2, 300)])
-def test_router_of_many_rows(G, oracle, monkeypatch, hidden, heads, kv, experts, k, batch, prompt):
+# hidden sizes that fill no row of lanes, four and eight column groups per lane, expert counts around eight; more rows than wavefronts;
+# and matrices that leave no room in LDS (fast: a block per row instead)
+@pytest.mark.parametrize("hidden,heads,kv,experts,k,batch,prompt,fast",
+                         [(48, 3, 1, 2, 1, 1, 3, True), (64, 4, 2, 9, 4, 3, 90, True), (528, 33, 11, 8, 2, 2, 40, True), (64, 4, 4, 64, 4, 1, 60, True), (64, 4, 2, 8, 2, 9, 500, True),
+                          (272, 17, 17, 16, 2, 2, 300, True), (1056, 33, 11, 8, 3, 1, 17, True), (1040, 65, 13, 7, 4, 2, 30, True), (2048, 32, 8, 3, 2, 1, 40, True),
+                          (1056, 33, 11, 12, 3, 1, 17, False), (2080, 65, 13, 7, 2, 1, 9, False)])
+def test_router_of_many_rows(G, oracle, monkeypatch, hidden, heads, kv, experts, k, batch, prompt, fast):
     cfg = synth.tiny_config(n_layers=3, hidden=hidden, n_heads=heads, n_kv_heads=kv, n_experts=experts, experts_per_token=k, norm_type=synth.LAYERNORM,
                             act=synth.RELU, dtype="f16", batch=batch, prompt=prompt, vocab=100)
     w = synth.make_weights(cfg, 63, random_bias=True)
     monkeypatch.setenv("TSHIP_MOE_ROUTER_ROWS", "0")
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
     seqs = synth.make_prompts(cfg, 163)
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 10)
     gpu.prefill(seqs)
+    routers = [s for s in gpu.profile_symbols() if "moe_router" in s]
+    assert routers and all(("moe_router_rows_kernel<%d>" % (4 if hidden <= 1024 else 8) in s) == fast for s in routers)
     orc = oracle.OracleGpt(cfg, w)
     _, lg = orc.step(seqs, use_cache=True)
     assert np.abs(gpu.logits() - lg).max() <= FP16_ABS
