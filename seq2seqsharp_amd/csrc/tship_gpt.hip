@@ -800,7 +800,7 @@ static AttnKernel pick_attn_d(int D, int G, AttnKind kind) {
     });
 }
 // decode attention of caches without the fragment layout
-typedef void (*AttnStepKernel)(const int*, const float*, void*, void*, const float*, const float*, int, unsigned, int, int, AttnArgs);
+typedef void (*AttnStepKernel)(const int*, const float*, void*, void*, const float*, int, unsigned, int, int, AttnArgs);
 template <typename T>
 static AttnStepKernel pick_attn_step(int D, int G) {
     return with_heads(D, G, [&](auto Dc, auto Gc) -> AttnStepKernel { return attn_decode_kernel<T, T, decltype(Dc)::value, decltype(Gc)::value>; });
@@ -950,7 +950,7 @@ static void launch_attn_decode(TSHipGpt* m, AttnArgs a, int B) {
                       "internal: attention counts beyond their packed fields");      // (at most 512 heads of 16, 16 splits, 31 groups)
         const unsigned counts = (unsigned)a.H | ((unsigned)a.Hkv << 10) | ((unsigned)a.KS << 20) | ((unsigned)a.kv_sub << 25);
         launch(m, "attn_decode", m->f16 ? pick_attn_step<half_t>(m->D, m->G) : pick_attn_step<float>(m->D, m->G), dim3(m->Hv, B), dim3(1024),
-               a.d_pos, a.qkv, a.kcache, a.vcache, a.rope_cos, a.rope_sin, (int)a.max_len, counts, (int)a.ldq, (int)a.split_stride, a);
+               a.d_pos, a.qkv, a.kcache, a.vcache, a.bias, (int)a.max_len, counts, (int)a.ldq, (int)a.split_stride, a);
         return;
     }
     const int S = attn_splits(m, B);

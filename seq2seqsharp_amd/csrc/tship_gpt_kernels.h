@@ -2539,14 +2539,20 @@ struct AttnSmem {
 // key/value to the cache in place, then attends over pos+1 positions.
 // Replaces: AsContiguous head split, RoPE, GQA Expand, Concate(cache), MulBatch, Softmax, MulBatch, transpose
 // (Seq2SeqSharp/Layers/GroupQueryAttention.cs:121-224, Layers/MultiHeadAttention.cs:133-230).
-// A small launch (8 heads, 100 positions) is a chain of round trips, so they are taken side by side: the leading arguments
-// are preloaded, the position heads the longest chain, and the first sweep of cached rows (16 wavefronts x 4 requests each)
-// and the rotation are requested before the partial sums are waited for; the new row is attended from LDS, not read back.
+// A small launch (8 heads, 100 positions) is a chain of round trips, so those that can be are taken side by side: the leading
+// arguments are preloaded, and the sums, the bias, the norm's tile sums and the rotation are requested before the first wait.
+// A long one is bound by the instructions of a position and by the cache's bytes: two requests of keys and of values per thread
+// are in flight (16 wavefronts x 4 KiB), more cost registers that the accumulators of many heads need.
+// Measured, us at 8 rows x 4 KV heads, one wait per request and four in flight -> cached rows requested in front of the
+// prologue -> this: fp32, head size 64, one head per KV head, 60 / 500 / 2000 positions 5.2 / 9.4 / 23.6 -> 4.8 / 9.6 / 24.1 -> 4.3 /
+// 8.6 / 22.7, five heads 11.0 / 16.6 / 39.6 -> 9.2 / 17.8 / 42.1 -> 8.2 / 15.5 / 39.3, eight heads 43 / 157 / 558 -> 15 / 38 / 133 -> 11 / 27 / 74;
+// fp16, head size 32, four heads 13.3 / 14.1 / 19.0 -> 13.7 / 15.8 / 23.5 -> 12.2 / 13.3 / 18.7, eight 36 / 41 / 79 -> 28 / 39 / 84 -> 26 / 35 / 73;
+// head size 16, one head 5.9 / 6.3 / 7.5 -> 6.1 / 6.5 / 8.5 -> 5.6 / 5.9 / 7.8.  Three or four in flight: slower from four heads on.
 template <typename CT, typename AT, int D, int G>
 __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict__ d_pos_, const float* __restrict__ qkv_, void* kcache_, void* vcache_,
-                                                           const float* __restrict__ rope_cos_, const float* __restrict__ rope_sin_, int max_len_, unsigned counts_, int ldq_, int split_stride_, AttnArgs a) {
+                                                           const float* __restrict__ bias_, int max_len_, unsigned counts_, int ldq_, int split_stride_, AttnArgs a) {
     constexpr int NW = 16, NTH = NW * 64;
-    constexpr int EPL = 16 / (int)sizeof(CT), LPR = D / EPL, RPW = 64 / LPR, UR = 4, SWEEP = NW * RPW * UR;
+    constexpr int EPL = 16 / (int)sizeof(CT), LPR = D / EPL, RPW = 64 / LPR, UR = 2, SWEEP = NW * RPW * UR;
     typedef CT vec_t __attribute__((ext_vector_type(EPL)));
     __shared__ AttnSmem<CT, D, G, NW> sm;
     __shared__ __align__(16) CT s_k[D], s_v[D];
@@ -2557,42 +2563,48 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
     CT* Kb = (CT*)kcache_ + ((long)b * Hkv + kvc) * max_len_ * D;
     CT* Vb = (CT*)vcache_ + ((long)b * Hkv + kvc) * max_len_ * D;
     const int HD = H * D, GD = Hkv * D;
-    // the projection's sums: thread t takes columns t and t + 1024 of the group's (G + 2) D
+    // everything the prologue needs, in front of its first wait: the projection's sums (thread t takes columns t and t + 1024 of
+    // the group's (G + 2) D; split-K partials, the first eight at once), ...
     constexpr int NC = ((G + 2) * D + NTH - 1) / NTH, NP = ((G + 1) * D / 2 + NTH - 1) / NTH;
-    int col[NC]; float p0[NC];
+    int col[NC]; float part[NC][8], bias[NC], lnc[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         const int idx = min(t + i * NTH, (G + 2) * D - 1);
         col[i] = idx < G * D ? kvh * G * D + idx : idx < (G + 1) * D ? HD + kvc * D + (idx - G * D) : HD + GD + kvc * D + (idx - (G + 1) * D);
-        p0[i] = qkv_[(long)b * ldq_ + col[i]];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) { part[i][k] = 0.0f; if (k < KS) part[i][k] = qkv_[k * (long)split_stride_ + (long)b * ldq_ + col[i]]; }
+        bias[i] = bias_[col[i]]; lnc[i] = 0.0f;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ... the norm's tile sums and the rotation
+    float ssq_v[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ssum_v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (sizeof(CT) == 2) {
+        if (a.ssq) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) ssq_v[u] = a.ssq[(long)min(lane + 64 * u, a.ssq_nt - 1) * a.ssq_ld + b];
+            if (a.ln) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) ssum_v[u] = a.ssq[(long)(a.ssq_nt + min(lane + 64 * u, a.ssq_nt - 1)) * a.ssq_ld + b];
+#pragma unroll
+                for (int i = 0; i < NC; ++i) lnc[i] = bias_[ldq_ + col[i]];
+            }
+        }
     }
     float rc[NP], rs[NP];
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
         const int p = (t + i * NTH) % (D / 2);
-        rc[i] = rope_cos_ ? rope_cos_[(long)pos * (D / 2) + p] : 1.0f; rs[i] = rope_cos_ ? rope_sin_[(long)pos * (D / 2) + p] : 0.0f;
+        rc[i] = a.rope_cos ? a.rope_cos[(long)pos * (D / 2) + p] : 1.0f; rs[i] = a.rope_cos ? a.rope_sin[(long)pos * (D / 2) + p] : 0.0f;
     }
-    vec_t kv[UR], vv[UR];
-    int tt[UR];
-#pragma unroll
-    for (int u = 0; u < UR; ++u) {
-        tt[u] = (u * NW + wave) * RPW + rg;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) { kv[u][e] = (CT)0.0f; vv[u][e] = (CT)0.0f; }
-        if (tt[u] < pos) {
-            kv[u] = load_once((const vec_t*)(Kb + (long)tt[u] * D + sub * EPL));
-            vv[u] = load_once((const vec_t*)(Vb + (long)tt[u] * D + sub * EPL));
-        }
-    }
+    __builtin_amdgcn_sched_barrier(0);
     float rinv = 1.0f, mean = 0.0f;
     if constexpr (sizeof(CT) == 2) {
-        if (a.ssq) {
-            float s = 0.0f;
-            for (int tt = lane; tt < a.ssq_nt; tt += 64) s += a.ssq[(long)tt * a.ssq_ld + b];
-            s = wave_sum(s);                                   // same butterfly in every wavefront: identical result
+        if (a.ssq) {      // (the same butterfly in every wavefront: identical result)
+            float s = 0.0f, sv = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) if (lane + 64 * u < a.ssq_nt) { s += ssq_v[u]; sv += ssum_v[u]; }
+            s = wave_sum(s);
             if (a.ln) {
-                float sv = 0.0f;
-                for (int tt = lane; tt < a.ssq_nt; tt += 64) sv += a.ssq[(long)(a.ssq_nt + tt) * a.ssq_ld + b];
                 mean = wave_sum(sv) * a.inv_h;
                 rinv = 1.0f / sqrtf(fmaxf(s * a.inv_h - mean * mean, 0.0f) + a.eps);
             } else {
@@ -2602,16 +2614,11 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
     }
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-        // split-K partials in index order, eight requested at a time (unconditionally, the index clamped to the last split)
-        float s = p0[i];
-        for (int k = 1; k < KS; k += 8) {
-            float pk[8];
+        float s = part[i][0];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pk[j] = qkv_[min(k + j, KS - 1) * (long)split_stride_ + (long)b * ldq_ + col[i]];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) if (k + j < KS) s += pk[j];
-        }
-        if (t + i * NTH < (G + 2) * D) sm.in[t + i * NTH] = a.ln ? (s - mean * a.bias[ldq_ + col[i]]) * rinv + a.bias[col[i]] : s * rinv + a.bias[col[i]];
+        for (int k = 1; k < 8; ++k) if (k < KS) s += part[i][k];
+        for (int k = 8; k < KS; ++k) s += qkv_[k * (long)split_stride_ + (long)b * ldq_ + col[i]];
+        if (t + i * NTH < (G + 2) * D) sm.in[t + i * NTH] = (s - mean * lnc[i]) * rinv + bias[i];
     }
     __syncthreads();
 #pragma unroll
@@ -2621,7 +2628,7 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
             const int vec = p / (D / 2), j = p % (D / 2);
             const float x0 = sm.in[vec * D + 2 * j], x1 = sm.in[vec * D + 2 * j + 1];
             float y0 = x0, y1 = x1;
-            if (rope_cos_) rope_pair(x0, x1, rc[i], rs[i], y0, y1);
+            if (a.rope_cos) rope_pair(x0, x1, rc[i], rs[i], y0, y1);
             if (vec < G) { sm.q[vec * D + 2 * j] = a.scale * y0; sm.q[vec * D + 2 * j + 1] = a.scale * y1; }
             else {
                 CT* dst = Kb + (long)pos * D + 2 * j;
@@ -2630,6 +2637,7 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
         }
     }
     for (int d = t; d < D; d += NTH) Vb[(long)pos * D + d] = s_v[d] = (CT)sm.in[(G + 1) * D + d];
+    __threadfence_block();
     __syncthreads();
 
     // fp16 cache: queries as packed halves and v_dot2_f32_f16 (fp32 accumulate); fp32 cache: fp32 multiply-add
@@ -2656,7 +2664,7 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
 #pragma unroll
         for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
     }
-    auto take = [&](const vec_t& kc, const vec_t& vc, bool ok) {
+    auto take = [&](const vec_t& kc, const float (&vf)[EPL], bool ok) {
         float s[G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -2682,25 +2690,49 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
                 const float corr = __expf(m[g] - mn), p = __expf(s[g] - mn);
                 l[g] = l[g] * corr + p;
 #pragma unroll
-                for (int e = 0; e < EPL; ++e) acc[g][e] = acc[g][e] * corr + p * (float)vc[e];
+                for (int e = 0; e < EPL; ++e) acc[g][e] = acc[g][e] * corr + p * vf[e];
                 m[g] = mn;
             }
         }
     };
-    for (int base = 0; base < pos; base += SWEEP) {
+    vec_t kv[UR], vv[UR];
+    int tt[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+        tt[u] = (u * NW + wave) * RPW + rg;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) { kv[u][e] = (CT)0.0f; vv[u][e] = (CT)0.0f; }
+        if (tt[u] < pos) {
+            kv[u] = load_once((const vec_t*)(Kb + (long)tt[u] * D + sub * EPL));
+            vv[u] = load_once((const vec_t*)(Vb + (long)tt[u] * D + sub * EPL));
+        }
+        // (the new row from LDS where the first sweep holds it; a later one reads it back)
+        if (tt[u] == pos) { kv[u] = *(const vec_t*)&s_k[sub * EPL]; vv[u] = *(const vec_t*)&s_v[sub * EPL]; }
+    }
+    const int T = pos + 1;
+    int base = 0;
+    for (; base + NW * RPW < T; base += SWEEP) {
 #pragma unroll
         for (int u = 0; u < UR; ++u) {
-            const bool ok = tt[u] < pos;
-            const vec_t kc = kv[u], vc = vv[u];
+            const bool ok = tt[u] < T;
+            const vec_t kc = kv[u];
+            float vf[EPL];
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) vf[e] = (float)vv[u][e];
             tt[u] += SWEEP;
-            if (tt[u] < pos) {
+            if (tt[u] < T) {
                 kv[u] = load_once((const vec_t*)(Kb + (long)tt[u] * D + sub * EPL));
                 vv[u] = load_once((const vec_t*)(Vb + (long)tt[u] * D + sub * EPL));
             }
-            if ((base / RPW + u * NW + wave) * RPW < pos) take(kc, vc, ok);      // (a wavefront whose rows are all behind the last one skips them)
+            take(kc, vf, ok);
         }
     }
-    if (wave == 0) take(*(const vec_t*)&s_k[sub * EPL], *(const vec_t*)&s_v[sub * EPL], rg == 0);      // the new position
+    if (base < T) {      // (one row per lane group is left)
+        float vf[EPL];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) vf[e] = (float)vv[0][e];
+        take(kv[0], vf, tt[0] < T);
+    }
     attn_merge<CT, D, G, NW>(m, l, acc, sm.m, sm.l, sm.acc, sm.out);
     if (a.out_kt > 0) {
         for (int idx = t; idx < G * D; idx += NTH) ((AT*)a.out)[xpack_index(b, kvh * G * D + idx, a.out_kt)] = (AT)sm.out[idx];
