@@ -746,6 +746,7 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
 // 128 rows per expert in the last tile.
 static void run_packed_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long total, int epi, BigArgs e) {
     const int E = e.packed_problems;
+    TSHIP_REQUIRE(E >= 1 && E <= 64, "internal: a packed launch gives each problem a lane");
     e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.splits = 1;
     const GemmCost& whole = gemm_costs().back();
     const long CT = ceil_div(w.NT, whole.cols), half_tiles = E * CT / 2, tiles = total / whole.rows * CT;

@@ -1378,22 +1378,22 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     const int wr = w >> 1, wn = w & 1;                   // 4 x 2 wavefronts
     const int CT = (a.NT + 7) / 8;
     int RT = (int)((a.R + 255) / 256);
-    const int packed_up = a.packed_whole ? 0 : 255;
+    // (a lane per problem, up to 64: their row tiles and the running sum.  Two scalar loops over 64 problems took 3 us.)
+    int rows_e = 0, upto = 0;
     if (a.packed_problems) {
-        RT = 0;
-        for (int i = 0; i < a.packed_problems; ++i) RT += (a.rows_tab[i] + packed_up) / 256;
+        if (lane < a.packed_problems) rows_e = a.rows_tab[lane];
+        upto = (rows_e + (a.packed_whole ? 0 : 255)) >> 8;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(upto, o, 64); if (lane >= o) upto += v; }
+        RT = __builtin_amdgcn_readlane(upto, 63);
     }
     int rtile, ctile;
     if (!xcd_tile(blockIdx.x, RT, CT, a.patch_rows ? a.patch_rows : 8, rtile, ctile)) return;
     if (a.packed_problems) {
-        // the problem whose tiles hold packed row tile `rtile` (block-uniform: the counts sit in scalar registers)
-        int e = -1, first = 0;
-        for (int i = 0; i < a.packed_problems; ++i) {
-            const int tiles = (a.rows_tab[i] + packed_up) / 256;
-            if (e < 0 && rtile < first + tiles) { e = i; rtile -= first; }
-            first += tiles;
-        }
-        a.R = a.rows_tab[e]; a.W = a.Wtab[e]; a.X += e * a.x_estride;
+        // the problem whose tiles hold packed row tile `rtile`: behind those that end in front of it
+        const int e = __popcll(__ballot(upto <= rtile));
+        if (e) rtile -= __builtin_amdgcn_readlane(upto, e - 1);
+        a.R = __builtin_amdgcn_readlane(rows_e, e); a.W = a.Wtab[e]; a.X += e * a.x_estride;
         if (a.out) a.out += e * a.out_estride;
         if (a.out16) a.out16 += e * a.out16_estride;
         if (a.row_idx) a.row_idx += e * a.idx_estride;

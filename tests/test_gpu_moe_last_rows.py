@@ -15,8 +15,8 @@ def G():
     return gpt
 
 
-# 512 rows: fewer than 256 per expert of eight (no whole row tile)
-@pytest.mark.parametrize("experts,k,batch,prompt,router_bias", [(8, 1, 4, 128, None), (4, 2, 5, 520, None), (16, 5, 1, 600, None),
+# 512 rows: fewer than 256 per expert of eight (no whole row tile); as many experts as lanes, some of them without rows
+@pytest.mark.parametrize("experts,k,batch,prompt,router_bias", [(64, 2, 3, 210, None), (64, 1, 2, 300, (60.0,) * 5 + (0.0,) * 59), (33, 3, 1, 700, None), (8, 1, 4, 128, None), (4, 2, 5, 520, None), (16, 5, 1, 600, None),
                                                                 (4, 2, 2, 256, (60.0, 0.0, 0.0, 0.0)), (4, 2, 3, 200, (-60.0, 0.0, 0.0, 0.0))])
 @pytest.mark.parametrize("tile", [11, 12, 14, 22, 24, None])
 def test_last_rows_by_themselves(G, oracle, monkeypatch, experts, k, batch, prompt, router_bias, tile):
