@@ -3049,11 +3049,13 @@ struct AttnPacked {
 };
 constexpr int MAX_ATTN_SPLITS = 16;
 // Most chunks of 32 positions that one block of a pair takes by itself: a round of chunks of all its wavefronts takes 1.1 us, the
-// exchange 2 (head size 128: 3).  Two or three blocks per pair mean that most of the chip's bandwidth is in use already.  One
+// exchange 2 (head size 128: 3).  Two or three blocks per pair mean that more of the chip's bandwidth is in use already.  One
 // block -> several, ms per 17 steps: 1B model, one row at 300 / 600 / 1000 / 2000 positions 10.39 / 10.72 / 11.21 / 12.44 -> (one) /
-// 10.75 (so one) / 10.91 / 11.06, 8 rows at 1500 12.30 -> 11.84, 16 rows at 1500 (two blocks) 12.87 -> 13.07 (so one); 8 layers of the
-// 7B one, one row at 1000 12.86 -> 12.22, 8 rows at 500 12.43 -> 12.57 (so one), 3 rows at 3000 14.01 -> 12.90.
-__host__ __device__ constexpr int attn_split_chunks(int D, int S) { return S < 4 ? (D == 128 ? 63 : 127) : (D == 128 ? 20 : 24); }
+// 10.75 (so one) / 10.91 / 11.06, 8 rows at 1500 12.30 -> 11.84; 8 layers of the 7B one, one row at 1000 12.86 -> 12.22, 8 rows at
+// 500 12.43 -> 12.57 (so one), 3 rows at 3000 14.01 -> 12.90.  Two launched, one -> two of them at work, us a step at 500 / 1000 / 1500 /
+// 2000 / 4030 positions: 4 layers of the 1B model, 16 rows 178 / 188 / 199 / 211 / 256 -> 181 / 188 / 197 / 207 / 245; 8 layers of 12 heads, 8 rows
+// 234 / 254 / 274 / 299 / 378 -> 239 / 250 / 264 / 277 / 334; 2 layers of the 7B one, 12 rows 200 / 205 / 215 / 224 / - -> 202 / 203 / 211 / 217 / -.
+__host__ __device__ constexpr int attn_split_chunks(int D, int S) { return S < 4 ? (D == 128 ? 36 : 30) : (D == 128 ? 20 : 24); }
 template <int D, int G, bool SPLIT, bool SUB = false>      // SUB: groups of query heads share a KV head (AttnArgs::kv_sub > 1)
 __global__ __launch_bounds__(D == 128 ? 256 : 512) void attn_mfma_kernel(void* kcache_, int d_vcache, int d_qkv, int d_pos, int d_bias, int d_ssq, int d_rope_cos,
                                                                        int d_rope_sin, int max_len_, unsigned counts, int ldq_, int split_stride_,

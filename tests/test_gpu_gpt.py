@@ -463,10 +463,12 @@ def test_decode_attention_split_over_blocks(G, oracle, monkeypatch, hidden, head
     gpu.close()
 
 
-@pytest.mark.parametrize("hidden,heads,kv_heads,batch,at", [(256, 4, 2, 1, 768), (256, 2, 1, 2, 640), (512, 8, 8, 5, 768)])
-def test_decode_attention_takes_more_blocks_as_the_context_grows(G, monkeypatch, hidden, heads, kv_heads, batch, at):
+@pytest.mark.parametrize("hidden,heads,kv_heads,batch,at,cache", [(256, 4, 2, 1, 768, 1100), (256, 2, 1, 2, 640, 1100), (512, 8, 8, 5, 768, 1100),
+                                                                  (512, 8, 8, 12, 960, 4100), (512, 4, 4, 25, 1152, 2100)])
+def test_decode_attention_takes_more_blocks_as_the_context_grows(G, monkeypatch, hidden, heads, kv_heads, batch, at, cache):
     """Head sizes 64 and 128: the captured step goes on from the last position that one block of a pair takes by itself to the
-    first that several share.  Against one block throughout, and against the prefill path."""
+    first that several share (the last two: two blocks, in caches long enough to launch them).  Against one block throughout, and
+    against the prefill path."""
     cfg = synth.tiny_config(dtype="f16", hidden=hidden, n_heads=heads, n_kv_heads=kv_heads, ffn_dim=2 * hidden, vocab=300, batch=batch, prompt=at - 3)
     w = synth.make_weights(cfg, 83, random_bias=True)
     seqs = synth.make_prompts(cfg, 84)
@@ -474,7 +476,7 @@ def test_decode_attention_takes_more_blocks_as_the_context_grows(G, monkeypatch,
     for splits in (None, "1"):
         if splits:
             monkeypatch.setenv("TSHIP_ATTN_SPLITS", splits)
-        gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=1100)
+        gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=cache)
         gpu.prefill(seqs)
         ids, _ = gpu.generate(6)
         ids = ids.reshape(6, batch)
