@@ -8,6 +8,8 @@
 // replays; eight launches with norm and activation kernels of their own -> these): one row of the 512-wide gated model
 // (context 64-96) QKV 5.2, attention 5.5, output 5.0 + norm 3.9, up 6.6 + activation 3.1, down 6.3 + norm 3.9 -> 3.9, 5.4, 4.8,
 // 4.1, 6.4; eight rows of the 768-wide one (context 300) 7.0, 9.4, 5.2 + 6.1, 7.8 + 3.3, 10.6 + 6.1 -> 4.6, 8.7, 5.8, 6.5, 8.6.
+// Whole steps of six layers at 8 / 16 / 17 / 32 rows (from 17 on in two groups of 16, which read the weights twice): 512 wide
+// 312 / 399 / 547 / 602 -> 195 / 232 / 240 / 247; 768 wide 347 / 452 / 712 / 820 -> 221 / 270 / 309 / 350; 2048 wide (ffn 5632) 689 / 941 / 1923 / 2192 -> 498 / 604 / 765 / 792 us.
 // An empty launch is 1.7 us.  Rows summed and normalised from the partial sums by every consumer, without the exchange in the
 // tails, were measured at one row: 1.5 us more in each consumer for 1.9 less in each producer, and 2.9 at two rows; not kept.
 #pragma once

@@ -793,18 +793,26 @@ static auto with_heads(int D, int G, F&& f) {
         default: throw Error("head_dim must be 16, 32, 64 or 128");
     }
 }
-template <typename CT, typename AT>
+// (fp16 caches with head sizes 64 and 128 have the fragment layout and kernels of their own)
+template <typename T, int D> constexpr bool row_major_cache = sizeof(T) == 4 || D <= 32;
+template <typename T>
 static AttnKernel pick_attn_d(int D, int G, AttnKind kind) {
     return with_heads(D, G, [&](auto Dc, auto Gc) -> AttnKernel {
-        if constexpr (sizeof(CT) == 4) { if (kind == ATTN_PREFILL_TILES) return attn_prefill_f32_kernel<decltype(Dc)::value, decltype(Gc)::value>; }
-        return attn_prefill_kernel<CT, AT, decltype(Dc)::value, decltype(Gc)::value>;
+        constexpr int HD = decltype(Dc)::value, HG = decltype(Gc)::value;
+        if constexpr (sizeof(T) == 4) { if (kind == ATTN_PREFILL_TILES) return attn_prefill_f32_kernel<HD, HG>; }
+        if constexpr (row_major_cache<T, HD>) return attn_prefill_kernel<T, T, HD, HG>;
+        else throw Error("internal: a cache of another layout");
     });
 }
 // decode attention of caches without the fragment layout
 typedef void (*AttnStepKernel)(const int*, const float*, void*, void*, const float*, int, unsigned, int, int, AttnArgs);
 template <typename T>
 static AttnStepKernel pick_attn_step(int D, int G) {
-    return with_heads(D, G, [&](auto Dc, auto Gc) -> AttnStepKernel { return attn_decode_kernel<T, T, decltype(Dc)::value, decltype(Gc)::value>; });
+    return with_heads(D, G, [&](auto Dc, auto Gc) -> AttnStepKernel {
+        constexpr int HD = decltype(Dc)::value;
+        if constexpr (row_major_cache<T, HD>) return attn_decode_kernel<T, T, HD, decltype(Gc)::value>;
+        else throw Error("internal: a cache of another layout");
+    });
 }
 template <int D>
 static AttnKernel pick_attn_mfma_prefill(int G, bool ragged, int nq) {
@@ -894,7 +902,7 @@ static AttnDecodeKernel pick_attn_mfma_decode(int G, bool split, bool sub) {
 }
 static AttnKernel pick_attn_prefill(TSHipGpt* m, AttnKind kind, bool ragged = false, int nq = 1) {
     if (m->vt) return m->D == 64 ? pick_attn_mfma_prefill<64>(m->G, ragged, nq) : pick_attn_mfma_prefill<128>(m->G, ragged, nq);
-    return m->f16 ? pick_attn_d<half_t, half_t>(m->D, m->G, kind) : pick_attn_d<float, float>(m->D, m->G, kind);
+    return m->f16 ? pick_attn_d<half_t>(m->D, m->G, kind) : pick_attn_d<float>(m->D, m->G, kind);
 }
 // Kernel of an fp32 prefill's attention: a block per query that reads the cache with all lanes, or tiles of 32 columns on the
 // matrix cores.  A tile takes the positions in steps of 128 however few of its columns are queries, so few queries of small

@@ -87,7 +87,9 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
     if (m->f16 && h % 4 == 0) {      // tree-order sums: an fp16 model's routing input is not the reference's to the last bit anyway
         // a row per wavefront for a prefill's rows, the matrix in 64 KiB of LDS; a block per row for the others, whose launch does not
         // wait for the matrix: 1024 columns, 8 experts, 512 / 1024 / 1536 / 2048 / 4096 / 8192 rows 7.3 / 9.7 / 12.0 / 14.7 / 24.6 / 50.4 us
-        // with it, 9.2 / 9.3 / 9.7 / 10.3 / 14.3 / 22.2 per wavefront
+        // with it, 9.2 / 9.3 / 9.7 / 10.3 / 14.3 / 22.2 per wavefront.  Other sizes meet before that line: us a prompt of three layers, one of
+        // them MoE, at 1000 and 1100 rows, block -> wavefront: 256 columns, 8 experts 255 / 260 -> 252 / 256, 1024 columns, 16 experts 436 / 463 ->
+        // 407 / 427, 1536 columns, 8 experts 586 / 600 -> 583 / 591, 2048 columns, 8 experts 711 / 767 -> 709 / 761
         const long shm = (h * round_up(E, 8) + 2L * h) * 4;
         if (batched && rows > g_hooks.moe_router_rows && !r.part && k <= 4 && h * round_up(E, 8) <= 16384) {
             r.rows = rows;
