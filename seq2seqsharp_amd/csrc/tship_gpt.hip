@@ -638,7 +638,7 @@ static GemmTile best_gemm_tile(int KT, int NT, long R, float own_cache_write = 0
     }
     return best;
 }
-static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) {
+static int pick_gemm_tile(const GemmW& w, long R) {
     const int forced = g_hooks.gemm_tile;
     if (forced == 0 && R >= 256) return 0;
     if (forced > 0) {
@@ -646,7 +646,7 @@ static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) 
         const bool fits = ceil_div(R, c.rows) * ceil_div(w.NT, c.cols) * (forced / 100) <= TSHipGpt::MID_XCHG_TILES;
         return forced % 100 + 100 * (forced >= 200 && fits ? mid_splits(w.KT, forced % 100, forced / 100) : 1);
     }
-    return best_gemm_tile(w.KT, w.NT, R, own_cache_write).tile;
+    return best_gemm_tile(w.KT, w.NT, R).tile;
 }
 // A launch whose last round holds few tiles leaves most of the chip idle for as long as a whole round takes: instead, the first
 // `cols` 32-column tiles in whole rounds of one tile, and the other columns in a launch of their own with the tile that is best for
@@ -655,6 +655,7 @@ static int pick_gemm_tile(const GemmW& w, long R, float own_cache_write = 0.0f) 
 // 8 layers of the 7B one, 700 / 4400 rows 3.6 / 17.0 -> 3.1 / 13.9; the 768-wide one, 6000 rows 3.8 -> 3.3.
 struct GemmMix { int tile, cols, rest; float us; };
 static GemmMix pick_gemm_mix(const GemmW& w, long R) {
+    if (g_hooks.gemm_tile >= 0) return {pick_gemm_tile(w, R), 0, 0, 0.0f};
     const long ncu = std::max(1, n_compute_units());
     const GemmTile one = best_gemm_tile(w.KT, w.NT, R);
     GemmMix mix = {one.tile, 0, 0, one.us};
@@ -716,27 +717,22 @@ static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, i
 }
 
 // Y = X * W for many rows (prefill), fp16, X row-major.
-static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, int tile = -1) {
+static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, BigArgs e, const GemmMix& mix) {
     e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.R = (int)R;
-    if (tile < 0 && g_hooks.gemm_tile < 0) {
-        const GemmMix mix = pick_gemm_mix(w, R);
-        tile = mix.tile;
-        if (mix.cols) {
-            const int off = epi == BEPI_ACT16 && e.gated ? 16 * mix.cols : 32 * mix.cols;       // outputs of the first part
-            TSHIP_REQUIRE(!e.kcache && !e.advance_pos && !e.ssq && off < e.n_valid, "internal: columns of this projection stay together");
-            BigArgs r = e;
-            e.NT = mix.cols; e.n_valid = off;
-            r.W += (long)mix.cols * w.KT * 512; r.NT -= mix.cols; r.n_valid -= off; r.bias += off;
-            if (r.bias2) r.bias2 += off;
-            if (epi == BEPI_ACT16) r.out16 += off; else r.out += off;
-            if (epi == BEPI_RESID && r.xg16) { r.xg16 += off; r.gamma += off; r.ssq_out += mix.cols * r.ssq_ld; }
-            launch_big_gemm(m, name, e, epi, mix.tile);
-            launch_big_gemm(m, name, r, epi, mix.rest);
-            return;
-        }
-    }
-    if (tile < 0) tile = pick_gemm_tile(w, R);
-    launch_big_gemm(m, name, e, epi, tile);
+    if (!mix.cols) { launch_big_gemm(m, name, e, epi, mix.tile); return; }
+    const int off = epi == BEPI_ACT16 && e.gated ? 16 * mix.cols : 32 * mix.cols;       // outputs of the first part
+    TSHIP_REQUIRE(!e.kcache && !e.advance_pos && !e.ssq && off < e.n_valid, "internal: columns of this projection stay together");
+    BigArgs r = e;
+    e.NT = mix.cols; e.n_valid = off;
+    r.W += (long)mix.cols * w.KT * 512; r.NT -= mix.cols; r.n_valid -= off; r.bias += off;
+    if (r.bias2) r.bias2 += off;
+    if (epi == BEPI_ACT16) r.out16 += off; else r.out += off;
+    if (epi == BEPI_RESID && r.xg16) { r.xg16 += off; r.gamma += off; r.ssq_out += mix.cols * r.ssq_ld; }
+    launch_big_gemm(m, name, e, epi, mix.tile);
+    launch_big_gemm(m, name, r, epi, mix.rest);
+}
+static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const void* X, long ldx, long R, int epi, const BigArgs& e, int tile) {
+    run_big_gemm(m, name, w, X, ldx, R, epi, e, GemmMix{tile, 0, 0, 0.0f});
 }
 
 // The experts of a MoE layer, e.packed_problems of them with `total` rows together (the device knows which has how many): one
@@ -1432,29 +1428,36 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     auto producer = [&](BigArgs& e, const float* gamma) {        // residual GEMM that also emits the next GEMM's input
         e.xg16 = pxn.as<half_t>(); e.ld_xg = (int)m->ldh; e.gamma = gamma; e.ssq_out = pssq.as<float>(); e.ssq_ld = R;
     };
-    auto big = [&](const char* name, const GemmW& w, const void* X, long ldx, int epi, BigArgs e, int tile = -1) { run_big_gemm(m, name, w, X, ldx, R, epi, e, tile); };
+    auto big = [&](const char* name, const GemmW& w, const void* X, long ldx, int epi, const BigArgs& e, const GemmMix& tiles) { run_big_gemm(m, name, w, X, ldx, R, epi, e, tiles); };
     DevBuf& zero_bias = m->pw_zero_bias; zero_bias.reserve((size_t)std::max<long>(std::max<long>(qp, m->F13), round_up(h, 32)) * sizeof(float));
+    // Tiles of the projections, chosen once for all layers (layer 0 has them all, and the others' shapes): a choice takes the host up to
+    // 3 us (five of them in every layer before: three layers of the 1B model at 100 / 333 / 1500 rows 256 / 378 / 784 -> 249 / 374 / 764 us).
+    // The QKV projection with 256 x 256 tiles can write keys and values into the fragment-major cache itself (rotation
+    // included) when its wavefronts' 64 x 128 tiles are whole chunks of whole heads.  That takes it about 7.5 us longer and
+    // saves a kernel whose time goes with rows x columns of keys and values (profiles/prefill_gemm_tiles.txt: 1024 columns,
+    // 1024 rows 49.0 + 7.4 against 62.5 us, 16384 rows 202 + 37 against 211); a kernel of its own does it where that is less.
+    const int HD = c.n_heads * m->D, GD = c.n_kv_heads * m->D;
+    GemmMix qkv_tiles = {}, wo_tiles = {}, w13_tiles = {}, w2_tiles = {};
+    bool fuse_kv = false;
+    if (m->f16) {
+        const LayerW& L = *m->L[0];
+        const bool can_fuse_kv = m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && L.qkv.KT % 2 == 0 && (m->D == 64 || m->D == 128);
+        const float fuse_saves = 1.9e-6f * (float)(R * 2 * GD) - 7.5f;
+        const float own_write = can_fuse_kv ? std::max(0.0f, fuse_saves) : 0.0f;
+        qkv_tiles = pick_gemm_mix(L.qkv, R);
+        if (g_hooks.gemm_tile < 0) {      // (two launches of different tiles where that is less than the saved kernel)
+            const GemmTile one = best_gemm_tile(L.qkv.KT, L.qkv.NT, R, own_write);
+            if (!qkv_tiles.cols || qkv_tiles.us >= one.us) qkv_tiles = {one.tile, 0, 0, one.us};
+        }
+        fuse_kv = can_fuse_kv && !qkv_tiles.tile && !qkv_tiles.cols && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
+        wo_tiles = pick_gemm_mix(L.wo, R); w13_tiles = pick_gemm_mix(L.w13, R); w2_tiles = pick_gemm_mix(L.w2, R);
+    }
     for (int l = 0; l < c.n_layers; ++l) {
         LayerW& L = *m->L[l];
         AttnArgs aa = attn_args(m, L);
         aa.qkv = pqkv.as<float>(); aa.KS = 1; aa.split_stride = 0; aa.ldq = qp; aa.pos0 = pos0; aa.Tq = Tp;
         aa.out = po.p; aa.ld_out = m->ldh;
         aa.lens = host_lens ? m->pw_lens.as<int>() : nullptr;
-        // The QKV projection with 256 x 256 tiles can write keys and values into the fragment-major cache itself (rotation
-        // included) when its wavefronts' 64 x 128 tiles are whole chunks of whole heads.  That takes it about 7.5 us longer and
-        // saves a kernel whose time goes with rows x columns of keys and values (profiles/prefill_gemm_tiles.txt: 1024 columns,
-        // 1024 rows 49.0 + 7.4 against 62.5 us, 16384 rows 202 + 37 against 211); a kernel of its own does it where that is less.
-        const int HD = c.n_heads * m->D, GD = c.n_kv_heads * m->D;
-        const bool can_fuse_kv = m->f16 && m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && L.qkv.KT % 2 == 0 &&
-                                 (m->D == 64 || m->D == 128);
-        const float fuse_saves = 1.9e-6f * (float)(R * 2 * GD) - 7.5f;
-        const float own_write = can_fuse_kv ? std::max(0.0f, fuse_saves) : 0.0f;
-        int qkv_tile = m->f16 ? pick_gemm_tile(L.qkv, R, own_write) : 0;
-        if (m->f16 && g_hooks.gemm_tile < 0) {      // (two launches of different tiles, -1, where that is less than the saved kernel)
-            const GemmMix mix = pick_gemm_mix(L.qkv, R);
-            if (mix.cols && mix.us < best_gemm_tile(L.qkv.KT, L.qkv.NT, R, own_write).us) qkv_tile = -1;
-        }
-        const bool fuse_kv = can_fuse_kv && !qkv_tile && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
         if (m->f16) {
             BigArgs e; std::memset(&e, 0, sizeof(e));
             e.out = pqkv.as<float>(); e.ld_out = (int)qp; e.bias = L.bqkv.as<float>(); e.n_valid = m->Nqkv;
@@ -1464,7 +1467,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
                 e.kcache = (half_t*)L.kc.p; e.vcache = (half_t*)L.vc.p; e.kv_max_len = m->ML; e.kv_col0 = HD; e.kv_gd = GD; e.kv_D = m->D;
                 e.kv_hkv = c.n_kv_heads; e.kv_Tq = Tp; e.kv_pos0 = pos0; e.rope_cos = aa.rope_cos; e.rope_sin = aa.rope_sin;
             }
-            big("p_gemm_qkv", L.qkv, pxn.p, m->ldh, BEPI_F32_BIAS, e, qkv_tile);
+            big("p_gemm_qkv", L.qkv, pxn.p, m->ldh, BEPI_F32_BIAS, e, qkv_tiles);
             aa.bias = zero_bias.as<float>();      // bias already added by the GEMM epilogue
         } else {
             run_gemm_f32(m, "p_gemm_qkv", L.qkv, pxn.as<float>(), m->ldh, (int)R, pqkv.as<float>(), qp, 0, 1);
@@ -1498,7 +1501,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             BigArgs e; std::memset(&e, 0, sizeof(e));
             e.out = px.as<float>(); e.ld_out = h; e.bias = L.bo.as<float>(); e.n_valid = h;
             if (deferred) producer(e, L.n2_g.as<float>());
-            big("p_gemm_wo", L.wo, po.p, m->ldh, BEPI_RESID, e);
+            big("p_gemm_wo", L.wo, po.p, m->ldh, BEPI_RESID, e, wo_tiles);
         } else {
             run_gemm_f32(m, "p_gemm_wo", L.wo, po.as<float>(), m->ldh, (int)R, pqkv.as<float>(), qp, 0, 1);
             a2.part = pqkv.as<float>(); a2.KS = 1; a2.ld_part = qp; a2.bias = L.bo.as<float>();
@@ -1521,11 +1524,11 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             e.bias = L.b1.as<float>(); e.bias2 = L.b3.as<float>(); e.out16 = pa.as<half_t>(); e.ld16 = (int)m->ldF;
             e.act = c.act; e.gated = m->gated; e.n_valid = F;
             if (deferred) e.rinv = prinv.as<float>();
-            big("p_gemm_ffn13", L.w13, pxn.p, m->ldh, BEPI_ACT16, e);
+            big("p_gemm_ffn13", L.w13, pxn.p, m->ldh, BEPI_ACT16, e, w13_tiles);
             BigArgs e2; std::memset(&e2, 0, sizeof(e2));
             e2.out = px.as<float>(); e2.ld_out = h; e2.bias = L.b2.as<float>(); e2.n_valid = h;
             if (deferred && l + 1 < c.n_layers) producer(e2, m->L[l + 1]->n1_g.as<float>());
-            big("p_gemm_ffn2", L.w2, pa.p, m->ldF, BEPI_RESID, e2);
+            big("p_gemm_ffn2", L.w2, pa.p, m->ldF, BEPI_RESID, e2, w2_tiles);
         } else {
             run_gemm_f32(m, "p_gemm_ffn13", L.w13, pxn.as<float>(), m->ldh, (int)R, pf.as<float>(), m->F13, 0, 1);
             long tot = R * F;

@@ -128,15 +128,16 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
         half_t* xg = (half_t*)(base + o.xg); half_t* mid = (half_t*)(base + o.mid);
         launch(m, "moe_gather", moe_gather_kernel<half_t>, dim3(rows, E), dim3(256), (const float*)xn32, h, (const int*)counts, (const int*)lists, (int)Bp, xg,
                m->ldh, xg_stride, 0);
-        const int tile = g_hooks.no_moe_batch ? 0 : -1;      // (the hook compares with the batched launches: same tile, same bits)
+        // (the hook compares with the batched launches: same tile, same bits)
+        auto tiles = [&](const GemmW& w, long R) { return g_hooks.no_moe_batch ? GemmMix{} : pick_gemm_mix(w, R); };
         for (int e = 0; e < E; ++e) {
             if (n_e[e] == 0) continue;
             BigArgs e1; std::memset(&e1, 0, sizeof(e1));
             e1.bias = zero; e1.out16 = mid + e * mid_stride; e1.ld16 = (int)o.ld4h; e1.act = c.act; e1.gated = 0; e1.n_valid = 4 * h;
-            run_big_gemm(m, "moe_gemm1", *L.e1[e], xg + e * xg_stride, m->ldh, n_e[e], BEPI_ACT16, e1, tile);
+            run_big_gemm(m, "moe_gemm1", *L.e1[e], xg + e * xg_stride, m->ldh, n_e[e], BEPI_ACT16, e1, tiles(*L.e1[e], n_e[e]));
             BigArgs e2; std::memset(&e2, 0, sizeof(e2));
             e2.bias = zero; e2.out = y + e * y_stride; e2.ld_out = (int)o.ldy; e2.n_valid = h;
-            run_big_gemm(m, "moe_gemm2", *L.e2[e], mid + e * mid_stride, o.ld4h, n_e[e], BEPI_F32_BIAS, e2, tile);
+            run_big_gemm(m, "moe_gemm2", *L.e2[e], mid + e * mid_stride, o.ld4h, n_e[e], BEPI_F32_BIAS, e2, tiles(*L.e2[e], n_e[e]));
         }
     } else if (m->f16) {
         half_t* xg = (half_t*)(base + o.xg); half_t* mid = (half_t*)(base + o.mid);
