@@ -1739,11 +1739,14 @@ TSHIP_API int TSHip_GptFinalize(TSHipGpt* m) {
         // residual-tail projections (N = hidden): split K so that the launch has about one block per compute unit
         // (more blocks than that run in a second wave, which measured 2 us slower)
         // (and every split costs the last block an exchange: us at 8 rows for 2 / 4 / 6 / 8 / 10 splits, 768 x 768 5.2 / 5.0 / 5.3 / 5.7 /
-        // 6.6, 3072 x 768 6.5 / 5.9 / 5.8 / 6.1 / 7.0)
+        // 6.6, 3072 x 768 6.5 / 5.9 / 5.8 / 6.1 / 7.0.  Steps of six layers of other widths, one / 32 rows: 512 wide, output projection in
+        // 2 / 4 splits 150 / 173 and 150 / 174 us, down (2048) in 6 / 8 / 16 148 / 174, 150 / 174 and 172 / 195; 1024 wide, output in 5 / 8
+        // 169 and 173 (one row), down (4096) in 6 / 8 / 16 169, 170 and 195.  With up to eight column tiles the last blocks have the
+        // chip to themselves: 256 wide, output in 1 / 2 splits 136 / 155 and 130 / 152 us, down (2048) in 5 / 8 / 12 142 / 162,
+        // 137 / 160 and 148 / 169; 128 wide, down (2048) in 5 / 8 136 / 155 and 134 / 150)
         auto tail_ks = [&](const GemmW& w) {
-            int ks = std::max(1, n_compute_units() / std::max(1, w.NT));
-            ks = std::min(ks, std::max(1, w.KT / 12));
-            return std::min(ks, 6);
+            const int ks = std::max(1, n_compute_units() / std::max(1, w.NT)), most = std::max(1, w.KT / 8);
+            return std::min(ks, w.NT <= 8 ? std::min(most, 8) : std::min(std::max(w.KT / 12, std::min(2, most)), 6));
         };
         for (auto& L : m->L) { L->wo.KS = tail_ks(L->wo); L->w2.KS = tail_ks(L->w2); }
     }

@@ -16,7 +16,9 @@ def G():
 
 
 # hidden -> fragments per wavefront of the vocabulary projection: 4, 5, 6, 7, 11 (and half of that or more splits elsewhere)
-@pytest.mark.parametrize("hidden,heads,kv,ffn", [(512, 8, 2, 832), (640, 10, 5, 448), (768, 12, 12, 3072), (896, 14, 2, 576), (1408, 11, 11, 256)])
+@pytest.mark.parametrize("hidden,heads,kv,ffn", [(512, 8, 2, 832), (640, 10, 5, 448), (768, 12, 12, 3072), (896, 14, 2, 576), (1408, 11, 11, 256),
+                                                   # few column tiles: tails of one, two and eight splits, ranges of uneven length
+                                                   (128, 2, 2, 2048), (256, 4, 2, 1072), (352, 11, 1, 32)])
 @pytest.mark.parametrize("norm,act", [(synth.RMSNORM, synth.SWIGLU), (synth.LAYERNORM, synth.RELU)])
 @pytest.mark.parametrize("max_batch,batch", [(1, 1), (32, 17), (64, 33), (128, 65)])
 def test_steps(G, oracle, hidden, heads, kv, ffn, norm, act, max_batch, batch):
