@@ -284,7 +284,10 @@ TSHIP_API int TSHip_GptStepBytes(TSHipGpt* m, int batch, double* weight_bytes, d
  *   TSHIP_ATTN_NQ=1|2         prefill attention: groups of 16 MFMA columns per wavefront
  *   TSHIP_NO_KV_FUSE=1        prefill: the QKV projection leaves the cache write to a kernel of its own
  *   TSHIP_NO_MOE_BATCH=1      prefill of MoE layers: the experts' row counts are read back, the rows gathered and one GEMM
- *                             launched per expert, instead of one launch per projection with everything on the device */
+ *                             launched per expert, instead of one launch per projection with everything on the device
+ *   TSHIP_MOE_REST=11|12|14|22|24   prefill of MoE layers: the experts' last rows (behind whole 256-row tiles) in a launch of this tile
+ *                             (default: where that is estimated faster)
+ *   TSHIP_MOE_ROUTER_ROWS=n   prefill of fp16 MoE layers: a wavefront per row in the router from n + 1 rows on (default 1024) */
 
 #ifdef __cplusplus
 }
