@@ -275,8 +275,9 @@ TSHIP_API int TSHip_GptStepBytes(TSHipGpt* m, int batch, double* weight_bytes, d
  *   TSHIP_NO_GRAPH=1          the generate loop launches its kernels one by one instead of replaying a captured HIP graph
  *   TSHIP_ATTN_SPLITS=n       decode attention: n blocks per (sequence, KV head) pair (default: chosen from the batch and context)
  *   TSHIP_FFN_TILES=10|15|20|30|40   decode FFN up projection: column tiles per block x 10 (15 = a tile and a half)
- *   TSHIP_GEMM_TILE=0|11|12|14|22|24   prefill GEMMs: tile of mid_gemm_f16_kernel (10 x 64-row groups + 32-column tiles), 0 = the
- *                             256 x 256 tile from 256 rows on; + 200 ... 400: so many blocks share a tile's K (default: by estimated time)
+ *   TSHIP_GEMM_TILE=0|11|12|14|22|24|42|43|45   prefill GEMMs: tile of mid_gemm_f16_kernel (10 x 64-row groups + 32-column tiles), 0 = the
+ *                             256 x 256 tile from 256 rows on, 42, 43, 45 = that tile with 128, 192 or 320 columns (even k-tile counts);
+ *                             11 ... 24 + 200 ... 400: so many blocks share a tile's K (default: by estimated time)
  *   TSHIP_F32_TILE=11|21|22|42    fp32 GEMMs from 33 rows on: tile in units of 32 rows (10 x) and 32 columns (default: by size)
  *   TSHIP_F32_ATTN=0|1        attention of fp32 prefills: a block per query, or tiles of 32 columns (default: by estimated time)
  *   TSHIP_RECORD_SYMBOLS=1    TSHip_GptProfileSymbols gives the kernels launched since the last prefill began

@@ -212,8 +212,9 @@ static void refresh_test_hooks() {
     if (const char* v = std::getenv("TSHIP_GEMM_TILE")) {
         h.gemm_tile = std::atoi(v);
         const int tile = h.gemm_tile % 100, splits = h.gemm_tile / 100;
-        TSHIP_REQUIRE((h.gemm_tile == 0 || tile == 11 || tile == 12 || tile == 14 || tile == 22 || tile == 24) && splits >= 0 && splits <= MID_SPLITS,
-                      "TSHIP_GEMM_TILE: 0, 11, 12, 14, 22 or 24, plus 100 x the blocks (2 to 4) that share a tile's K");
+        TSHIP_REQUIRE((h.gemm_tile == 0 || tile == 11 || tile == 12 || tile == 14 || tile == 22 || tile == 24 ||
+                       h.gemm_tile == 42 || h.gemm_tile == 43 || h.gemm_tile == 45) && splits >= 0 && splits <= MID_SPLITS,
+                      "TSHIP_GEMM_TILE: 0, 11, 12, 14, 22 or 24, plus 100 x the blocks (2 to 4) that share a tile's K; 42, 43 or 45");
     }
     if (const char* v = std::getenv("TSHIP_F32_TILE")) {
         h.f32_tile = std::atoi(v);
@@ -616,24 +617,38 @@ static const std::vector<GemmCost>& gemm_costs() {
     typedef GemmCost Cost;
     static const Cost costs[] = {{11, 64, 1, 3.5f, 0.031f}, {12, 64, 2, 4.4f, 0.046f}, {14, 64, 4, 6.5f, 0.077f},
                                  {22, 128, 2, 5.2f, 0.072f}, {24, 128, 4, 8.1f, 0.111f}, {0, 256, 8, 11.0f, 0.315f}};
-    static const std::vector<GemmCost> v(std::begin(costs), std::end(costs));
+    // Other widths of the 256-row tile, for even k-tile counts: 128, 192 and 320 columns.  A launch of a few rounds is as long as its
+    // rounds, and with a width to choose the tiles fill them: of 108 launches (12 pairs of K and N, 333 ... 16384 rows, profiles/prefill_gemm_wide_tiles.txt)
+    // the choice among 128 x 64, 128 x 128 and 256 x 256 costs 5.7 % over the best tile on average, with these 0.13 %.
+    static const Cost wide[] = {{0, 256, 4, 5.8f, 0.198f}, {0, 256, 6, 8.5f, 0.254f}, {0, 256, 10, 13.5f, 0.385f}};
+    static const std::vector<GemmCost> v = [] {
+        std::vector<GemmCost> all(std::begin(costs), std::end(costs));
+        all.insert(all.end(), std::begin(wide), std::end(wide));
+        return all;
+    }();
     return v;
 }
+// the tile's name in a choice: that of mid_gemm_f16_kernel, 0 for 256 x 256, 40 + half its column tiles for the other widths
+static int gemm_tile_code(const GemmCost& c) { return c.tile ? c.tile : c.cols == 8 ? 0 : 40 + c.cols / 2; }
+static bool is_wide_tile(int tile) { return tile == 42 || tile == 43 || tile == 45; }
+static bool gemm_tile_takes(const GemmCost& c, int KT, long R) { return c.tile || (R >= 256 && (c.cols == 8 || KT % 2 == 0)); }
 static float gemm_tile_us(const GemmCost& c, int KT, long n_tiles, int splits) {
     const float ncu = (float)std::max(1, n_compute_units()), tiles = (float)(n_tiles * splits), rounds = std::ceil(tiles / ncu);
     float us = rounds * (c.a + c.b * (float)ceil_div(KT, splits)) * (1.0f + (c.tile ? 0.2f : 0.35f) * tiles / (rounds * ncu));
     if (splits > 1) us += 1.16f + 0.08f * (float)splits + 0.7f * (float)(c.rows * c.cols) / 64.0f;
     return us;
 }
-static GemmTile best_gemm_tile(int KT, int NT, long R, float own_cache_write = 0.0f) {
+// (all_widths: false leaves out the 256-row tiles of other widths than 256)
+static GemmTile best_gemm_tile(int KT, int NT, long R, float own_cache_write = 0.0f, bool all_widths = true) {
     GemmTile best = {111, 1e30f};
     for (const GemmCost& c : gemm_costs()) {
-        if (c.tile == 0 && R < 256) continue;
+        if (!gemm_tile_takes(c, KT, R) || (!all_widths && is_wide_tile(gemm_tile_code(c)))) continue;
         const long n_tiles = ceil_div(R, c.rows) * ceil_div(NT, c.cols);
         for (int splits = 1; splits <= (c.tile ? MID_SPLITS : 1); ++splits) {
             if (mid_splits(KT, c.tile, splits) != splits || (splits > 1 && (n_tiles * splits > TSHipGpt::MID_XCHG_TILES || n_tiles * splits > n_compute_units()))) continue;
-            const float us = gemm_tile_us(c, KT, n_tiles, splits) - (c.tile == 0 ? own_cache_write : 0.0f);
-            if (us < best.us) best = {c.tile ? c.tile + 100 * splits : 0, us};
+            const int code = gemm_tile_code(c);
+            const float us = gemm_tile_us(c, KT, n_tiles, splits) - (code == 0 ? own_cache_write : 0.0f);
+            if (us < best.us) best = {c.tile ? code + 100 * splits : code, us};
         }
     }
     return best;
@@ -641,6 +656,7 @@ static GemmTile best_gemm_tile(int KT, int NT, long R, float own_cache_write = 0
 static int pick_gemm_tile(const GemmW& w, long R) {
     const int forced = g_hooks.gemm_tile;
     if (forced == 0 && R >= 256) return 0;
+    if (is_wide_tile(forced)) return R >= 256 && w.KT % 2 == 0 ? forced : best_gemm_tile(w.KT, w.NT, R).tile;
     if (forced > 0) {
         const GemmCost& c = *std::find_if(gemm_costs().begin(), gemm_costs().end(), [&](const GemmCost& k) { return k.tile == forced % 100; });
         const bool fits = ceil_div(R, c.rows) * ceil_div(w.NT, c.cols) * (forced / 100) <= TSHipGpt::MID_XCHG_TILES;
@@ -653,21 +669,27 @@ static int pick_gemm_tile(const GemmW& w, long R) {
 // them.  cols 0: one launch.  The second launch costs 2 us.  ms per prompt, one launch per projection -> two: 1B model, 1500 / 1665 /
 // 2200 / 5000 / 8750 rows 4.4 / 4.5 / 6.6 / 10.4 / 17.9 -> 3.9 / 4.2 / 5.3 / 9.5 / 15.8 (with the tiles' even shares of xcd_tile);
 // 8 layers of the 7B one, 700 / 4400 rows 3.6 / 17.0 -> 3.1 / 13.9; the 768-wide one, 6000 rows 3.8 -> 3.3.
+// The other widths of the 256-row tile mostly fill the rounds of one launch.  Estimates are off by 10 %, so they take the place of two
+// launches of the other tiles only where they promise 7.5 %: 2048 x 11264 at 1500 rows 81 us for 83, so two launches; at 1665 rows 83 for 95.
 struct GemmMix { int tile, cols, rest; float us; };
-static GemmMix pick_gemm_mix(const GemmW& w, long R) {
-    if (g_hooks.gemm_tile >= 0) return {pick_gemm_tile(w, R), 0, 0, 0.0f};
+static GemmMix pick_gemm_mix(const GemmW& w, long R, bool all_widths) {
     const long ncu = std::max(1, n_compute_units());
-    const GemmTile one = best_gemm_tile(w.KT, w.NT, R);
+    const GemmTile one = best_gemm_tile(w.KT, w.NT, R, 0.0f, all_widths);
     GemmMix mix = {one.tile, 0, 0, one.us};
     for (const GemmCost& c : gemm_costs()) {
-        if (c.tile == 0 && R < 256) continue;
+        if (!gemm_tile_takes(c, w.KT, R) || (!all_widths && is_wide_tile(gemm_tile_code(c)))) continue;
         const long RT = ceil_div(R, c.rows), CT = ceil_div(w.NT, c.cols), cols = RT * CT / ncu * ncu / RT;      // column tiles of whole rounds
         if (cols < 1 || cols >= CT) continue;
-        const GemmTile rest = best_gemm_tile(w.KT, w.NT - (int)(cols * c.cols), R);
+        const GemmTile rest = best_gemm_tile(w.KT, w.NT - (int)(cols * c.cols), R, 0.0f, all_widths);
         const float us = gemm_tile_us(c, w.KT, RT * cols, 1) + rest.us + 2.0f;
-        if (us < mix.us && us < 0.97f * one.us) mix = {c.tile ? c.tile + 100 : 0, (int)(cols * c.cols), rest.tile, us};
+        if (us < mix.us && us < 0.97f * one.us) mix = {c.tile ? c.tile + 100 : gemm_tile_code(c), (int)(cols * c.cols), rest.tile, us};
     }
     return mix;
+}
+static GemmMix pick_gemm_mix(const GemmW& w, long R) {
+    if (g_hooks.gemm_tile >= 0) return {pick_gemm_tile(w, R), 0, 0, 0.0f};
+    const GemmMix other = pick_gemm_mix(w, R, false), all = pick_gemm_mix(w, R, true);
+    return other.cols && all.us >= 0.925f * other.us ? other : all;
 }
 static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int mid) {
     e.splits = mid / 100; mid %= 100;
@@ -696,18 +718,21 @@ static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int 
 
 static bool big_gemm_packed_ok(int KT, long R) { return R >= 512 && KT % 2 == 0; }
 static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int tile) {
-    TSHIP_REQUIRE(!e.packed_problems || (!tile && e.KT % 2 == 0), "internal: packed launch of a GEMM shape the LDS-tiled kernel does not take");
-    if (!tile) {          // 256 x 256 block tile
+    const bool rows256 = !tile || is_wide_tile(tile);
+    TSHIP_REQUIRE(!e.packed_problems || (rows256 && e.KT % 2 == 0), "internal: packed launch of a GEMM shape the LDS-tiled kernel does not take");
+    TSHIP_REQUIRE(!e.kcache || !tile, "internal: only the 256 x 256 tile writes the cache");
+    if (rows256) {        // 256-row block tiles
+        e.patch_rows = g_hooks.patch_rows;
+        if (e.KT % 2 == 0) {      // asynchronous staging: four stages of two k-tiles, eight wavefronts
+            const WideGemm wide = tile ? wide_gemm(tile, epi) : WideGemm{epi == BEPI_F32_BIAS ? big_gemm3_f16_kernel<BEPI_F32_BIAS> : epi == BEPI_RESID ? big_gemm3_f16_kernel<BEPI_RESID> : big_gemm3_f16_kernel<BEPI_ACT16>, 8, BigShape<4>::SHM};
+            const dim3 grid((unsigned)xcd_tile_blocks(ceil_div(e.NT, wide.cols) * ceil_div((long)e.R, 256)));
+            launch_shm(m, name, wide.kernel, grid, dim3(512), wide.shm, e);
+            return;
+        }
+        TSHIP_REQUIRE(!tile, "internal: the other widths of the 256-row tile need an even number of k-tiles");
         constexpr int CK = 4;
         const unsigned shm = 2u * 2u * 8u * CK * 1024u;
         const dim3 grid((unsigned)xcd_tile_blocks(ceil_div(e.NT, 8) * ceil_div((long)e.R, 256)));
-        e.patch_rows = g_hooks.patch_rows;
-        if (e.KT % 2 == 0) {      // asynchronous staging: four stages of two k-tiles, eight wavefronts
-            if (epi == BEPI_F32_BIAS) launch_shm(m, name, big_gemm3_f16_kernel<BEPI_F32_BIAS>, grid, dim3(512), shm, e);
-            else if (epi == BEPI_RESID) launch_shm(m, name, big_gemm3_f16_kernel<BEPI_RESID>, grid, dim3(512), shm, e);
-            else launch_shm(m, name, big_gemm3_f16_kernel<BEPI_ACT16>, grid, dim3(512), shm, e);
-            return;
-        }
         if (epi == BEPI_F32_BIAS) launch_shm(m, name, big_gemm2_f16_kernel<BEPI_F32_BIAS, CK>, grid, dim3(256), shm, e);
         else if (epi == BEPI_RESID) launch_shm(m, name, big_gemm2_f16_kernel<BEPI_RESID, CK>, grid, dim3(256), shm, e);
         else launch_shm(m, name, big_gemm2_f16_kernel<BEPI_ACT16, CK>, grid, dim3(256), shm, e);
@@ -744,19 +769,25 @@ static void run_packed_gemm(TSHipGpt* m, const char* name, const GemmW& w, const
     const int E = e.packed_problems;
     TSHIP_REQUIRE(E >= 1 && E <= 64, "internal: a packed launch gives each problem a lane");
     e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.splits = 1;
-    const GemmCost& whole = gemm_costs().back();
-    const long CT = ceil_div(w.NT, whole.cols), half_tiles = E * CT / 2, tiles = total / whole.rows * CT;
     int rest = 0; float rest_us = 1e30f;
     for (const GemmCost& c : gemm_costs()) {
         if (!c.tile) continue;
         const float us = gemm_tile_us(c, w.KT, E * (c.rows + 256) / (2 * c.rows) * ceil_div(w.NT, c.cols), 1);
         if (us < rest_us) { rest_us = us; rest = c.tile; }
     }
-    bool two = tiles > half_tiles && gemm_tile_us(whole, w.KT, tiles - half_tiles, 1) + rest_us + 2.0f < 0.97f * gemm_tile_us(whole, w.KT, tiles + half_tiles, 1);
+    bool two = false; int tile = 0; float best_us = 1e30f;
+    for (const GemmCost& c : gemm_costs()) {
+        if (c.tile) continue;
+        const long CT = ceil_div(w.NT, c.cols), half_tiles = E * CT / 2, tiles = total / c.rows * CT;
+        const float one_us = gemm_tile_us(c, w.KT, tiles + half_tiles, 1), two_us = tiles > half_tiles ? gemm_tile_us(c, w.KT, tiles - half_tiles, 1) + rest_us + 2.0f : 1e30f;
+        if (one_us < best_us) { best_us = one_us; tile = gemm_tile_code(c); two = false; }
+        if (two_us < 0.97f * best_us) { best_us = two_us; tile = gemm_tile_code(c); two = true; }
+    }
     if (g_hooks.moe_rest) { two = true; rest = g_hooks.moe_rest; }
+    if (is_wide_tile(g_hooks.gemm_tile) || g_hooks.gemm_tile == 0) tile = g_hooks.gemm_tile;
     e.packed_whole = two ? 1 : 0;
     e.R = (int)(256 * (total / 256 + (two ? 0 : E)));      // >= 256 x the sum over the experts of their (whole) row tiles
-    if (e.R) launch_big_gemm(m, name, e, epi, 0);
+    if (e.R) launch_big_gemm(m, name, e, epi, tile);
     if (two) {
         e.R = 255;
         run_mid_gemm(m, name, e, epi, rest + 100);
@@ -1445,7 +1476,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         const float fuse_saves = 1.9e-6f * (float)(R * 2 * GD) - 7.5f;
         const float own_write = can_fuse_kv ? std::max(0.0f, fuse_saves) : 0.0f;
         qkv_tiles = pick_gemm_mix(L.qkv, R);
-        if (g_hooks.gemm_tile < 0) {      // (two launches of different tiles where that is less than the saved kernel)
+        if (g_hooks.gemm_tile < 0 && own_write > 0.0f) {      // (two launches of different tiles where that is less than the saved kernel)
             const GemmTile one = best_gemm_tile(L.qkv.KT, L.qkv.NT, R, own_write);
             if (!qkv_tiles.cols || qkv_tiles.us >= one.us) qkv_tiles = {one.tile, 0, 0, one.us};
         }

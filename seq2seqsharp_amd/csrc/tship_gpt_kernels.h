@@ -1,4 +1,4 @@
-// Device kernels of the fused GPTDecoder path (gfx950).  Included by tship_gpt.hip only.
+// Device kernels of the fused GPTDecoder path (gfx950).  Included by tship_gpt.hip and tship_wide_gemm.hip.
 //
 // Data layout in HBM
 //   residual stream x      fp32 [rows][hidden]
@@ -94,7 +94,7 @@ enum { PACK_PLAIN = 0, PACK_INTERLEAVE16 = 1 };
 // PACK_PLAIN: destination column = n_off + n.  PACK_INTERLEAVE16: destination column =
 // (n/16)*32 + n_off + n%16 with n_off in {0,16}: column tile j then holds 16 columns of the first matrix
 // followed by the same 16 columns of the second, so a gated FFN epilogue finds both factors in one tile.
-__global__ void pack_w_kernel(const float* __restrict__ src, long ld, int K, int N, half_t* __restrict__ dst, int KT,
+static __global__ void pack_w_kernel(const float* __restrict__ src, long ld, int K, int N, half_t* __restrict__ dst, int KT,
                               int mode, int n_off) {
     long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     long total = (long)N * KT * 2;
@@ -118,7 +118,7 @@ __global__ void pack_w_kernel(const float* __restrict__ src, long ld, int K, int
 // W being the fp16 values the GEMM multiplies with; sums in double, k ascending.  bias_mode 0: bias[n] (plain layout);
 // 1: the gated interleave (packed column 32 g + j stands for column 16 g + j of W1 when j < 16, of W3 otherwise: bias1 /
 // bias2); a null bias counts as zero.  One thread per packed column.
-__global__ void ln_fold_kernel(const half_t* __restrict__ W, int KT, int NT, int K, const float* __restrict__ gamma, const float* __restrict__ beta,
+static __global__ void ln_fold_kernel(const half_t* __restrict__ W, int KT, int NT, int K, const float* __restrict__ gamma, const float* __restrict__ beta,
                                const float* __restrict__ bias1, const float* __restrict__ bias2, int bias_mode, int n_logical,
                                float* __restrict__ c_out, float* __restrict__ d_out) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
@@ -831,13 +831,13 @@ struct BigArgs {
 // that rows leave as whole 128-byte lines (eight lanes x 16 bytes per row, eight rows per store instruction) instead of
 // 32 pieces of 16 bytes per instruction: the fragmented form takes four times the store requests.  `stage`: 64 rows x 72
 // halfs of LDS owned by this wavefront (row stride 144 bytes: 16-byte aligned pieces, rows spread over the banks).  Whole tiles only.
-template <int ACT>
-__device__ __forceinline__ void gated_store_lines(const BigArgs& a, floatx16 (&acc)[4][2], int nt_first, long row_first, int lane, half_t* stage,
+template <int ACT, int NJ>
+__device__ __forceinline__ void gated_store_lines(const BigArgs& a, floatx16 (&acc)[NJ][2], int nt_first, long row_first, int lane, half_t* stage,
                                                   const float (&rinv2)[2]) {
-    constexpr int LDSROW = 72;
+    constexpr int LDSROW = 16 * NJ + 8, PPR = 2 * NJ;      // (PPR: 16-byte pieces of a row)
     const int lh = lane >> 5, r = lane & 31;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NJ; ++j) {
         float b1[8], b2[8];
 #pragma unroll
         for (int v = 0; v < 8; ++v) {
@@ -857,12 +857,12 @@ __device__ __forceinline__ void gated_store_lines(const BigArgs& a, floatx16 (&a
     }
     __builtin_amdgcn_wave_barrier();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int piece = lane & 7, rr = lane >> 3;
-    half8 line[8];
+    half8 line[PPR];
 #pragma unroll
-    for (int ps = 0; ps < 8; ++ps) line[ps] = *(const half8*)(stage + (8 * ps + rr) * LDSROW + 8 * piece);
+    for (int ps = 0; ps < PPR; ++ps) line[ps] = *(const half8*)(stage + ((64 * ps + lane) / PPR) * LDSROW + 8 * ((64 * ps + lane) % PPR));
 #pragma unroll
-    for (int ps = 0; ps < 8; ++ps) *(half8*)(a.out16 + (row_first + 8 * ps + rr) * a.ld16 + (long)nt_first * 16 + 8 * piece) = line[ps];
+    for (int ps = 0; ps < PPR; ++ps)
+        *(half8*)(a.out16 + (row_first + (64 * ps + lane) / PPR) * a.ld16 + (long)nt_first * 16 + 8 * ((64 * ps + lane) % PPR)) = line[ps];
 }
 
 // The same for one 32-column tile of a residual projection (64 rows x 32 fp32 columns = one 128-byte line per row): the
@@ -920,15 +920,16 @@ __device__ __forceinline__ void resid_store_lines(const BigArgs& a, const floatx
 
 // Ungated activation output (ReLU / SiLU / LeakyReLU feed-forward, MoE experts): a wavefront's 64 rows x 128 columns go
 // out in two halves of 64 columns (one 128-byte line per row each) through the same 64 x 72 halfs of LDS.
-template <int ACT>
-__device__ __forceinline__ void act_store_lines(const BigArgs& a, floatx16 (&acc)[4][2], int nt_first, long row_first, int lane, half_t* stage,
+template <int ACT, int NJ>
+__device__ __forceinline__ void act_store_lines(const BigArgs& a, floatx16 (&acc)[NJ][2], int nt_first, long row_first, int lane, half_t* stage,
                                                 const float (&rinv2)[2]) {
     constexpr int LDSROW = 72;
-    const int lh = lane >> 5, r = lane & 31, piece = lane & 7, rr = lane >> 3;
+    const int lh = lane >> 5, r = lane & 31;
 #pragma unroll
-    for (int hj = 0; hj < 2; ++hj) {
+    for (int hj = 0; hj < (NJ + 1) / 2; ++hj) {
+        const int tiles = 2 * hj + 1 < NJ ? 2 : 1, ppr = 4 * tiles;      // (compile-time after unrolling: column tiles of this pass, 16-byte pieces of a row)
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
+        for (int jj = 0; jj < tiles; ++jj) {
             const int j = 2 * hj + jj;
             float bb[16];
 #pragma unroll
@@ -947,10 +948,11 @@ __device__ __forceinline__ void act_store_lines(const BigArgs& a, floatx16 (&acc
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         half8 line[8];
 #pragma unroll
-        for (int ps = 0; ps < 8; ++ps) line[ps] = *(const half8*)(stage + (8 * ps + rr) * LDSROW + 8 * piece);
+        for (int ps = 0; ps < ppr; ++ps) line[ps] = *(const half8*)(stage + ((64 * ps + lane) / ppr) * LDSROW + 8 * ((64 * ps + lane) % ppr));
 #pragma unroll
-        for (int ps = 0; ps < 8; ++ps) *(half8*)(a.out16 + (row_first + 8 * ps + rr) * a.ld16 + (long)(nt_first + 2 * hj) * 32 + 8 * piece) = line[ps];
-        __builtin_amdgcn_wave_barrier();          // the second half overwrites the stage
+        for (int ps = 0; ps < ppr; ++ps)
+            *(half8*)(a.out16 + (row_first + (64 * ps + lane) / ppr) * a.ld16 + (long)(nt_first + 2 * hj) * 32 + 8 * ((64 * ps + lane) % ppr)) = line[ps];
+        __builtin_amdgcn_wave_barrier();          // the next pass overwrites the stage
     }
 }
 
@@ -1057,9 +1059,10 @@ __device__ __forceinline__ void kv_store_frags(const BigArgs& a, floatx16 (&acc)
     }
 }
 
-template <int EPI, int NI = 4>      // NI: 32-row tiles per wavefront (the wavefront's rows start at 32 NI wr)
-__device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)[4][NI], int nt0, long row0, int wr, int wn, int lane, half_t* stage = nullptr) {
-    // accumulator (j, i), lane l, register v = 4 g + e: column (nt0 + 4 wn + j) * 32 + 8 g + 4 (l / 32) + e,
+// NI: 32-row tiles per wavefront (the wavefront's rows start at 32 NI wr), NJ: its 32-column tiles
+template <int EPI, int NI = 4, int NJ = 4>
+__device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)[NJ][NI], int nt0, long row0, int wr, int wn, int lane, half_t* stage = nullptr) {
+    // accumulator (j, i), lane l, register v = 4 g + e: column (nt0 + NJ wn + j) * 32 + 8 g + 4 (l / 32) + e,
     // row row0 + 128 wr + 32 i + l % 32.  Biases (and the residual) are fetched in batches before the first store
     // of a column tile, and the four consecutive columns of a group go out as one 16-byte (fp32) or 8-byte (fp16) store.
     const int lh = lane >> 5;
@@ -1071,25 +1074,25 @@ __device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)
         rinv4[i] = (a.rinv && row < a.R) ? a.rinv[row] : 1.0f;
     }
     if constexpr (EPI == BEPI_ACT16 && NI == 2) {
-        // whole 64 x 64 output block of a gated projection with 16-byte aligned rows: line stores through LDS
+        // whole outputs of a wavefront with 16-byte aligned rows: line stores through LDS
         const long rf = row0 + 64 * wr;
-        const int ntf = nt0 + 4 * wn;
-        if (stage && a.gated && rf + 64 <= a.R && ntf + 4 <= a.NT && (ntf + 4) * 16 <= a.n_valid && (a.ld16 & 7) == 0) {
+        const int ntf = nt0 + NJ * wn;
+        if (stage && a.gated && rf + 64 <= a.R && ntf + NJ <= a.NT && (ntf + NJ) * 16 <= a.n_valid && (a.ld16 & 7) == 0) {
             const float r2[2] = {rinv4[0], rinv4[1]};
-            with_act(a.act, [&](auto A) { gated_store_lines<decltype(A)::value>(a, acc, ntf, rf, lane, stage, r2); });
+            with_act(a.act, [&](auto A) { gated_store_lines<decltype(A)::value, NJ>(a, acc, ntf, rf, lane, stage, r2); });
             return;
         }
-        if (stage && !a.gated && rf + 64 <= a.R && ntf + 4 <= a.NT && (ntf + 4) * 32 <= a.n_valid && (a.ld16 & 7) == 0) {
+        if (stage && !a.gated && rf + 64 <= a.R && ntf + NJ <= a.NT && (ntf + NJ) * 32 <= a.n_valid && (a.ld16 & 7) == 0) {
             const float r2[2] = {rinv4[0], rinv4[1]};
-            with_act(a.act, [&](auto A) { act_store_lines<decltype(A)::value>(a, acc, ntf, rf, lane, stage, r2); });
+            with_act(a.act, [&](auto A) { act_store_lines<decltype(A)::value, NJ>(a, acc, ntf, rf, lane, stage, r2); });
             return;
         }
     }
     if constexpr ((EPI == BEPI_RESID || EPI == BEPI_F32_BIAS) && NI == 2) {
         const long rf = row0 + 64 * wr;
-        const int ntf = nt0 + 4 * wn;
+        const int ntf = nt0 + NJ * wn;
         constexpr bool RS = EPI == BEPI_RESID;
-        if constexpr (!RS) {
+        if constexpr (!RS && NJ == 4) {
             // key and value columns of a QKV projection that writes the cache itself (whole wavefronts: the column counts
             // are multiples of 128, the launch code checks the rest)
             if (stage && a.kcache && ntf * 32 >= a.kv_col0) {
@@ -1101,19 +1104,17 @@ __device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)
                 return;
             }
         }
-        if (stage && rf + 64 <= a.R && ntf + 4 <= a.NT && (ntf + 4) * 32 <= a.n_valid && (a.ld_out & 3) == 0 && (!RS || !a.xg16 || (a.ld_xg & 3) == 0)) {
+        if (stage && rf + 64 <= a.R && ntf + NJ <= a.NT && (ntf + NJ) * 32 <= a.n_valid && (a.ld_out & 3) == 0 && (!RS || !a.xg16 || (a.ld_xg & 3) == 0)) {
             const float r2[2] = {rinv4[0], rinv4[1]};
-            resid_store_lines<RS>(a, acc[0], ntf + 0, rf, lane, (float*)stage, r2);
-            resid_store_lines<RS>(a, acc[1], ntf + 1, rf, lane, (float*)stage, r2);
-            resid_store_lines<RS>(a, acc[2], ntf + 2, rf, lane, (float*)stage, r2);
-            resid_store_lines<RS>(a, acc[3], ntf + 3, rf, lane, (float*)stage, r2);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) resid_store_lines<RS>(a, acc[j], ntf + j, rf, lane, (float*)stage, r2);
             return;
         }
     }
     // one column tile per call with a compile-time tile number: the accumulators must only ever be indexed statically
     auto tile_out = [&](auto J) {
         constexpr int j = decltype(J)::value;
-        const int nt = nt0 + 4 * wn + j;
+        const int nt = nt0 + NJ * wn + j;
         if (nt >= a.NT) return;
         if (EPI == BEPI_ACT16 && a.gated) {
             float b1[8], b2[8];
@@ -1238,8 +1239,9 @@ __device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)
     };
     tile_out(std::integral_constant<int, 0>{});
     tile_out(std::integral_constant<int, 1>{});
-    tile_out(std::integral_constant<int, 2>{});
-    tile_out(std::integral_constant<int, 3>{});
+    if constexpr (NJ > 2) tile_out(std::integral_constant<int, 2>{});
+    if constexpr (NJ > 3) tile_out(std::integral_constant<int, 3>{});
+    if constexpr (NJ > 4) tile_out(std::integral_constant<int, 4>{});
 }
 
 // LDS-tiled prefill GEMM.  Block tile 256 rows x 256 columns, 4 wavefronts, each owning 128 x 128 (4 x 4 MFMA
@@ -1349,34 +1351,56 @@ __global__ __launch_bounds__(256) void big_gemm2_f16_kernel(BigArgs a) {
 // queue for the pipes: the gated up projection of 32 768 x 2048 x 11 264 took 1.21 ms that way against 1.07 ms.
 // (Four wavefronts of 128 x 128 each, 16 fragment reads per 32 MFMAs and two thirds of the LDS traffic, measured
 // slower still: the loop is bound by exposed waits, not by LDS bandwidth.)
-__device__ __forceinline__ void lds_read_frags(unsigned wa, unsigned xa, half8 (&wf)[4], half8 (&xf)[2]) {
-    asm volatile(
-        "ds_read_b128 %0, %6\n\t"
-        "ds_read_b128 %1, %6 offset:2048\n\t"
-        "ds_read_b128 %2, %6 offset:4096\n\t"
-        "ds_read_b128 %3, %6 offset:6144\n\t"
-        "ds_read_b128 %4, %7\n\t"
-        "ds_read_b128 %5, %7 offset:2048"
-        : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(wf[2]), "=&v"(wf[3]), "=&v"(xf[0]), "=&v"(xf[1])
-        : "v"(wa), "v"(xa)
-        : "memory");
+template <int NJ>
+__device__ __forceinline__ void lds_read_frags(unsigned wa, unsigned xa, half8 (&wf)[NJ], half8 (&xf)[2]) {
+    static_assert(NJ >= 2 && NJ <= 5, "column tiles of a wavefront");
+    if constexpr (NJ == 5)
+        asm volatile("ds_read_b128 %0, %7\n\tds_read_b128 %1, %7 offset:2048\n\tds_read_b128 %2, %7 offset:4096\n\tds_read_b128 %3, %7 offset:6144\n\t"
+                     "ds_read_b128 %4, %7 offset:8192\n\tds_read_b128 %5, %8\n\tds_read_b128 %6, %8 offset:2048"
+                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(wf[2]), "=&v"(wf[3]), "=&v"(wf[4]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa) : "memory");
+    else if constexpr (NJ == 4)
+        asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:2048\n\tds_read_b128 %2, %6 offset:4096\n\tds_read_b128 %3, %6 offset:6144\n\t"
+                     "ds_read_b128 %4, %7\n\tds_read_b128 %5, %7 offset:2048"
+                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(wf[2]), "=&v"(wf[3]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa) : "memory");
+    else if constexpr (NJ == 3)
+        asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %5 offset:2048\n\tds_read_b128 %2, %5 offset:4096\n\tds_read_b128 %3, %6\n\tds_read_b128 %4, %6 offset:2048"
+                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(wf[2]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa) : "memory");
+    else
+        asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\tds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:2048"
+                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa) : "memory");
 }
-template <int N>
-__device__ __forceinline__ void lds_wait_frags(half8 (&wf)[4], half8 (&xf)[2]) {
-    asm volatile("s_waitcnt lgkmcnt(%6)"
-                 : "+v"(wf[0]), "+v"(wf[1]), "+v"(wf[2]), "+v"(wf[3]), "+v"(xf[0]), "+v"(xf[1])
-                 : "n"(N)
-                 : "memory");
+template <int N, int NJ>
+__device__ __forceinline__ void lds_wait_frags(half8 (&wf)[NJ], half8 (&xf)[2]) {
+    if constexpr (NJ == 5)
+        asm volatile("s_waitcnt lgkmcnt(%7)" : "+v"(wf[0]), "+v"(wf[1]), "+v"(wf[2]), "+v"(wf[3]), "+v"(wf[4]), "+v"(xf[0]), "+v"(xf[1]) : "n"(N) : "memory");
+    else if constexpr (NJ == 4)
+        asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(wf[0]), "+v"(wf[1]), "+v"(wf[2]), "+v"(wf[3]), "+v"(xf[0]), "+v"(xf[1]) : "n"(N) : "memory");
+    else if constexpr (NJ == 3)
+        asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(wf[0]), "+v"(wf[1]), "+v"(wf[2]), "+v"(xf[0]), "+v"(xf[1]) : "n"(N) : "memory");
+    else
+        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(wf[0]), "+v"(wf[1]), "+v"(xf[0]), "+v"(xf[1]) : "n"(N) : "memory");
 }
 
-template <int EPI>
+// NJ: 32-column tiles of a wavefront, 2 NJ of the block (the loop above with NJ = 4).  A launch of one to four rounds is as long as its
+// rounds of tiles over the 256 units, so the width is chosen for them (pick_gemm_tile; the wider ones also read less per product).  us at
+// 128 / 192 / 256 / 320 columns, 128 x 128 tiles of mid_gemm_f16_kernel behind the bar: gated 2048 x 11264 at 333 rows 33 / 40 / 47 / 56 | 44, at 1665
+// 102 / 93 / 105 / 83 | 122; 2048 x 3072 at 1665 rows 33 / 40 / 47 / 56 | 41; 5632 x 2048 at 9000 284 / 262 / 299 / 234 | 267; all sizes in
+// profiles/prefill_gemm_wide_tiles.txt.  An odd NJ gives the first four wavefronts one weight fragment more per chunk to stage than the others.
+// bytes of a stage (two k-tiles of 2 NJ column tiles and of 256 rows) and dynamic LDS of a launch
+template <int NJ> struct BigShape {
+    static constexpr int NST = 4, STAGE = (4 * NJ + 16) * 1024;
+    static constexpr unsigned SHM = NST * STAGE;
+};
+template <int EPI, int NJ = 4>
 __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     extern __shared__ __attribute__((aligned(16))) half_t big_smem[];
-    constexpr int CK = 2, NST = 4, FR = 8 * CK, PF = NST - 1;          // k-tiles per stage, stages, fragments per operand and stage, chunks requested ahead
-    constexpr int STAGE = 2 * FR * 512;                  // halfs per stage: weight fragments, then activation fragments
+    constexpr int CK = 2, NST = BigShape<NJ>::NST, WFR = 2 * NJ * CK, PF = NST - 1;          // k-tiles per stage, stages, weight fragments per stage, chunks requested ahead
+    constexpr int STAGE = BigShape<NJ>::STAGE / 2;       // halfs per stage: weight fragments, then 16 activation fragments
+    constexpr int LW = (WFR + 7) / 8;                    // weight fragments that a wavefront stages; with an odd NJ the last half of them belongs to the first four
+    constexpr bool HALF = WFR % 8 != 0;
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = w >> 1, wn = w & 1;                   // 4 x 2 wavefronts
-    const int CT = (a.NT + 7) / 8;
+    const int CT = (a.NT + 2 * NJ - 1) / (2 * NJ);
     int RT = (int)((a.R + 255) / 256);
     // (a lane per problem, up to 64: their row tiles and the running sum.  Two scalar loops over 64 problems took 3 us.)
     int rows_e = 0, upto = 0;
@@ -1398,11 +1422,11 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
         if (a.out16) a.out16 += e * a.out16_estride;
         if (a.row_idx) a.row_idx += e * a.idx_estride;
     }
-    const int nt0 = ctile * 8;
+    const int nt0 = ctile * 2 * NJ;
     const long row0 = (long)rtile * 256;
-    floatx16 acc[4][2];
+    floatx16 acc[NJ][2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1412,12 +1436,16 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     // Activations: 1 KiB block f holds 16 rows x 64 bytes (both k-tiles of the chunk); lane l fetches 16-byte piece
     // s = (l % 4) ^ ((row / 4) % 4) of row 16 f + l / 4, so that four lanes read one contiguous 64-byte run and the
     // fragment reads below (32 rows x 2 pieces) spread evenly over the LDS banks
-    const half_t* wsrc[2]; const half_t* xsrc[2];
+    const half_t* wsrc[LW]; const half_t* xsrc[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int f = i * 8 + w, tl = f >> 1, ktl = f & 1;
+    for (int i = 0; i < LW; ++i) {
+        const int f = min(i * 8 + w, WFR - 1), tl = f >> 1, ktl = f & 1;
         const int nt = min(nt0 + tl, a.NT - 1);
         wsrc[i] = a.W + (((long)nt * a.KT + ktl) * 64 + lane) * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int f = i * 8 + w;
         const int rl = f * 16 + (lane >> 2);
         long row = min(row0 + rl, (long)a.R - 1);
         if (a.row_idx) row = a.row_idx[row];
@@ -1425,22 +1453,24 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     }
     typedef const void __attribute__((address_space(1)))* gptr_t;
     typedef void __attribute__((address_space(3)))* lptr_t;
+    const int g = w >> 2;
     auto issue = [&](int c) {
         half_t* st = big_smem + (c % NST) * STAGE;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int f = i * 8 + w;
-            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (long)c * (CK * 512)), (lptr_t)(st + f * 512), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (long)c * (CK * 16)), (lptr_t)(st + (FR + f) * 512), 16, 0, 0);
-        }
+        for (int i = 0; i < LW; ++i)
+            if (!HALF || i + 1 < LW || g == 0)
+                __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (long)c * (CK * 512)), (lptr_t)(st + (i * 8 + w) * 512), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (long)c * (CK * 16)), (lptr_t)(st + (WFR + i * 8 + w) * 512), 16, 0, 0);
     };
     const int NC = a.KT / CK;
     const unsigned lds0 = (unsigned)(size_t)(lptr_t)big_smem;
-    const unsigned woff = (unsigned)(((4 * wn) * CK) * 1024 + lane * 16);
+    const unsigned woff = (unsigned)(((NJ * wn) * CK) * 1024 + lane * 16);
     const int xr = 64 * wr + (lane & 31);
     const unsigned xsw = (unsigned)((xr >> 2) & 3);
-    const unsigned xoff0 = (unsigned)(FR * 1024 + xr * 64 + 16 * (((lane >> 5)) ^ xsw));          // k-tile 0: s = l / 32
-    const unsigned xoff1 = (unsigned)(FR * 1024 + xr * 64 + 16 * ((2 + (lane >> 5)) ^ xsw));      // k-tile 1: s = 2 + l / 32
+    const unsigned xoff0 = (unsigned)(WFR * 1024 + xr * 64 + 16 * (((lane >> 5)) ^ xsw));          // k-tile 0: s = l / 32
+    const unsigned xoff1 = (unsigned)(WFR * 1024 + xr * 64 + 16 * ((2 + (lane >> 5)) ^ xsw));      // k-tile 1: s = 2 + l / 32
     issue(0);
     if (NC > 1) issue(1);
     if (NC > 2) issue(2);
@@ -1450,46 +1480,48 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     // registers, then the first multiplies chunk c while the second reads it.  Before barrier c every wavefront has
     // waited for its own part of chunk c and has read chunk c - 1, so the loads of chunk c + 3 may overwrite that stage.
     // Both groups pass the same number of barriers.
-    const int g = w >> 2;
-    half8 wfA[4], xfA[2], wfB[4], xfB[2];
-    auto wait_loads = [&](int c) {          // this wavefront's part of chunk c + 1 has landed
+    half8 wfA[NJ], xfA[2], wfB[NJ], xfB[2];
+    // (loads per chunk: those of the first group, and of the second, which has one less with an odd NJ)
+    auto wait_loads = [&](int c, auto group) {          // this wavefront's part of chunk c + 1 has landed
+        constexpr int LPC = LW + 2 - (HALF && decltype(group)::value ? 1 : 0);
         const int later = max(0, min(PF - 1, NC - 2 - c));
-        if (later == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else if (later == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        if (later == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPC) : "memory");
+        else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPC) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
+    typedef std::integral_constant<int, 0> group0; typedef std::integral_constant<int, 1> group1;
     auto R = [&](int c, bool wait_now) {
         const unsigned sb = lds0 + (unsigned)((c % NST) * STAGE * 2);
-        lds_read_frags(sb + woff, sb + xoff0, wfA, xfA);                   // k-tile 0
-        lds_read_frags(sb + woff + 1024, sb + xoff1, wfB, xfB);            // k-tile 1
+        lds_read_frags<NJ>(sb + woff, sb + xoff0, wfA, xfA);                   // k-tile 0
+        lds_read_frags<NJ>(sb + woff + 1024, sb + xoff1, wfB, xfB);            // k-tile 1
         if (c + PF < NC) issue(c + PF);
-        if (wait_now) wait_loads(c);
-        lds_wait_frags<0>(wfA, xfA);
-        lds_wait_frags<0>(wfB, xfB);
+        if (wait_now) wait_loads(c, group1());      // (the second group)
+        lds_wait_frags<0, NJ>(wfA, xfA);
+        lds_wait_frags<0, NJ>(wfB, xfB);
         __builtin_amdgcn_sched_barrier(0);
     };
     auto M = [&]() {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wfA[j], xfA[i], acc[j][i], 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wfB[j], xfB[i], acc[j][i], 0, 0, 0);
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
     };
-    wait_loads(-1);
+    if (g == 0) wait_loads(-1, group0()); else wait_loads(-1, group1());
     __builtin_amdgcn_s_barrier();                       // chunk 0 is in LDS
     if (g == 0) {
         for (int c = 0; c < NC; ++c) {
             if (c) { __builtin_amdgcn_s_barrier(); __builtin_amdgcn_sched_barrier(0); }
             R(c, false);
             M();
-            wait_loads(c);          // (behind the products: half a period more for the loads than in front of them)
+            wait_loads(c, group0());          // (behind the products: half a period more for the loads than in front of them)
         }
     } else {
         R(0, true);
@@ -1501,10 +1533,17 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
         M();
     }
     // (the first group is here while the second may still be reading the last chunk: the stages are dead, and each
-    // wavefront owns 64 x 72 halfs of them for its epilogue, once every wavefront has passed this barrier)
+    // wavefront owns 64 x 72 halfs of them (88 with five column tiles) for its epilogue, once every wavefront has passed this barrier)
     __builtin_amdgcn_s_barrier();
-    big_gemm_store<EPI, 2>(a, acc, nt0, row0, wr, wn, lane, big_smem + w * (64 * 72));
+    constexpr int OWN = 64 * (NJ > 4 ? 16 * NJ + 8 : 72);
+    static_assert(8 * OWN * 2 <= (int)BigShape<NJ>::SHM, "the epilogue's rows fit the stages");
+    big_gemm_store<EPI, 2, NJ>(a, acc, nt0, row0, wr, wn, lane, big_smem + w * OWN);
 }
+
+// (tship_wide_gemm.hip) the kernel of another width of the 256-row tile, its 32-column tiles and dynamic LDS
+typedef void (*BigKernel)(BigArgs);
+struct WideGemm { BigKernel kernel; int cols; unsigned shm; };
+WideGemm wide_gemm(int tile, int epi);
 
 // Prefill GEMM for launches that 256 x 256 tiles would leave most of the chip idle in (up to a few thousand rows).  Block tile
 // 64 WR rows x 32 NJ columns, eight wavefronts: a wavefront owns 64 rows x all the columns (NJ x 2 MFMA tiles of 32 x 32), and
@@ -2276,7 +2315,7 @@ __global__ __launch_bounds__(256) void resid_norm_kernel(ResidNormArgs a) {
 }
 
 // 1 / rms of every row from the per-tile sums of squares (deferred RMSNorm, prefill): one thread per row
-__global__ __launch_bounds__(256) void rinv_rows_kernel(const float* __restrict__ ssq, int ntiles, long ld, float inv_h, float eps,
+static __global__ __launch_bounds__(256) void rinv_rows_kernel(const float* __restrict__ ssq, int ntiles, long ld, float inv_h, float eps,
                                                         float* __restrict__ rinv, long rows) {
     const long r = (long)blockIdx.x * 256 + threadIdx.x;
     if (r >= rows) return;
@@ -3872,7 +3911,7 @@ __device__ __forceinline__ int greedy_row(const float* __restrict__ logits, long
     __syncthreads();
     return s_tok;
 }
-__global__ __launch_bounds__(1024) void greedy_kernel(const float* __restrict__ logits, long ld, int V, int* __restrict__ next_ids,
+static __global__ __launch_bounds__(1024) void greedy_kernel(const float* __restrict__ logits, long ld, int V, int* __restrict__ next_ids,
                                                       int* __restrict__ gen_out, const int* __restrict__ d_step,
                                                       int* __restrict__ last_pos, long last_ld, const int* __restrict__ d_len,
                                                       const unsigned char* __restrict__ blocked) {

@@ -1,0 +1,115 @@
+"""The other widths of the 256-row prefill GEMM tile (TSHIP_GEMM_TILE 42, 43, 45: 128, 192 and 320 columns) at the edges of their range."""
+import os
+import re
+import subprocess
+
+import numpy as np
+import pytest
+
+from parity_util import FP16_SENSITIVE_REL, sensitive
+from seq2seqsharp_amd import build as B
+from seq2seqsharp_amd import synth
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def G():
+    from seq2seqsharp_amd import gpt
+    return gpt
+
+
+# hidden, heads, kv heads, ffn, norm, activation: even k-tile counts; columns below, between and behind whole tiles of each width
+# (QKV 288, 448 and 1280 columns; up projections of 384, 1408 and 640), the last wavefront's columns partly or wholly beyond the matrix
+SHAPES = {
+    "rms_gated": (96, 6, 6, 192, synth.RMSNORM, synth.SWIGLU),
+    "rms_silu_gate": (320, 5, 1, 704, synth.RMSNORM, synth.SWIGLU_SILU),
+    "layer_norm_relu": (640, 10, 5, 640, synth.LAYERNORM, synth.RELU),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("batch,prompt", [(1, 256), (1, 257), (3, 90), (2, 256), (5, 128), (1, 895)])      # row tiles whole, by one row, by part of a wavefront
+def test_widths_of_the_256_row_tile(G, oracle, monkeypatch, shape, batch, prompt):
+    hidden, heads, kv, ffn, norm, act = SHAPES[shape]
+    cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=ffn, vocab=157, attn_type=synth.GQA, norm_type=norm, act=act,
+                     batch=batch, prompt=prompt, steps=2, dtype="f16")
+    w = sensitive(synth.make_weights(cfg, 51, random_bias=True), hidden)
+    seqs = synth.make_prompts(cfg, 52)
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(seqs, use_cache=True)
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
+    for tile in (0, 42, 43, 45):
+        monkeypatch.setenv("TSHIP_GEMM_TILE", str(tile))
+        gpu.reset()
+        gpu.prefill(seqs)
+        used = sum(bool(re.search(r"big_gemm3_f16_kernel<\d, %d>" % (tile % 10 or 4), s)) for s in gpu.profile_symbols())
+        assert used == 8, tile                     # four projections of two layers
+        got = gpu.logits()
+        assert np.abs(got - lg).max() <= FP16_SENSITIVE_REL * np.abs(lg).max(), tile
+        k, v = gpu.get_kv(1, 0), gpu.get_kv(1, 1)
+        if not tile:
+            k0, v0 = k, v
+        # every output's k-tiles are added in the same order with each width; what is left is where the gated product is rounded to
+        # fp16, once or twice (2^-11 of it), in front of the second layer's sums
+        assert np.abs(k - k0).max() <= 4e-3 * np.abs(k0).max() and np.abs(v - v0).max() <= 4e-3 * np.abs(v0).max(), tile
+    gpu.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("experts,k,batch,prompt", [(8, 2, 4, 300), (4, 1, 3, 200), (33, 3, 1, 700)])
+@pytest.mark.parametrize("tile", [42, 43, 45])
+def test_experts_with_each_width(G, oracle, monkeypatch, experts, k, batch, prompt, tile):
+    """The packed launches of MoE prefills: row tiles of several problems behind each other."""
+    cfg = synth.tiny_config(n_layers=3, n_experts=experts, experts_per_token=k, norm_type=synth.LAYERNORM, act=synth.RELU, dtype="f16", batch=batch, prompt=prompt, vocab=300)
+    w = synth.make_weights(cfg, 62, random_bias=True)
+    seqs = synth.make_prompts(cfg, 162)
+    orc = oracle.OracleGpt(cfg, w)
+    _, lg = orc.step(seqs, use_cache=True)
+    monkeypatch.setenv("TSHIP_GEMM_TILE", str(tile))
+    gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 10)
+    gpu.prefill(seqs)
+    assert np.abs(gpu.logits() - lg).max() <= 3e-2        # (the bar of the other MoE prefill tests)
+    gpu.close()
+
+
+@pytest.mark.timeout(900)
+def test_no_width_touches_a_read_in_flight(tmp_path):
+    """The scan of test_asm_hazards over these kernels' translation unit."""
+    from test_asm_hazards import _kernels, reads_in_flight_on_paths
+    if not os.path.exists(B.HIPCC):
+        pytest.skip("hipcc is not installed")
+    out = tmp_path / "wide.s"
+    r = subprocess.run([B.HIPCC] + B.FLAGS + ["--cuda-device-only", "-S", os.path.join(B.CSRC, "tship_wide_gemm.hip"), "-o", str(out)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernels = {n: i for n, i in _kernels(out.read_text()).items() if any(a and s.startswith("ds_read_b128") for _, s, a in i)}
+    assert sum("big_gemm3_f16_kernel" in n for n in kernels) == 9
+    for name, instrs in kernels.items():
+        assert reads_in_flight_on_paths(instrs) == [], name
+
+
+def test_the_rule_with_all_widths():
+    """The estimates with the constants of the source pick a tile within 1 % of the best on average, against the measured launches."""
+    source = open(os.path.join(ROOT, "seq2seqsharp_amd", "csrc", "tship_gpt.hip")).read()
+    table = open(os.path.join(ROOT, "profiles", "prefill_gemm_wide_tiles.txt")).read().split("\n")
+    numbers = lambda text: [[float(x.rstrip("f")) for x in c.split(",")] for c in re.findall(r"\{([\d., f]+)\}", text)]
+    other = numbers(re.search(r"static const Cost costs\[\] = \{(\{11, 64.*?)\};", source, re.S).group(1))
+    wide = numbers(re.search(r"static const Cost wide\[\] = \{(.*?)\};", source, re.S).group(1))
+    costs = {(40 + int(c[2]) // 2 if not c[0] else int(c[0])): c for c in other + wide}
+    over = []
+    for line in table:
+        m = re.fullmatch(r"(\d+) x (\d+) (\d+): (.*)", line)
+        if not m:
+            continue
+        k, n, rows = (int(m.group(i)) for i in (1, 2, 3))
+        us = {int(t): float(v) for t, v in re.findall(r"(\d+):([\d.]+)", m.group(4))}
+
+        def estimate(tile):
+            _, tr, tc, a, b = costs[tile]
+            tiles = -(-rows // int(tr)) * -(-(n // 32) // int(tc))
+            rounds = -(-tiles // 256)
+            return rounds * (a + b * (k // 16)) * (1 + (0.2 if tile < 40 else 0.35) * tiles / (rounds * 256))
+        over.append(us[min(us, key=estimate)] / min(us.values()) - 1)
+    assert len(over) > 100 and np.mean(over) <= 0.01 and np.mean(np.array(over) > 0.1) <= 0.03, (np.mean(over), max(over))
