@@ -1560,17 +1560,17 @@ WideGemm wide_gemm(int tile, int epi);
 //   1665 rows  2048 x 3072  45 -> 39    2048 x 2048  57 -> 27   2048 x 11264  109 (256 x 256)   5632 x 2048  124 -> 53
 // Two resident blocks per unit (three stages, half the reduction area) measured 8-25 % slower at one round of tiles and
 // gained only from three rounds on, where a larger tile is faster still.
-template <int NJ, int KG>
+template <int NJ, int CK>
 __device__ __forceinline__ void mid_read_frags(unsigned wa, unsigned xa, half8 (&wf)[NJ], half8 (&xf)[2]) {
-    constexpr int XO = 32 * KG * 32;      // bytes of 32 rows of a stage
+    constexpr int XO = 32 * CK * 32;      // bytes of 32 rows of a stage
     if constexpr (NJ == 4)
         asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:%8\n\tds_read_b128 %2, %6 offset:%9\n\tds_read_b128 %3, %6 offset:%10\n\t"
                      "ds_read_b128 %4, %7\n\tds_read_b128 %5, %7 offset:%11"
                      : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(wf[2]), "=&v"(wf[3]), "=&v"(xf[0]), "=&v"(xf[1])
-                     : "v"(wa), "v"(xa), "n"(KG * 1024), "n"(2 * KG * 1024), "n"(3 * KG * 1024), "n"(XO) : "memory");
+                     : "v"(wa), "v"(xa), "n"(CK * 1024), "n"(2 * CK * 1024), "n"(3 * CK * 1024), "n"(XO) : "memory");
     else if constexpr (NJ == 2)
         asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:%6\n\tds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:%7"
-                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa), "n"(KG * 1024), "n"(XO) : "memory");
+                     : "=&v"(wf[0]), "=&v"(wf[1]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa), "n"(CK * 1024), "n"(XO) : "memory");
     else
         asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %4\n\tds_read_b128 %2, %4 offset:%5"
                      : "=&v"(wf[0]), "=&v"(xf[0]), "=&v"(xf[1]) : "v"(wa), "v"(xa), "n"(XO) : "memory");
@@ -1582,9 +1582,11 @@ __device__ __forceinline__ void mid_wait_frags(half8 (&wf)[NJ], half8 (&xf)[2]) 
     else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wf[0]), "+v"(xf[0]), "+v"(xf[1])::"memory");
 }
 constexpr int MID_SPLITS = 4;        // at most so many blocks share the K of a tile
-// stages and LDS bytes of a launch
+// stages and LDS bytes of a launch.  A chunk holds U k-tiles of each wavefront: with two a barrier serves twice the products, which the
+// 128 x 64 tile has LDS for (three stages of 48 KiB; us at 96 rows, weights from HBM, one -> two: gated 2048 x 11264 20.2 -> 19.6, 5632 x 2048
+// 35.7 -> 34.4, 11008 x 4096 65.2 -> 62.6).  The 64 x 32 tile lost 1.5 % with two, the others have no LDS for a third stage.
 template <int WR, int NJ> struct MidShape {
-    static constexpr int KG = 8 / WR, STAGE = KG * (NJ + 2 * WR) * 1024, NST = STAGE > 40960 ? 3 : 4;
+    static constexpr int KG = 8 / WR, U = NJ == 2 && WR == 2 ? 2 : 1, CK = KG * U, STAGE = CK * (NJ + 2 * WR) * 1024, NST = STAGE > 49152 ? 2 : STAGE > 40960 ? 3 : 4;
     static constexpr int UP = NJ == 1 ? 2 : 4, RED = 8 * UP * 32 * 36 * 4;
     static constexpr unsigned SHM = NST * STAGE > RED ? NST * STAGE : RED;
 };
@@ -1595,7 +1597,7 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     extern __shared__ __attribute__((aligned(16))) half_t big_smem[];
     __shared__ float ssq_part[512];                     // [512 / (64 WR)][64 WR rows]: shares of the rows' sums of squares
     using S = MidShape<WR, NJ>;
-    constexpr int KG = S::KG, NST = S::NST, PF = NST - 1, STAGE = S::STAGE, LW = NJ * KG / 8, PPR = 2 * KG, LPC = LW + 2;      // LPC: loads per wavefront and chunk
+    constexpr int KG = S::KG, U = S::U, CK = S::CK, NST = S::NST, PF = NST - 1, STAGE = S::STAGE, LW = NJ * CK / 8, LX = 2 * U, PPR = 2 * CK, LPC = LW + LX;      // LPC: loads per wavefront and chunk
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = WR == 2 ? w >> 2 : 0, kg = WR == 2 ? w & 3 : w;
     int first = 0;      // first row
@@ -1635,13 +1637,13 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
 #pragma unroll
     for (int i = 0; i < LW; ++i) {
         const int p = i * 8 + w;
-        wsrc[i] = a.W + ((long)min(nt0 + p / KG, a.NT - 1) * a.KT * 64 + lane) * 8;
-        wkt[i] = p % KG;
+        wsrc[i] = a.W + ((long)min(nt0 + p / CK, a.NT - 1) * a.KT * 64 + lane) * 8;
+        wkt[i] = p % CK;
     }
-    auto swz = [](int row) { return KG == 4 ? (row >> 1) & 7 : row & 15; };
-    const half_t* xsrc[2]; int xkt[2];
+    auto swz = [](int row) { return PPR == 8 ? (row >> 1) & 7 : row & (PPR - 1); };
+    const half_t* xsrc[LX]; int xkt[LX];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < LX; ++i) {
         const int rl = (i * 8 + w) * (64 / PPR) + lane / PPR, s = (lane % PPR) ^ swz(rl);
         long row = min(row0 + rl, (long)a.R - 1);
         if (PACKED && a.row_idx) row = a.row_idx[row];
@@ -1654,16 +1656,20 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
         char* st = (char*)big_smem + (c % NST) * STAGE;
 #pragma unroll
         for (int i = 0; i < LW; ++i)
-            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (long)min(kt_first + c * KG + wkt[i], kt_end - 1) * 512), (lptr_t)(st + (i * 8 + w) * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(wsrc[i] + (long)min(kt_first + c * CK + wkt[i], kt_end - 1) * 512), (lptr_t)(st + (i * 8 + w) * 1024), 16, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (long)min(kt_first + c * KG + xkt[i], kt_end - 1) * 16), (lptr_t)(st + NJ * KG * 1024 + (i * 8 + w) * 1024), 16, 0, 0);
+        for (int i = 0; i < LX; ++i)
+            __builtin_amdgcn_global_load_lds((gptr_t)(xsrc[i] + (long)min(kt_first + c * CK + xkt[i], kt_end - 1) * 16), (lptr_t)(st + NJ * CK * 1024 + (i * 8 + w) * 1024), 16, 0, 0);
     };
-    const int NC = (kt_end - kt_first + KG - 1) / KG;
+    const int NC = (kt_end - kt_first + CK - 1) / CK;
     const unsigned lds0 = (unsigned)(size_t)(lptr_t)big_smem;
     const int xr = 64 * wr + (lane & 31);
-    const unsigned woff = (unsigned)(kg * 1024 + lane * 16);
-    const unsigned xoff = (unsigned)(NJ * KG * 1024 + xr * (PPR * 16) + 16 * ((2 * kg + (lane >> 5)) ^ swz(xr)));
+    unsigned woff[U], xoff[U];      // of this wavefront's k-tiles of a chunk
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        woff[u] = (unsigned)((u * KG + kg) * 1024 + lane * 16);
+        xoff[u] = (unsigned)(NJ * CK * 1024 + xr * (PPR * 16) + 16 * ((2 * (u * KG + kg) + (lane >> 5)) ^ swz(xr)));
+    }
     issue(0);
     if (NC > 1) issue(1);
     if (PF > 2 && NC > 2) issue(2);
@@ -1676,7 +1682,7 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
         ssq_part[t] = s;
     }
     if (a.advance_pos && blockIdx.x == 0 && blockIdx.y == 0 && t == 0) { a.advance_pos[0] += 1; a.advance_pos[1] += 1; }
-    half8 wf[NJ], xf[2];
+    half8 wf[U][NJ], xf[U][2];
     auto wait_loads = [&](int c) {          // this wavefront's part of chunk c + 1 has landed
         const int later = max(0, min(PF - 1, NC - 2 - c));
         if (later == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPC) : "memory");
@@ -1685,22 +1691,26 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
     };
     auto R = [&](int c, bool wait_now) {
         const unsigned sb = lds0 + (unsigned)((c % NST) * STAGE);
-        mid_read_frags<NJ, KG>(sb + woff, sb + xoff, wf, xf);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mid_read_frags<NJ, CK>(sb + woff[u], sb + xoff[u], wf[u], xf[u]);
         if (c + PF < NC) issue(c + PF);
         if (wait_now) wait_loads(c);
-        mid_wait_frags<NJ>(wf, xf);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mid_wait_frags<NJ>(wf[u], xf[u]);
         __builtin_amdgcn_sched_barrier(0);
     };
     auto M = [&](int c) {
         __builtin_amdgcn_sched_barrier(0);
-        if (kt_first + c * KG + kg < kt_end) {           // (wavefront-uniform: the last chunk may hold fewer than KG k-tiles)
-            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
+        for (int u = 0; u < U; ++u)
+            if (kt_first + c * CK + u * KG + kg < kt_end) {           // (wavefront-uniform: the last chunk may hold fewer than CK k-tiles)
+                __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-                for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[j], xf[i], acc[j][i], 0, 0, 0);
-            __builtin_amdgcn_s_setprio(0);
-        }
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[u][j], xf[u][i], acc[j][i], 0, 0, 0);
+                __builtin_amdgcn_s_setprio(0);
+            }
         __builtin_amdgcn_sched_barrier(0);
     };
     wait_loads(-1);
