@@ -691,6 +691,21 @@ static GemmMix pick_gemm_mix(const GemmW& w, long R) {
     const GemmMix other = pick_gemm_mix(w, R, false), all = pick_gemm_mix(w, R, true);
     return other.cols && all.us >= 0.925f * other.us ? other : all;
 }
+// Whether the blocks of a projection with these tiles form its rows' 1 / rms themselves (BigArgs::ssq): a kernel in front of it takes 5 us
+// and the gap behind it, forming it delays every round of tiles by the sums' loads, some hundred ns.  ms per prompt of the 1B model with at
+// most 0 / 1 / 2 / 4 / 8 / any rounds: 600 rows 2.27 / 2.17 / 2.16 / 2.14 / 2.16 / 2.15, 1665 rows 3.71 / 3.59 / 3.57 / 3.54 / 3.56 / 3.57, 5328 rows
+// 8.97 / 8.97 / 8.93 / 8.87 / 8.87 / 8.87, 32768 rows 49.9 / 49.8 / 49.8 / 50.2 / 50.0 / 50.6 (no tile of it in four rounds; +-0.3 between runs).
+static bool forms_rms(const GemmW& w, const GemmMix& mix, long R) {
+    const long ncu = std::max(1, n_compute_units());
+    long rounds = 0;
+    auto part = [&](int tile, int columns) {
+        for (const GemmCost& c : gemm_costs())
+            if (gemm_tile_code(c) == (tile >= 100 ? tile % 100 : tile)) rounds += ceil_div(ceil_div(R, c.rows) * ceil_div(columns, c.cols) * std::max(1, tile / 100), ncu);
+        return tile != 0 || w.KT % 2 == 0;      // (the kernel for odd k-tile counts does not)
+    };
+    const bool able = mix.cols ? part(mix.tile, mix.cols) && part(mix.rest, w.NT - mix.cols) : part(mix.tile, w.NT);
+    return able && rounds <= 4;
+}
 static void run_mid_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int mid) {
     e.splits = mid / 100; mid %= 100;
     e.xchg = m->mid_xchg.as<float>(); e.tile_count = m->mid_count.as<int>();
@@ -746,7 +761,7 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
     e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.R = (int)R;
     if (!mix.cols) { launch_big_gemm(m, name, e, epi, mix.tile); return; }
     const int off = epi == BEPI_ACT16 && e.gated ? 16 * mix.cols : 32 * mix.cols;       // outputs of the first part
-    TSHIP_REQUIRE(!e.kcache && !e.advance_pos && !e.ssq && off < e.n_valid, "internal: columns of this projection stay together");
+    TSHIP_REQUIRE(!e.kcache && !e.advance_pos && off < e.n_valid, "internal: columns of this projection stay together");
     BigArgs r = e;
     e.NT = mix.cols; e.n_valid = off;
     r.W += (long)mix.cols * w.KT * 512; r.NT -= mix.cols; r.n_valid -= off; r.bias += off;
@@ -1448,7 +1463,6 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         if (h <= 2048) launch(m, "p_embed_prepare", fn_prepare_kernel<8>, dim3((unsigned)R), dim3(256), a);
         else if (h <= 4096) launch(m, "p_embed_prepare", fn_prepare_kernel<16>, dim3((unsigned)R), dim3(256), a);
         else launch(m, "p_embed_prepare", fn_prepare_kernel<32>, dim3((unsigned)R), dim3(256), a);
-        make_rinv("p_rinv_attn");
     } else {
         ResidNormArgs a = rn;
         a.ids = ids.as<int>(); a.emb = m->emb.p; a.emb_f16 = m->f16; a.emb_scale = (float)std::sqrt((double)h);
@@ -1483,6 +1497,13 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         fuse_kv = can_fuse_kv && !qkv_tiles.tile && !qkv_tiles.cols && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
         wo_tiles = pick_gemm_mix(L.wo, R); w13_tiles = pick_gemm_mix(L.w13, R); w2_tiles = pick_gemm_mix(L.w2, R);
     }
+    // 1 / rms of a deferred norm: from the tile sums, by the consuming projection itself or by a kernel in front of it
+    const bool rms_qkv = deferred && forms_rms(m->L[0]->qkv, qkv_tiles, R), rms_w13 = deferred && forms_rms(m->L[0]->w13, w13_tiles, R);
+    auto consumer = [&](BigArgs& e, bool forms, const char* name) {
+        if (!deferred) return;
+        if (forms) { e.ssq = pssq.as<float>(); e.ssq_nt = NTh; e.ssq_in_ld = R; e.inv_h = 1.0f / (float)h; e.eps = c.norm_eps; }
+        else { make_rinv(name); e.rinv = prinv.as<float>(); }
+    };
     for (int l = 0; l < c.n_layers; ++l) {
         LayerW& L = *m->L[l];
         AttnArgs aa = attn_args(m, L);
@@ -1492,7 +1513,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         if (m->f16) {
             BigArgs e; std::memset(&e, 0, sizeof(e));
             e.out = pqkv.as<float>(); e.ld_out = (int)qp; e.bias = L.bqkv.as<float>(); e.n_valid = m->Nqkv;
-            if (deferred) e.rinv = prinv.as<float>();
+            consumer(e, rms_qkv, "p_rinv_attn");
             if (fuse_kv) {
                 TSHIP_REQUIRE((long)round_up(pos0 + Tp, 32) <= m->ML, "internal: cache chunk beyond the allocation");
                 e.kcache = (half_t*)L.kc.p; e.vcache = (half_t*)L.vc.p; e.kv_max_len = m->ML; e.kv_col0 = HD; e.kv_gd = GD; e.kv_D = m->D;
@@ -1546,15 +1567,14 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             // experts' output is added to the residual stream by the norm kernel that follows (a combine kernel of its own
             // behind the last layer of an fp16 model, which no norm kernel follows)
             run_moe_ffn_prefill(m, L, (int)R, a2, rowmap.as<int>(), B, norm_after ? &a3 : nullptr);
-        } else if (deferred) make_rinv("p_rinv_ffn");
-        else run_resid_norm(m, "p_norm_ffn", (int)R, a2);
+        } else if (!deferred) run_resid_norm(m, "p_norm_ffn", (int)R, a2);
         if (L.moe) {
             // (nothing more: no dense feed-forward in this layer)
         } else if (m->f16) {
             BigArgs e; std::memset(&e, 0, sizeof(e));
             e.bias = L.b1.as<float>(); e.bias2 = L.b3.as<float>(); e.out16 = pa.as<half_t>(); e.ld16 = (int)m->ldF;
             e.act = c.act; e.gated = m->gated; e.n_valid = F;
-            if (deferred) e.rinv = prinv.as<float>();
+            consumer(e, rms_w13, "p_rinv_ffn");
             big("p_gemm_ffn13", L.w13, pxn.p, m->ldh, BEPI_ACT16, e, w13_tiles);
             BigArgs e2; std::memset(&e2, 0, sizeof(e2));
             e2.out = px.as<float>(); e2.ld_out = h; e2.bias = L.b2.as<float>(); e2.n_valid = h;
@@ -1568,8 +1588,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             run_gemm_f32(m, "p_gemm_ffn2", L.w2, pa.as<float>(), m->ldF, (int)R, pqkv.as<float>(), qp, 0, 1);
             a3.part = pqkv.as<float>(); a3.KS = 1; a3.ld_part = qp; a3.bias = L.b2.as<float>();
         }
-        if (deferred) { if (l + 1 < c.n_layers) make_rinv("p_rinv_attn"); }
-        else if (norm_after && !L.moe) run_resid_norm(m, "p_norm_attn", (int)R, a3);
+        if (norm_after && !L.moe) run_resid_norm(m, "p_norm_attn", (int)R, a3);
     }
     // last position of every sequence (Decoder.cs:705-716) -> final norm -> vocabulary projection
     if (m->fused_norm && !m->ln) {

@@ -797,7 +797,7 @@ struct BigArgs {
     // deferred RMSNorm (LDS-tiled kernels only).  Consumers: X holds half(gamma * x) and every output row is scaled by
     // rinv[row] before the bias.  Producers (BEPI_RESID): besides the residual stream, store half(gamma * x) row-major
     // into xg16 and the sum of squares of every (32-column tile, row) into ssq_out[tile * ssq_ld + row].
-    // (mid_gemm_f16_kernel: with ssq instead of rinv it forms them itself from the ssq_nt tile sums [tile][ssq_in_ld rows])
+    // (mid_gemm_f16_kernel, big_gemm3_f16_kernel: with ssq instead of rinv they form it themselves from the ssq_nt tile sums [tile][ssq_in_ld rows])
     const float* rinv;
     const float* ssq; int ssq_nt; long ssq_in_ld; float inv_h, eps;
     int splits; float* xchg; int* tile_count;      // mid_gemm_f16_kernel: blocks that share a tile's K (0 or 1: one), their exchange area and counters
@@ -1060,8 +1060,10 @@ __device__ __forceinline__ void kv_store_frags(const BigArgs& a, floatx16 (&acc)
 }
 
 // NI: 32-row tiles per wavefront (the wavefront's rows start at 32 NI wr), NJ: its 32-column tiles
+// ssq_part: with a.ssq, two shares of each of the tile's 256 rows' sums of squares
 template <int EPI, int NI = 4, int NJ = 4>
-__device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)[NJ][NI], int nt0, long row0, int wr, int wn, int lane, half_t* stage = nullptr) {
+__device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)[NJ][NI], int nt0, long row0, int wr, int wn, int lane, half_t* stage = nullptr,
+                                               const float* ssq_part = nullptr) {
     // accumulator (j, i), lane l, register v = 4 g + e: column (nt0 + NJ wn + j) * 32 + 8 g + 4 (l / 32) + e,
     // row row0 + 128 wr + 32 i + l % 32.  Biases (and the residual) are fetched in batches before the first store
     // of a column tile, and the four consecutive columns of a group go out as one 16-byte (fp32) or 8-byte (fp16) store.
@@ -1072,6 +1074,10 @@ __device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)
     for (int i = 0; i < NI; ++i) {
         const long row = row0 + 32 * NI * wr + 32 * i + (lane & 31);
         rinv4[i] = (a.rinv && row < a.R) ? a.rinv[row] : 1.0f;
+        if (ssq_part && a.ssq) {
+            const int rl = 32 * NI * wr + 32 * i + (lane & 31);
+            rinv4[i] = 1.0f / sqrtf((ssq_part[rl] + ssq_part[256 + rl]) * a.inv_h + a.eps);
+        }
     }
     if constexpr (EPI == BEPI_ACT16 && NI == 2) {
         // whole outputs of a wavefront with 16-byte aligned rows: line stores through LDS
@@ -1394,6 +1400,7 @@ template <int NJ> struct BigShape {
 template <int EPI, int NJ = 4>
 __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     extern __shared__ __attribute__((aligned(16))) half_t big_smem[];
+    __shared__ float ssq_part[512];                      // (a.ssq) two shares of every row's sum of squares
     constexpr int CK = 2, NST = BigShape<NJ>::NST, WFR = 2 * NJ * CK, PF = NST - 1;          // k-tiles per stage, stages, weight fragments per stage, chunks requested ahead
     constexpr int STAGE = BigShape<NJ>::STAGE / 2;       // halfs per stage: weight fragments, then 16 activation fragments
     constexpr int LW = (WFR + 7) / 8;                    // weight fragments that a wavefront stages; with an odd NJ the last half of them belongs to the first four
@@ -1474,6 +1481,13 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     issue(0);
     if (NC > 1) issue(1);
     if (NC > 2) issue(2);
+    if (a.ssq) {      // (behind the first requests, as in mid_gemm_f16_kernel; sixteen at a time)
+        const float* src = a.ssq + min(row0 + (t & 255), (long)a.R - 1);
+        float s = 0.0f;
+#pragma unroll 16
+        for (int i = t >> 8; i < a.ssq_nt; i += 2) s += src[i * a.ssq_in_ld];
+        ssq_part[t] = s;
+    }
     // Two groups of four wavefronts (one per SIMD each; wavefronts w and w + 4 share a SIMD: grouping by w % 2 instead
     // measured 30 % slower) run the same chunks half a period apart with one block barrier per chunk: behind barrier c
     // the first group reads its fragments of chunk c from LDS while the second multiplies chunk c - 1 out of its
@@ -1537,7 +1551,7 @@ __global__ __launch_bounds__(512) void big_gemm3_f16_kernel(BigArgs a) {
     __builtin_amdgcn_s_barrier();
     constexpr int OWN = 64 * (NJ > 4 ? 16 * NJ + 8 : 72);
     static_assert(8 * OWN * 2 <= (int)BigShape<NJ>::SHM, "the epilogue's rows fit the stages");
-    big_gemm_store<EPI, 2, NJ>(a, acc, nt0, row0, wr, wn, lane, big_smem + w * OWN);
+    big_gemm_store<EPI, 2, NJ>(a, acc, nt0, row0, wr, wn, lane, big_smem + w * OWN, ssq_part);
 }
 
 // (tship_wide_gemm.hip) the kernel of another width of the 256-row tile, its 32-column tiles and dynamic LDS
