@@ -2421,6 +2421,7 @@ struct AttnArgs {
     const int* d_pos;                              // decode: number of cached positions, read on the device
     int pos0;                                      // prefill: cache offset of the first query row
     int Tq;                                        // prefill: query rows per sequence
+    int q_skip;                                    // prefill: blocks of query rows at the front of every sequence that the launch leaves out
     void* out; long ld_out;                        // [rows][H*D] in the activation type
     int out_kt;                                    // > 0: out is fragment packed with this many k-tiles
     float scale;
@@ -2907,7 +2908,7 @@ __global__ __launch_bounds__(D * 4) void kv_write_frag_kernel(AttnArgs a) {
 template <typename CT, typename AT, int D, int G>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
     __shared__ AttnSmem<CT, D, G, 4> sm;
-    const int tq = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z, t = threadIdx.x;
+    const int tq = blockIdx.x + a.q_skip, kvh = blockIdx.y, b = blockIdx.z, t = threadIdx.x;
     const int kvc = a.kv_sub > 1 ? kvh / a.kv_sub : kvh;
     const long row = (long)b * a.Tq + tq;
     const int pos = a.pos0 + tq;
@@ -2948,7 +2949,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float af_smem[];       // queries [32][LDQ]; later O [4][D][33], then m, l [4][32]
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, l32 = lane & 31, half = lane >> 5;
     const int kvh = blockIdx.y, b = blockIdx.z, kvc = a.kv_sub > 1 ? kvh / a.kv_sub : kvh;
-    const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * QB, nq = min(QB, a.Tq - q0);
+    const int q0 = (a.q_skip + (int)gridDim.x - 1 - (int)blockIdx.x) * QB, nq = min(QB, a.Tq - q0);
     for (int p = t; p < 32 * (D / 2); p += 256) {
         const int c = p / (D / 2), i = p % (D / 2), tq = q0 + c / G;
         float y0 = 0.0f, y1 = 0.0f;
@@ -3535,11 +3536,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? (
     const int r16 = lane & 15, q = lane >> 4;
     const int kvh = blockIdx.y, b = blockIdx.z;
     const int kvc = a.kv_sub > 1 ? kvh / a.kv_sub : kvh;       // (groups of query heads that share a KV head, see AttnArgs::kv_sub)
-    const int tq0 = (blockIdx.x * NW + w) * (QB * NQ);
+    const int qb = (int)blockIdx.x + a.q_skip, tq0 = (qb * NW + w) * (QB * NQ);
     const bool active = tq0 < a.Tq;          // wavefronts beyond the prompt still fetch their share of every chunk
     const int pos_base = a.pos0 + tq0, T = min(pos_base + QB * NQ, a.pos0 + a.Tq);
     // chunks of the block: up to the last position of its last active wavefront
-    const int tq_last = min(a.Tq, (int)(blockIdx.x + 1) * NW * QB * NQ);
+    const int tq_last = min(a.Tq, (qb + 1) * NW * QB * NQ);
     const int len_b = RAGGED ? a.lens[b] : 0x7fffffff;
     const int Ttot = a.pos0 + a.Tq;
     const int nchunks = (RAGGED && tq_last > len_b) ? (Ttot + 31) / 32 : (a.pos0 + tq_last + 31) / 32;
