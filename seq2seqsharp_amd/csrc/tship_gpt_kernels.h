@@ -3890,10 +3890,12 @@ __device__ __forceinline__ int greedy_row(const float* __restrict__ logits, long
                                           const unsigned char* __restrict__ blocked) {
     __shared__ float sv[16];
     __shared__ int si[16];
-    __shared__ int s_tok;
     const int b = blockIdx.x, t = threadIdx.x;
     const float* row = logits + (long)b * ld;
     float best = -INFINITY; int bi = 0x7fffffff;
+    // (requested in front of the logits: behind the choice they would be a round trip between it and the embedding's rows)
+    const long step = gen_out && d_step ? (long)*d_step : 0;
+    const int len = last_pos ? *d_len : 0;
     // eight 16-byte requests per thread at a time, all in flight before the first comparison (32 768 logits: one round trip;
     // 4-byte requests took four); rows start at multiples of 32 floats, the indices are clamped to the row's last 16 bytes
     for (int i0 = 4 * t; i0 < V; i0 += 1024 * 4 * 8) {
@@ -3925,16 +3927,21 @@ __device__ __forceinline__ int greedy_row(const float* __restrict__ logits, long
     }
     if ((t & 63) == 0) { sv[t >> 6] = best; si[t >> 6] = bi; }
     __syncthreads();
-    if (t == 0) {
-        for (int w = 1; w < 16; ++w) if (sv[w] > best || (sv[w] == best && si[w] < bi)) { best = sv[w]; bi = si[w]; }
-        if (bi == 0x7fffffff) bi = 0;   // a row of NaNs: the reference's scan never moves off index 0
-        next_ids[b] = bi;
-        if (gen_out) gen_out[(d_step ? (long)*d_step * gridDim.x : 0) + b] = bi;
-        if (last_pos) last_pos[(long)b * last_ld + bi] = *d_len;
-        s_tok = bi;
+    // every wavefront finishes the choice for itself: one barrier
+    best = sv[t & 15]; bi = si[t & 15];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) {
+        const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(bi, o, 64);
+        if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
     }
-    __syncthreads();
-    return s_tok;
+    bi = __builtin_amdgcn_readfirstlane(bi);
+    if (bi == 0x7fffffff) bi = 0;   // a row of NaNs: the reference's scan never moves off index 0
+    if (t == 0) {
+        next_ids[b] = bi;
+        if (gen_out) gen_out[step * gridDim.x + b] = bi;
+        if (last_pos) last_pos[(long)b * last_ld + bi] = len;
+    }
+    return bi;
 }
 static __global__ __launch_bounds__(1024) void greedy_kernel(const float* __restrict__ logits, long ld, int V, int* __restrict__ next_ids,
                                                       int* __restrict__ gen_out, const int* __restrict__ d_step,
