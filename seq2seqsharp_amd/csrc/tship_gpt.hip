@@ -749,7 +749,7 @@ static bool big_gemm_packed_ok(int KT, long R) { return R >= 512 && KT % 2 == 0;
 static void launch_big_gemm(TSHipGpt* m, const char* name, BigArgs e, int epi, int tile) {
     const bool rows256 = !tile || is_wide_tile(tile);
     TSHIP_REQUIRE(!e.packed_problems || (rows256 && e.KT % 2 == 0), "internal: packed launch of a GEMM shape the LDS-tiled kernel does not take");
-    TSHIP_REQUIRE(!e.kcache || !tile, "internal: only the 256 x 256 tile writes the cache");
+    TSHIP_REQUIRE(!e.kcache || e.kv_scatter || !tile, "internal: only the 256 x 256 tile writes whole fragments of the cache");
     if (rows256) {        // 256-row block tiles
         e.patch_rows = g_hooks.patch_rows;
         if (e.KT % 2 == 0) {      // asynchronous staging: four stages of two k-tiles, eight wavefronts
@@ -775,10 +775,10 @@ static void run_big_gemm(TSHipGpt* m, const char* name, const GemmW& w, const vo
     e.W = w.buf.as<half_t>(); e.KT = w.KT; e.NT = w.NT; e.X = (const half_t*)X; e.ldx = (int)ldx; e.R = (int)R;
     if (!mix.cols) { launch_big_gemm(m, name, e, epi, mix.tile); return; }
     const int off = epi == BEPI_ACT16 && e.gated ? 16 * mix.cols : 32 * mix.cols;       // outputs of the first part
-    TSHIP_REQUIRE(!e.kcache && !e.advance_pos && off < e.n_valid, "internal: columns of this projection stay together");
+    TSHIP_REQUIRE((!e.kcache || e.kv_scatter) && !e.advance_pos && off < e.n_valid, "internal: columns of this projection stay together");
     BigArgs r = e;
     e.NT = mix.cols; e.n_valid = off;
-    r.W += (long)mix.cols * w.KT * 512; r.NT -= mix.cols; r.n_valid -= off; r.bias += off;
+    r.W += (long)mix.cols * w.KT * 512; r.NT -= mix.cols; r.n_valid -= off; r.bias += off; r.kv_col0 -= off;
     if (r.bias2) r.bias2 += off;
     if (epi == BEPI_ACT16) r.out16 += off; else r.out += off;
     if (epi == BEPI_RESID && r.xg16) { r.xg16 += off; r.gamma += off; r.ssq_out += mix.cols * r.ssq_ld; }
@@ -1494,10 +1494,10 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     // The QKV projection with 256 x 256 tiles can write keys and values into the fragment-major cache itself (rotation
     // included) when its wavefronts' 64 x 128 tiles are whole chunks of whole heads.  That takes it about 7.5 us longer and
     // saves a kernel whose time goes with rows x columns of keys and values (profiles/prefill_gemm_tiles.txt: 1024 columns,
-    // 1024 rows 49.0 + 7.4 against 62.5 us, 16384 rows 202 + 37 against 211); a kernel of its own does it where that is less.
+    // 1024 rows 49.0 + 7.4 against 62.5 us, 16384 rows 202 + 37 against 211); elsewhere the tile with the least time writes it in pieces.
     const int HD = c.n_heads * m->D, GD = c.n_kv_heads * m->D;
     GemmMix qkv_tiles = {}, wo_tiles = {}, w13_tiles = {}, w2_tiles = {};
-    bool fuse_kv = false;
+    bool fuse_kv = false, scatter_kv = false;
     if (m->f16) {
         const LayerW& L = *m->L[0];
         const bool can_fuse_kv = m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && L.qkv.KT % 2 == 0 && (m->D == 64 || m->D == 128);
@@ -1509,6 +1509,8 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             if (!qkv_tiles.cols || qkv_tiles.us >= one.us) qkv_tiles = {one.tile, 0, 0, one.us};
         }
         fuse_kv = can_fuse_kv && !qkv_tiles.tile && !qkv_tiles.cols && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
+        // (any other tile and prompt length: in pieces, BigArgs::kv_scatter; the kernel of its own is left to the tests that compare with it)
+        scatter_kv = m->vt && !fuse_kv && g_hooks.gemm_tile != 0 && !g_hooks.no_kv_fuse;
         wo_tiles = pick_gemm_mix(L.wo, R); w13_tiles = pick_gemm_mix(L.w13, R); w2_tiles = pick_gemm_mix(L.w2, R);
     }
     // 1 / rms of a deferred norm: from the tile sums, by the consuming projection itself or by a kernel in front of it
@@ -1539,7 +1541,8 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             BigArgs e; std::memset(&e, 0, sizeof(e));
             e.out = pqkv.as<float>(); e.ld_out = (int)qp; e.bias = L.bqkv.as<float>(); e.n_valid = m->Nqkv;
             consumer(e, rms_qkv, "p_rinv_attn");
-            if (fuse_kv) {
+            if (fuse_kv || scatter_kv) {
+                e.kv_scatter = scatter_kv ? 1 : 0;
                 TSHIP_REQUIRE((long)round_up(pos0 + Tp, 32) <= m->ML, "internal: cache chunk beyond the allocation");
                 e.kcache = (half_t*)L.kc.p; e.vcache = (half_t*)L.vc.p; e.kv_max_len = m->ML; e.kv_col0 = HD; e.kv_gd = GD; e.kv_D = m->D;
                 e.kv_hkv = c.n_kv_heads; e.kv_Tq = Tp; e.kv_pos0 = pos0; e.rope_cos = aa.rope_cos; e.rope_sin = aa.rope_sin;
@@ -1549,7 +1552,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         } else {
             run_gemm_f32(m, "p_gemm_qkv", L.qkv, pxn.as<float>(), m->ldh, (int)R, pqkv.as<float>(), qp, 0, 1);
         }
-        if (fuse_kv) {
+        if (fuse_kv || scatter_kv) {
             // (cache written by the projection)
         } else if (m->vt && aa.pos0 % 32 == 0) {      // whole fragments, one block per 32-position chunk
             TSHIP_REQUIRE(qp % 4 == 0 && (long)round_up(aa.pos0 + Tp, 32) <= m->ML, "internal: cache chunk beyond the allocation");

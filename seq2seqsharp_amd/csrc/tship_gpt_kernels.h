@@ -810,6 +810,12 @@ struct BigArgs {
     // [sequence][kv_hkv heads][kv_max_len x kv_D]; only the query columns are stored to `out`.  kcache null: off.
     half_t* kcache; half_t* vcache; long kv_max_len; int kv_col0, kv_gd, kv_D, kv_hkv, kv_Tq, kv_pos0;
     const float* rope_cos; const float* rope_sin;
+    // kv_scatter: the same with any kernel and any kv_Tq and kv_pos0 (the column counts are multiples of 64): four columns of a row at a time,
+    // 8 bytes of a key fragment or four values of value fragments, whose whole runs the block's stores put together in L2.  A kernel of its
+    // own for them took 5 to 20 us a layer, most of it the round trip to what the projection had just written.  ms per prompt, kernel -> this: 1B
+    // model 1 x 37 1.05 -> 0.99, 2 x 100 1.39 -> 1.31, 16 x 333 8.71 -> 8.60, 32 x 1000 48.2 -> 47.6; 768-wide one 2 x 100 0.64 -> 0.58, 32 x 511
+    // 5.95 -> 5.50; 4 layers of the 7B one 1 x 100 0.66 -> 0.62, 1 x 8001 11.14 -> 11.05; none of 25 sizes slower
+    int kv_scatter;
     // Several problems of one shape in one launch (the experts of a MoE layer at prefill; packed_problems > 0): problem e takes its
     // weights from Wtab[e], its row count from rows_tab[e] (read on the device) and its activations / outputs at fixed strides.
     // The LDS-tiled asynchronous kernel packs the problems' row tiles one behind the other: the launch covers R / 256 row tiles,
@@ -869,6 +875,7 @@ __device__ __forceinline__ void gated_store_lines(const BigArgs& a, floatx16 (&a
 // old residual values are requested in line layout first, the accumulators cross through LDS (64 rows x 36 floats), and
 // x, half(gamma x) and the tile's sums of squares leave from the line layout (a row's 32 columns sit in eight lanes).
 // Same arithmetic per element as the direct form (acc * rinv + bias, then + old); the sums of squares add in another order.
+__device__ __forceinline__ void kv_scatter4(const BigArgs& a, long row, int c0, floatx4 x);
 template <bool RESID>     // false: plain fp32 output with bias (no old values, no fp16 copy)
 __device__ __forceinline__ void resid_store_lines(const BigArgs& a, const floatx16 (&acc2)[2], int nt, long row_first, int lane, float* stage,
                                                   const float (&rinv2)[2]) {
@@ -902,6 +909,7 @@ __device__ __forceinline__ void resid_store_lines(const BigArgs& a, const floatx
         floatx4 sv;
 #pragma unroll
         for (int e = 0; e < 4; ++e) sv[e] = RESID ? v[ps][e] + old[ps][e] : v[ps][e];
+        if (!RESID && a.kcache && nt * 32 >= a.kv_col0) { kv_scatter4(a, row, nt * 32 + 4 * piece, sv); continue; }
         __builtin_nontemporal_store(sv, (floatx4*)(a.out + row * a.ld_out + (long)nt * 32 + 4 * piece));
         if (RESID && a.xg16) {
             half4v xg;
@@ -916,6 +924,60 @@ __device__ __forceinline__ void resid_store_lines(const BigArgs& a, const floatx
         }
     }
     __builtin_amdgcn_wave_barrier();          // the next tile's accumulators overwrite the stage
+}
+
+// Fragment-major KV cache of the MFMA attention kernels (fp16, head_dim 64 or 128).  Positions are grouped in chunks
+// of 32; within a chunk every 1 KiB block is exactly one A operand of v_mfma_f32_16x16x32_f16 (64 lanes x 8 halfs),
+// so a wavefront's load instruction reads 1 KiB contiguous.
+//   keys:   block (chunk, tile, kd), lane r + 16 qq holds K[t = 32 chunk + 8 (r / 4) + 4 tile + r % 4][d = 32 kd + 8 qq + j]
+//   values: block (chunk, dt),       lane r + 16 qq holds V[t = 32 chunk + 8 qq + j][d = 16 dt + r]
+__host__ __device__ inline long kfrag_index(int t, int d, int D) {
+    const int c = t >> 5, tin = t & 31, q8 = tin >> 3, rem = tin & 7, tile = rem >> 2, r = 4 * q8 + (rem & 3);
+    const int kd = d >> 5, qq = (d & 31) >> 3, j = d & 7;
+    return ((((long)c * 2 + tile) * (D / 32) + kd) * 64 + r + 16 * qq) * 8 + j;
+}
+__host__ __device__ inline long vfrag_index(int t, int d, int D) {
+    const int c = t >> 5, qq = (t & 31) >> 3, j = t & 7;
+    return (((long)c * (D / 16) + (d >> 4)) * 64 + (d & 15) + 16 * qq) * 8 + j;
+}
+// Columns c0 ... c0 + 3 of the projection's row `row`, key or value columns, to the cache (BigArgs::kv_scatter).  The same value as through memory and
+// kv_write_frag_kernel: rounded to fp32, rotated with two roundings per output, rounded to fp16.  Where the prompt begins a 32-position chunk, what is
+// left of its last one becomes zero, as there (behind a context it keeps what it held, as with kv_write_kernel).
+__device__ __forceinline__ void kv_scatter4(const BigArgs& a, long row, int c0, floatx4 x) {
+    const int rel = c0 - a.kv_col0, D = a.kv_D, sh = D == 64 ? 6 : 7;
+    const bool is_k = rel < a.kv_gd;
+    const int rc = is_k ? rel : rel - a.kv_gd, kvh = rc >> sh, d = rc & (D - 1);
+    const unsigned bq = (unsigned)row / (unsigned)a.kv_Tq;
+    const int tq = (int)((unsigned)row - bq * (unsigned)a.kv_Tq), pos = a.kv_pos0 + tq;
+    half_t* base = (is_k ? a.kcache : a.vcache) + ((long)bq * a.kv_hkv + kvh) * a.kv_max_len * D;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { float xe = x[e]; asm volatile("" : "+v"(xe)); x[e] = xe; }
+    half4v o;
+    if (is_k && a.rope_cos) {
+        const long ro = (long)pos * (D / 2) + d / 2;
+        const floatx2 cs = *(const floatx2*)(a.rope_cos + ro), sn = *(const floatx2*)(a.rope_sin + ro);
+#pragma unroll
+        for (int pr = 0; pr < 2; ++pr) {
+            float y0, y1;
+            rope_pair(x[2 * pr], x[2 * pr + 1], cs[pr], sn[pr], y0, y1);
+            o[2 * pr] = (half_t)y0; o[2 * pr + 1] = (half_t)y1;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (half_t)x[e];
+    }
+    auto store = [&](int p, half4v v) {
+        if (is_k) *(half4v*)(base + kfrag_index(p, d, D)) = v;
+        else {
+            half_t* dst = base + vfrag_index(p, d, D);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dst[8 * e] = v[e];
+        }
+    };
+    store(pos, o);
+    // the rest of the last chunk: a position for each of the last rows (by the last row alone: 5 x 333 tokens of the 1B model 3.61 ms for 3.53)
+    const int end = a.kv_pos0 + a.kv_Tq;
+    if ((a.kv_pos0 & 31) == 0) for (int p = end + a.kv_Tq - 1 - tq; p < ((end + 31) & ~31); p += a.kv_Tq) store(p, half4v{0, 0, 0, 0});
 }
 
 // Ungated activation output (ReLU / SiLU / LeakyReLU feed-forward, MoE experts): a wavefront's 64 rows x 128 columns go
@@ -1101,7 +1163,7 @@ __device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)
         if constexpr (!RS && NJ == 4) {
             // key and value columns of a QKV projection that writes the cache itself (whole wavefronts: the column counts
             // are multiples of 128, the launch code checks the rest)
-            if (stage && a.kcache && ntf * 32 >= a.kv_col0) {
+            if (stage && a.kcache && !a.kv_scatter && ntf * 32 >= a.kv_col0) {
                 if (ntf >= a.NT) return;
                 const float r2[2] = {rinv4[0], rinv4[1]};
                 const bool is_k = ntf * 32 < a.kv_col0 + a.kv_gd;
@@ -1222,6 +1284,10 @@ __device__ __forceinline__ void big_gemm_store(const BigArgs& a, floatx16 (&acc)
                                     for (int e = 0; e < 4; ++e) if (c0 + e < a.n_valid) xd[e] = xg[e];
                                 }
                             }
+                        }
+                        if (EPI == BEPI_F32_BIAS && a.kcache && c0 >= a.kv_col0) {
+                            if (c0 < a.n_valid) kv_scatter4(a, row, c0, s);
+                            continue;
                         }
                         float* dst = a.out + row * a.ld_out + c0;
                         if (vec_ok && c0 + 3 < a.n_valid) *(floatx4*)dst = s;
@@ -1875,6 +1941,10 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
             if (EPI == BEPI_RESID) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s[e] = s[e] + old[q][e];
+            }
+            if (EPI == BEPI_F32_BIAS && a.kcache && c0 >= a.kv_col0) {
+                if (ok && c0 < a.n_valid) kv_scatter4(a, row, c0, s);
+                continue;
             }
             if (ok) {
                 float* dst = a.out + row * a.ld_out + c0;
@@ -2804,21 +2874,6 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
         AT* out = (AT*)a.out + (long)b * a.ld_out + kvh * G * D;
         for (int idx = t; idx < G * D; idx += NTH) out[idx] = (AT)sm.out[idx];
     }
-}
-
-// Fragment-major KV cache of the MFMA attention kernels (fp16, head_dim 64 or 128).  Positions are grouped in chunks
-// of 32; within a chunk every 1 KiB block is exactly one A operand of v_mfma_f32_16x16x32_f16 (64 lanes x 8 halfs),
-// so a wavefront's load instruction reads 1 KiB contiguous.
-//   keys:   block (chunk, tile, kd), lane r + 16 qq holds K[t = 32 chunk + 8 (r / 4) + 4 tile + r % 4][d = 32 kd + 8 qq + j]
-//   values: block (chunk, dt),       lane r + 16 qq holds V[t = 32 chunk + 8 qq + j][d = 16 dt + r]
-__host__ __device__ inline long kfrag_index(int t, int d, int D) {
-    const int c = t >> 5, tin = t & 31, q8 = tin >> 3, rem = tin & 7, tile = rem >> 2, r = 4 * q8 + (rem & 3);
-    const int kd = d >> 5, qq = (d & 31) >> 3, j = d & 7;
-    return ((((long)c * 2 + tile) * (D / 32) + kd) * 64 + r + 16 * qq) * 8 + j;
-}
-__host__ __device__ inline long vfrag_index(int t, int d, int D) {
-    const int c = t >> 5, qq = (t & 31) >> 3, j = t & 7;
-    return (((long)c * (D / 16) + (d >> 4)) * 64 + (d & 15) + 16 * qq) * 8 + j;
 }
 
 // prefill, step 1: grid (Tq, batch).  Rotates the keys of every position and writes keys and values into the cache.
