@@ -1456,8 +1456,8 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     rn.x = px.as<float>(); rn.ldx = h; rn.h = h; rn.eps = c.norm_eps; rn.norm_type = c.norm_type;
     rn.xn = pxn.p; rn.ldxn = m->ldh;
     // Deferred RMSNorm (fp16 RMSNorm models, from 512 rows on): no norm kernels.  The producer of the residual stream
-    // stores half(gamma * x) and per-(32-column tile, row) sums of squares, a one-thread-per-row kernel turns those into
-    // 1 / rms, and the consuming GEMMs scale their output rows by it.  half(gamma * x) is infinite from 65504 on; prompts of
+    // stores half(gamma * x) and per-(32-column tile, row) sums of squares, the consuming GEMMs or a one-thread-per-row kernel in
+    // front of them (forms_rms) turn those into 1 / rms, and the consuming GEMMs scale their output rows by it.  half(gamma * x) is infinite from 65504 on; prompts of
     // fewer rows keep the norm kernels, which store normalised rows whatever the residual's size, in as many launches.
     const bool deferred = m->fused_norm && !m->ln && R >= 512;
     const int NTh = (int)(round_up(h, 32) / 32);

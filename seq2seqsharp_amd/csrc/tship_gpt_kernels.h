@@ -1629,7 +1629,7 @@ WideGemm wide_gemm(int tile, int epi);
 // 64 WR rows x 32 NJ columns, eight wavefronts: a wavefront owns 64 rows x all the columns (NJ x 2 MFMA tiles of 32 x 32), and
 // the KG = 8 / WR wavefronts of a row group take the k-tiles in turn, so that a small tile still has two wavefronts per SIMD
 // and the fragment reads of a large one (NJ + 2 per 2 NJ MFMAs).  Staging, waits and the half-period offset between the two
-// wavefronts of a SIMD are those of big_gemm3_f16_kernel; a stage is KG k-tiles (a row's 128 or 256 contiguous bytes of
+// wavefronts of a SIMD are those of big_gemm3_f16_kernel; a stage is KG k-tiles, or 2 KG (a row's 128 or 256 contiguous bytes of
 // activations: whole lines).  The KG partial accumulators cross through the dead stages at the end, so outputs leave in line
 // layout.  Any number of k-tiles (those beyond the last are fetched again and not multiplied); rows and columns beyond the
 // matrix are clamped on load and dropped on store.
