@@ -273,6 +273,7 @@ TSHIP_API int TSHip_GptStepBytes(TSHipGpt* m, int batch, double* weight_bytes, d
  * TSHip_GptGenerate*, TSHip_GptProfileDecode call; a value outside the listed ones makes the call fail).  None of them
  * changes results beyond what the tests that use them state; production runs set none.
  *   TSHIP_NO_GRAPH=1          the generate loop launches its kernels one by one instead of replaying a captured HIP graph
+ *   TSHIP_FAIL_STEPS_GRAPH=1  the generate loop's graph of eight steps counts as one that cannot be made; the graph of one step serves
  *   TSHIP_ATTN_SPLITS=n       decode attention: n blocks per (sequence, KV head) pair (default: chosen from the batch and context)
  *   TSHIP_FFN_TILES=10|15|20|30|40   decode FFN up projection: column tiles per block x 10 (15 = a tile and a half)
  *   TSHIP_GEMM_TILE=0|11|12|14|22|24|42|43|45   prefill GEMMs: tile of mid_gemm_f16_kernel (10 x 64-row groups + 32-column tiles), 0 = the

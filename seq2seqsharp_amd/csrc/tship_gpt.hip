@@ -137,17 +137,17 @@ struct TSHipGpt {
     long ML = 0;                   // cache rows per (sequence, KV head): max_seq_len rounded up to 32
     // one decode step (sample + decode) captured as a HIP graph; valid for one (batch, sampling mode) at a time
     hipGraphExec_t step_graph = nullptr;
-    // The same for GRAPH_STEPS steps, captured once the graph of one has run GRAPH_STEPS_AFTER times: between two launches of a graph the GPU
-    // idles for 8.5 us, inside one for none; a capture takes the host longer than that saves in a first call.
-    // ms for 32 tokens of the small fp32 model (one row) 5.47 -> 5.32 and of the 768-wide fp16 one (8 rows) 11.44 -> 11.31, 16 of the 1B model (32
-    // rows) 14.21 -> 14.14.
-    static constexpr int GRAPH_STEPS = 8, GRAPH_STEPS_AFTER = 64;
+    // The same for GRAPH_STEPS steps: between two launches of a graph the GPU idles for 8.5 us, inside one for none.  A capture of eight steps
+    // takes the host 0.8 to 1.9 ms, two to five steps' time on the GPU.  It is made behind the launch of a call's GRAPH_STEPS_AHEAD-th single step,
+    // while the GPU works through those: there the host would wait for it anyway.  Its first launch costs 0.1 ms more than later ones, 25 steps' gain
+    // (the 768-wide fp32 model with two rows, 24 / 32 tokens 8.62 / 11.29 -> 8.69 / 11.38 ms with it), so a call has to have GRAPH_STEPS_FIRST steps left for it.
+    static constexpr int GRAPH_STEPS = 8, GRAPH_STEPS_AHEAD = 16, GRAPH_STEPS_FIRST = 32;
     hipGraphExec_t steps_graph = nullptr;
-    int graph_steps_run = 0;
+    bool steps_graph_failed = false, steps_graph_ran = false;      // (failed: could not be made; the single step's graph serves until both are dropped)
     void drop_graphs() {
         if (step_graph) (void)hipGraphExecDestroy(step_graph);
         if (steps_graph) (void)hipGraphExecDestroy(steps_graph);
-        step_graph = steps_graph = nullptr; graph_steps_run = 0;
+        step_graph = steps_graph = nullptr; steps_graph_failed = steps_graph_ran = false;
     }
     int graph_batch = 0, graph_mode = -1; float graph_top_p = 0.0f, graph_temp = 0.0f;
     const float* graph_uniforms = nullptr; int* graph_gen = nullptr;
@@ -207,6 +207,7 @@ struct TestHooks {
     int moe_rest = 0;         // TSHIP_MOE_REST: tile of a launch of its own for the experts' last rows (see run_packed_gemm)
     bool record_symbols = false;      // TSHIP_RECORD_SYMBOLS: TSHip_GptProfileSymbols gives the kernels launched since the last prefill began
     bool no_graph = false;    // TSHIP_NO_GRAPH: the generate loop launches its kernels one by one
+    bool fail_steps_graph = false;    // TSHIP_FAIL_STEPS_GRAPH: the graph of several steps counts as one that cannot be made
     bool all_rows = false;    // TSHIP_GEMM_TILE, TSHIP_MOE_ROUTER_ROWS, TSHIP_MOE_REST or TSHIP_RECORD_SYMBOLS is set: the last layer of a prefill computes all rows
 };
 static TestHooks g_hooks;
@@ -243,6 +244,7 @@ static void refresh_test_hooks() {
         TSHIP_REQUIRE(h.moe_rest == 11 || h.moe_rest == 12 || h.moe_rest == 14 || h.moe_rest == 22 || h.moe_rest == 24, "TSHIP_MOE_REST: 11, 12, 14, 22 or 24");
     }
     h.no_graph = std::getenv("TSHIP_NO_GRAPH") != nullptr;
+    h.fail_steps_graph = std::getenv("TSHIP_FAIL_STEPS_GRAPH") != nullptr;
     for (const char* v : {"TSHIP_GEMM_TILE", "TSHIP_MOE_ROUTER_ROWS", "TSHIP_MOE_REST", "TSHIP_RECORD_SYMBOLS"}) h.all_rows = h.all_rows || std::getenv(v);
     g_hooks = h;
 }
@@ -2018,6 +2020,23 @@ static int generate_impl(TSHipGpt* m, int n_steps, int mode, float top_p, float 
         const size_t need = topp_scratch_bytes(m->Bpad, m->c.vocab);
         if (m->topp_scratch.bytes < need) m->topp_scratch.alloc(need);
     }
+    auto capture = [&](hipGraphExec_t& exec, int steps) {
+        hipGraph_t graph = nullptr;
+        TSHIP_CHECK_HIP(hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal));
+        const int saved_pos = m->pos;
+        try {
+            for (int s = 0; s < steps; ++s) {
+                sample_tokens(m, mode, top_p, temperature, nullptr, uni_base, B, gen.as<int>(), d_step, true, true);
+                decode_step(m, m->ids.as<int>(), B);
+            }
+        } catch (...) { hipGraph_t g2 = nullptr; (void)hipStreamEndCapture(stream(), &g2); if (g2) (void)hipGraphDestroy(g2); m->pos = saved_pos; m->embed_done = false; throw; }
+        m->pos = saved_pos;                    // capturing launched nothing
+        TSHIP_CHECK_HIP(hipStreamEndCapture(stream(), &graph));
+        const hipError_t ge = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(graph);
+        if (ge != hipSuccess) exec = nullptr;
+        TSHIP_CHECK_HIP(ge);
+    };
     if (use_graph) {
         // (sample -> decode) of one step is captured once; every replay reads the position, the step counter and the
         // token ids from device memory, so identical launches walk through the sequence
@@ -2025,30 +2044,13 @@ static int generate_impl(TSHipGpt* m, int n_steps, int mode, float top_p, float 
                               m->graph_uniforms != uni_base || m->graph_gen != gen.as<int>() || m->graph_penalty != m->repeat_penalty)) {
             m->drop_graphs();
         }
-        auto capture = [&](hipGraphExec_t& exec, int steps) {
-            hipGraph_t graph = nullptr;
+        if (!m->step_graph) {
             m->clear_counters();      // (every replay of the graph starts from what is there)
             TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
-            TSHIP_CHECK_HIP(hipStreamBeginCapture(stream(), hipStreamCaptureModeThreadLocal));
-            const int saved_pos = m->pos;
-            try {
-                for (int s = 0; s < steps; ++s) {
-                    sample_tokens(m, mode, top_p, temperature, nullptr, uni_base, B, gen.as<int>(), d_step, true, true);
-                    decode_step(m, m->ids.as<int>(), B);
-                }
-            } catch (...) { hipGraph_t g2 = nullptr; (void)hipStreamEndCapture(stream(), &g2); if (g2) (void)hipGraphDestroy(g2); m->pos = saved_pos; m->embed_done = false; throw; }
-            m->pos = saved_pos;                    // capturing launched nothing
-            TSHIP_CHECK_HIP(hipStreamEndCapture(stream(), &graph));
-            hipError_t ge = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            TSHIP_CHECK_HIP(ge);
-        };
-        if (!m->step_graph) {
             capture(m->step_graph, 1);
             m->graph_batch = B; m->graph_mode = mode; m->graph_top_p = top_p; m->graph_temp = temperature;
             m->graph_uniforms = uni_base; m->graph_gen = gen.as<int>(); m->graph_penalty = m->repeat_penalty;
         }
-        if (!m->steps_graph && eos_id < 0 && n_steps >= TSHipGpt::GRAPH_STEPS && m->graph_steps_run >= TSHipGpt::GRAPH_STEPS_AFTER) capture(m->steps_graph, TSHipGpt::GRAPH_STEPS);
     }
     struct EventPair {      // destroyed on every path out of the function
         hipEvent_t a = nullptr, b = nullptr;
@@ -2059,12 +2061,27 @@ static int generate_impl(TSHipGpt* m, int n_steps, int mode, float top_p, float 
     const hipEvent_t e0 = ev.a, e1 = ev.b;
     TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
     TSHIP_CHECK_HIP(hipEventRecord(e0, stream()));
+    // The graph of several steps, behind single ones that the GPU is still busy with (their counters are back at zero whenever a step ends).
+    // Host ms of a state's first call of 32 / 64 / 128 / 512 tokens, all of it, single steps only -> with it: the small fp32 model (one row) 5.29 / 10.36 /
+    // 20.76 / 87.1 -> 5.29 / 10.27 / 20.34 / 85.0, the 768-wide fp32 one (2 rows) 11.28 / 22.42 / 44.8 / 188.6 -> 11.32 / 22.27 / 44.5 / 187.0, the 1B one (32
+    // rows) 22.79 / 44.85 / 89.5 / 363.5 -> 22.77 / 44.95 / 89.1 / 360.4; of a later one, of 32 tokens, 5.10, 10.98 and 22.56 -> 4.97, 10.86 and 22.35.  Captured in
+    // front of a call's first step instead, that call took 0.6 to 1.6 ms longer.
+    auto capture_steps = [&]() {
+        try {
+            capture(m->steps_graph, TSHipGpt::GRAPH_STEPS);
+            if (g_hooks.fail_steps_graph) { (void)hipGraphExecDestroy(m->steps_graph); m->steps_graph = nullptr; throw Error("TSHIP_FAIL_STEPS_GRAPH"); }
+        } catch (const std::exception&) { m->steps_graph_failed = true; (void)hipGetLastError(); }
+    };
     int done = 0;
     for (int s = 0; s < n_steps; ++s) {
-        if (use_graph && eos_id < 0 && m->steps_graph && s + TSHipGpt::GRAPH_STEPS <= n_steps) {
+        if (use_graph && eos_id < 0 && m->steps_graph && n_steps - s >= (m->steps_graph_ran ? TSHipGpt::GRAPH_STEPS : TSHipGpt::GRAPH_STEPS_FIRST)) {
             TSHIP_CHECK_HIP(hipGraphLaunch(m->steps_graph, stream()));
+            m->steps_graph_ran = true;
             m->pos += TSHipGpt::GRAPH_STEPS; s += TSHipGpt::GRAPH_STEPS - 1;
-        } else if (use_graph) { TSHIP_CHECK_HIP(hipGraphLaunch(m->step_graph, stream())); m->pos += 1; m->graph_steps_run += 1; }
+        } else if (use_graph) {
+            TSHIP_CHECK_HIP(hipGraphLaunch(m->step_graph, stream())); m->pos += 1;
+            if (eos_id < 0 && s + 1 == TSHipGpt::GRAPH_STEPS_AHEAD && n_steps >= TSHipGpt::GRAPH_STEPS_FIRST && !m->steps_graph && !m->steps_graph_failed) capture_steps();
+        }
         else {
             sample_tokens(m, mode, top_p, temperature, nullptr, uni_base, B, gen.as<int>(), d_step, true, true);
             decode_step(m, m->ids.as<int>(), B);

@@ -1,5 +1,5 @@
-"""Token loops long enough for the captured graph of several steps (from 64 steps of a loop on, eight at a time): the tokens and
-logits of steps launched one by one."""
+"""Token loops long enough for the captured graph of eight steps, which a call of 32 steps or more makes behind its sixteenth and
+which runs from the first call on that has 32 left: the tokens and logits of steps launched one by one."""
 import numpy as np
 import pytest
 
@@ -18,8 +18,9 @@ def G():
                                                       ("f16", synth.LAYERNORM, 4, 4)])
 @pytest.mark.parametrize("sampled", [False, True])
 def test_loops_of_many_steps(G, monkeypatch, dtype, norm, batch, experts, sampled):
-    """Loops below, at and between multiples of eight steps, with a rewind, single steps, a loop that looks for an end token and
-    blocked tokens (which drop the graphs) between them."""
+    """Loops that make the long graph and run it at once (64), make it and leave it to a later one (32, 47), are too short (31), and find it
+    there, below, at and between multiples of eight steps; a rewind, single steps, a loop that looks for an end token and blocked tokens
+    (which drop the graphs) between them; the same where the long graph cannot be made."""
     cfg = synth.tiny_config(n_layers=3, dtype=dtype, norm_type=norm, n_experts=experts, experts_per_token=min(2, experts), batch=batch, prompt=8, vocab=300,
                              act=synth.RELU if experts > 1 else synth.SWIGLU)
     w = synth.make_weights(cfg, 101, random_bias=True)
@@ -42,13 +43,22 @@ def test_loops_of_many_steps(G, monkeypatch, dtype, norm, batch, experts, sample
         gpu.decode((np.arange(batch) + 4).astype(np.int32))
         out += [loop(19), loop(9, until=2), loop(16)]
         gpu.set_blocked_tokens([5, 6, 7])
-        out += [loop(17)]
+        out += [loop(31), loop(20)]
+        for n, later in ((32, 33), (47, 9)):
+            gpu.set_blocked_tokens([])
+            gpu.set_seq_len(batch, 40)
+            gpu.decode((np.arange(batch) + 4).astype(np.int32))
+            out += [loop(n), loop(later), loop(10)]
+            gpu.set_blocked_tokens([5])
         return out
 
     first, second = run(), run()
+    monkeypatch.setenv("TSHIP_FAIL_STEPS_GRAPH", "1")
+    gpu.set_blocked_tokens([5])
+    without = run()
     monkeypatch.setenv("TSHIP_NO_GRAPH", "1")
     want = run()
-    for got in (first, second):
+    for got in (first, second, without):
         for (a, la), (b, lb) in zip(got, want):
             assert np.array_equal(a, b) and np.array_equal(la, lb)
     gpu.close()
