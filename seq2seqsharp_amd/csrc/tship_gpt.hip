@@ -1644,6 +1644,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         ResidNormArgs a = rn;
         a.row_map = rowmap.as<int>(); a.xn = m->xn.p; a.ldxn = m->ldh; a.xn_kt = m->f16 ? (int)(m->ldh / 16) : 0;
         a.gamma = m->fn_g.as<float>(); a.beta = m->fn_b.as<float>();
+        if (m->fused_norm) a.x_rows = m->x.as<float>();      // (LayerNorm: TSHip_GptGetHidden reads the residual stream of the rows there)
         run_resid_norm(m, "p_final_norm", B, a);
     }
     const long Vp = round_up(c.vocab, 32);

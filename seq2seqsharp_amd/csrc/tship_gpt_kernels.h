@@ -2237,6 +2237,7 @@ struct ResidNormArgs {
     void* xn; long ldxn;
     int xn_kt;              // > 0 (fp16 only): xn is fragment packed with this many k-tiles; 0: row-major with ldxn
     const int* row_map;     // optional: block r works on row row_map[r] of x and writes row r of xn
+    float* x_rows;          // optional: row r of x (as it is behind this kernel) also goes to row r of [rows][h]
     int* advance_pos;       // optional: block 0 increments this device counter (end of a decode step)
     // optional source: x += the MoE experts' outputs, each scaled by its router probability and added in expert order
     // (MoEFeedForward.cs:167-178; IndexSelectGrad, TensorApplyCPU.cs:1336-1356).  y[e][slot][col], slot[row * k + j] =
@@ -2369,6 +2370,7 @@ __global__ __launch_bounds__(256) void resid_norm_kernel(ResidNormArgs a) {
         int c = t + i * 256;
         if (c < a.h) {
             if (a.ids || part || a.moe_y) a.x[xr * a.ldx + c] = v[i];
+            if (a.x_rows) a.x_rows[(long)r * a.h + c] = v[i];
             sum += v[i]; sq += v[i] * v[i];
         }
     }
