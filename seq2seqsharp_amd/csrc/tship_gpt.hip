@@ -121,7 +121,7 @@ struct TSHipGpt {
 
     // decode state
     DevBuf x, xn, o, a, part_qkv, part_h, part_f, logits, ids, d_pos, hidden;
-    DevBuf moe_ws, topp_scratch, topp_uni, gen_buf, uni_buf, tile_count;
+    DevBuf moe_ws, moe_zero_bias, topp_scratch, topp_uni, gen_buf, uni_buf, tile_count;
     DevBuf pw_lens, pw_ids, pw_x, pw_xn, pw_qkv, pw_o, pw_a, pw_f, pw_rowmap, pw_ssq, pw_rinv, pw_zero_bias, pw_moe;     // prefill workspace
     DevBuf xn_rows, o_rows, a_rows, zero_qkv; // row-major activations of models that step by rows (xn, and o and a of the other models, hold packed ones)
     // prefill GEMMs whose tiles' K several blocks share: partial sums of up to 256 tiles x splits of 128 x 128, a counter per tile

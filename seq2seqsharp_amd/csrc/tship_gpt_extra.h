@@ -5,7 +5,7 @@
 namespace tship {
 
 struct MoeLayout {
-    size_t xn32, probs, top_val, top_idx, counts, lists, slot, xg, mid, y, zero, total;
+    size_t xn32, probs, top_val, top_idx, counts, lists, slot, xg, mid, y, total;
     long ld4h, ldy;
 };
 
@@ -21,7 +21,6 @@ static MoeLayout moe_layout(TSHipGpt* m, long cap) {
     o.xg = take(E * Bp * m->ldh * m->esz());
     o.mid = take(E * Bp * o.ld4h * m->esz());
     o.y = take(E * Bp * o.ldy * 4);
-    o.zero = take(std::max<long>(4 * h, 64) * 4);
     o.total = at;
     return o;
 }
@@ -29,6 +28,7 @@ static MoeLayout moe_layout(TSHipGpt* m, long cap) {
 static void moe_alloc(TSHipGpt* m) {
     TSHIP_REQUIRE(m->c.hidden <= 4096, "TSHip_GptCreate: MoE layers support hidden up to 4096");
     m->moe_ws.alloc(moe_layout(m, m->Bpad).total);
+    m->moe_zero_bias.alloc((size_t)std::max<long>(4L * m->c.hidden, 64) * sizeof(float));
     // the experts' row counters start at zero and every layer's combine kernel leaves them so (the fp16 router adds to them)
     TSHIP_CHECK_HIP(hipMemsetAsync(m->moe_ws.p, 0, m->moe_ws.bytes, stream()));
 }
@@ -67,7 +67,9 @@ static void run_moe_ffn_impl(TSHipGpt* m, LayerW& L, int rows, const ResidNormAr
     float* top_val = batched ? (float*)(base + o.top_val) : lroute + (size_t)m->Bpad * E;
     float* top_idx = batched ? (float*)(base + o.top_idx) : lroute + (size_t)m->Bpad * (E + k);
     int* counts = (int*)(base + o.counts); int* lists = (int*)(base + o.lists); int* slot = (int*)(base + o.slot);
-    float* y = (float*)(base + o.y); float* zero = (float*)(base + o.zero);
+    float* y = (float*)(base + o.y);
+    // the experts have no biases.  (Not in the workspace: a prompt of another size lays that out anew and finds the last one's data there.)
+    const float* zero = m->moe_zero_bias.as<float>();
 
     MoeRouterArgs r; std::memset(&r, 0, sizeof(r));
     r.x = pre.x; r.ldx = pre.ldx; r.h = h;
