@@ -282,8 +282,8 @@ TSHIP_API int TSHip_GptStepBytes(TSHipGpt* m, int batch, double* weight_bytes, d
  *   TSHIP_F32_TILE=11|21|22|42    fp32 GEMMs from 33 rows on: tile in units of 32 rows (10 x) and 32 columns (default: by size)
  *   TSHIP_F32_ATTN=0|1        attention of fp32 prefills: a block per query, or tiles of 32 columns (default: by estimated time)
  *   TSHIP_RECORD_SYMBOLS=1    TSHip_GptProfileSymbols gives the kernels launched since the last prefill began
- *                             (with it, TSHIP_GEMM_TILE, TSHIP_MOE_ROUTER_ROWS or TSHIP_MOE_REST the last layer of a prefill computes all its
- *                             rows; otherwise, behind its keys and values, those of the last positions, which are all that is read)
+ *   TSHIP_ALL_ROWS=1          the last layer of a prefill computes all its rows, as the others do (default: behind its keys and values, those
+ *                             of the last positions, which are all that is read)
  *   TSHIP_PATCH_ROWS=1|2|4|8  prefill GEMM: most row tiles of a band of tiles
  *   TSHIP_ATTN_NQ=1|2         prefill attention: groups of 16 MFMA columns per wavefront
  *   TSHIP_NO_KV_FUSE=1        prefill: the QKV projection leaves the cache write to a kernel of its own (so does TSHIP_GEMM_TILE=0 where

@@ -208,7 +208,7 @@ struct TestHooks {
     bool record_symbols = false;      // TSHIP_RECORD_SYMBOLS: TSHip_GptProfileSymbols gives the kernels launched since the last prefill began
     bool no_graph = false;    // TSHIP_NO_GRAPH: the generate loop launches its kernels one by one
     bool fail_steps_graph = false;    // TSHIP_FAIL_STEPS_GRAPH: the graph of several steps counts as one that cannot be made
-    bool all_rows = false;    // TSHIP_GEMM_TILE, TSHIP_MOE_ROUTER_ROWS, TSHIP_MOE_REST or TSHIP_RECORD_SYMBOLS is set: the last layer of a prefill computes all rows
+    bool all_rows = false;    // TSHIP_ALL_ROWS: the last layer of a prefill computes all rows
 };
 static TestHooks g_hooks;
 static void refresh_test_hooks() {
@@ -245,7 +245,7 @@ static void refresh_test_hooks() {
     }
     h.no_graph = std::getenv("TSHIP_NO_GRAPH") != nullptr;
     h.fail_steps_graph = std::getenv("TSHIP_FAIL_STEPS_GRAPH") != nullptr;
-    for (const char* v : {"TSHIP_GEMM_TILE", "TSHIP_MOE_ROUTER_ROWS", "TSHIP_MOE_REST", "TSHIP_RECORD_SYMBOLS"}) h.all_rows = h.all_rows || std::getenv(v);
+    h.all_rows = std::getenv("TSHIP_ALL_ROWS") != nullptr;
     g_hooks = h;
 }
 
@@ -1524,9 +1524,8 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     };
     // Behind the last layer's keys and values only the last position of every sequence is needed: the attention of the blocks that hold
     // them, and the output projection and feed-forward of those B rows, which lie Tp rows apart in po and px and close together in what
-    // follows; nothing else of the layer is ever read.  (Not where a test forces or records kernels: those tests are about all rows of all
-    // layers.)  ms per prompt, all rows -> these: 1B model (16 layers) 32 x 1024 49.9 -> 47.2, 5 x 333 3.55 -> 3.47; 8 layers of the 7B one, 8000
-    // positions 27.3 -> 24.5; 12-layer mixture of experts, 64 x 256 10.2 -> 9.5.
+    // follows; nothing else of the layer is ever read.  ms per prompt, all rows (TSHIP_ALL_ROWS) -> these: 1B model (16 layers) 32 x 1024
+    // 49.9 -> 47.2, 5 x 333 3.55 -> 3.47; 8 layers of the 7B one, 8000 positions 27.3 -> 24.5; 12-layer mixture of experts, 64 x 256 10.2 -> 9.5.
     const bool last_rows_only = Tp > 1 && !g_hooks.all_rows && (long)Tp * std::max<long>(m->ldh, h) <= INT32_MAX;
     for (int l = 0; l < c.n_layers; ++l) {
         LayerW& L = *m->L[l];

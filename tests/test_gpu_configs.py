@@ -347,6 +347,7 @@ def large_tile(monkeypatch):
     """The 256 x 256 tile of the prefill GEMMs, which prompts of these tests' sizes do not take by themselves, and a check
     of the kernels that the last prefill launched."""
     monkeypatch.setenv("TSHIP_GEMM_TILE", "0")
+    monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
 
     def launched(gpu, cache_write=None):

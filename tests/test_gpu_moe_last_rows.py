@@ -20,7 +20,8 @@ def G():
                                                                 (4, 2, 2, 256, (60.0, 0.0, 0.0, 0.0)), (4, 2, 3, 200, (-60.0, 0.0, 0.0, 0.0))])
 @pytest.mark.parametrize("tile", [11, 12, 14, 22, 24, None])
 def test_last_rows_by_themselves(G, oracle, monkeypatch, experts, k, batch, prompt, router_bias, tile):
-    cfg = synth.tiny_config(n_layers=3, n_experts=experts, experts_per_token=k, norm_type=synth.LAYERNORM, act=synth.RELU, dtype="f16",
+    """In the third layer of four (the last one computes the last positions only, as a decode step)."""
+    cfg = synth.tiny_config(n_layers=4, n_experts=experts, experts_per_token=k, norm_type=synth.LAYERNORM, act=synth.RELU, dtype="f16",
                             batch=batch, prompt=prompt, vocab=300)
     w = synth.make_weights(cfg, 62, random_bias=True)
     if router_bias is not None:
@@ -48,6 +49,7 @@ def test_router_of_many_rows(G, oracle, monkeypatch, hidden, heads, kv, experts,
                             act=synth.RELU, dtype="f16", batch=batch, prompt=prompt, vocab=100)
     w = synth.make_weights(cfg, 63, random_bias=True)
     monkeypatch.setenv("TSHIP_MOE_ROUTER_ROWS", "0")
+    monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
     seqs = synth.make_prompts(cfg, 163)
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 10)

@@ -105,6 +105,7 @@ def test_columns_in_two_launches(G, monkeypatch, norm, act, batch, prompt):
                      batch=batch, prompt=prompt, steps=2, dtype="f16")
     w = synth.make_weights(cfg, 91, random_bias=True)
     seqs = synth.make_prompts(cfg, 92)
+    monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
     got = []

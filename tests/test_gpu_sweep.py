@@ -205,6 +205,7 @@ def test_large_prefill_paths_agree_bit_for_bit(monkeypatch, seed):
     seqs = synth.make_prompts(cfg, 200 + seed)
     gpu = G.HipGpt(cfg, w, max_batch=cfg["batch"], max_seq_len=cfg["prompt"] + 8)
     monkeypatch.setenv("TSHIP_GEMM_TILE", "0")
+    monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
 
     def launched(cache_write):

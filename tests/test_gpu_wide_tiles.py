@@ -39,6 +39,7 @@ def test_widths_of_the_256_row_tile(G, oracle, monkeypatch, shape, batch, prompt
     seqs = synth.make_prompts(cfg, 52)
     orc = oracle.OracleGpt(cfg, w)
     _, lg = orc.step(seqs, use_cache=True)
+    monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 8)
     for tile in (0, 42, 43, 45):
@@ -69,6 +70,7 @@ def test_experts_with_each_width(G, oracle, monkeypatch, experts, k, batch, prom
     orc = oracle.OracleGpt(cfg, w)
     _, lg = orc.step(seqs, use_cache=True)
     monkeypatch.setenv("TSHIP_GEMM_TILE", str(tile))
+    monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 10)
     gpu.prefill(seqs)
     assert np.abs(gpu.logits() - lg).max() <= 3e-2        # (the bar of the other MoE prefill tests)
