@@ -366,8 +366,8 @@ def test_moe_prefill_runs_the_experts_on_gathered_rows(G, oracle, dtype, batch, 
     rows gathered for it (about 660 rows per expert in the first case: one launch for all experts; fewer than 512 in the
     others: one per expert), and the scaled outputs are added back in expert order.  Logits of the last position and the routing of the
     last position against the oracle, then decode steps on top of the cache the prefill wrote."""
-    cfg = synth.tiny_config(n_layers=3, n_experts=4, experts_per_token=2, norm_type=synth.LAYERNORM, act=synth.RELU, dtype=dtype,
-                            batch=batch, prompt=prompt, vocab=300)
+    cfg = synth.tiny_config(n_layers=4, n_experts=4, experts_per_token=2, norm_type=synth.LAYERNORM, act=synth.RELU, dtype=dtype,
+                            batch=batch, prompt=prompt, vocab=300)      # (the third layer; the last one computes the last positions only)
     orc, gpu, out, cur = _teacher_forced(G, oracle, cfg, 61, 3)
     for lg, gl in out:
         if dtype == "f32":
@@ -377,10 +377,11 @@ def test_moe_prefill_runs_the_experts_on_gathered_rows(G, oracle, dtype, batch, 
     if dtype == "f32":
         gpu.reset()
         gpu.prefill(cur)
-        ti, tv, pr = gpu.moe_routing(2)                      # last MoE layer, last position of every sequence
-        oi, ov, op = orc.moe_trace(0, batch)
-        assert np.array_equal(ti, oi)
-        assert np.allclose(pr, op, rtol=1e-6)
+        for layer in (2, 3):                                 # the last position of every sequence
+            ti, tv, pr = gpu.moe_routing(layer)
+            oi, ov, op = orc.moe_trace(layer - 2, batch)
+            assert np.array_equal(ti, oi)
+            assert np.allclose(pr, op, rtol=1e-6)
     gpu.close()
 
 
@@ -658,8 +659,10 @@ def test_moe_prefill_one_launch_for_all_experts_equals_one_per_expert(G, oracle,
     pointer table, the problem of a tile found on the device from the counts), and the up projection reads its rows
     through the token lists.  Same logits, bit for bit, as the path with the counts on the host, gathered rows and one
     launch per expert (TSHIP_NO_MOE_BATCH=1): with an expert that holds far fewer rows than the largest one, one with no
-    rows at all, one with every row, and row counts that fill no tile.  And the logits against the oracle."""
-    cfg = synth.tiny_config(n_layers=3, n_experts=experts, experts_per_token=k, norm_type=synth.LAYERNORM, act=synth.RELU, dtype="f16",
+    rows at all, one with every row, and row counts that fill no tile.  And the logits against the oracle.  (In the third layer of
+    four: the keys and values of the last one follow from all its rows.)"""
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
+    cfg = synth.tiny_config(n_layers=4, n_experts=experts, experts_per_token=k, norm_type=synth.LAYERNORM, act=synth.RELU, dtype="f16",
                             batch=batch, prompt=prompt, vocab=300)
     w = synth.make_weights(cfg, 62, random_bias=True)
     if router_bias is not None:
@@ -668,7 +671,8 @@ def test_moe_prefill_one_launch_for_all_experts_equals_one_per_expert(G, oracle,
     seqs = synth.make_prompts(cfg, 162)
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 10)
     gpu.prefill(seqs)
-    one = gpu.logits()
+    one, cache = gpu.logits(), [gpu.get_kv(3, i) for i in range(2)]
+    assert not any("moe_gather_kernel" in s for s in gpu.profile_symbols())
     if router_bias is not None:
         ti, _, _ = gpu.moe_routing(2)
         assert (ti == 0).any(axis=1).all() if router_bias[0] > 0 else not (ti == 0).any()
@@ -676,7 +680,8 @@ def test_moe_prefill_one_launch_for_all_experts_equals_one_per_expert(G, oracle,
     gpu.reset()
     gpu.prefill(seqs)
     monkeypatch.delenv("TSHIP_NO_MOE_BATCH")
-    assert np.array_equal(one, gpu.logits())
+    assert any("moe_gather_kernel" in s for s in gpu.profile_symbols())
+    assert np.array_equal(one, gpu.logits()) and all(np.array_equal(cache[i], gpu.get_kv(3, i)) for i in range(2))
     _, lg = oracle.OracleGpt(cfg, w).step(seqs, use_cache=True)
     assert np.abs(one - lg).max() <= FP16_ABS
     gpu.close()
