@@ -1512,7 +1512,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         }
         fuse_kv = can_fuse_kv && !qkv_tiles.tile && !qkv_tiles.cols && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
         // (any other tile and prompt length: in pieces, BigArgs::kv_scatter; the kernel of its own is left to the tests that compare with it)
-        scatter_kv = m->vt && !fuse_kv && g_hooks.gemm_tile != 0 && !g_hooks.no_kv_fuse;
+        scatter_kv = m->vt && !fuse_kv && !g_hooks.no_kv_fuse;
         wo_tiles = pick_gemm_mix(L.wo, R); w13_tiles = pick_gemm_mix(L.w13, R); w2_tiles = pick_gemm_mix(L.w2, R);
     }
     // 1 / rms of a deferred norm: from the tile sums, by the consuming projection itself or by a kernel in front of it

@@ -30,7 +30,8 @@ def test_cache_in_pieces(G, monkeypatch, shape, batch, prompt, context):
     seqs = synth.make_prompts(cfg, 112)
     longer = np.random.default_rng(113).integers(4, 157, size=(batch, context + prompt + 40)).astype(np.int32)
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=context + prompt + 48)
-    for tile in (None, "11", "14", "222", "24", "42", "43", "45"):
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
+    for tile in (None, "0", "11", "14", "222", "24", "42", "43", "45"):
         if tile:
             monkeypatch.setenv("TSHIP_GEMM_TILE", tile)
         got = []
@@ -43,6 +44,7 @@ def test_cache_in_pieces(G, monkeypatch, shape, batch, prompt, context):
             if context:
                 gpu.prefill(seqs[:, :context])
             gpu.prefill(seqs[:, context:])
+            assert any("kv_write" in s for s in gpu.profile_symbols()) == separate, tile
             out = [gpu.logits()] + [gpu.get_kv(l, i) for l in range(2) for i in range(2)]
             for _ in range(2):
                 gpu.decode((np.arange(batch) + 5).astype(np.int32))
