@@ -617,7 +617,7 @@ static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const fl
 // (L2, HBM, power).  A launch that leaves half of the units idle may have up to four blocks share the K of a tile (100 x their
 // number in the result); the exchange costs 1.2 us, a little per block and 0.7 us per 64 x 32 values of the tile that each
 // block stores and the last one adds.
-// own_cache_write: us that a launch saves with the 256 x 256 tile, which can write the key-value cache itself.
+// whole_saves: us that the 256 x 256 tile is credited with, which can write whole fragments of the key-value cache (see prefill).
 // a, b and the exchange are fits to 8707 times (33 ... 16384 rows, 27 pairs of K and N from 128 to 22016, every tile and
 // split; profiles/prefill_gemm_tiles.txt): over the best tile of each of the 916 sizes the choice costs 0.6 % on average,
 // more than 15 % in 9.  Without the exchange's growth with the tile it was 2.5 % and 53: 4096 x 1024 at 1024 rows 27.5 us for 17.5.
@@ -655,7 +655,7 @@ static float gemm_tile_us(const GemmCost& c, int KT, long n_tiles, int splits) {
     return us;
 }
 // (all_widths: false leaves out the 256-row tiles of other widths than 256)
-static GemmTile best_gemm_tile(int KT, int NT, long R, float own_cache_write = 0.0f, bool all_widths = true) {
+static GemmTile best_gemm_tile(int KT, int NT, long R, float whole_saves = 0.0f, bool all_widths = true) {
     GemmTile best = {111, 1e30f};
     for (const GemmCost& c : gemm_costs()) {
         if (!gemm_tile_takes(c, KT, R) || (!all_widths && is_wide_tile(gemm_tile_code(c)))) continue;
@@ -663,7 +663,7 @@ static GemmTile best_gemm_tile(int KT, int NT, long R, float own_cache_write = 0
         for (int splits = 1; splits <= (c.tile ? MID_SPLITS : 1); ++splits) {
             if (mid_splits(KT, c.tile, splits) != splits || (splits > 1 && (n_tiles * splits > TSHipGpt::MID_XCHG_TILES || n_tiles * splits > n_compute_units()))) continue;
             const int code = gemm_tile_code(c);
-            const float us = gemm_tile_us(c, KT, n_tiles, splits) - (code == 0 ? own_cache_write : 0.0f);
+            const float us = gemm_tile_us(c, KT, n_tiles, splits) - (code == 0 ? whole_saves : 0.0f);
             if (us < best.us) best = {c.tile ? code + 100 * splits : code, us};
         }
     }
@@ -1493,25 +1493,25 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
     DevBuf& zero_bias = m->pw_zero_bias; zero_bias.reserve((size_t)std::max<long>(std::max<long>(qp, m->F13), round_up(h, 32)) * sizeof(float));
     // Tiles of the projections, chosen once for all layers (layer 0 has them all, and the others' shapes): a choice takes the host up to
     // 3 us (five of them in every layer before: three layers of the 1B model at 100 / 333 / 1500 rows 256 / 378 / 784 -> 249 / 374 / 764 us).
-    // The QKV projection with 256 x 256 tiles can write keys and values into the fragment-major cache itself (rotation
-    // included) when its wavefronts' 64 x 128 tiles are whole chunks of whole heads.  That takes it about 7.5 us longer and
-    // saves a kernel whose time goes with rows x columns of keys and values (profiles/prefill_gemm_tiles.txt: 1024 columns,
-    // 1024 rows 49.0 + 7.4 against 62.5 us, 16384 rows 202 + 37 against 211); elsewhere the tile with the least time writes it in pieces.
+    // Every tile of the QKV projection writes keys and values into the fragment-major cache, rotation included: the 256 x 256 one as
+    // whole fragments where its wavefronts' 64 x 128 tiles are whole chunks of whole heads, the others in pieces (BigArgs::kv_scatter).  With the same
+    // tile pieces take 4 us longer and 0.44 us per million keys and values (183 sizes, profiles/prefill_qkv_cache_write.txt); against other tiles
+    // whole fragments are worth more where there are many, as a launch of several rounds with pieces takes longer than its estimate: 1.6 us per
+    // million less 8.  The choice with that loses 85 us over those launches, always whole fragments 1090, never 1157, 1.9 less 7.5 135.
     const int HD = c.n_heads * m->D, GD = c.n_kv_heads * m->D;
     GemmMix qkv_tiles = {}, wo_tiles = {}, w13_tiles = {}, w2_tiles = {};
     bool fuse_kv = false, scatter_kv = false;
     if (m->f16) {
         const LayerW& L = *m->L[0];
         const bool can_fuse_kv = m->vt && pos0 % 32 == 0 && Tp % 32 == 0 && HD % 128 == 0 && GD % 128 == 0 && L.qkv.KT % 2 == 0 && (m->D == 64 || m->D == 128);
-        const float fuse_saves = 1.9e-6f * (float)(R * 2 * GD) - 7.5f;
-        const float own_write = can_fuse_kv ? std::max(0.0f, fuse_saves) : 0.0f;
+        const float whole_saves = can_fuse_kv ? std::max(0.0f, 1.6e-6f * (float)(R * 2 * GD) - 8.0f) : 0.0f;
         qkv_tiles = pick_gemm_mix(L.qkv, R);
-        if (g_hooks.gemm_tile < 0 && own_write > 0.0f) {      // (two launches of different tiles where that is less than the saved kernel)
-            const GemmTile one = best_gemm_tile(L.qkv.KT, L.qkv.NT, R, own_write);
+        if (g_hooks.gemm_tile < 0 && whole_saves > 0.0f) {      // (two launches of different tiles only where they are less than that one)
+            const GemmTile one = best_gemm_tile(L.qkv.KT, L.qkv.NT, R, whole_saves);
             if (!qkv_tiles.cols || qkv_tiles.us >= one.us) qkv_tiles = {one.tile, 0, 0, one.us};
         }
-        fuse_kv = can_fuse_kv && !qkv_tiles.tile && !qkv_tiles.cols && (fuse_saves > 0.0f || g_hooks.gemm_tile == 0) && !g_hooks.no_kv_fuse;
-        // (any other tile and prompt length: in pieces, BigArgs::kv_scatter; the kernel of its own is left to the tests that compare with it)
+        fuse_kv = can_fuse_kv && !qkv_tiles.tile && !qkv_tiles.cols && !g_hooks.no_kv_fuse;
+        // (kernels of their own for the cache, kv_write_frag_kernel and kv_write_kernel, are left to the tests that compare with them, TSHIP_NO_KV_FUSE)
         scatter_kv = m->vt && !fuse_kv && !g_hooks.no_kv_fuse;
         wo_tiles = pick_gemm_mix(L.wo, R); w13_tiles = pick_gemm_mix(L.w13, R); w2_tiles = pick_gemm_mix(L.w2, R);
     }
