@@ -622,7 +622,7 @@ static void run_gemm_f32(TSHipGpt* m, const char* name, const GemmW& w, const fl
 // split; profiles/prefill_gemm_tiles.txt): over the best tile of each of the 916 sizes the choice costs 0.6 % on average,
 // more than 15 % in 9.  Without the exchange's growth with the tile it was 2.5 % and 53: 4096 x 1024 at 1024 rows 27.5 us for 17.5.
 struct GemmTile { int tile; float us; };      // (tile as above, plus 100 x the blocks that share its K)
-// the most blocks up to `splits` that leave none of their ranges of whole chunks empty
+// the most blocks up to `splits` that leave none of their ranges (multiples of a k-tile per wavefront of a row group) empty
 static int mid_splits(int KT, int tile, int splits) {
     const int kg = tile >= 20 ? 4 : 8;
     while (splits > 1 && (splits - 1) * (int)ceil_div(KT, kg * splits) * kg >= KT) --splits;
@@ -1106,7 +1106,7 @@ static void decode_step_rows(TSHipGpt* m, const int* d_ids, int B) {
     const long hp = round_up(h, 32), qp = round_up(m->Nqkv, 32), Vp = round_up(c.vocab, 32);
     const int NTh = (int)(hp / 32);
     float* ssq = m->ssq.as<float>();
-    // (the 256 x 256 tile neither forms 1 / rms nor fits these row counts: pick_gemm_tile offers it from 256 rows on)
+    // (up to 128 rows: pick_gemm_tile offers the 256-row tiles from 256 on)
     auto gemm = [&](const char* name, const GemmW& w, const DevBuf& X, long ldx, int epi, BigArgs e) { run_big_gemm(m, name, w, X.p, ldx, B, epi, e, pick_gemm_tile(w, B)); };
     auto with_ssq = [&](BigArgs& e) { e.ssq = ssq; e.ssq_nt = NTh; e.ssq_in_ld = m->Bpad; e.inv_h = 1.0f / (float)h; e.eps = c.norm_eps; };
     auto resid = [&](const char* name, const GemmW& w, const DevBuf& X, long ldx, const DevBuf& bias, const DevBuf& gamma) {

@@ -1666,7 +1666,8 @@ constexpr int MID_SPLITS = 4;        // at most so many blocks share the K of a 
 // 128 x 64 tile has LDS for (three stages of 48 KiB; us at 96 rows, weights from HBM, one -> two: gated 2048 x 11264 20.2 -> 19.6, 5632 x 2048
 // 35.7 -> 34.4, 11008 x 4096 65.2 -> 62.6).  The 64 x 32 tile lost 1.5 % with two, the others have no LDS for a third stage.
 template <int WR, int NJ> struct MidShape {
-    static constexpr int KG = 8 / WR, U = NJ == 2 && WR == 2 ? 2 : 1, CK = KG * U, STAGE = CK * (NJ + 2 * WR) * 1024, NST = STAGE > 49152 ? 2 : STAGE > 40960 ? 3 : 4;
+    static constexpr int KG = 8 / WR, U = NJ == 2 && WR == 2 ? 2 : 1, CK = KG * U, STAGE = CK * (NJ + 2 * WR) * 1024, NST = STAGE > 40960 ? 3 : 4;
+    static_assert(NST * STAGE + 2048 <= 163840, "the stages and ssq_part fit a compute unit's LDS");
     static constexpr int UP = NJ == 1 ? 2 : 4, RED = 8 * UP * 32 * 36 * 4;
     static constexpr unsigned SHM = NST * STAGE > RED ? NST * STAGE : RED;
 };
@@ -1698,7 +1699,9 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
         ctile = i >> (RT - 1); rtile = i - ctile * RT;
     } else if (!xcd_tile(blockIdx.x, RT, CT, 8, rtile, ctile)) return;
     const int tile = ctile * RT + rtile;
-    // k-tiles of this block: all, or (a.splits > 1) one of as many ranges of whole chunks, blockIdx.y
+    // k-tiles of this block: all, or (a.splits > 1) one of as many ranges, blockIdx.y.  They are cut in multiples of KG, a k-tile per wavefront: the
+    // longest holds as many chunks as with a cut in CK (n KG-steps over s blocks, two to a chunk: ceil(ceil(n / s) / 2) = ceil(ceil(n / 2) / s)), and
+    // the steps are shared more evenly (16 over 3: 6, 5, 5 for 6, 6, 4)
     const int kt_per = a.splits > 1 ? ((a.KT + KG * a.splits - 1) / (KG * a.splits)) * KG : a.KT;
     const int kt_first = a.splits > 1 ? (int)blockIdx.y * kt_per : 0, kt_end = min(a.KT, kt_first + kt_per);      // (the host leaves no range empty)
     const int nt0 = ctile * NJ;
@@ -1711,7 +1714,7 @@ __global__ __launch_bounds__(512) void mid_gemm_f16_kernel(BigArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[j][i][v] = 0.0f;
 
-    // 1 KiB pieces of a stage: NJ KG weight fragments [column tile][k-tile], then 16 pieces of activations (row-major, a row's
+    // 1 KiB pieces of a stage: NJ CK weight fragments [column tile][k-tile], then 16 U pieces of activations (row-major, a row's
     // 16-byte units at position unit ^ swz(row): the fragment reads of 32 rows x 2 units then spread evenly over the banks)
     const half_t* wsrc[LW]; int wkt[LW];
 #pragma unroll
