@@ -286,7 +286,7 @@ TSHIP_API int TSHip_GptStepBytes(TSHipGpt* m, int batch, double* weight_bytes, d
  *                             of the last positions, which are all that is read)
  *   TSHIP_PATCH_ROWS=1|2|4|8  prefill GEMM: most row tiles of a band of tiles
  *   TSHIP_ATTN_NQ=1|2         prefill attention: groups of 16 MFMA columns per wavefront
- *   TSHIP_NO_KV_FUSE=1        prefill: the QKV projection leaves the cache write to a kernel of its own
+ *   TSHIP_NO_KV_FUSE=1        prefill: the QKV projection's 256 x 256 tile writes the cache in pieces, as the others do, instead of whole fragments
  *   TSHIP_NO_MOE_BATCH=1      prefill of MoE layers: the experts' row counts are read back, the rows gathered and one GEMM
  *                             launched per expert, instead of one launch per projection with everything on the device
  *   TSHIP_MOE_REST=11|12|14|22|24   prefill of MoE layers: the experts' last rows (behind whole 256-row tiles) in a launch of this tile

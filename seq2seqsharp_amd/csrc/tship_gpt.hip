@@ -201,7 +201,7 @@ struct TestHooks {
     int f32_tile = 0;         // TSHIP_F32_TILE: tile of the fp32 GEMMs from 33 rows on (pick_f32_tile)
     int f32_attn = -1;        // TSHIP_F32_ATTN: attention of fp32 prefills: 0 a block per query, 1 tiles of 32 columns (f32_attn_by_query)
     int attn_nq = 0;          // TSHIP_ATTN_NQ: 1 or 2 groups of 16 MFMA columns per wavefront in prefill attention
-    bool no_kv_fuse = false;  // TSHIP_NO_KV_FUSE: the QKV projection of a prefill does not write the cache itself
+    bool no_kv_fuse = false;  // TSHIP_NO_KV_FUSE: the QKV projection of a prefill writes the cache in pieces with every tile
     bool no_moe_batch = false;// TSHIP_NO_MOE_BATCH: one prefill GEMM launch per expert
     int moe_router_rows = 1024;       // TSHIP_MOE_ROUTER_ROWS: prefills of more rows route a row per wavefront
     int moe_rest = 0;         // TSHIP_MOE_REST: tile of a launch of its own for the experts' last rows (see run_packed_gemm)
@@ -978,22 +978,21 @@ static bool f32_attn_by_query(const TSHipGpt* m, int B, int Tp, int pos0) {
     const float tiles = m->D == 128 ? 7.0f + 1.83f * steps : m->D == 64 ? 2.0f + 1.23f * steps : 1.15f * steps;
     return by_query < tiles;
 }
-template <typename CT>
-static AttnKernel pick_kvw_t(int D) {
-    switch (D) {
-        case 16: return kv_write_kernel<CT, 16>;
-        case 32: return kv_write_kernel<CT, 32>;
-        case 64: return kv_write_kernel<CT, 64>;
-        case 128: return kv_write_kernel<CT, 128>;
-        default: throw Error("head_dim must be 16, 32, 64 or 128");
+static AttnKernel pick_kvw(TSHipGpt* m) {      // (fp16 caches of head sizes 64 and 128 are fragment-major)
+    switch (m->D) {
+        case 16: return m->f16 ? kv_write_kernel<half_t, 16> : kv_write_kernel<float, 16>;
+        case 32: return m->f16 ? kv_write_kernel<half_t, 32> : kv_write_kernel<float, 32>;
+        case 64: if (!m->f16) return kv_write_kernel<float, 64>; break;
+        case 128: if (!m->f16) return kv_write_kernel<float, 128>; break;
+        default: break;
     }
+    throw Error("internal: no kernel writes a cache of this head size");
 }
-static AttnKernel pick_kvw(TSHipGpt* m) { return m->f16 ? pick_kvw_t<half_t>(m->D) : pick_kvw_t<float>(m->D); }
 
 static AttnArgs attn_args(TSHipGpt* m, LayerW& L) {
     AttnArgs a; std::memset(&a, 0, sizeof(a));
     a.bias = L.bqkv.as<float>(); a.H = m->c.n_heads; a.Hkv = m->c.n_kv_heads; a.kv_sub = m->SG;
-    a.kcache = L.kc.p; a.vcache = L.vc.p; a.max_len = m->ML; a.vt = m->vt ? 1 : 0;
+    a.kcache = L.kc.p; a.vcache = L.vc.p; a.max_len = m->ML;
     if (m->c.use_rope) { a.rope_cos = m->rope_cos.as<float>(); a.rope_sin = m->rope_sin.as<float>(); }
     a.d_pos = m->d_pos.as<int>();
     a.scale = 1.0f / (float)std::sqrt((double)m->D);   // GroupQueryAttention.cs:193
@@ -1511,8 +1510,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
             if (!qkv_tiles.cols || qkv_tiles.us >= one.us) qkv_tiles = {one.tile, 0, 0, one.us};
         }
         fuse_kv = can_fuse_kv && !qkv_tiles.tile && !qkv_tiles.cols && !g_hooks.no_kv_fuse;
-        // (kernels of their own for the cache, kv_write_frag_kernel and kv_write_kernel, are left to the tests that compare with them, TSHIP_NO_KV_FUSE)
-        scatter_kv = m->vt && !fuse_kv && !g_hooks.no_kv_fuse;
+        scatter_kv = m->vt && !fuse_kv;
         wo_tiles = pick_gemm_mix(L.wo, R); w13_tiles = pick_gemm_mix(L.w13, R); w2_tiles = pick_gemm_mix(L.w2, R);
     }
     // 1 / rms of a deferred norm: from the tile sums, by the consuming projection itself or by a kernel in front of it
@@ -1553,16 +1551,7 @@ static void prefill(TSHipGpt* m, const int32_t* host_ids, int B, int Tp, const i
         } else {
             run_gemm_f32(m, "p_gemm_qkv", L.qkv, pxn.as<float>(), m->ldh, (int)R, pqkv.as<float>(), qp, 0, 1);
         }
-        if (fuse_kv || scatter_kv) {
-            // (cache written by the projection)
-        } else if (m->vt && aa.pos0 % 32 == 0) {      // whole fragments, one block per 32-position chunk
-            TSHIP_REQUIRE(qp % 4 == 0 && (long)round_up(aa.pos0 + Tp, 32) <= m->ML, "internal: cache chunk beyond the allocation");
-            dim3 grid((unsigned)ceil_div(Tp, 32), c.n_kv_heads, B);
-            if (m->D == 64) launch(m, "p_kv_write", kv_write_frag_kernel<64>, grid, dim3(256), aa);
-            else launch(m, "p_kv_write", kv_write_frag_kernel<128>, grid, dim3(512), aa);
-        } else {
-            launch(m, "p_kv_write", pick_kvw(m), dim3(Tp, B), dim3(256), aa);
-        }
+        if (!m->vt) launch(m, "p_kv_write", pick_kvw(m), dim3(Tp, B), dim3(256), aa);      // (the other caches are written by the projection)
         auto q_blocks = [&](int per_block) {
             const int n = (int)ceil_div(Tp, per_block);
             aa.q_skip = last ? n - 1 : 0;

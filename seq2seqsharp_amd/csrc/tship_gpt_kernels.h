@@ -940,9 +940,9 @@ __host__ __device__ inline long vfrag_index(int t, int d, int D) {
     const int c = t >> 5, qq = (t & 31) >> 3, j = t & 7;
     return (((long)c * (D / 16) + (d >> 4)) * 64 + (d & 15) + 16 * qq) * 8 + j;
 }
-// Columns c0 ... c0 + 3 of the projection's row `row`, key or value columns, to the cache (BigArgs::kv_scatter).  The same value as through memory and
-// kv_write_frag_kernel: rounded to fp32, rotated with two roundings per output, rounded to fp16.  Where the prompt begins a 32-position chunk, what is
-// left of its last one becomes zero, as there (behind a context it keeps what it held, as with kv_write_kernel).
+// Columns c0 ... c0 + 3 of the projection's row `row`, key or value columns, to the cache (BigArgs::kv_scatter).  The same value as kv_store_frags
+// writes: rounded to fp32, rotated with two roundings per output, rounded to fp16.  Where the prompt begins a 32-position chunk, what is
+// left of its last one becomes zero (behind a context it keeps what it held).
 __device__ __forceinline__ void kv_scatter4(const BigArgs& a, long row, int c0, floatx4 x) {
     const int rel = c0 - a.kv_col0, D = a.kv_D, sh = D == 64 ? 6 : 7;
     const bool is_k = rel < a.kv_gd;
@@ -1023,8 +1023,7 @@ __device__ __forceinline__ void act_store_lines(const BigArgs& a, floatx16 (&acc
 // go in row-major (keys rotated first: a lane holds both elements of a pair), whole fragments come out, 16 bytes per lane
 // and 1 KiB per store instruction.  Key fragment (tile, kd) of a chunk: lane (r, qq) holds position 8 (r / 4) + 4 tile +
 // r % 4, elements 32 kd + 8 qq .. + 7; value fragment dt: lane (r, qq) holds element 16 dt + r at positions 8 qq .. + 7
-// (the layouts kv_write_frag_kernel writes).  Same arithmetic per element as the unfused path: acc * rinv + bias, rotation
-// with two roundings per output, one rounding to fp16.
+// (kfrag_index, vfrag_index).  Per element acc * rinv + bias, rotation with two roundings per output, one rounding to fp16.
 template <int D, bool IS_K>
 __device__ __forceinline__ void kv_store_frags(const BigArgs& a, floatx16 (&acc)[4][2], int nt_first, long row_first, int lane, half_t* stage,
                                                const float (&rinv2)[2]) {
@@ -2502,7 +2501,6 @@ struct AttnArgs {
     float scale;
     const float* ssq; int ssq_nt; int ssq_ld; float inv_h; float eps;   // deferred RMSNorm of the projection input (see SkinnyArgs)
     int ln;      // deferred LayerNorm (see SkinnyArgs): plain sums behind the sums of squares, `bias` holds d[ldq] followed by c[ldq]
-    int vt;      // 1: keys and values are stored fragment-major (kfrag_index / vfrag_index) for the MFMA attention kernels
     // decode with several blocks per (row, KV head): their number, the exchange area [pairs][S][G D + 2 G] floats and one counter per pair
     int S; float* xchg; int* xcount; int s_fixed;      // (s_fixed: all S take part whatever the position, for tests)
     // prefill of sequences padded to one length (Decoder.cs:656, 687-690): original lengths [batch], null = none were padded.
@@ -2881,7 +2879,8 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const int* __restrict
     }
 }
 
-// prefill, step 1: grid (Tq, batch).  Rotates the keys of every position and writes keys and values into the cache.
+// prefill, step 1: grid (Tq, batch).  Rotates the keys of every position and writes keys and values into the row-major cache (the
+// fragment-major one is written by the QKV projection).
 template <typename CT, int D>
 __global__ __launch_bounds__(256) void kv_write_kernel(AttnArgs a) {
     const int tq = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
@@ -2896,69 +2895,13 @@ __global__ __launch_bounds__(256) void kv_write_kernel(AttnArgs a) {
         float x0 = a.qkv[row * a.ldq + col] + a.bias[col], x1 = a.qkv[row * a.ldq + col + 1] + a.bias[col + 1], y0 = x0, y1 = x1;
         if (a.rope_cos) rope_pair(x0, x1, a.rope_cos[(long)pos * (D / 2) + i], a.rope_sin[(long)pos * (D / 2) + i], y0, y1);
         CT* Kh = Kb + (long)kvh * a.max_len * D;
-        if (a.vt) { Kh[kfrag_index(pos, 2 * i, D)] = (CT)y0; Kh[kfrag_index(pos, 2 * i + 1, D)] = (CT)y1; }
-        else { Kh[(long)pos * D + 2 * i] = (CT)y0; Kh[(long)pos * D + 2 * i + 1] = (CT)y1; }
+        Kh[(long)pos * D + 2 * i] = (CT)y0; Kh[(long)pos * D + 2 * i + 1] = (CT)y1;
     }
     for (int p = t; p < GD; p += 256) {
         int kvh = p / D, d = p % D;
         int col = HD + GD + p;
         const float val = a.qkv[row * a.ldq + col] + a.bias[col];
-        if (a.vt) Vb[(long)kvh * a.max_len * D + vfrag_index(pos, d, D)] = (CT)val;
-        else Vb[((long)kvh * a.max_len + pos) * D + d] = (CT)val;
-    }
-}
-
-// prefill, step 1 for the fragment-major fp16 cache when the first position starts a 32-position chunk: one block per
-// (chunk, KV head, batch row) writes the chunk's key and value fragments whole, 16 bytes per lane (the kernel above
-// scatters two-byte elements from one small block per position).  Wavefront w: key fragment w (tile w / KD, kd w % KD)
-// and value fragment w (dt = w).  grid (ceil(Tq / 32), Hkv, batch), D / 16 wavefronts.
-template <int D>
-__global__ __launch_bounds__(D * 4) void kv_write_frag_kernel(AttnArgs a) {
-    constexpr int KD = D / 32;
-    const int chunk = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int r = lane & 15, qq = lane >> 4;
-    const int HD = a.H * D, GD = a.Hkv * D;
-    const long cabs = (a.pos0 >> 5) + chunk;                     // chunk index in the cache (pos0 is a multiple of 32)
-    half_t* Kh = (half_t*)a.kcache + ((long)b * a.Hkv + kvh) * a.max_len * D + cabs * (32 * D);
-    half_t* Vh = (half_t*)a.vcache + ((long)b * a.Hkv + kvh) * (long)D * a.max_len + cabs * (32 * D);
-    {   // keys: lane (r, qq) of fragment (tile, kd) holds position 8 (r / 4) + 4 tile + r % 4, d = 32 kd + 8 qq .. + 7
-        const int tile = w / KD, kd = w % KD;
-        const int tq = chunk * 32 + 8 * (r >> 2) + 4 * tile + (r & 3);
-        const int d0 = 32 * kd + 8 * qq;
-        half8 o = half8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (tq < a.Tq) {
-            const long row = (long)b * a.Tq + tq;
-            const int pos = a.pos0 + tq;
-            const int col = HD + kvh * D + d0;
-            const floatx4 x0 = *(const floatx4*)(a.qkv + row * a.ldq + col), x1 = *(const floatx4*)(a.qkv + row * a.ldq + col + 4);
-            const floatx4 b0 = *(const floatx4*)(a.bias + col), b1 = *(const floatx4*)(a.bias + col + 4);
-            float x[8];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) { x[j] = x0[j] + b0[j]; x[4 + j] = x1[j] + b1[j]; }
-#pragma unroll
-            for (int pr = 0; pr < 4; ++pr) {
-                float y0 = x[2 * pr], y1 = x[2 * pr + 1];
-                if (a.rope_cos) {
-                    const int i = d0 / 2 + pr;
-                    rope_pair(x[2 * pr], x[2 * pr + 1], a.rope_cos[(long)pos * (D / 2) + i], a.rope_sin[(long)pos * (D / 2) + i], y0, y1);
-                }
-                o[2 * pr] = (half_t)y0; o[2 * pr + 1] = (half_t)y1;
-            }
-        }
-        *(half8*)(Kh + (long)w * 512 + lane * 8) = o;
-    }
-    {   // values: lane (r, qq) of fragment dt holds d = 16 dt + r at positions 8 qq .. 8 qq + 7
-        const int d = 16 * w + r;
-        const int col = HD + GD + kvh * D + d;
-        const float bv = a.bias[col];
-        half8 o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int tq = chunk * 32 + 8 * qq + j;
-            o[j] = tq < a.Tq ? (half_t)(a.qkv[((long)b * a.Tq + tq) * a.ldq + col] + bv) : (half_t)0.0f;
-        }
-        *(half8*)(Vh + (long)w * 512 + lane * 8) = o;
+        Vb[((long)kvh * a.max_len + pos) * D + d] = (CT)val;
     }
 }
 

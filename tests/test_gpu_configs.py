@@ -350,11 +350,10 @@ def large_tile(monkeypatch):
     monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
 
-    def launched(gpu, cache_write=None):
+    def launched(gpu, projection_writes_cache=False):
         kernels = gpu.profile_symbols()
         assert any("big_gemm" in k for k in kernels) and not any("mid_gemm" in k for k in kernels), kernels
-        if cache_write is not None:
-            assert any("kv_write_frag_kernel" in k for k in kernels) == cache_write, kernels
+        assert not projection_writes_cache or not any("kv_write" in k for k in kernels), kernels
     return launched
 
 
@@ -403,23 +402,23 @@ def test_eight_query_heads_per_kv_head(G, oracle, dtype, hidden, heads, kv, batc
     (1024, 8, 2, 3, 192),      # head size 128: a wavefront's 128 columns are one head, written in two passes
     (512, 8, 4, 1, 544),       # one sequence of 17 chunks: the last wavefront's second chunk lies beyond the rows
 ])
-def test_projection_writes_the_cache_like_the_separate_kernel(G, oracle, monkeypatch, large_tile, hidden, heads, kv, batch, prompt):
+def test_projection_writes_whole_fragments_like_pieces(G, oracle, monkeypatch, large_tile, hidden, heads, kv, batch, prompt):
     """With the 256 x 256 tile and whole 32-position chunks, the QKV projection's epilogue rotates the keys and writes keys
-    and values into the fragment-major cache itself.  Same cache contents and logits as with the separate cache-write kernel
-    (TSHIP_NO_KV_FUSE=1), and the cache against the oracle's keys and values."""
+    and values into the fragment-major cache as whole fragments.  Same cache contents and logits as in pieces of four
+    columns of a row (TSHIP_NO_KV_FUSE=1), and the logits of tokens behind it against the oracle's."""
     cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=2 * hidden, vocab=157, attn_type=synth.GQA,
                      norm_type=synth.RMSNORM, act=synth.SWIGLU, batch=batch, prompt=prompt, steps=2, dtype="f16")
     w = synth.make_weights(cfg, 77, random_bias=True)
     seqs = synth.make_prompts(cfg, 78)
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 136)
     gpu.prefill(seqs)
-    large_tile(gpu, cache_write=False)
+    large_tile(gpu, projection_writes_cache=True)
     fused = [(gpu.get_kv(l, 0), gpu.get_kv(l, 1)) for l in range(2)]
     lg_fused = gpu.logits()
     monkeypatch.setenv("TSHIP_NO_KV_FUSE", "1")
     gpu.reset()
     gpu.prefill(seqs)
-    large_tile(gpu, cache_write=True)
+    large_tile(gpu, projection_writes_cache=True)
     monkeypatch.delenv("TSHIP_NO_KV_FUSE")
     for l in range(2):
         k, v = gpu.get_kv(l, 0), gpu.get_kv(l, 1)
@@ -427,13 +426,13 @@ def test_projection_writes_the_cache_like_the_separate_kernel(G, oracle, monkeyp
         assert np.array_equal(fused[l][1], v), "values of layer %d" % l
     assert np.array_equal(lg_fused, gpu.logits())
     # appended tokens behind the fused prefill continue the same cache: 128 more per sequence (with three or five sequences
-    # written by the projection at a cache offset; the 128 rows of one sequence take smaller tiles and the separate kernel)
+    # written as whole fragments at a cache offset; the 128 rows of one sequence take smaller tiles, which write pieces)
     more = synth.make_prompts(dict(cfg, prompt=128), 79)
     gpu.reset()
     gpu.prefill(seqs)
     gpu.prefill(more)
     if batch > 1:
-        large_tile(gpu, cache_write=False)
+        large_tile(gpu, projection_writes_cache=True)
     lg_app = gpu.logits()
     k_app = gpu.get_kv(1, 0)
     orc = oracle.OracleGpt(cfg, w)

@@ -79,7 +79,7 @@ def test_padded_batch_fp16_mfma_attention(G, oracle, monkeypatch, hidden, heads,
     orc, gpu, out, ids = _run(G, oracle, cfg, lens, 9)
     if tile == "large" and lens.size == 9:      # (symbols since the prefill: the steps launch no cache write of this kind)
         kernels = gpu.profile_symbols()
-        assert any("big_gemm" in k for k in kernels) and not any("kv_write_frag_kernel" in k for k in kernels), kernels
+        assert any("big_gemm" in k for k in kernels) and not any("kv_write" in k for k in kernels), kernels
     fr = []
     for lg, gl in out:
         assert np.abs(gl - lg).max() <= 3e-2

@@ -57,9 +57,9 @@ def test_prefill_gemm_tiles(G, oracle, monkeypatch, shape, batch, prompt):
 
 
 @pytest.mark.parametrize("hidden,heads,kv,batch,prompt", [(512, 8, 2, 5, 128), (1024, 8, 2, 3, 192), (512, 8, 4, 1, 544)])
-def test_large_tile_writes_the_cache_like_the_separate_kernel(G, monkeypatch, hidden, heads, kv, batch, prompt):
-    """The 256 x 256 tile forced: the QKV projection's own cache write (head sizes 64 and 128, a wavefront partly beyond the
-    rows) against the separate kernel, and the heights of the tile patches against each other, bit for bit."""
+def test_large_tile_writes_whole_fragments_like_pieces(G, monkeypatch, hidden, heads, kv, batch, prompt):
+    """The 256 x 256 tile forced: whole fragments of the cache (head sizes 64 and 128, a wavefront partly beyond the
+    rows) against pieces, and the heights of the tile patches against each other, bit for bit."""
     cfg = synth._cfg(n_layers=2, hidden=hidden, n_heads=heads, n_kv_heads=kv, ffn_dim=2 * hidden, vocab=157, attn_type=synth.GQA,
                      norm_type=synth.RMSNORM, act=synth.SWIGLU, batch=batch, prompt=prompt, steps=2, dtype="f16")
     w = synth.make_weights(cfg, 77, random_bias=True)

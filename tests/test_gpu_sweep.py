@@ -196,8 +196,8 @@ def _big_prefill_cfg(seed):
 
 @pytest.mark.parametrize("seed", range(16))
 def test_large_prefill_paths_agree_bit_for_bit(monkeypatch, seed):
-    """The cache written by the QKV projection's epilogue and the tile patches chosen from the launch size, against the
-    separate cache-write kernel and fixed 8 x 4 patches: same logits, keys and values.  (The 256 x 256 tile is forced: most
+    """The cache written as whole fragments by the QKV projection's epilogue and the tile patches chosen from the launch size,
+    against the cache written in pieces and fixed 8 x 4 patches: same logits, keys and values.  (The 256 x 256 tile is forced: most
     of these sizes take smaller ones by themselves.)"""
     from seq2seqsharp_amd import gpt as G
     cfg = _big_prefill_cfg(seed)
@@ -208,19 +208,18 @@ def test_large_prefill_paths_agree_bit_for_bit(monkeypatch, seed):
     monkeypatch.setenv("TSHIP_ALL_ROWS", "1")
     monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
 
-    def launched(cache_write):
+    def launched():
         kernels = gpu.profile_symbols()
-        assert any("big_gemm3" in x for x in kernels) and not any("mid_gemm" in x for x in kernels), kernels
-        assert any("kv_write_frag_kernel" in x for x in kernels) == cache_write, kernels
+        assert any("big_gemm3" in x for x in kernels) and not any("mid_gemm" in x or "kv_write" in x for x in kernels), kernels
 
     gpu.prefill(seqs)
-    launched(False)
+    launched()
     lg, k, v = gpu.logits(), gpu.get_kv(1, 0), gpu.get_kv(1, 1)
     assert np.isfinite(lg).all()
     monkeypatch.setenv("TSHIP_NO_KV_FUSE", "1")
     monkeypatch.setenv("TSHIP_PATCH_ROWS", "8")
     gpu.reset()
     gpu.prefill(seqs)
-    launched(True)
+    launched()
     assert np.array_equal(lg, gpu.logits()) and np.array_equal(k, gpu.get_kv(1, 0)) and np.array_equal(v, gpu.get_kv(1, 1))
     gpu.close()
