@@ -138,16 +138,17 @@ struct TSHipGpt {
     // one decode step (sample + decode) captured as a HIP graph; valid for one (batch, sampling mode) at a time
     hipGraphExec_t step_graph = nullptr;
     // The same for GRAPH_STEPS steps: between two launches of a graph the GPU idles for 8.5 us, inside one for none.  A capture of eight steps
-    // takes the host 0.8 to 1.9 ms, two to five steps' time on the GPU.  It is made behind the launch of a call's GRAPH_STEPS_AHEAD-th single step,
-    // while the GPU works through those: there the host would wait for it anyway.  Its first launch costs 0.1 ms more than later ones, 25 steps' gain
-    // (the 768-wide fp32 model with two rows, 24 / 32 tokens 8.62 / 11.29 -> 8.69 / 11.38 ms with it), so a call has to have GRAPH_STEPS_FIRST steps left for it.
-    static constexpr int GRAPH_STEPS = 8, GRAPH_STEPS_AHEAD = 16, GRAPH_STEPS_FIRST = 32;
+    // takes the host 0.6 to 1.4 ms.  It is made behind the launch of a call's GRAPH_STEPS_AHEAD-th single step, while the GPU works through
+    // those and the host would wait for it anyway; in shorter calls behind the last, once GRAPH_STEPS_AFTER steps say that a loop goes on.  Not in
+    // models with experts, which take 2 us a step longer in the long graph (12 layers, 8 rows, 16 / 24 tokens 8.38 / 12.52 -> 8.41 / 12.56 ms).
+    static constexpr int GRAPH_STEPS = 8, GRAPH_STEPS_AHEAD = 16, GRAPH_STEPS_AFTER = 64;
     hipGraphExec_t steps_graph = nullptr;
-    bool steps_graph_failed = false, steps_graph_ran = false;      // (failed: could not be made; the single step's graph serves until both are dropped)
+    bool steps_graph_failed = false;      // could not be made; the single step's graph serves until both are dropped
+    int graph_steps_run = 0;              // single steps since then
     void drop_graphs() {
         if (step_graph) (void)hipGraphExecDestroy(step_graph);
         if (steps_graph) (void)hipGraphExecDestroy(steps_graph);
-        step_graph = steps_graph = nullptr; steps_graph_failed = steps_graph_ran = false;
+        step_graph = steps_graph = nullptr; steps_graph_failed = false; graph_steps_run = 0;
     }
     int graph_batch = 0, graph_mode = -1; float graph_top_p = 0.0f, graph_temp = 0.0f;
     const float* graph_uniforms = nullptr; int* graph_gen = nullptr;
@@ -2051,10 +2052,11 @@ static int generate_impl(TSHipGpt* m, int n_steps, int mode, float top_p, float 
     TSHIP_CHECK_HIP(hipStreamSynchronize(stream()));
     TSHIP_CHECK_HIP(hipEventRecord(e0, stream()));
     // The graph of several steps, behind single ones that the GPU is still busy with (their counters are back at zero whenever a step ends).
-    // Host ms of a state's first call of 32 / 64 / 128 / 512 tokens, all of it, single steps only -> with it: the small fp32 model (one row) 5.29 / 10.36 /
-    // 20.76 / 87.1 -> 5.29 / 10.27 / 20.34 / 85.0, the 768-wide fp32 one (2 rows) 11.28 / 22.42 / 44.8 / 188.6 -> 11.32 / 22.27 / 44.5 / 187.0, the 1B one (32
-    // rows) 22.79 / 44.85 / 89.5 / 363.5 -> 22.77 / 44.95 / 89.1 / 360.4; of a later one, of 32 tokens, 5.10, 10.98 and 22.56 -> 4.97, 10.86 and 22.35.  Captured in
-    // front of a call's first step instead, that call took 0.6 to 1.6 ms longer.
+    // Host us of a state's first, second and third call against single steps only, all of the call: 16 tokens of the small fp32 model (one row, 2.6 ms)
+    // -50 / +4 / -79, the 768-wide fp32 one (2 rows, 5.6) +12 / +28 / -60, the 768-wide fp16 one (8 rows, 5.2) -1 / -89 / -70, the 1B one (32 rows, 11.2)
+    // +12 / -18 / -82; 24 tokens +1 / -117 / -118, +7 / -91 / -98, -47 / -116 / -119, -64 / -124 / -227; 128 tokens, the first call, -414, -268, -471, -496.
+    // Calls of 8 tokens: the eighth 0 to +80, later ones -40, -27, -40 and -40 of 1.3 to 5.6 ms.  (+-50 between runs.)  Captured in front of a
+    // call's first step instead, that call took 0.6 to 1.6 ms longer.
     auto capture_steps = [&]() {
         try {
             capture(m->steps_graph, TSHipGpt::GRAPH_STEPS);
@@ -2063,13 +2065,13 @@ static int generate_impl(TSHipGpt* m, int n_steps, int mode, float top_p, float 
     };
     int done = 0;
     for (int s = 0; s < n_steps; ++s) {
-        if (use_graph && eos_id < 0 && m->steps_graph && n_steps - s >= (m->steps_graph_ran ? TSHipGpt::GRAPH_STEPS : TSHipGpt::GRAPH_STEPS_FIRST)) {
+        if (use_graph && eos_id < 0 && m->steps_graph && n_steps - s >= TSHipGpt::GRAPH_STEPS) {
             TSHIP_CHECK_HIP(hipGraphLaunch(m->steps_graph, stream()));
-            m->steps_graph_ran = true;
             m->pos += TSHipGpt::GRAPH_STEPS; s += TSHipGpt::GRAPH_STEPS - 1;
         } else if (use_graph) {
-            TSHIP_CHECK_HIP(hipGraphLaunch(m->step_graph, stream())); m->pos += 1;
-            if (eos_id < 0 && s + 1 == TSHipGpt::GRAPH_STEPS_AHEAD && n_steps >= TSHipGpt::GRAPH_STEPS_FIRST && !m->steps_graph && !m->steps_graph_failed) capture_steps();
+            TSHIP_CHECK_HIP(hipGraphLaunch(m->step_graph, stream())); m->pos += 1; m->graph_steps_run += 1;
+            const bool behind = s + 1 == TSHipGpt::GRAPH_STEPS_AHEAD || (s + 1 == n_steps && n_steps >= TSHipGpt::GRAPH_STEPS && m->graph_steps_run >= TSHipGpt::GRAPH_STEPS_AFTER);
+            if (eos_id < 0 && m->c.n_experts <= 1 && behind && !m->steps_graph && !m->steps_graph_failed) capture_steps();
         }
         else {
             sample_tokens(m, mode, top_p, temperature, nullptr, uni_base, B, gen.as<int>(), d_step, true, true);

@@ -1,5 +1,5 @@
-"""Token loops long enough for the captured graph of eight steps, which a call of 32 steps or more makes behind its sixteenth and
-which runs from the first call on that has 32 left: the tokens and logits of steps launched one by one."""
+"""Token loops long enough for the captured graph of eight steps, which a call of 16 steps or more makes behind its sixteenth, a shorter one
+behind its last once 64 steps have run: the tokens and logits of steps launched one by one."""
 import numpy as np
 import pytest
 
@@ -18,9 +18,10 @@ def G():
                                                       ("f16", synth.LAYERNORM, 4, 4)])
 @pytest.mark.parametrize("sampled", [False, True])
 def test_loops_of_many_steps(G, monkeypatch, dtype, norm, batch, experts, sampled):
-    """Loops that make the long graph and run it at once (64), make it and leave it to a later one (32, 47), are too short (31), and find it
-    there, below, at and between multiples of eight steps; a rewind, single steps, a loop that looks for an end token and blocked tokens
-    (which drop the graphs) between them; the same where the long graph cannot be made."""
+    """Loops that make the long graph and run it at once (64, 47, 24), make it and leave it to a later one (16 to 23; the last of them at the
+    cache's end), are too short for it (15, the first calls of 8), and find it there, below, at and between multiples of eight steps; a rewind, single
+    steps, a loop that looks for an end token and blocked tokens (which drop the graphs) between them; the same where the long graph
+    cannot be made.  (Models with experts make none.)"""
     cfg = synth.tiny_config(n_layers=3, dtype=dtype, norm_type=norm, n_experts=experts, experts_per_token=min(2, experts), batch=batch, prompt=8, vocab=300,
                              act=synth.RELU if experts > 1 else synth.SWIGLU)
     w = synth.make_weights(cfg, 101, random_bias=True)
@@ -44,12 +45,17 @@ def test_loops_of_many_steps(G, monkeypatch, dtype, norm, batch, experts, sample
         out += [loop(19), loop(9, until=2), loop(16)]
         gpu.set_blocked_tokens([5, 6, 7])
         out += [loop(31), loop(20)]
-        for n, later in ((32, 33), (47, 9)):
-            gpu.set_blocked_tokens([])
-            gpu.set_seq_len(batch, 40)
+
+        def again(at, *lengths):
+            gpu.set_seq_len(batch, at)
             gpu.decode((np.arange(batch) + 4).astype(np.int32))
-            out += [loop(n), loop(later), loop(10)]
+            return [loop(n) for n in lengths]
+
+        for lengths in ((32, 33, 10), (47, 9, 10), (24, 8), (15, 16, 23), (8,) * 10):
+            gpu.set_blocked_tokens([])
+            out += again(40, *lengths)
             gpu.set_blocked_tokens([5])
+        out += again(160 - 17, 16) + again(40, 24)
         return out
 
     first, second = run(), run()
