@@ -361,14 +361,17 @@ def test_moe_model(G, oracle, dtype, act):
 
 
 @pytest.mark.parametrize("dtype,batch,prompt", [("f16", 4, 330), ("f16", 3, 70), ("f32", 2, 40)])
-def test_moe_prefill_runs_the_experts_on_gathered_rows(G, oracle, dtype, batch, prompt):
+def test_moe_prefill_runs_the_experts_on_gathered_rows(G, oracle, monkeypatch, dtype, batch, prompt):
     """Prefill of a model with MoE layers: all prompt rows are routed at once, every expert runs the prefill GEMMs on the
     rows gathered for it (about 660 rows per expert in the first case: one launch for all experts; fewer than 512 in the
     others: one per expert), and the scaled outputs are added back in expert order.  Logits of the last position and the routing of the
     last position against the oracle, then decode steps on top of the cache the prefill wrote."""
     cfg = synth.tiny_config(n_layers=4, n_experts=4, experts_per_token=2, norm_type=synth.LAYERNORM, act=synth.RELU, dtype=dtype,
                             batch=batch, prompt=prompt, vocab=300)      # (the third layer; the last one computes the last positions only)
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
     orc, gpu, out, cur = _teacher_forced(G, oracle, cfg, 61, 3)
+    kernels = gpu.profile_symbols()
+    assert any("moe_lists_big_kernel" in s for s in kernels) and any("moe_gather_kernel" in s for s in kernels) == (batch * prompt < 512)
     for lg, gl in out:
         if dtype == "f32":
             assert _rel(gl, lg) <= FP32_REL

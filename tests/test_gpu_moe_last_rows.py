@@ -30,8 +30,13 @@ def test_last_rows_by_themselves(G, oracle, monkeypatch, experts, k, batch, prom
     if tile is not None:
         monkeypatch.setenv("TSHIP_MOE_REST", str(tile))
     gpu = G.HipGpt(cfg, w, max_batch=batch, max_seq_len=prompt + 10)
+    monkeypatch.setenv("TSHIP_RECORD_SYMBOLS", "1")
     gpu.prefill(seqs)
     got = gpu.logits()
+    kernels = gpu.profile_symbols()
+    assert any("moe_lists_big_kernel" in s for s in kernels) and not any("moe_gather_kernel" in s for s in kernels)      # one launch for all experts
+    if tile is not None:      # (its last template argument: the last rows of several problems)
+        assert sum("mid_gemm_f16_kernel" in s and ", %d, %d, true>" % (tile // 10, tile % 10) in s for s in kernels) == 2
     orc = oracle.OracleGpt(cfg, w)
     _, lg = orc.step(seqs, use_cache=True)
     assert np.abs(got - lg).max() <= FP16_ABS
